@@ -9,7 +9,7 @@
 
 // Kernel-choice overrides of a context (tuning and tests).  Read from the environment ONCE, when the context is created
 // (SOFIE_HIP_SWIZZLE, SOFIE_HIP_I8_TILE, SOFIE_HIP_F8_TILE, SOFIE_HIP_GEMM_VARIANT, SOFIE_HIP_CONV_EXPLICIT,
-// SOFIE_HIP_F32_SKINNY, SOFIE_HIP_F32_CHAIN), afterwards changed only through sofie_hip_ctx_set_option.
+// SOFIE_HIP_F32_SKINNY, SOFIE_HIP_F32_CHAIN, SOFIE_HIP_F32_TILE), afterwards changed only through sofie_hip_ctx_set_option.
 struct sofie_hip_options {
    int swizzle = 4;       // tile order: XCD regrouping, bands of 4 tile rows
    int i8_tile = 0;       // 0 = heuristic
@@ -18,6 +18,7 @@ struct sofie_hip_options {
    int conv_explicit = 0; // int8 convolution through a column matrix whenever the workspace holds one
    int f32_skinny = -1;   // -1 = heuristic
    int f32_chain = -1;
+   int f32_tile = 0;      // 0 = heuristic
 };
 
 struct sofie_hip_ctx {

@@ -1,0 +1,681 @@
+// fp32 products on the matrix cores (v_mfma_f32_32x32x2_f32, v_mfma_f32_16x16x4_f32: full fp32 multiply-adds at twice the rate of the unpacked vector
+// instructions), for Gemm / MatMul and for convolutions as implicit GEMM.  Two kernels:
+//   f32_tile_kernel     a workgroup of four waves owns a BM x BN tile; slabs of k go straight from memory into a ring in LDS
+//   f32_direct_kernel   small products: a workgroup owns one small tile and its waves split the reduction; every fragment is
+//                       loaded from memory into the registers the MFMA reads, with many loads in flight and no LDS in the loop
+//
+// Both feed an MFMA the n side as first operand and the m side as second, so a lane ends up with 4 consecutive columns n of one
+// row m.  Four MFMAs take four consecutive k from every lane: which k a lane supplies to which MFMA only has to agree between the
+// operands, and this order lets an operand that is contiguous in k be read as one 16-byte word per lane.
+#pragma once
+#include "mfma8_common.hpp"
+#include "mfma8_gemm_dma.hpp"
+
+namespace sofie_hip {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+// What loads of positions outside an operand read.
+static __device__ __attribute__((aligned(256))) float f32_zero_page[64] = {};
+
+__device__ __forceinline__ v4f mfma_f32_step(const v4f &n_side, const v4f &m_side, v4f acc)
+{
+#pragma unroll
+   for (int j = 0; j < 4; ++j)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(n_side[j], m_side[j], acc, 0, 0, 0);
+   return acc;
+}
+
+// ---- operands ---------------------------------------------------------------------------------------------------------------
+// An operand is a matrix of `rows` (m or n) by K.  KC: contiguous in k (a row's k neighbours lie side by side); otherwise
+// contiguous along the rows.  VEC: floats per load; 4 needs 16-byte aligned pieces (the host checks that the address, the
+// pitch and the extent along the contiguous direction are multiples of 16 bytes).
+template <bool KC_, int VEC_>
+struct F32Matrix {
+   static constexpr int kLeastRows = 16; // of a tile of the tile kernel
+   static constexpr bool KC = KC_;
+   static constexpr int VEC = VEC_;
+   const float *p;
+   long long ld;
+   int rows, K;
+   __device__ __forceinline__ void shift(long long elements) { p += elements; }
+   __device__ __forceinline__ void select_group(int) {}
+
+   // what a lane keeps per load instruction of a slab: the address at k = 0
+   template <int LD>
+   struct lane_state {
+      const float *at[LD];
+   };
+   template <int LD>
+   __device__ __forceinline__ void init(lane_state<LD> &st, int i, int row, int kk) const
+   {
+      // rows past the edge re-read the last piece (their results are not stored)
+      const int r = row < rows ? row : (KC || VEC == 1 ? rows - 1 : rows - VEC);
+      st.at[i] = KC ? p + (long long)r * ld + kk : p + (long long)kk * ld + r;
+   }
+   // address of load i of the slab at k0 (kk: the lane's k within the slab; WHOLE: no k of the slab lies past K)
+   template <bool WHOLE, int LD>
+   __device__ __forceinline__ const float *load_ptr(const lane_state<LD> &st, int i, int kk, int k0) const
+   {
+      const float *a = st.at[i] + (KC ? (long long)k0 : (long long)k0 * ld);
+      return WHOLE || k0 + kk < K ? a : f32_zero_page;
+   }
+
+   // direct fetch of row `row`, k..k+3
+   struct row_state {
+      const float *at;
+   };
+   __device__ __forceinline__ row_state row_of(int row) const
+   {
+      const int r = row < rows ? row : rows - 1;
+      return row_state{KC ? p + (long long)r * ld : p + r};
+   }
+   __device__ __forceinline__ v4f fetch(const row_state &st, int k) const
+   {
+      v4f v = {0.f, 0.f, 0.f, 0.f};
+      if (KC && VEC == 4) {
+         if (k < K)
+            v = *(const v4f *)(st.at + k);
+      } else {
+#pragma unroll
+         for (int j = 0; j < 4; ++j)
+            if (k + j < K)
+               v[j] = st.at[KC ? (long long)(k + j) : (long long)(k + j) * ld];
+      }
+      return v;
+   }
+};
+
+// The column matrix of a convolution, gathered from the NCHW input as it is asked for: row m = (image, output position), column
+// k = (channel, kernel position), zero outside the image -- the index arithmetic of the reference's Im2col / Im2col_3d
+// (core/src/utils/SOFIE_common_helpers.cxx:47-139).  Neighbouring rows are neighbouring output positions of one image row, so a
+// load instruction (64 rows, one k) reads (almost) consecutive floats; what depends on k alone is scalar arithmetic.
+struct F32ConvShape {
+   int C, D, H, W, kd, kh, kw, OD, OH, OW; // input channels (all groups); a 2-D convolution has D = kd = OD = 1
+   int pad_d, pad_h, pad_w, stride_d, stride_h, stride_w, dil_d, dil_h, dil_w;
+   int Cg;                                 // channels per group
+   unsigned kw_mul, kh_mul, kd_mul;        // ceil(2^31 / extent): k / extent == umulhi(2 k, mul) while k * extent < 2^31 (checked on the host)
+};
+template <bool VOLUME> // three spatial axes
+struct F32ConvRows {
+   static constexpr int kLeastRows = 64; // a load instruction covers one k: what depends on k is scalar
+   static constexpr bool KC = false;
+   static constexpr int VEC = 1;
+   const float *X;
+   F32ConvShape s;
+   int rows, K;
+   long long image, channel; // elements per image and per channel
+   __device__ __forceinline__ void shift(long long) {}
+   __device__ __forceinline__ void select_group(int g) { X += (long long)g * s.Cg * channel; }
+
+   struct row_state {
+      const float *at; // element of channel 0 at (id0, ih0, iw0): dereferenced only inside the image
+      int id0, ih0, iw0;
+   };
+   __device__ __forceinline__ row_state row_of(int row) const
+   {
+      const int m = row < rows ? row : rows - 1;
+      int ow = m % s.OW, t = m / s.OW;
+      int oh = t % s.OH;
+      t /= s.OH;
+      int od = 0, img = t;
+      if (VOLUME) {
+         od = t % s.OD;
+         img = t / s.OD;
+      }
+      row_state r;
+      r.id0 = VOLUME ? od * s.stride_d - s.pad_d : 0;
+      r.ih0 = oh * s.stride_h - s.pad_h;
+      r.iw0 = ow * s.stride_w - s.pad_w;
+      r.at = X + (long long)img * image + ((long long)r.id0 * s.H + r.ih0) * s.W + r.iw0;
+      return r;
+   }
+   static __device__ __forceinline__ int divide(int k, unsigned mul) { return (int)__umulhi((unsigned)k * 2u, mul); }
+   // address of column k of a row, or of a zero
+   __device__ __forceinline__ const float *element(const row_state &r, int k) const
+   {
+      const int t = divide(k, s.kw_mul), kx = k - t * s.kw;
+      const int u = divide(t, s.kh_mul), ky = t - u * s.kh;
+      int ci = u, kz = 0;
+      if (VOLUME) {
+         ci = divide(u, s.kd_mul);
+         kz = u - ci * s.kd;
+      }
+      const int dz = kz * s.dil_d, dy = ky * s.dil_h, dx = kx * s.dil_w;
+      bool inside = k < K && (unsigned)(r.ih0 + dy) < (unsigned)s.H && (unsigned)(r.iw0 + dx) < (unsigned)s.W;
+      if (VOLUME)
+         inside = inside && (unsigned)(r.id0 + dz) < (unsigned)s.D;
+      const float *p = r.at + ((long long)ci * channel + ((long long)dz * s.H + dy) * s.W + dx);
+      return inside ? p : f32_zero_page;
+   }
+   // a lane keeps the same row through all load instructions of a slab (tiles of 64 rows or more, four waves)
+   template <int LD>
+   struct lane_state {
+      row_state r;
+   };
+   template <int LD>
+   __device__ __forceinline__ void init(lane_state<LD> &st, int i, int row, int) const
+   {
+      if (i == 0)
+         st.r = row_of(row);
+   }
+   template <bool WHOLE, int LD>
+   __device__ __forceinline__ const float *load_ptr(const lane_state<LD> &st, int, int kk, int k0) const
+   {
+      return element(st.r, k0 + __builtin_amdgcn_readfirstlane(kk));
+   }
+   __device__ __forceinline__ v4f fetch(const row_state &st, int k) const
+   {
+      v4f v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+         v[j] = *element(st, k + j);
+      return v;
+   }
+};
+
+// ---- stores -----------------------------------------------------------------------------------------------------------------
+struct F32Epilogue {
+   float alpha, beta;
+   const float *C;
+   int bias_mode;
+   long long ldc;
+   PostChain chain; // the activation, then the caller's chain of one-to-one operators
+   const float *R;  // tensor of Y's shape added before the activation, or nullptr
+   long long ldr;
+};
+
+// one activation and no further link: the cases worth a straight path (a chain of count 0 is a chain of "none")
+__device__ __forceinline__ float f32_activate(float v, const PostChain &chain)
+{
+   if (chain.count == 0)
+      return v;
+   if (chain.count == 1 && chain.op0 == SOFIE_ACT_RELU)
+      return v > 0.0f ? v : 0.0f;
+   return apply_chain(v, chain);
+}
+
+// everything before the activation
+__device__ __forceinline__ float f32_linear(const F32Epilogue &ep, float acc, int m, int n)
+{
+   float v = ep.alpha * acc;
+   switch (ep.bias_mode) {
+   case SOFIE_BIAS_ROW: v += ep.C[n]; break;
+   case SOFIE_BIAS_COL: v += ep.C[m]; break;
+   case SOFIE_BIAS_SCALAR: v += ep.C[0]; break;
+   case SOFIE_BIAS_FULL: v += ep.beta * ep.C[m * ep.ldc + n]; break;
+   default: break;
+   }
+   if (ep.R)
+      v += ep.R[m * ep.ldr + n];
+   return v;
+}
+__device__ __forceinline__ float f32_epilogue(const F32Epilogue &ep, float acc, int m, int n)
+{
+   return f32_activate(f32_linear(ep, acc, m, n), ep.chain);
+}
+
+// Row-major results of a product.
+struct F32RowStore {
+   static constexpr bool kAlongRows = false; // neighbouring lanes store neighbouring columns
+   float *Y;
+   long long ldy;
+   F32Epilogue ep;
+   int vec; // rows may be written 16 bytes at a time
+   long long strideC, strideY;
+   __device__ __forceinline__ void select_batch(int b)
+   {
+      Y += b * strideY;
+      if (ep.C)
+         ep.C += b * strideC;
+      if (ep.R)
+         ep.R += b * strideY;
+   }
+   __device__ __forceinline__ void put(float acc, int m, int n) const { Y[m * ldy + n] = f32_epilogue(ep, acc, m, n); }
+   // columns n..n+3 of row m (those before N)
+   __device__ __forceinline__ void put4(v4f a, int m, int n, int N) const
+   {
+      v4f v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+         v[e] = f32_linear(ep, a[e], m, n + e < N ? n + e : N - 1);
+      if (ep.chain.count != 0) {
+#pragma unroll
+         for (int e = 0; e < 4; ++e)
+            v[e] = f32_activate(v[e], ep.chain);
+      }
+      float *y = Y + m * ldy + n;
+      if (vec && n + 4 <= N) {
+         *(v4f *)y = v;
+      } else {
+#pragma unroll
+         for (int e = 0; e < 4; ++e)
+            if (n + e < N)
+               y[e] = v[e];
+      }
+   }
+};
+
+// NCHW results of a convolution: row m = (image, position), column n = output channel of the group.
+struct F32ConvStore {
+   static constexpr bool kAlongRows = true; // neighbouring lanes store neighbouring positions of one channel
+   float *Y;
+   const float *bias;
+   const float *R; // tensor of Y's shape added before the activation, or nullptr
+   PostChain chain;
+   int Cout, Cout_g, positions, first;
+   __device__ __forceinline__ void select_batch(int g) { first = g * Cout_g; }
+   struct row_state {
+      size_t at;
+   };
+   __device__ __forceinline__ row_state row_of(int m) const
+   {
+      const int img = m / positions;
+      return row_state{(size_t)img * Cout * positions + (m - img * positions)};
+   }
+   __device__ __forceinline__ void put_at(float v, const row_state &r, int n) const
+   {
+      const int co = first + n;
+      const size_t at = r.at + (size_t)co * positions;
+      if (bias)
+         v += bias[co];
+      if (R)
+         v += R[at];
+      Y[at] = f32_activate(v, chain);
+   }
+   __device__ __forceinline__ void put(float v, int m, int n) const { put_at(v, row_of(m), n); }
+};
+
+// ---- the tile kernel ----------------------------------------------------------------------------------------------------------
+// Its fragments are those of v_mfma_f32_32x32x2_f32: a step is 8 k, lane (lk = lane / 32, c = lane % 32) supplies k = 4 lk + j of row
+// c to MFMA j, and ends up with columns 8 g + 4 lk + e (g, e = 0..3) of row c.
+
+// Position of (row r, k) of an operand's slab of BK k in LDS, in floats.  Contiguous in k: rows of BK floats whose 16-byte chunks
+// are permuted by the row, free of bank conflicts for the fragment read (32 rows, chunks lk = 0, 1).  Contiguous along the
+// rows: BK lines of R floats; the two k of a fragment read lie four lines apart, and a gap of 32 floats behind every fourth line
+// puts them in different banks (R >= 64: a load instruction never crosses such a gap).
+template <int BK>
+__device__ __forceinline__ int f32_row_swizzle(int r)
+{
+   return BK == 16 ? (r >> 2) & 3 : (r >> 1) & 7;
+}
+template <bool KC, int R>
+__device__ __forceinline__ int f32_gap(int k)
+{
+   return !KC && R >= 64 ? (k >> 2) * 32 : 0;
+}
+template <bool KC, int R, int BK>
+constexpr int f32_slab_floats()
+{
+   return R * BK + (!KC && R >= 64 ? BK / 4 * 32 : 0);
+}
+
+template <class SRC, int R, int BK, int NW>
+struct F32Slab {
+   static constexpr int VEC = SRC::VEC;
+   static constexpr int TOTAL = R * BK / (64 * VEC);  // wave-wide load instructions per slab
+   static constexpr int LD = (TOTAL + NW - 1) / NW;   // per wave; where they do not divide, some waves repeat a load
+   static constexpr bool KC = SRC::KC;
+   static constexpr int FLOATS = f32_slab_floats<SRC::KC, R, BK>();
+   typename SRC::template lane_state<LD> st;
+
+   // (row, k) of the slab that load i of this wave brings to this lane's place in LDS
+   static __device__ __forceinline__ void place(int i, int wave, int lane, int &row, int &kk)
+   {
+      const int f = (((i * NW + wave) % TOTAL) * 64 + lane) * VEC;
+      if (SRC::KC) {
+         row = f / BK;
+         const int pos = f % BK;
+         kk = (((pos >> 2) ^ f32_row_swizzle<BK>(row)) << 2) + (pos & 3);
+      } else {
+         kk = f / R;
+         row = f % R;
+      }
+   }
+   __device__ __forceinline__ void init(const SRC &src, int r0, int wave, int lane)
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i) {
+         int row, kk;
+         place(i, wave, lane, row, kk);
+         src.template init<LD>(st, i, r0 + row, kk);
+      }
+   }
+   template <bool WHOLE>
+   __device__ __forceinline__ void issue(const SRC &src, float *lds, int k0, int wave, int lane) const
+   {
+      static_for<LD>([&](auto ic) {
+         constexpr int i = decltype(ic)::value;
+         int row, kk;
+         place(i, wave, lane, row, kk);
+         const int f = ((i * NW + wave) % TOTAL) * 64 * VEC;
+         global_void_t *from = (global_void_t *)src.template load_ptr<WHOLE, LD>(st, i, kk, k0);
+         lds_void_t *to = (lds_void_t *)(lds + f + f32_gap<SRC::KC, R>(f / R));
+         if constexpr (VEC == 4)
+            __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
+         else
+            __builtin_amdgcn_global_load_lds(from, to, 4, 0, 0);
+      });
+   }
+   // fragment of k = 8 g .. 8 g + 7 of the 32 rows from r on
+   static __device__ __forceinline__ v4f fragment(const float *lds, int r, int g, int lane)
+   {
+      const int lk = lane >> 5, row = r + (lane & 31);
+      if (SRC::KC)
+         return *(const v4f *)(lds + row * BK + (((2 * g + lk) ^ f32_row_swizzle<BK>(row)) << 2));
+      v4f v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+         v[j] = lds[(8 * g + 4 * lk + j) * R + f32_gap<SRC::KC, R>(8 * g + 4 * lk) + row];
+      return v;
+   }
+};
+
+template <int TM, int TN, bool ALONG_ROWS>
+constexpr int f32_store_floats()
+{
+   return ALONG_ROWS ? TN * (TM + 4) : TM * (TN + 4);
+}
+template <int BM, int BN, int BK, int STAGES, int WAVES_M, int WAVES_N, int WAVES_K, bool KCA, bool KCB, bool ALONG_ROWS>
+constexpr size_t f32_tile_lds_bytes()
+{
+   constexpr size_t ring = (size_t)STAGES * (f32_slab_floats<KCA, BM, BK>() + f32_slab_floats<KCB, BN, BK>()) * 4;
+   constexpr size_t store = (size_t)WAVES_M * WAVES_N * WAVES_K * f32_store_floats<BM / WAVES_M, BN / WAVES_N, ALONG_ROWS>() * 4;
+   return ring > store ? ring : store;
+}
+
+// Ring of STAGES slabs, one barrier per slab.  An fp32 MFMA is slow against what it reads (a 32 x 32 wave tile: 8 KB from LDS per
+// 1024 cycles), so neither LDS nor L2 bounds the loop; the matrix cores do where there are enough tiles, and the last, partly
+// filled round of tiles where there are not.  WAVES_K waves share a wave tile: each takes its part of the k of every slab,
+// which puts all four SIMDs of a CU to work on tiles smaller than four blocks of 32 x 32.
+template <class ASRC, class BSRC, class STORE, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int WAVES_K, int STAGES>
+__global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_kernel(ASRC A, BSRC B, STORE out, int M, int N, int K, int tiles_m,
+                                                                                   int tiles_n, long long strideA, long long strideB)
+{
+   constexpr int NW = WAVES_M * WAVES_N * WAVES_K;
+   constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N, MT = TM / 32, NT = TN / 32;
+   constexpr int GS = BK / 8 / WAVES_K; // steps of 8 k per slab and wave
+   static_assert(TM % 32 == 0 && TN % 32 == 0 && GS >= 1 && GS * WAVES_K * 8 == BK, "wave tile of 32 x 32 blocks");
+   typedef F32Slab<ASRC, BM, BK, NW> SA;
+   typedef F32Slab<BSRC, BN, BK, NW> SB;
+   constexpr int LPT = SA::LD + SB::LD;
+   constexpr int STAGE = SA::FLOATS + SB::FLOATS;
+   static_assert((STAGES - 1) * LPT < 64, "vmcnt counts fewer than 64 loads");
+   extern __shared__ __attribute__((aligned(16))) float f32_lds[];
+
+   const int z = blockIdx.z;
+   A.shift(z * strideA);
+   B.shift(z * strideB);
+   A.select_group(z);
+   out.select_batch(z);
+   int tm, tn;
+   tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, 4, tm, tn);
+   const int m0 = tm * BM, n0 = tn * BN;
+   const int lane = threadIdx.x & 63;
+   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+   const int wk = wave % WAVES_K, wm = wave / WAVES_K / WAVES_N, wn = wave / WAVES_K % WAVES_N;
+
+   SA sa;
+   SB sb;
+   sa.init(A, m0, wave, lane);
+   sb.init(B, n0, wave, lane);
+   v16f acc[MT][NT];
+#pragma unroll
+   for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+         for (int e = 0; e < 16; ++e)
+            acc[i][j][e] = 0.0f;
+
+   const int KT = (K + BK - 1) / BK;
+   // a slab past the end is asked for as the last one again: filler that keeps the number of loads per step the same
+   auto issue = [&](int kt, int stage, auto whole) {
+      const int k0 = (kt < KT ? kt : KT - 1) * BK;
+      float *s = f32_lds + stage * STAGE;
+      sa.template issue<decltype(whole)::value>(A, s, k0, wave, lane);
+      sb.template issue<decltype(whole)::value>(B, s + SA::FLOATS, k0, wave, lane);
+   };
+   constexpr std::false_type any{};
+   v4f fa[2][GS][MT], fb[2][GS][NT];
+   auto read = [&](int stage, v4f(&a)[GS][MT], v4f(&b)[GS][NT]) {
+      const float *cA = f32_lds + stage * STAGE, *cB = cA + SA::FLOATS;
+#pragma unroll
+      for (int g = 0; g < GS; ++g) {
+#pragma unroll
+         for (int i = 0; i < MT; ++i)
+            a[g][i] = SA::fragment(cA, wm * TM + i * 32, wk * GS + g, lane);
+#pragma unroll
+         for (int j = 0; j < NT; ++j)
+            b[g][j] = SB::fragment(cB, wn * TN + j * 32, wk * GS + g, lane);
+      }
+   };
+   if (KT > 0) { // an empty reduction reads nothing
+#pragma unroll
+      for (int s = 0; s < STAGES; ++s)
+         issue(s, s, any);
+      wait_vmcnt<(STAGES - 1) * LPT>();
+      __builtin_amdgcn_s_barrier();
+      read(0, fa[0], fb[0]);
+   }
+   int stage = 0;
+   // Slab kt: its fragments are in registers.  Behind the barrier slab kt + 1 has landed for every wave and slab kt has been read by
+   // every wave: the next fragments are asked for and slab kt + STAGES takes the place of slab kt.  The barrier sits between
+   // two halves of the MFMAs, and what is issued behind it is dealt out among those of the second half: a wave that runs alone
+   // on its SIMD keeps the matrix core busy.
+   auto step = [&](int kt, auto parity, auto whole) {
+      constexpr int cur = decltype(parity)::value;
+      const int next = stage + 1 == STAGES ? 0 : stage + 1;
+      constexpr int QS = GS * 4, HALF = QS / 2;
+      auto multiply = [&](auto from, auto to) {
+         static_for<decltype(to)::value - decltype(from)::value>([&](auto qc) {
+            constexpr int q = decltype(from)::value + decltype(qc)::value;
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+               for (int j = 0; j < NT; ++j)
+                  acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[cur][q / 4][j][q % 4], fa[cur][q / 4][i][q % 4], acc[i][j], 0, 0, 0);
+         });
+      };
+      multiply(std::integral_constant<int, 0>{}, std::integral_constant<int, HALF>{});
+      __builtin_amdgcn_sched_barrier(0);
+      wait_vmcnt<(STAGES - 2) * LPT>();
+      __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0): all of this wave's fragments of slab kt are in registers
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      read(next, fa[cur ^ 1], fb[cur ^ 1]);
+      issue(kt + STAGES, stage, whole);
+      multiply(std::integral_constant<int, HALF>{}, std::integral_constant<int, QS>{});
+      constexpr int GROUPS = (QS - HALF) * MT * NT;
+      constexpr int READS = GS * ((SA::KC ? MT : 2 * MT) + (SB::KC ? NT : 2 * NT)); // pairs of dwords go into one instruction
+#pragma unroll
+      for (int g = 0; g < GROUPS; ++g) {
+         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+         __builtin_amdgcn_sched_group_barrier(0x100, (READS + GROUPS - 1) / GROUPS, 0);
+         __builtin_amdgcn_sched_group_barrier(0x020, (LPT + GROUPS - 1) / GROUPS, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      stage = next;
+   };
+   constexpr std::integral_constant<int, 0> even{};
+   constexpr std::integral_constant<int, 1> odd{};
+   int kt = 0;
+   // as long as what is asked for is a whole slab, no load looks at its k (the comparison and the selection of an address per load
+   // cost 5 - 8 % of the loop)
+   for (; kt + 1 + STAGES < K / BK; kt += 2) {
+      step(kt, even, std::true_type{});
+      step(kt + 1, odd, std::true_type{});
+   }
+   for (; kt < KT; kt += 2) {
+      step(kt, even, any);
+      if (kt + 1 < KT)
+         step(kt + 1, odd, any);
+   }
+
+   // The tile store reuses the ring, one region per wave: the wave's tile is laid out as the result is (rows of columns, or columns
+   // of rows), and read back in one rolled loop, so that a wave instruction stores whole lines and the code of the
+   // activations exists once.  Waves that share a tile add their parts up as they read, each for its share of the lines.
+   wait_vmcnt<0>();
+   __syncthreads();
+   const int lk = lane >> 5, c = lane & 31;
+   constexpr int REGION = f32_store_floats<TM, TN, STORE::kAlongRows>();
+   float *mine = f32_lds + wave * REGION, *first = f32_lds + (wave - wk) * REGION;
+#pragma unroll
+   for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+         for (int g = 0; g < 4; ++g) {
+            if constexpr (!STORE::kAlongRows)
+               *(v4f *)(mine + (i * 32 + c) * (TN + 4) + j * 32 + g * 8 + lk * 4) =
+                  v4f{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+            else
+#pragma unroll
+               for (int e = 0; e < 4; ++e)
+                  mine[(j * 32 + g * 8 + lk * 4 + e) * (TM + 4) + i * 32 + c] = acc[i][j][4 * g + e];
+         }
+   if constexpr (WAVES_K > 1)
+      __syncthreads();
+   else
+      __builtin_amdgcn_wave_barrier();
+   if constexpr (!STORE::kAlongRows) {
+      constexpr int LPR = TN / 4, RPP = 64 / LPR; // lanes per row, rows per pass
+      const int n = n0 + wn * TN + (lane % LPR) * 4;
+#pragma unroll 1
+      for (int r = wk * RPP + lane / LPR; r < TM; r += RPP * WAVES_K) {
+         const int m = m0 + wm * TM + r;
+         const float *at = first + r * (TN + 4) + (lane % LPR) * 4;
+         v4f v = *(const v4f *)at;
+#pragma unroll
+         for (int w = 1; w < WAVES_K; ++w)
+            v += *(const v4f *)(at + w * REGION);
+         if (m < M && n < N)
+            out.put4(v, m, n, N);
+      }
+   } else {
+      constexpr int RPP = TM >= 64 ? 1 : 64 / TM; // columns per pass
+      static_assert(TM <= 64, "a column of the wave tile is at most one lane per row");
+      const int m = m0 + wm * TM + lane % TM;
+      const auto where = out.row_of(m < M ? m : M - 1);
+#pragma unroll 1
+      for (int r = wk * RPP + lane / TM; r < TN; r += RPP * WAVES_K) {
+         const int n = n0 + wn * TN + r;
+         const float *at = first + r * (TM + 4) + lane % TM;
+         float v = *at;
+#pragma unroll
+         for (int w = 1; w < WAVES_K; ++w)
+            v += at[w * REGION];
+         if (m < M && n < N)
+            out.put_at(v, where, n);
+      }
+   }
+}
+
+// ---- the direct kernel --------------------------------------------------------------------------------------------------------
+// W waves split the reduction of one (16 MB) x (16 NB) tile in steps of 16 k (v_mfma_f32_16x16x4_f32: lane (lk = lane / 16, c = lane
+// % 16) supplies k = 4 lk + j of row c to MFMA j); the partial tiles meet in LDS.  What such a product
+// costs is one trip to memory for its operands: every wave has UNROLL steps of loads in flight at once.
+template <class ASRC, class BSRC, class STORE, int MB, int NB, int W, int UNROLL>
+__global__ __launch_bounds__(W * 64) void f32_direct_kernel(ASRC A, BSRC B, STORE out, int M, int N, int K, int tiles_m, int tiles_n, long long strideA,
+                                                            long long strideB)
+{
+   constexpr int TM = MB * 16, TN = NB * 16, PITCH = TN + 4;
+   __shared__ __attribute__((aligned(16))) float part[W][TM][PITCH];
+   const int z = blockIdx.z;
+   A.shift(z * strideA);
+   B.shift(z * strideB);
+   A.select_group(z);
+   out.select_batch(z);
+   int tm, tn;
+   tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, 4, tm, tn);
+   const int m0 = tm * TM, n0 = tn * TN;
+   const int lane = threadIdx.x & 63;
+   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+   const int lk = lane >> 4, c = lane & 15;
+   typename ASRC::row_state ra[MB];
+   typename BSRC::row_state rb[NB];
+#pragma unroll
+   for (int i = 0; i < MB; ++i)
+      ra[i] = A.row_of(m0 + i * 16 + c);
+#pragma unroll
+   for (int j = 0; j < NB; ++j)
+      rb[j] = B.row_of(n0 + j * 16 + c);
+   v4f acc[MB][NB];
+#pragma unroll
+   for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+         acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+   const int KS = (K + 15) / 16;
+   for (int s0 = wave; s0 < KS; s0 += W * UNROLL) {
+      v4f fa[UNROLL][MB], fb[UNROLL][NB];
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+         const int k = (s0 + u * W) * 16 + lk * 4; // steps past the end fetch zeros
+#pragma unroll
+         for (int i = 0; i < MB; ++i)
+            fa[u][i] = A.fetch(ra[i], k);
+#pragma unroll
+         for (int j = 0; j < NB; ++j)
+            fb[u][j] = B.fetch(rb[j], k);
+      }
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+         for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+               acc[i][j] = mfma_f32_step(fb[u][j], fa[u][i], acc[i][j]);
+   }
+#pragma unroll
+   for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+         *(v4f *)&part[wave][i * 16 + c][j * 16 + lk * 4] = acc[i][j];
+   __syncthreads();
+#pragma unroll 1
+   for (int e = threadIdx.x; e < TM * TN; e += W * 64) {
+      // neighbouring threads store neighbouring elements of the direction that is contiguous in the result
+      const int r = STORE::kAlongRows ? e % TM : e / TN, q = STORE::kAlongRows ? e / TM : e % TN;
+      float v = part[0][r][q];
+#pragma unroll
+      for (int w = 1; w < W; ++w)
+         v += part[w][r][q];
+      const int m = m0 + r, n = n0 + q;
+      if (m < M && n < N)
+         out.put(v, m, n);
+   }
+}
+
+// ---- launches -----------------------------------------------------------------------------------------------------------------
+template <class ASRC, class BSRC, class STORE, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int WAVES_K, int STAGES>
+static int launch_f32_tile(hipStream_t stream, const ASRC &A, const BSRC &B, const STORE &out, int M, int N, int K, int batch, long long strideA, long long strideB)
+{
+   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+   const long long nwg = (long long)tiles_m * tiles_n;
+   if (nwg > 0x7fffffffLL)
+      return fail(SOFIE_HIP_ERR_INVALID, "fp32 product: too many tiles");
+   constexpr size_t smem = f32_tile_lds_bytes<BM, BN, BK, STAGES, WAVES_M, WAVES_N, WAVES_K, ASRC::KC, BSRC::KC, STORE::kAlongRows>();
+   auto kern = f32_tile_kernel<ASRC, BSRC, STORE, BM, BN, BK, WAVES_M, WAVES_N, WAVES_K, STAGES>;
+   static_assert(smem <= 160 * 1024, "LDS of a CU");
+   static bool configured[64] = {};
+   if (int st = configure_lds_once(kern, smem, configured))
+      return st;
+   hipLaunchKernelGGL(kern, dim3((unsigned)nwg, 1, (unsigned)batch), dim3(WAVES_M * WAVES_N * WAVES_K * 64), smem, stream, A, B, out, M, N, K, tiles_m, tiles_n, strideA,
+                      strideB);
+   return launch_status("f32_tile_kernel");
+}
+
+template <class ASRC, class BSRC, class STORE, int MB, int NB, int W, int UNROLL>
+static int launch_f32_direct(hipStream_t stream, const ASRC &A, const BSRC &B, const STORE &out, int M, int N, int K, int batch, long long strideA, long long strideB)
+{
+   const int tiles_m = (M + MB * 16 - 1) / (MB * 16), tiles_n = (N + NB * 16 - 1) / (NB * 16);
+   const long long nwg = (long long)tiles_m * tiles_n;
+   if (nwg > 0x7fffffffLL)
+      return fail(SOFIE_HIP_ERR_INVALID, "fp32 product: too many tiles");
+   hipLaunchKernelGGL((f32_direct_kernel<ASRC, BSRC, STORE, MB, NB, W, UNROLL>), dim3((unsigned)nwg, 1, (unsigned)batch), dim3(W * 64), 0, stream, A, B, out, M, N, K,
+                      tiles_m, tiles_n, strideA, strideB);
+   return launch_status("f32_direct_kernel");
+}
+
+} // namespace sofie_hip

@@ -1,329 +1,8 @@
-// fp32 Gemm / MatMul and fp32 convolution (implicit GEMM) with the bias + activation epilogue fused
-// into the store.  These are the small-batch, HBM/latency-bound operators of the fp32 path: tiles of
-// 64x64 outputs, K walked in slabs of 16 staged through LDS, 4x4 outputs per lane, fp32 FMA.
-// The operand fetch is a functor, so the same tile loop serves a strided/transposed Gemm and a
-// convolution whose column matrix is gathered on the fly (no materialised im2col).
-#include "common.hpp"
-#include <cstdlib>
-
-namespace sofie_hip {
-
-constexpr int F32_BM = 64, F32_BN = 64, F32_BK = 16;
-
-struct GemmOperandA {
-   const float *p;
-   long long sm, sk; // element strides of op(A)[m,k]
-   __device__ __forceinline__ float operator()(int m, int k) const { return p[m * sm + k * sk]; }
-};
-struct GemmOperandB {
-   const float *p;
-   long long sk, sn; // element strides of op(B)[k,n]
-   __device__ __forceinline__ float operator()(int k, int n) const { return p[k * sk + n * sn]; }
-};
-
-struct F32Epilogue {
-   float alpha, beta;
-   const float *C;
-   int bias_mode;
-   long long ldc;
-   PostChain chain; // the activation, then the caller's chain of one-to-one operators
-   const float *R;  // tensor of Y's shape added before the activation, or nullptr
-   long long ldr;
-};
-
-__device__ __forceinline__ float f32_epilogue(const F32Epilogue &ep, float acc, int m, int n)
-{
-   float v = ep.alpha * acc;
-   switch (ep.bias_mode) {
-   case SOFIE_BIAS_ROW: v += ep.C[n]; break;
-   case SOFIE_BIAS_COL: v += ep.C[m]; break;
-   case SOFIE_BIAS_SCALAR: v += ep.C[0]; break;
-   case SOFIE_BIAS_FULL: v += ep.beta * ep.C[m * ep.ldc + n]; break;
-   default: break;
-   }
-   if (ep.R)
-      v += ep.R[m * ep.ldr + n];
-   return apply_chain(v, ep.chain);
-}
-
-// The tile loop: acc[4][4] per lane over a 64x64 tile.  LA(m,k), LB(k,n) return 0-safe values only for
-// in-range indices; the loop bounds-checks before calling them.
-template <class LA, class LB>
-__device__ __forceinline__ void f32_tile_loop(const LA &la, const LB &lb, int M, int N, int K, int m0, int n0,
-                                              float (&acc)[4][4])
-{
-   __shared__ float sA[F32_BK][F32_BM + 4];
-   __shared__ float sB[F32_BK][F32_BN + 4];
-   const int t = threadIdx.x;
-   const int tx = t & 15, ty = t >> 4; // 16x16 lanes, each 4x4 outputs
-#pragma unroll
-   for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-         acc[i][j] = 0.0f;
-
-   for (int k0 = 0; k0 < K; k0 += F32_BK) {
-      // 64x16 elements of each operand, 256 threads -> 4 each
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-         int id = t + i * 256;
-         int kk = id & 15, mm = id >> 4; // k fastest for A: consecutive lanes walk k
-         int m = m0 + mm, k = k0 + kk;
-         sA[kk][mm] = (m < M && k < K) ? la(m, k) : 0.0f;
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-         int id = t + i * 256;
-         int nn = id & 63, kk = id >> 6; // n fastest for B
-         int n = n0 + nn, k = k0 + kk;
-         sB[kk][nn] = (n < N && k < K) ? lb(k, n) : 0.0f;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int kk = 0; kk < F32_BK; ++kk) {
-         float a[4], b[4];
-#pragma unroll
-         for (int i = 0; i < 4; ++i)
-            a[i] = sA[kk][ty * 4 + i];
-#pragma unroll
-         for (int j = 0; j < 4; ++j)
-            b[j] = sB[kk][tx * 4 + j];
-#pragma unroll
-         for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-               acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-      }
-      __syncthreads();
-   }
-}
-
-__global__ __launch_bounds__(256) void gemm_f32_kernel(GemmOperandA la, GemmOperandB lb, int M, int N, int K, float *Y,
-                                                        long long ldy, F32Epilogue ep, long long strideA, long long strideB,
-                                                        long long strideC, long long strideY)
-{
-   const int b = blockIdx.z;
-   la.p += b * strideA;
-   lb.p += b * strideB;
-   if (ep.C)
-      ep.C += b * strideC;
-   if (ep.R)
-      ep.R += b * strideY;
-   Y += b * strideY;
-   const int m0 = blockIdx.x * F32_BM, n0 = blockIdx.y * F32_BN;
-   float acc[4][4];
-   f32_tile_loop(la, lb, M, N, K, m0, n0, acc);
-   const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-#pragma unroll
-   for (int i = 0; i < 4; ++i) {
-      int m = m0 + ty * 4 + i;
-      if (m >= M)
-         continue;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-         int n = n0 + tx * 4 + j;
-         if (n < N)
-            Y[m * ldy + n] = f32_epilogue(ep, acc[i][j], m, n);
-      }
-   }
-}
-
-// Small products (the fp32 MLP at batch 64 has 64x128, 64x64 and 64x10 outputs): the 64x64 tiles above would
-// occupy a handful of CUs and spend their time waiting for one 16-wide K slab after another.  Here a
-// workgroup is ONE wave that owns an 8x8 tile, one output per lane, so even these products spread over
-// more than a hundred CUs.  K is walked in chunks of 256: the 8 rows of op(A) and the 8 columns of op(B)
-// are staged in LDS with K contiguous (row pitch 260 floats: the 8 rows a wave reads at once fall into
-// different banks), the next chunk's loads are issued before the current chunk is consumed, and a lane
-// reads 4 K values of its row and its column per step into four partial sums (k mod 4), added at the end.
-constexpr int SK_T = 8, SK_KC = 256, SK_PITCH = SK_KC + 4;
-
-template <bool VEC_A, bool VEC_B>
-__global__ __launch_bounds__(64) void gemm_f32_skinny_kernel(GemmOperandA la, GemmOperandB lb, int M, int N, int K, float *Y,
-                                                              long long ldy, F32Epilogue ep, long long strideA, long long strideB,
-                                                              long long strideC, long long strideY)
-{
-   __shared__ __attribute__((aligned(16))) float sA[2][SK_T][SK_PITCH];
-   __shared__ __attribute__((aligned(16))) float sB[2][SK_T][SK_PITCH];
-   const int b = blockIdx.z;
-   la.p += b * strideA;
-   lb.p += b * strideB;
-   if (ep.C)
-      ep.C += b * strideC;
-   if (ep.R)
-      ep.R += b * strideY;
-   Y += b * strideY;
-   const int lane = threadIdx.x;
-   const int tm = lane >> 3, tn = lane & 7;
-   const int m0 = blockIdx.x * SK_T, n0 = blockIdx.y * SK_T;
-
-   // staging registers of one chunk: row i of the tile, K values 4*lane..4*lane+3 (vector form), or
-   // element lane + 64*j of the 8x256 block (scalar form, any strides)
-   float4 ra[SK_T], rb[SK_T];
-   float qa[VEC_A ? 1 : 32], qb[VEC_B ? 1 : 32];
-   auto fetch = [&](int k0) {
-      if (VEC_A) {
-#pragma unroll
-         for (int i = 0; i < SK_T; ++i) {
-            const int m = m0 + i, k = k0 + lane * 4;
-            ra[i] = (m < M && k < K) ? *(const float4 *)(la.p + m * la.sm + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-         }
-      } else {
-#pragma unroll
-         for (int j = 0; j < 32; ++j) {
-            const int id = lane + 64 * j, row = id & 7, kk = id >> 3; // rows fastest: a transposed operand is contiguous there
-            const int m = m0 + row, k = k0 + kk;
-            qa[j] = (m < M && k < K) ? la(m, k) : 0.0f;
-         }
-      }
-      if (VEC_B) {
-#pragma unroll
-         for (int i = 0; i < SK_T; ++i) {
-            const int n = n0 + i, k = k0 + lane * 4;
-            rb[i] = (n < N && k < K) ? *(const float4 *)(lb.p + n * lb.sn + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-         }
-      } else {
-#pragma unroll
-         for (int j = 0; j < 32; ++j) {
-            const int id = lane + 64 * j, row = id & 7, kk = id >> 3;
-            const int n = n0 + row, k = k0 + kk;
-            qb[j] = (n < N && k < K) ? lb(k, n) : 0.0f;
-         }
-      }
-   };
-   auto stage = [&](int buf) {
-      if (VEC_A) {
-#pragma unroll
-         for (int i = 0; i < SK_T; ++i)
-            *(float4 *)&sA[buf][i][lane * 4] = ra[i];
-      } else {
-#pragma unroll
-         for (int j = 0; j < 32; ++j) {
-            const int id = lane + 64 * j;
-            sA[buf][id & 7][id >> 3] = qa[j];
-         }
-      }
-      if (VEC_B) {
-#pragma unroll
-         for (int i = 0; i < SK_T; ++i)
-            *(float4 *)&sB[buf][i][lane * 4] = rb[i];
-      } else {
-#pragma unroll
-         for (int j = 0; j < 32; ++j) {
-            const int id = lane + 64 * j;
-            sB[buf][id & 7][id >> 3] = qb[j];
-         }
-      }
-   };
-
-   float acc4[4] = {0.0f, 0.0f, 0.0f, 0.0f}; // k = 0,1,2,3 (mod 4): four independent FMA chains, added at the end
-   fetch(0);
-   int buf = 0;
-   for (int k0 = 0; k0 < K; k0 += SK_KC) {
-      stage(buf);
-      if (k0 + SK_KC < K)
-         fetch(k0 + SK_KC); // in flight while this chunk is consumed
-      __builtin_amdgcn_wave_barrier();
-      const int kc = (K - k0) < SK_KC ? (K - k0) : SK_KC;
-#pragma unroll 4
-      for (int kk = 0; kk < kc; kk += 4) {
-         const float4 a = *(const float4 *)&sA[buf][tm][kk];
-         const float4 c = *(const float4 *)&sB[buf][tn][kk];
-         acc4[0] = fmaf(a.x, c.x, acc4[0]);
-         acc4[1] = fmaf(a.y, c.y, acc4[1]);
-         acc4[2] = fmaf(a.z, c.z, acc4[2]);
-         acc4[3] = fmaf(a.w, c.w, acc4[3]);
-      }
-      buf ^= 1;
-   }
-   const float acc = (acc4[0] + acc4[1]) + (acc4[2] + acc4[3]);
-   const int m = m0 + tm, n = n0 + tn;
-   if (m < M && n < N)
-      Y[m * ldy + n] = f32_epilogue(ep, acc, m, n);
-}
-
-// Column-matrix element (row m = (image, oh, ow), column k = (ci, kh, kw)) gathered from NCHW input;
-// the same index arithmetic as the reference's Im2col, zero outside the image.
-struct ConvOperandA {
-   const float *X;
-   int C, H, W, kh, kw, OH, OW, pad_h0, pad_w0, stride_h, stride_w, dil_h, dil_w;
-   int c_first; // first input channel of this group
-   __device__ __forceinline__ float operator()(int m, int k) const
-   {
-      int ow = m % OW, t = m / OW;
-      int oh = t % OH, img = t / OH;
-      int kx = k % kw, t2 = k / kw;
-      int ky = t2 % kh, ci = t2 / kh;
-      int ih = oh * stride_h - pad_h0 + ky * dil_h;
-      int iw = ow * stride_w - pad_w0 + kx * dil_w;
-      if ((unsigned)ih >= (unsigned)H || (unsigned)iw >= (unsigned)W)
-         return 0.0f;
-      return X[(((size_t)img * C + c_first + ci) * H + ih) * W + iw];
-   }
-};
-// The same for three spatial dimensions (the reference's Im2col_3d): row m = (image, od, oh, ow), column k = (ci, kd, kh, kw).
-struct Conv3dOperandA {
-   const float *X;
-   int C, D, H, W, kd, kh, kw, OD, OH, OW, pad_d0, pad_h0, pad_w0, stride_d, stride_h, stride_w, dil_d, dil_h, dil_w;
-   int c_first;
-   __device__ __forceinline__ float operator()(int m, int k) const
-   {
-      int ow = m % OW, t = m / OW;
-      int oh = t % OH;
-      t /= OH;
-      int od = t % OD, img = t / OD;
-      int kx = k % kw, t2 = k / kw;
-      int ky = t2 % kh;
-      t2 /= kh;
-      int kz = t2 % kd, ci = t2 / kd;
-      int id = od * stride_d - pad_d0 + kz * dil_d;
-      int ih = oh * stride_h - pad_h0 + ky * dil_h;
-      int iw = ow * stride_w - pad_w0 + kx * dil_w;
-      if ((unsigned)id >= (unsigned)D || (unsigned)ih >= (unsigned)H || (unsigned)iw >= (unsigned)W)
-         return 0.0f;
-      return X[((((size_t)img * C + c_first + ci) * D + id) * H + ih) * W + iw];
-   }
-};
-struct ConvOperandB {
-   const float *Wt; // [Cout_g][Kg] rows of this group
-   int Kg;
-   __device__ __forceinline__ float operator()(int k, int n) const { return Wt[(size_t)n * Kg + k]; }
-};
-
-template <class LA>
-__global__ __launch_bounds__(256) void conv_f32_kernel(LA la, const float *Wt, const float *bias, float *Y, int M,
-                                                        int Cout_g, int Kg, int Cg, int Cout, int OHW, PostChain chain, const float *R)
-{
-   const int g = blockIdx.z;
-   la.c_first = g * Cg;
-   ConvOperandB lb{Wt + (size_t)g * Cout_g * Kg, Kg};
-   const int m0 = blockIdx.x * F32_BM, n0 = blockIdx.y * F32_BN;
-   float acc[4][4];
-   f32_tile_loop(la, lb, M, Cout_g, Kg, m0, n0, acc);
-   const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-#pragma unroll
-   for (int i = 0; i < 4; ++i) {
-      int m = m0 + ty * 4 + i;
-      if (m >= M)
-         continue;
-      int img = m / OHW, pix = m % OHW;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-         int n = n0 + tx * 4 + j;
-         if (n < Cout_g) {
-            int co = g * Cout_g + n;
-            float v = acc[i][j];
-            if (bias)
-               v += bias[co];
-            const size_t at = ((size_t)img * Cout + co) * OHW + pix;
-            if (R)
-               v += R[at];
-            Y[at] = apply_chain(v, chain);
-         }
-      }
-   }
-}
-
-} // namespace sofie_hip
+// fp32 Gemm / MatMul and fp32 convolution (implicit GEMM) with the bias + activation epilogue fused into the store: the entry
+// points and the choice among the kernels of f32_mfma.hpp, and the kernel that runs a chain of small products in one launch.
+#include "f32_mfma.hpp"
+#include <algorithm>
+#include <cmath>
 
 namespace sofie_hip {
 
@@ -453,6 +132,86 @@ __global__ __launch_bounds__(CHAIN_THREADS) void gemm_chain_f32_kernel(ChainArgs
 
 } // namespace sofie_hip
 
+namespace sofie_hip {
+
+// The kernel for a product of M x N x K, `batch` times: the one whose time, estimated from what each was measured to do, is the
+// shortest.  A CU multiplies a 32 x 32 block by 32 k in 256 cycles at best; the tile kernels reach 0.66 (32 x 32 tiles), 0.78
+// (64 x 64) and 0.84 (128 x 128) of that and take 4.2 / 5 / 5.5 us on top (launch, first loads, store), in as many rounds as the tiles
+// need over 256 CUs.  The direct kernel costs a launch and a trip to memory per 512 k (2.0 and 1.35 us), or the 9.4 TB/s at which
+// its fragments, which nothing shares, arrive.
+enum F32Tile { F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128 = 128 };
+static int pick_f32_tile(int M, int N, int K, int batch, int least_rows)
+{
+   auto tiles = [&](int bm, int bn) { return (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
+   auto tiled = [&](int bm, int bn, double rate, double fixed) {
+      const double rounds = std::ceil(tiles(bm, bn) / 256.0), blocks = (bm / 32) * (bn / 32);
+      return fixed + rounds * ((K + 31) / 32) * blocks * 256.0 / (2400.0 * rate);
+   };
+   const double steps = (K + 15) / 16;
+   int best = F32_DIRECT;
+   double least = std::max(2.0 + 1.35 * std::ceil(steps / 32.0), tiles(16, 16) * steps * 2048.0 / 9.4e6 + 2.0);
+   auto offer = [&](int tile, double t) {
+      if (t < least)
+         least = t, best = tile;
+   };
+   if (least_rows <= 32)
+      offer(F32_TILE_32, tiled(32, 32, 0.66, 4.2));
+   offer(F32_TILE_64x32, tiled(64, 32, 0.70, 4.6));
+   offer(F32_TILE_64, tiled(64, 64, 0.78, 5.0));
+   offer(F32_TILE_128, tiled(128, 128, 0.84, 5.5));
+   return best;
+}
+
+template <class ASRC, class BSRC, class STORE>
+static int launch_f32_product(sofie_hip_ctx *ctx, const ASRC &A, const BSRC &B, const STORE &out, int M, int N, int K, int batch, long long strideA, long long strideB)
+{
+   hipStream_t s = ctx->stream;
+   int tile = ctx->opt.f32_tile;
+   if (ctx->opt.f32_skinny == 1 || K == 0)
+      tile = F32_DIRECT;
+   else if (ctx->opt.f32_skinny == 0 && !tile)
+      tile = F32_TILE_64;
+   if (!tile)
+      tile = pick_f32_tile(M, N, K, batch, ASRC::kLeastRows);
+   switch (tile) {
+   case F32_DIRECT: return launch_f32_direct<ASRC, BSRC, STORE, 1, 1, 8, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
+   case F32_TILE_32:
+      if constexpr (ASRC::kLeastRows <= 32)
+         return launch_f32_tile<ASRC, BSRC, STORE, 32, 32, 32, 1, 1, 4, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
+      [[fallthrough]];
+   case F32_TILE_64x32: return launch_f32_tile<ASRC, BSRC, STORE, 64, 32, 32, 2, 1, 2, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
+   case F32_TILE_64: return launch_f32_tile<ASRC, BSRC, STORE, 64, 64, 32, 2, 2, 2, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
+   case F32_TILE_128: return launch_f32_tile<ASRC, BSRC, STORE, 128, 128, 16, 2, 2, 1, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
+   default: return fail(SOFIE_HIP_ERR_INVALID, "fp32 product: unknown tile %d", tile);
+   }
+}
+
+// A convolution of `group` groups as products of M = images x positions rows and Cout / group columns.
+template <bool VOLUME>
+static int launch_f32_conv(sofie_hip_ctx *ctx, const float *X, F32ConvShape s, const float *W, const F32ConvStore &out, long long M, int group, const char *who)
+{
+   const int taps = s.kd * s.kh * s.kw, K = s.Cg * taps, N = out.Cout_g;
+   auto reciprocal = [](int d) { return (unsigned)(((1ull << 31) + d - 1) / (unsigned)d); };
+   s.kw_mul = reciprocal(s.kw), s.kh_mul = reciprocal(s.kh), s.kd_mul = reciprocal(s.kd);
+   // umulhi(2 k, ceil(2^31 / d)) is k / d while k * d < 2^31; a slab or two past K are divided as well
+   const long long longest = std::max(s.kw, std::max(s.kh, s.kd));
+   SOFIE_HIP_REQUIRE((K + 1024LL) * longest < (1LL << 31), "%s: reduction too long", who);
+   F32ConvRows<VOLUME> A;
+   A.X = X;
+   A.s = s;
+   A.rows = (int)M;
+   A.K = K;
+   A.channel = (long long)s.D * s.H * s.W;
+   A.image = A.channel * s.C;
+   SOFIE_HIP_REQUIRE(group <= 65535, "%s: too many groups for one launch", who);
+   const long long strideB = (long long)N * K;
+   if (((uintptr_t)W & 15) == 0 && K % 4 == 0)
+      return launch_f32_product(ctx, A, F32Matrix<true, 4>{W, K, N, K}, out, (int)M, N, K, group, 0, strideB);
+   return launch_f32_product(ctx, A, F32Matrix<true, 1>{W, K, N, K}, out, (int)M, N, K, group, 0, strideB);
+}
+
+} // namespace sofie_hip
+
 using namespace sofie_hip;
 
 extern "C" {
@@ -478,8 +237,6 @@ int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *d)
    const long long ldy = d->ldy ? d->ldy : N;
    SOFIE_HIP_REQUIRE(lda >= (d->transA ? M : K) && ldb >= (d->transB ? K : N) && ldy >= N,
                      "sofie_hip_gemm_f32: leading dimension too small");
-   GemmOperandA la{d->A, d->transA ? 1 : lda, d->transA ? lda : 1};
-   GemmOperandB lb{d->B, d->transB ? 1 : ldb, d->transB ? ldb : 1};
    ep.alpha = d->alpha;
    ep.beta = d->beta;
    ep.C = d->bias_mode == SOFIE_BIAS_NONE ? nullptr : d->C;
@@ -487,32 +244,27 @@ int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *d)
    ep.ldc = N;
    ep.R = d->residual;
    ep.ldr = ldy;
-   const unsigned gy = (M + F32_BM - 1) / F32_BM, gx = (N + F32_BN - 1) / F32_BN;
-   SOFIE_HIP_REQUIRE(gx <= 65535 && d->batch <= 65535, "sofie_hip_gemm_f32: N or batch too large for one launch");
-   // few 64x64 tiles: one-wave workgroups with 8x8 tiles reach every CU (SOFIE_HIP_F32_SKINNY=0/1 overrides)
-   const bool skinny = ctx->opt.f32_skinny >= 0 ? ctx->opt.f32_skinny != 0 : ((long long)gy * gx * d->batch < 192);
-   if (skinny && K > 0 && (N + SK_T - 1) / SK_T <= 65535) {
-      auto aligned16 = [](const void *p) { return ((uintptr_t)p & 15) == 0; };
-      const bool va = !d->transA && K % 4 == 0 && lda % 4 == 0 && aligned16(d->A) && d->strideA % 4 == 0;
-      const bool vb = d->transB && K % 4 == 0 && ldb % 4 == 0 && aligned16(d->B) && d->strideB % 4 == 0;
-      const dim3 grid((M + SK_T - 1) / SK_T, (N + SK_T - 1) / SK_T, (unsigned)d->batch);
-#define SOFIE_SKINNY(VA, VB)                                                                                              \
-   hipLaunchKernelGGL((gemm_f32_skinny_kernel<VA, VB>), grid, dim3(64), 0, ctx->stream, la, lb, M, N, K, d->Y, ldy, ep,   \
-                      (long long)d->strideA, (long long)d->strideB, (long long)d->strideC, (long long)d->strideY)
-      if (va && vb)
-         SOFIE_SKINNY(true, true);
-      else if (va)
-         SOFIE_SKINNY(true, false);
-      else if (vb)
-         SOFIE_SKINNY(false, true);
-      else
-         SOFIE_SKINNY(false, false);
-#undef SOFIE_SKINNY
-      return launch_status("gemm_f32_skinny_kernel");
-   }
-   hipLaunchKernelGGL(gemm_f32_kernel, dim3(gy, gx, (unsigned)d->batch), dim3(256), 0, ctx->stream, la, lb, M, N, K, d->Y, ldy, ep,
-                      (long long)d->strideA, (long long)d->strideB, (long long)d->strideC, (long long)d->strideY);
-   return launch_status("gemm_f32_kernel");
+   SOFIE_HIP_REQUIRE(d->batch <= 65535, "sofie_hip_gemm_f32: batch too large for one launch");
+   auto in_vectors = [](const void *p, long long a, long long b, long long c) { return ((uintptr_t)p & 15) == 0 && a % 4 == 0 && b % 4 == 0 && c % 4 == 0; };
+   F32RowStore out;
+   out.Y = d->Y;
+   out.ldy = ldy;
+   out.ep = ep;
+   out.vec = in_vectors(d->Y, ldy, d->strideY, 0);
+   out.strideC = d->strideC;
+   out.strideY = d->strideY;
+   // 16-byte loads where both operands allow them: address, pitch, and the extent along the contiguous direction
+   const bool vec = in_vectors(d->A, lda, d->strideA, d->transA ? M : K) && in_vectors(d->B, ldb, d->strideB, d->transB ? K : N);
+   auto with_b = [&](const auto &A) {
+      auto go = [&](const auto &B) {
+         return launch_f32_product(ctx, A, B, out, M, N, K, d->batch, d->strideA, d->strideB);
+      };
+      constexpr int VEC = std::remove_reference_t<decltype(A)>::VEC;
+      return d->transB ? go(F32Matrix<true, VEC>{d->B, ldb, N, K}) : go(F32Matrix<false, VEC>{d->B, ldb, N, K});
+   };
+   if (vec)
+      return d->transA ? with_b(F32Matrix<false, 4>{d->A, lda, M, K}) : with_b(F32Matrix<true, 4>{d->A, lda, M, K});
+   return d->transA ? with_b(F32Matrix<false, 1>{d->A, lda, M, K}) : with_b(F32Matrix<true, 1>{d->A, lda, M, K});
 }
 
 int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *layers, int32_t count)
@@ -641,13 +393,11 @@ int sofie_hip_conv_f32(sofie_hip_ctx *ctx, const sofie_conv_desc *d, const float
    SOFIE_HIP_REQUIRE(X && W && Y, "sofie_hip_conv_f32: NULL pointer");
    const long long M = (long long)d->N * OH * OW;
    SOFIE_HIP_REQUIRE(M < (1LL << 31), "sofie_hip_conv_f32: too many output pixels");
-   const int Cg = d->C / d->group, Cout_g = d->Cout / d->group, Kg = Cg * d->kh * d->kw;
-   ConvOperandA la{X, d->C, d->H, d->W, d->kh, d->kw, OH, OW, d->pad_h0, d->pad_w0, d->stride_h, d->stride_w, d->dil_h, d->dil_w, 0};
-   const unsigned gy = (unsigned)((M + F32_BM - 1) / F32_BM), gx = (Cout_g + F32_BN - 1) / F32_BN;
-   SOFIE_HIP_REQUIRE(gx <= 65535 && d->group <= 65535, "sofie_hip_conv_f32: too many channels or groups for one launch");
-   hipLaunchKernelGGL(conv_f32_kernel<ConvOperandA>, dim3(gy, gx, (unsigned)d->group), dim3(256), 0, ctx->stream, la, W, bias, Y, (int)M, Cout_g, Kg,
-                      Cg, d->Cout, OH * OW, chain, residual);
-   return launch_status("conv_f32_kernel");
+   SOFIE_HIP_REQUIRE((long long)(d->C / d->group) * d->kh * d->kw < (1LL << 31), "sofie_hip_conv_f32: reduction too long");
+   const F32ConvShape s{d->C, 1, d->H, d->W, 1, d->kh, d->kw, 1, OH, OW, 0, d->pad_h0, d->pad_w0, 1, d->stride_h, d->stride_w, 1, d->dil_h, d->dil_w,
+                        d->C / d->group, 0, 0, 0};
+   const F32ConvStore out{Y, bias, residual, chain, d->Cout, d->Cout / d->group, OH * OW, 0};
+   return launch_f32_conv<false>(ctx, X, s, W, out, M, d->group, "sofie_hip_conv_f32");
 }
 
 int sofie_hip_conv3d_f32(sofie_hip_ctx *ctx, const sofie_conv3d_desc *d, const float *X, const float *W, const float *bias,
@@ -679,14 +429,10 @@ int sofie_hip_conv3d_f32(sofie_hip_ctx *ctx, const sofie_conv3d_desc *d, const f
    SOFIE_HIP_REQUIRE(M < (1LL << 31) && (long long)d->C * d->D * d->H * d->W < (1LL << 31), "sofie_hip_conv3d_f32: too many output or input elements");
    const long long Kg64 = (long long)(d->C / d->group) * d->kd * d->kh * d->kw;
    SOFIE_HIP_REQUIRE(Kg64 < (1LL << 31), "sofie_hip_conv3d_f32: reduction too long");
-   const int Cg = d->C / d->group, Cout_g = d->Cout / d->group, Kg = (int)Kg64;
-   Conv3dOperandA la{X, d->C, d->D, d->H, d->W, d->kd, d->kh, d->kw, outd[0], outd[1], outd[2], d->pad[0], d->pad[1], d->pad[2],
-                     d->stride[0], d->stride[1], d->stride[2], d->dil[0], d->dil[1], d->dil[2], 0};
-   const unsigned gy = (unsigned)((M + F32_BM - 1) / F32_BM), gx = (Cout_g + F32_BN - 1) / F32_BN;
-   SOFIE_HIP_REQUIRE(gx <= 65535 && d->group <= 65535, "sofie_hip_conv3d_f32: too many channels or groups for one launch");
-   hipLaunchKernelGGL(conv_f32_kernel<Conv3dOperandA>, dim3(gy, gx, (unsigned)d->group), dim3(256), 0, ctx->stream, la, W, bias, Y, (int)M,
-                      Cout_g, Kg, Cg, d->Cout, (int)plane, chain, residual);
-   return launch_status("conv_f32_kernel (3-D)");
+   const F32ConvShape s{d->C, d->D, d->H, d->W, d->kd, d->kh, d->kw, outd[0], outd[1], outd[2], d->pad[0], d->pad[1], d->pad[2],
+                        d->stride[0], d->stride[1], d->stride[2], d->dil[0], d->dil[1], d->dil[2], d->C / d->group, 0, 0, 0};
+   const F32ConvStore out{Y, bias, residual, chain, d->Cout, d->Cout / d->group, (int)plane, 0};
+   return launch_f32_conv<true>(ctx, X, s, W, out, M, d->group, "sofie_hip_conv3d_f32");
 }
 
 } // extern "C"

@@ -53,6 +53,7 @@ const OptionName kOptionNames[] = {
    {"conv_explicit", "SOFIE_HIP_CONV_EXPLICIT", &sofie_hip_options::conv_explicit},
    {"f32_skinny", "SOFIE_HIP_F32_SKINNY", &sofie_hip_options::f32_skinny},
    {"f32_chain", "SOFIE_HIP_F32_CHAIN", &sofie_hip_options::f32_chain},
+   {"f32_tile", "SOFIE_HIP_F32_TILE", &sofie_hip_options::f32_tile},
 };
 } // namespace
 
