@@ -51,7 +51,8 @@ int sofie_hip_ctx_destroy(sofie_hip_ctx *ctx);
  * reference, whose GPU path has no such choice): "i8_tile" / "f8_tile" (64, 128, 256; 258 and 512 ask for the two-per-CU and the
  * persistent kernel; 0 = heuristic), "gemm_variant" (1: alternative pipelined kernel, -1: general kernel only), "swizzle"
  * (tile order), "conv_explicit" (1: int8 convolutions through a column matrix whenever the workspace holds one), "f32_skinny",
- * "f32_chain" (0 / 1, -1 = heuristic).  Each is also read once, at sofie_hip_ctx_create, from the environment variable
+ * "f32_chain" (0 / 1, -1 = heuristic), "f32_tile" (fp32 products and convolutions: 16 the direct kernel; 32, 62, 64, 126, 128 the tile
+ * kernel with tiles of 32 x 32, 64 x 32, 64 x 64, 128 x 32 (convolutions), 128 x 128 (products); 0 = heuristic).  Each is also read once, at sofie_hip_ctx_create, from the environment variable
  * SOFIE_HIP_<NAME IN CAPITALS>; nothing reads the environment after that. */
 int sofie_hip_ctx_set_option(sofie_hip_ctx *ctx, const char *name, int32_t value);
 const char *sofie_hip_last_error(void);

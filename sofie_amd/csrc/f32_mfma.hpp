@@ -26,6 +26,18 @@ __device__ __forceinline__ v4f mfma_f32_step(const v4f &n_side, const v4f &m_sid
    return acc;
 }
 
+// tile_of_block; a single column of tiles (the usual convolution) needs none of its divisions
+__device__ __forceinline__ void f32_tile_of_block(int tiles_m, int tiles_n, int &tm, int &tn)
+{
+   if (tiles_n == 1) {
+      const int bid = blockIdx.x, per = tiles_m / 8, rem = tiles_m % 8, xcd = bid % 8;
+      tm = xcd * per + (xcd < rem ? xcd : rem) + bid / 8;
+      tn = 0;
+   } else {
+      tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, 4, tm, tn);
+   }
+}
+
 // ---- operands ---------------------------------------------------------------------------------------------------------------
 // An operand is a matrix of `rows` (m or n) by K.  KC: contiguous in k (a row's k neighbours lie side by side); otherwise
 // contiguous along the rows.  VEC: floats per load; 4 needs 16-byte aligned pieces (the host checks that the address, the
@@ -53,9 +65,12 @@ struct F32Matrix {
       const int r = row < rows ? row : (KC || VEC == 1 ? rows - 1 : rows - VEC);
       st.at[i] = KC ? p + (long long)r * ld + kk : p + (long long)kk * ld + r;
    }
+   struct walk_state {};
+   __device__ __forceinline__ void walk_start(walk_state &, int, int, int) const {}
+   __device__ __forceinline__ void walk_on(walk_state &, int) const {}
    // address of load i of the slab at k0 (kk: the lane's k within the slab; WHOLE: no k of the slab lies past K)
    template <bool WHOLE, int LD>
-   __device__ __forceinline__ const float *load_ptr(const lane_state<LD> &st, int i, int kk, int k0) const
+   __device__ __forceinline__ const float *load_ptr(const lane_state<LD> &st, const walk_state &, int i, int kk, int k0) const
    {
       const float *a = st.at[i] + (KC ? (long long)k0 : (long long)k0 * ld);
       return WHOLE || k0 + kk < K ? a : f32_zero_page;
@@ -94,9 +109,14 @@ struct F32ConvShape {
    int C, D, H, W, kd, kh, kw, OD, OH, OW; // input channels (all groups); a 2-D convolution has D = kd = OD = 1
    int pad_d, pad_h, pad_w, stride_d, stride_h, stride_w, dil_d, dil_h, dil_w;
    int Cg;                                 // channels per group
-   unsigned kw_mul, kh_mul, kd_mul;        // ceil(2^31 / extent): k / extent == umulhi(2 k, mul) while k * extent < 2^31 (checked on the host)
+   int positions;                          // kd * kh * kw
+   unsigned long long ow_mul, oh_mul, od_mul; // ceil(2^64 / extent), 0 for an extent of 1: m / extent == umul64hi(m, mul) for 32-bit m
+   unsigned kw_mul, kh_mul, kd_mul, positions_mul; // ceil(2^31 / extent): k / extent == umulhi(2 k, mul) while k * extent < 2^31 (checked on the host)
 };
-template <bool VOLUME> // three spatial axes
+// MASKED (at most 31 kernel positions): a lane keeps one bit per kernel position that lies inside the image; lane i walks along the
+// k of load instruction i, from slab to slab, and the instructions take offset and kernel position from there as scalars.
+// About ten instructions per 64 elements, a quarter of what decomposing every k by scalar arithmetic took.
+template <bool MASKED>
 struct F32ConvRows {
    static constexpr int kLeastRows = 64; // a load instruction covers one k: what depends on k is scalar
    static constexpr bool KC = false;
@@ -114,17 +134,13 @@ struct F32ConvRows {
    };
    __device__ __forceinline__ row_state row_of(int row) const
    {
+      auto quotient = [](int n, unsigned long long mul) { return mul ? (int)__umul64hi((unsigned long long)(unsigned)n, mul) : n; };
       const int m = row < rows ? row : rows - 1;
-      int ow = m % s.OW, t = m / s.OW;
-      int oh = t % s.OH;
-      t /= s.OH;
-      int od = 0, img = t;
-      if (VOLUME) {
-         od = t % s.OD;
-         img = t / s.OD;
-      }
+      const int t = quotient(m, s.ow_mul), ow = m - t * s.OW;
+      const int u = quotient(t, s.oh_mul), oh = t - u * s.OH;
+      const int img = quotient(u, s.od_mul), od = u - img * s.OD;
       row_state r;
-      r.id0 = VOLUME ? od * s.stride_d - s.pad_d : 0;
+      r.id0 = od * s.stride_d - s.pad_d;
       r.ih0 = oh * s.stride_h - s.pad_h;
       r.iw0 = ow * s.stride_w - s.pad_w;
       r.at = X + (long long)img * image + ((long long)r.id0 * s.H + r.ih0) * s.W + r.iw0;
@@ -136,32 +152,82 @@ struct F32ConvRows {
    {
       const int t = divide(k, s.kw_mul), kx = k - t * s.kw;
       const int u = divide(t, s.kh_mul), ky = t - u * s.kh;
-      int ci = u, kz = 0;
-      if (VOLUME) {
-         ci = divide(u, s.kd_mul);
-         kz = u - ci * s.kd;
-      }
+      const int ci = divide(u, s.kd_mul), kz = u - ci * s.kd;
       const int dz = kz * s.dil_d, dy = ky * s.dil_h, dx = kx * s.dil_w;
-      bool inside = k < K && (unsigned)(r.ih0 + dy) < (unsigned)s.H && (unsigned)(r.iw0 + dx) < (unsigned)s.W;
-      if (VOLUME)
-         inside = inside && (unsigned)(r.id0 + dz) < (unsigned)s.D;
+      const bool inside = k < K && (unsigned)(r.id0 + dz) < (unsigned)s.D && (unsigned)(r.ih0 + dy) < (unsigned)s.H && (unsigned)(r.iw0 + dx) < (unsigned)s.W;
       const float *p = r.at + ((long long)ci * channel + ((long long)dz * s.H + dy) * s.W + dx);
       return inside ? p : f32_zero_page;
    }
-   // a lane keeps the same row through all load instructions of a slab (tiles of 64 rows or more, four waves)
+   // a lane keeps the same row through all load instructions of a slab (tiles of 64 rows or more, an even number of waves)
    template <int LD>
    struct lane_state {
       row_state r;
+      unsigned inside; // bit t: kernel position t of this row lies inside the image
    };
    template <int LD>
    __device__ __forceinline__ void init(lane_state<LD> &st, int i, int row, int) const
    {
-      if (i == 0)
-         st.r = row_of(row);
+      if (i != 0)
+         return;
+      st.r = row_of(row);
+      if constexpr (MASKED) {
+         unsigned columns = 0, lines = 0;
+         for (int kx = 0; kx < s.kw; ++kx)
+            columns |= ((unsigned)(st.r.iw0 + kx * s.dil_w) < (unsigned)s.W ? 1u : 0u) << kx;
+         for (int ky = 0; ky < s.kh; ++ky)
+            lines |= ((unsigned)(st.r.ih0 + ky * s.dil_h) < (unsigned)s.H ? columns : 0u) << (ky * s.kw);
+         st.inside = 0;
+         for (int kz = 0; kz < s.kd; ++kz)
+            st.inside |= ((unsigned)(st.r.id0 + kz * s.dil_d) < (unsigned)s.D ? lines : 0u) << (kz * s.kh * s.kw);
+      }
+   }
+   // For MASKED, lane i: the k of load i of the slab to be asked for, its kernel position and the offsets of its channel and position.
+   struct walk_state {
+      int k, position, channel_offset;
+      int step_channels, step_rest; // a slab's worth of k in channels (as an offset) and kernel positions: uniform
+      int table;  // lane t: offset of kernel position t
+      int offset; // of k: what load i adds to the address of its row
+   };
+   __device__ __forceinline__ void walk_settle(walk_state &w) const
+   {
+      w.offset = w.channel_offset + __builtin_amdgcn_ds_bpermute(w.position << 2, w.table);
+      if (w.k >= K)
+         w.offset = 0;
+   }
+   __device__ __forceinline__ void walk_start(walk_state &w, int k, int lane, int step) const
+   {
+      if constexpr (MASKED) {
+         const int t = divide(lane, s.kw_mul), kx = lane - t * s.kw, kz = divide(t, s.kh_mul), ky = t - kz * s.kh;
+         w.table = (kz * s.dil_d * s.H + ky * s.dil_h) * s.W + kx * s.dil_w; // lanes past the last position are not asked
+         const int ci = divide(k, s.positions_mul), channels = divide(step, s.positions_mul);
+         w.k = k;
+         w.position = k - ci * s.positions;
+         w.channel_offset = ci * (int)channel;
+         w.step_channels = channels * (int)channel;
+         w.step_rest = step - channels * s.positions;
+         walk_settle(w);
+      }
+   }
+   __device__ __forceinline__ void walk_on(walk_state &w, int step) const // by the `step` of walk_start
+   {
+      if constexpr (MASKED) {
+         w.k += step;
+         w.position += w.step_rest;
+         w.channel_offset += w.step_channels;
+         const bool over = w.position >= s.positions;
+         w.position -= over ? s.positions : 0;
+         w.channel_offset += over ? (int)channel : 0;
+         walk_settle(w);
+      }
    }
    template <bool WHOLE, int LD>
-   __device__ __forceinline__ const float *load_ptr(const lane_state<LD> &st, int, int kk, int k0) const
+   __device__ __forceinline__ const float *load_ptr(const lane_state<LD> &st, const walk_state &w, int i, int kk, int k0) const
    {
+      if constexpr (MASKED) {
+         const int offset = __builtin_amdgcn_readlane(w.offset, i);
+         const int position = __builtin_amdgcn_readlane(WHOLE || w.k < K ? w.position : 31, i); // no lane has bit 31 set
+         return (st.inside >> position) & 1u ? st.r.at + (long long)offset : f32_zero_page;
+      }
       return element(st.r, k0 + __builtin_amdgcn_readfirstlane(kk));
    }
    __device__ __forceinline__ v4f fetch(const row_state &st, int k) const
@@ -273,17 +339,36 @@ struct F32ConvStore {
       const int img = m / positions;
       return row_state{(size_t)img * Cout * positions + (m - img * positions)};
    }
-   __device__ __forceinline__ void put_at(float v, const row_state &r, int n) const
+   // C columns of one row; those from N on are left out
+   template <int C>
+   __device__ __forceinline__ void put_columns(float (&v)[C], const row_state &r, const int (&n)[C], int N) const
    {
-      const int co = first + n;
-      const size_t at = r.at + (size_t)co * positions;
-      if (bias)
-         v += bias[co];
-      if (R)
-         v += R[at];
-      Y[at] = f32_activate(v, chain);
+      size_t at[C];
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+         const int co = first + (n[i] < N ? n[i] : N - 1);
+         at[i] = r.at + (size_t)co * positions;
+         if (bias)
+            v[i] += bias[co];
+         if (R)
+            v[i] += R[at[i]];
+      }
+      if (chain.count != 0) {
+#pragma unroll
+         for (int i = 0; i < C; ++i)
+            v[i] = f32_activate(v[i], chain);
+      }
+#pragma unroll
+      for (int i = 0; i < C; ++i)
+         if (n[i] < N)
+            Y[at[i]] = v[i];
    }
-   __device__ __forceinline__ void put(float v, int m, int n) const { put_at(v, row_of(m), n); }
+   __device__ __forceinline__ void put(float v, int m, int n) const
+   {
+      float one[1] = {v};
+      const int col[1] = {n};
+      put_columns<1>(one, row_of(m), col, n + 1);
+   }
 };
 
 // ---- the tile kernel ----------------------------------------------------------------------------------------------------------
@@ -318,6 +403,7 @@ struct F32Slab {
    static constexpr bool KC = SRC::KC;
    static constexpr int FLOATS = f32_slab_floats<SRC::KC, R, BK>();
    typename SRC::template lane_state<LD> st;
+   typename SRC::walk_state walk;
 
    // (row, k) of the slab that load i of this wave brings to this lane's place in LDS
    static __device__ __forceinline__ void place(int i, int wave, int lane, int &row, int &kk)
@@ -340,22 +426,25 @@ struct F32Slab {
          place(i, wave, lane, row, kk);
          src.template init<LD>(st, i, r0 + row, kk);
       }
+      src.walk_start(walk, ((lane * NW + wave) % TOTAL) * 64 * VEC / R, lane, BK); // the k of the load whose number is the lane's
    }
+   // asks for the slab at k0; the slabs are asked for one after the other
    template <bool WHOLE>
-   __device__ __forceinline__ void issue(const SRC &src, float *lds, int k0, int wave, int lane) const
+   __device__ __forceinline__ void issue(const SRC &src, float *lds, int k0, int wave, int lane)
    {
       static_for<LD>([&](auto ic) {
          constexpr int i = decltype(ic)::value;
          int row, kk;
          place(i, wave, lane, row, kk);
          const int f = ((i * NW + wave) % TOTAL) * 64 * VEC;
-         global_void_t *from = (global_void_t *)src.template load_ptr<WHOLE, LD>(st, i, kk, k0);
+         global_void_t *from = (global_void_t *)src.template load_ptr<WHOLE, LD>(st, walk, i, kk, k0);
          lds_void_t *to = (lds_void_t *)(lds + f + f32_gap<SRC::KC, R>(f / R));
          if constexpr (VEC == 4)
             __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
          else
             __builtin_amdgcn_global_load_lds(from, to, 4, 0, 0);
       });
+      src.walk_on(walk, BK);
    }
    // fragment of k = 8 g .. 8 g + 7 of the 32 rows from r on
    static __device__ __forceinline__ v4f fragment(const float *lds, int r, int g, int lane)
@@ -376,11 +465,12 @@ constexpr int f32_store_floats()
 {
    return ALONG_ROWS ? TN * (TM + 4) : TM * (TN + 4);
 }
-template <int BM, int BN, int BK, int STAGES, int WAVES_M, int WAVES_N, int WAVES_K, bool KCA, bool KCB, bool ALONG_ROWS>
-constexpr size_t f32_tile_lds_bytes()
+// LDS of a tile kernel with a ring of `stages` slabs
+template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int WAVES_K, bool KCA, bool KCB, bool ALONG_ROWS>
+constexpr size_t f32_tile_lds_bytes(int stages)
 {
-   constexpr size_t ring = (size_t)STAGES * (f32_slab_floats<KCA, BM, BK>() + f32_slab_floats<KCB, BN, BK>()) * 4;
-   constexpr size_t store = (size_t)WAVES_M * WAVES_N * WAVES_K * f32_store_floats<BM / WAVES_M, BN / WAVES_N, ALONG_ROWS>() * 4;
+   const size_t ring = (size_t)stages * (f32_slab_floats<KCA, BM, BK>() + f32_slab_floats<KCB, BN, BK>()) * 4;
+   const size_t store = (size_t)WAVES_M * WAVES_N * WAVES_K * f32_store_floats<BM / WAVES_M, BN / WAVES_N, ALONG_ROWS>() * 4;
    return ring > store ? ring : store;
 }
 
@@ -409,7 +499,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_ke
    A.select_group(z);
    out.select_batch(z);
    int tm, tn;
-   tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, 4, tm, tn);
+   f32_tile_of_block(tiles_m, tiles_n, tm, tn);
    const int m0 = tm * BM, n0 = tn * BN;
    const int lane = threadIdx.x & 63;
    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -429,13 +519,21 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_ke
             acc[i][j][e] = 0.0f;
 
    const int KT = (K + BK - 1) / BK;
-   // a slab past the end is asked for as the last one again: filler that keeps the number of loads per step the same
    auto issue = [&](int kt, int stage, auto whole) {
-      const int k0 = (kt < KT ? kt : KT - 1) * BK;
       float *s = f32_lds + stage * STAGE;
-      sa.template issue<decltype(whole)::value>(A, s, k0, wave, lane);
-      sb.template issue<decltype(whole)::value>(B, s + SA::FLOATS, k0, wave, lane);
+      sa.template issue<decltype(whole)::value>(A, s, kt * BK, wave, lane);
+      sb.template issue<decltype(whole)::value>(B, s + SA::FLOATS, kt * BK, wave, lane);
    };
+   // until at most `slabs` of the slabs asked for last are still on their way (counts past STAGES - 2 wait for that many)
+   auto wait_slabs = [&](int slabs) {
+      if (slabs >= STAGES - 2)
+         wait_vmcnt<(STAGES - 2) * LPT>();
+      else if (STAGES > 3 && slabs == 1)
+         wait_vmcnt<LPT>();
+      else
+         wait_vmcnt<0>();
+   };
+   static_assert(STAGES == 3 || STAGES == 4, "the cases of wait_slabs");
    constexpr std::false_type any{};
    v4f fa[2][GS][MT], fb[2][GS][NT];
    auto read = [&](int stage, v4f(&a)[GS][MT], v4f(&b)[GS][NT]) {
@@ -453,8 +551,12 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_ke
    if (KT > 0) { // an empty reduction reads nothing
 #pragma unroll
       for (int s = 0; s < STAGES; ++s)
-         issue(s, s, any);
-      wait_vmcnt<(STAGES - 1) * LPT>();
+         if (s < KT)
+            issue(s, s, any);
+      if (KT >= STAGES)
+         wait_vmcnt<(STAGES - 1) * LPT>();
+      else
+         wait_slabs(KT - 1);
       __builtin_amdgcn_s_barrier();
       read(0, fa[0], fb[0]);
    }
@@ -465,6 +567,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_ke
    // on its SIMD keeps the matrix core busy.
    auto step = [&](int kt, auto parity, auto whole) {
       constexpr int cur = decltype(parity)::value;
+      constexpr bool WHOLE = decltype(whole)::value;
       const int next = stage + 1 == STAGES ? 0 : stage + 1;
       constexpr int QS = GS * 4, HALF = QS / 2;
       auto multiply = [&](auto from, auto to) {
@@ -479,12 +582,17 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_ke
       };
       multiply(std::integral_constant<int, 0>{}, std::integral_constant<int, HALF>{});
       __builtin_amdgcn_sched_barrier(0);
-      wait_vmcnt<(STAGES - 2) * LPT>();
+      if constexpr (WHOLE)
+         wait_vmcnt<(STAGES - 2) * LPT>();
+      else
+         wait_slabs(KT - 2 - kt);
       __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0): all of this wave's fragments of slab kt are in registers
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      read(next, fa[cur ^ 1], fb[cur ^ 1]);
-      issue(kt + STAGES, stage, whole);
+      if (WHOLE || kt + 1 < KT)
+         read(next, fa[cur ^ 1], fb[cur ^ 1]);
+      if (WHOLE || kt + STAGES < KT)
+         issue(kt + STAGES, stage, whole);
       multiply(std::integral_constant<int, HALF>{}, std::integral_constant<int, QS>{});
       constexpr int GROUPS = (QS - HALF) * MT * NT;
       constexpr int READS = GS * ((SA::KC ? MT : 2 * MT) + (SB::KC ? NT : 2 * NT)); // pairs of dwords go into one instruction
@@ -557,16 +665,24 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_ke
       static_assert(TM <= 64, "a column of the wave tile is at most one lane per row");
       const int m = m0 + wm * TM + lane % TM;
       const auto where = out.row_of(m < M ? m : M - 1);
+      // four columns at a time: their biases (and residuals) are on their way together
+      constexpr int STEP = RPP * WAVES_K, C = TN / STEP >= 4 ? 4 : TN / STEP;
+      static_assert(TN % (STEP * C) == 0, "columns divide over the passes");
 #pragma unroll 1
-      for (int r = wk * RPP + lane / TM; r < TN; r += RPP * WAVES_K) {
-         const int n = n0 + wn * TN + r;
-         const float *at = first + r * (TM + 4) + lane % TM;
-         float v = *at;
+      for (int r = wk * RPP + lane / TM; r < TN; r += STEP * C) {
+         float v[C];
+         int n[C];
 #pragma unroll
-         for (int w = 1; w < WAVES_K; ++w)
-            v += at[w * REGION];
-         if (m < M && n < N)
-            out.put_at(v, where, n);
+         for (int i = 0; i < C; ++i) {
+            n[i] = n0 + wn * TN + r + i * STEP;
+            const float *at = first + (r + i * STEP) * (TM + 4) + lane % TM;
+            v[i] = *at;
+#pragma unroll
+            for (int w = 1; w < WAVES_K; ++w)
+               v[i] += at[w * REGION];
+         }
+         if (m < M)
+            out.template put_columns<C>(v, where, n, N);
       }
    }
 }
@@ -587,7 +703,7 @@ __global__ __launch_bounds__(W * 64) void f32_direct_kernel(ASRC A, BSRC B, STOR
    A.select_group(z);
    out.select_batch(z);
    int tm, tn;
-   tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, 4, tm, tn);
+   f32_tile_of_block(tiles_m, tiles_n, tm, tn);
    const int m0 = tm * TM, n0 = tn * TN;
    const int lane = threadIdx.x & 63;
    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -655,11 +771,15 @@ static int launch_f32_tile(hipStream_t stream, const ASRC &A, const BSRC &B, con
    const long long nwg = (long long)tiles_m * tiles_n;
    if (nwg > 0x7fffffffLL)
       return fail(SOFIE_HIP_ERR_INVALID, "fp32 product: too many tiles");
-   constexpr size_t smem = f32_tile_lds_bytes<BM, BN, BK, STAGES, WAVES_M, WAVES_N, WAVES_K, ASRC::KC, BSRC::KC, STORE::kAlongRows>();
+   // a reduction of fewer slabs than the ring holds takes only their places: more workgroups share a CU (first convolution of a
+   // 64-image network, one slab: 40 -> 32 us)
+   const int slabs = K > BK * (STAGES - 1) ? STAGES : K > BK ? (K + BK - 1) / BK : 1;
+   const size_t smem = f32_tile_lds_bytes<BM, BN, BK, WAVES_M, WAVES_N, WAVES_K, ASRC::KC, BSRC::KC, STORE::kAlongRows>(slabs);
+   constexpr size_t most = f32_tile_lds_bytes<BM, BN, BK, WAVES_M, WAVES_N, WAVES_K, ASRC::KC, BSRC::KC, STORE::kAlongRows>(STAGES);
+   static_assert(most <= 160 * 1024, "LDS of a CU");
    auto kern = f32_tile_kernel<ASRC, BSRC, STORE, BM, BN, BK, WAVES_M, WAVES_N, WAVES_K, STAGES>;
-   static_assert(smem <= 160 * 1024, "LDS of a CU");
    static bool configured[64] = {};
-   if (int st = configure_lds_once(kern, smem, configured))
+   if (int st = configure_lds_once(kern, most, configured))
       return st;
    hipLaunchKernelGGL(kern, dim3((unsigned)nwg, 1, (unsigned)batch), dim3(WAVES_M * WAVES_N * WAVES_K * 64), smem, stream, A, B, out, M, N, K, tiles_m, tiles_n, strideA,
                       strideB);

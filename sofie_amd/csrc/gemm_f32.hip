@@ -139,8 +139,8 @@ namespace sofie_hip {
 // (64 x 64) and 0.84 (128 x 128) of that and take 4.2 / 5 / 5.5 us on top (launch, first loads, store), in as many rounds as the tiles
 // need over 256 CUs.  The direct kernel costs a launch and a trip to memory per 512 k (2.0 and 1.35 us), or the 9.4 TB/s at which
 // its fragments, which nothing shares, arrive.
-enum F32Tile { F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128 = 128 };
-static int pick_f32_tile(int M, int N, int K, int batch, int least_rows)
+enum F32Tile { F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
+static int pick_f32_tile(int M, int N, int K, int batch)
 {
    auto tiles = [&](int bm, int bn) { return (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
    auto tiled = [&](int bm, int bn, double rate, double fixed) {
@@ -154,11 +154,32 @@ static int pick_f32_tile(int M, int N, int K, int batch, int least_rows)
       if (t < least)
          least = t, best = tile;
    };
-   if (least_rows <= 32)
-      offer(F32_TILE_32, tiled(32, 32, 0.66, 4.2));
+   offer(F32_TILE_32, tiled(32, 32, 0.66, 4.2));
    offer(F32_TILE_64x32, tiled(64, 32, 0.70, 4.6));
    offer(F32_TILE_64, tiled(64, 64, 0.78, 5.0));
    offer(F32_TILE_128, tiled(128, 128, 0.84, 5.5));
+   return best;
+}
+// The same for a convolution, whose tiles carry the arithmetic of the gather: 0.62 of the matrix rate in the loop and 0.7 us per
+// 32 x 32 block of a tile for its start and its store, and not less than 0.75 us per slab where a CU has one tile only.  The direct
+// kernel gathers for every 16 columns anew.
+static int pick_f32_conv_tile(int M, int N, int K, int group)
+{
+   auto tiles = [&](int bm, int bn) { return (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * group; };
+   auto tiled = [&](int bm, int bn) {
+      const double rounds = std::ceil(tiles(bm, bn) / 256.0), blocks = (bm / 32) * (bn / 32), slabs = (K + 31) / 32;
+      return 3.0 + std::max(rounds * blocks * (slabs * 256.0 / (2400.0 * 0.62) + 0.7), 0.75 * slabs + 1.4);
+   };
+   int best = F32_DIRECT;
+   double least = 5.3 + tiles(16, 16) / 256.0 * (0.9 + 0.17 * ((K + 15) / 16));
+   auto offer = [&](int tile, double t) {
+      if (t < least)
+         least = t, best = tile;
+   };
+   offer(F32_TILE_64x32, tiled(64, 32));
+   offer(F32_TILE_64, tiled(64, 64));
+   if (N <= 32 && tiles(128, 32) >= 1024) // a start per 128 rows instead of 64: first convolution of a 64-image network 29.7 -> 27.6 us
+      offer(F32_TILE_128x32, 0.95 * tiled(128, 32));
    return best;
 }
 
@@ -171,43 +192,65 @@ static int launch_f32_product(sofie_hip_ctx *ctx, const ASRC &A, const BSRC &B, 
       tile = F32_DIRECT;
    else if (ctx->opt.f32_skinny == 0 && !tile)
       tile = F32_TILE_64;
+   constexpr bool CONV = ASRC::kLeastRows == 64;
    if (!tile)
-      tile = pick_f32_tile(M, N, K, batch, ASRC::kLeastRows);
+      tile = CONV ? pick_f32_conv_tile(M, N, K, batch) : pick_f32_tile(M, N, K, batch);
+   if (CONV ? tile == F32_TILE_32 || tile == F32_TILE_128 : tile == F32_TILE_128x32)
+      tile = F32_TILE_64; // a request for a tile that the other kind of product has
+   if constexpr (CONV) {
+      switch (tile) {
+      case F32_TILE_64x32: return launch_f32_tile<ASRC, BSRC, STORE, 64, 32, 32, 2, 1, 2, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
+      case F32_TILE_128x32: return launch_f32_tile<ASRC, BSRC, STORE, 128, 32, 32, 4, 1, 1, 3>(s, A, B, out, M, N, K, batch, strideA, strideB);
+      }
+   } else {
+      switch (tile) {
+      case F32_TILE_32: return launch_f32_tile<ASRC, BSRC, STORE, 32, 32, 32, 1, 1, 4, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
+      case F32_TILE_64x32: return launch_f32_tile<ASRC, BSRC, STORE, 64, 32, 32, 2, 1, 2, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
+      case F32_TILE_128: return launch_f32_tile<ASRC, BSRC, STORE, 128, 128, 16, 2, 2, 1, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
+      }
+   }
    switch (tile) {
    case F32_DIRECT: return launch_f32_direct<ASRC, BSRC, STORE, 1, 1, 8, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
-   case F32_TILE_32:
-      if constexpr (ASRC::kLeastRows <= 32)
-         return launch_f32_tile<ASRC, BSRC, STORE, 32, 32, 32, 1, 1, 4, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
-      [[fallthrough]];
-   case F32_TILE_64x32: return launch_f32_tile<ASRC, BSRC, STORE, 64, 32, 32, 2, 1, 2, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
    case F32_TILE_64: return launch_f32_tile<ASRC, BSRC, STORE, 64, 64, 32, 2, 2, 2, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
-   case F32_TILE_128: return launch_f32_tile<ASRC, BSRC, STORE, 128, 128, 16, 2, 2, 1, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
    default: return fail(SOFIE_HIP_ERR_INVALID, "fp32 product: unknown tile %d", tile);
    }
 }
 
 // A convolution of `group` groups as products of M = images x positions rows and Cout / group columns.
-template <bool VOLUME>
-static int launch_f32_conv(sofie_hip_ctx *ctx, const float *X, F32ConvShape s, const float *W, const F32ConvStore &out, long long M, int group, const char *who)
+template <bool MASKED>
+static int launch_f32_conv_rows(sofie_hip_ctx *ctx, const F32ConvRows<MASKED> &A, const float *W, const F32ConvStore &out, int M, int group)
 {
-   const int taps = s.kd * s.kh * s.kw, K = s.Cg * taps, N = out.Cout_g;
-   auto reciprocal = [](int d) { return (unsigned)(((1ull << 31) + d - 1) / (unsigned)d); };
-   s.kw_mul = reciprocal(s.kw), s.kh_mul = reciprocal(s.kh), s.kd_mul = reciprocal(s.kd);
-   // umulhi(2 k, ceil(2^31 / d)) is k / d while k * d < 2^31; a slab or two past K are divided as well
-   const long long longest = std::max(s.kw, std::max(s.kh, s.kd));
-   SOFIE_HIP_REQUIRE((K + 1024LL) * longest < (1LL << 31), "%s: reduction too long", who);
-   F32ConvRows<VOLUME> A;
-   A.X = X;
-   A.s = s;
-   A.rows = (int)M;
-   A.K = K;
-   A.channel = (long long)s.D * s.H * s.W;
-   A.image = A.channel * s.C;
-   SOFIE_HIP_REQUIRE(group <= 65535, "%s: too many groups for one launch", who);
+   const int K = A.K, N = out.Cout_g;
    const long long strideB = (long long)N * K;
    if (((uintptr_t)W & 15) == 0 && K % 4 == 0)
-      return launch_f32_product(ctx, A, F32Matrix<true, 4>{W, K, N, K}, out, (int)M, N, K, group, 0, strideB);
-   return launch_f32_product(ctx, A, F32Matrix<true, 1>{W, K, N, K}, out, (int)M, N, K, group, 0, strideB);
+      return launch_f32_product(ctx, A, F32Matrix<true, 4>{W, K, N, K}, out, M, N, K, group, 0, strideB);
+   return launch_f32_product(ctx, A, F32Matrix<true, 1>{W, K, N, K}, out, M, N, K, group, 0, strideB);
+}
+static int launch_f32_conv(sofie_hip_ctx *ctx, const float *X, F32ConvShape s, const float *W, const F32ConvStore &out, long long M, int group, const char *who)
+{
+   const int taps = s.kd * s.kh * s.kw, K = s.Cg * taps;
+   auto reciprocal = [](int d) { return (unsigned)(((1ull << 31) + d - 1) / (unsigned)d); };
+   s.kw_mul = reciprocal(s.kw), s.kh_mul = reciprocal(s.kh), s.kd_mul = reciprocal(s.kd), s.positions_mul = reciprocal(taps);
+   // umulhi(2 k, ceil(2^31 / d)) is k / d while k * d < 2^31; a few slabs past K are divided as well
+   const long long longest = taps;
+   SOFIE_HIP_REQUIRE((K + 4096LL) * longest < (1LL << 31), "%s: reduction too long", who);
+   SOFIE_HIP_REQUIRE(group <= 65535, "%s: too many groups for one launch", who);
+   auto rows = [&](auto A) {
+      A.X = X;
+      A.s = s;
+      A.rows = (int)M;
+      A.K = K;
+      A.channel = (long long)s.D * s.H * s.W;
+      A.image = A.channel * s.C;
+      return launch_f32_conv_rows(ctx, A, W, out, (int)M, group);
+   };
+   s.positions = taps;
+   auto reciprocal64 = [](unsigned d) -> unsigned long long { return d <= 1 ? 0ull : (~0ull / d) + 1; };
+   s.ow_mul = reciprocal64(s.OW), s.oh_mul = reciprocal64(s.OH), s.od_mul = reciprocal64(s.OD);
+   // one bit per kernel position, and offsets inside an image (a few channels past the last one included) in 32 bits
+   if (taps <= 31 && ((long long)s.C + 4096) * s.D * s.H * s.W + ((long long)s.kd * s.dil_d * s.H + (long long)s.kh * s.dil_h) * s.W < (1LL << 31))
+      return rows(F32ConvRows<true>{});
+   return rows(F32ConvRows<false>{});
 }
 
 } // namespace sofie_hip
@@ -395,9 +438,9 @@ int sofie_hip_conv_f32(sofie_hip_ctx *ctx, const sofie_conv_desc *d, const float
    SOFIE_HIP_REQUIRE(M < (1LL << 31), "sofie_hip_conv_f32: too many output pixels");
    SOFIE_HIP_REQUIRE((long long)(d->C / d->group) * d->kh * d->kw < (1LL << 31), "sofie_hip_conv_f32: reduction too long");
    const F32ConvShape s{d->C, 1, d->H, d->W, 1, d->kh, d->kw, 1, OH, OW, 0, d->pad_h0, d->pad_w0, 1, d->stride_h, d->stride_w, 1, d->dil_h, d->dil_w,
-                        d->C / d->group, 0, 0, 0};
+                        d->C / d->group, 0, 0, 0, 0, 0, 0, 0, 0};
    const F32ConvStore out{Y, bias, residual, chain, d->Cout, d->Cout / d->group, OH * OW, 0};
-   return launch_f32_conv<false>(ctx, X, s, W, out, M, d->group, "sofie_hip_conv_f32");
+   return launch_f32_conv(ctx, X, s, W, out, M, d->group, "sofie_hip_conv_f32");
 }
 
 int sofie_hip_conv3d_f32(sofie_hip_ctx *ctx, const sofie_conv3d_desc *d, const float *X, const float *W, const float *bias,
@@ -430,9 +473,9 @@ int sofie_hip_conv3d_f32(sofie_hip_ctx *ctx, const sofie_conv3d_desc *d, const f
    const long long Kg64 = (long long)(d->C / d->group) * d->kd * d->kh * d->kw;
    SOFIE_HIP_REQUIRE(Kg64 < (1LL << 31), "sofie_hip_conv3d_f32: reduction too long");
    const F32ConvShape s{d->C, d->D, d->H, d->W, d->kd, d->kh, d->kw, outd[0], outd[1], outd[2], d->pad[0], d->pad[1], d->pad[2],
-                        d->stride[0], d->stride[1], d->stride[2], d->dil[0], d->dil[1], d->dil[2], d->C / d->group, 0, 0, 0};
+                        d->stride[0], d->stride[1], d->stride[2], d->dil[0], d->dil[1], d->dil[2], d->C / d->group, 0, 0, 0, 0, 0, 0, 0, 0};
    const F32ConvStore out{Y, bias, residual, chain, d->Cout, d->Cout / d->group, (int)plane, 0};
-   return launch_f32_conv<true>(ctx, X, s, W, out, M, d->group, "sofie_hip_conv3d_f32");
+   return launch_f32_conv(ctx, X, s, W, out, M, d->group, "sofie_hip_conv3d_f32");
 }
 
 } // extern "C"

@@ -14,7 +14,7 @@ from tests.test_gpu_f32 import conv_desc, gemm
 
 pytestmark = pytest.mark.gpu
 
-TILES = [16, 32, 62, 64, 128]
+TILES = [16, 32, 62, 64, 126, 128]
 
 
 @pytest.fixture
