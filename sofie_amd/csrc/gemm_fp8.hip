@@ -231,18 +231,6 @@ int sofie_hip_gemm_fp8(sofie_hip_ctx *ctx, const sofie_gemm_fp8_desc *d)
    int ldb = d->ldb ? d->ldb : (d->transB ? K : N);
    int ldy = d->ldy ? d->ldy : N;
    SOFIE_HIP_REQUIRE(lda >= K && ldb >= (d->transB ? K : N) && ldy >= N, "sofie_hip_gemm_fp8: leading dimension too small");
-   const int8_t *A = (const int8_t *)d->A, *Bt = (const int8_t *)d->B;
-   if (K > 0 && !d->transB) {
-      size_t need = (((size_t)K * (size_t)N) + 255) & ~(size_t)255;
-      SOFIE_HIP_REQUIRE(d->workspace != nullptr && d->workspace_bytes >= need,
-                        "sofie_hip_gemm_fp8: B is [K,N]; a workspace of %zu bytes is needed to re-lay it out", need);
-      SOFIE_HIP_REQUIRE(((uintptr_t)d->workspace & 255) == 0, "sofie_hip_gemm_fp8: workspace must be 256-byte aligned");
-      int st = transpose_i8(ctx->stream, (int8_t *)d->workspace, (const int8_t *)d->B, K, N, ldb, K);
-      if (st)
-         return st;
-      Bt = (const int8_t *)d->workspace;
-      ldb = K;
-   }
    F8Epilogue ep;
    ep.bias = d->bias;
    ep.scale = d->scale;
@@ -253,6 +241,20 @@ int sofie_hip_gemm_fp8(sofie_hip_ctx *ctx, const sofie_gemm_fp8_desc *d)
    ep.N = N;
    const size_t esz = d->out == SOFIE_F8OUT_F32 ? 4 : 2;
    ep.stage_ok = (((size_t)ldy * esz) % 16 == 0) && (((uintptr_t)d->Y & 15) == 0);
+   const int8_t *A = (const int8_t *)d->A, *Bt = (const int8_t *)d->B;
+   if (K > 0 && !d->transB) {
+      size_t need = (((size_t)K * (size_t)N) + 255) & ~(size_t)255;
+      SOFIE_HIP_REQUIRE(d->workspace != nullptr && d->workspace_bytes >= need,
+                        "sofie_hip_gemm_fp8: B is [K,N]; a workspace of %zu bytes is needed to re-lay it out", need);
+      SOFIE_HIP_REQUIRE(((uintptr_t)d->workspace & 255) == 0, "sofie_hip_gemm_fp8: workspace must be 256-byte aligned");
+      if (mfma8_columns_preferred(launch_cfg_f8(ctx), M, N, K, K % 128 == 0 && lda % 16 == 0 && ((uintptr_t)A & 15) == 0))
+         return launch_mfma8_general<MfmaF8, StagedColumns, F8Epilogue>(launch_cfg_f8(ctx), A, lda, StagedColumns{Bt, ldb, N}, M, N, K, ep);
+      int st = transpose_i8(ctx->stream, (int8_t *)d->workspace, (const int8_t *)d->B, K, N, ldb, K);
+      if (st)
+         return st;
+      Bt = (const int8_t *)d->workspace;
+      ldb = K;
+   }
    if (K == 0) {
       A = (const int8_t *)d->Y;
       Bt = (const int8_t *)d->Y;

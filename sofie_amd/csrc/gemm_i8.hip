@@ -7,25 +7,49 @@
 
 namespace sofie_hip {
 
-// dst[c][r] = src[r][c] for an int8 matrix, through a 64x64 LDS tile.
+// dst[c][r] = src[r][c] for an int8 matrix.  A workgroup takes 128 rows x 64 columns: 8 bytes of four rows per thread, transposed four
+// bytes by four in registers, laid out as rows of the result in LDS and stored 16 bytes per thread (any alignment).  Bound by
+// memory; 4096 x 4096: XX us (a byte per thread through LDS: YY us).
 __global__ __launch_bounds__(256) void transpose_i8_kernel(int8_t *__restrict__ dst, const int8_t *__restrict__ src,
                                                             int rows, int cols, int ld_src, int ld_dst)
 {
-   __shared__ int8_t tile[64][64 + 4];
-   const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
-   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-   for (int i = ty; i < 64; i += 4) {
-      int r = r0 + i, c = c0 + tx;
-      tile[i][tx] = (r < rows && c < cols) ? src[(size_t)r * ld_src + c] : (int8_t)0;
-   }
+   __shared__ __attribute__((aligned(16))) int8_t tile[64 * 128];
+   const int r0 = blockIdx.y * 128, c0 = blockIdx.x * 64, t = threadIdx.x;
+   const StagedColumns s{src, ld_src, cols};
+   StagedSlab<StagedColumns, 64, 128, 256> slab;
+   if (r0 + 128 <= rows)
+      slab.load(s, c0, r0, rows, t);
+   else
+      slab.load_last(s, c0, r0, rows, t);
+   if (c0 + 64 > cols)
+      slab.align_edge(s, c0, t);
+   slab.store(tile, t);
    __syncthreads();
-   for (int i = ty; i < 64; i += 4) {
-      int c = c0 + i, r = r0 + tx;
-      if (c < cols && r < rows)
-         dst[(size_t)c * ld_dst + r] = tile[tx][i];
+#pragma unroll
+   for (int i = 0; i < 2; ++i) {
+      const int id = t + i * 256, c = id / 8, k = id % 8 * 16;
+      if (c0 + c >= cols || r0 + k >= rows)
+         continue;
+      const v4i v = *(const v4i *)(tile + lds_chunk_offset<128>(c, id % 8));
+      int8_t *p = dst + (size_t)(c0 + c) * ld_dst + r0 + k;
+      if (r0 + k + 16 <= rows) {
+         *(v4i_unaligned *)p = v;
+      } else {
+         for (int e = 0; e < rows - r0 - k; ++e)
+            p[e] = (int8_t)(v[e >> 2] >> (8 * (e & 3)));
+      }
    }
 }
 
+// The same for a handful of columns, a byte per thread.
+__global__ __launch_bounds__(256) void transpose_few_columns_i8_kernel(int8_t *__restrict__ dst, const int8_t *__restrict__ src, int rows, int cols, int ld_src,
+                                                                       int ld_dst)
+{
+   const int r = blockIdx.x * 256 + threadIdx.x;
+   if (r < rows)
+      for (int c = 0; c < cols; ++c)
+         dst[(size_t)c * ld_dst + r] = src[(size_t)r * ld_src + c];
+}
 
 // The fields of the epilogue that follow from the others: what the stores may assume about alignment, and whether the
 // quotient of SOFIE_I8OUT_I8_DQQ may be formed from the reciprocal (a per-tensor scale known here, in a safe range).
@@ -74,7 +98,11 @@ int conv_i8_few_channels(const LaunchCfg &lc, const FewChannelConv &src, const i
 
 int transpose_i8(hipStream_t stream, int8_t *dst, const int8_t *src, int rows, int cols, int ld_src, int ld_dst)
 {
-   dim3 grid((cols + 63) / 64, (rows + 63) / 64);
+   if (cols < 8) {
+      hipLaunchKernelGGL(transpose_few_columns_i8_kernel, dim3((rows + 255) / 256), dim3(256), 0, stream, dst, src, rows, cols, ld_src, ld_dst);
+      return launch_status("transpose_few_columns_i8_kernel");
+   }
+   dim3 grid((cols + 63) / 64, (rows + 127) / 128);
    hipLaunchKernelGGL(transpose_i8_kernel, grid, dim3(256), 0, stream, dst, src, rows, cols, ld_src, ld_dst);
    return launch_status("transpose_i8_kernel");
 }
@@ -133,6 +161,21 @@ static int gemm_i8_with_workspace(sofie_hip_ctx *ctx, const sofie_gemm_i8_desc *
    SOFIE_HIP_REQUIRE(lda >= (d->transA ? M : K) && ldb >= (d->transB ? K : N) && ldy >= N,
                      "sofie_hip_gemm_i8: leading dimension too small");
 
+   I8Epilogue ep;
+   ep.bias = d->bias;
+   ep.scale = d->scale;
+   ep.scale_scalar = d->scale_scalar;
+   ep.q_scale = d->q_scale;
+   ep.relu_acc = d->relu_acc;
+   ep.relu_out = d->relu_out;
+   ep.out = d->out;
+   ep.Y = d->Y;
+   ep.ldy = ldy;
+   ep.stage_ok = 0;
+   ep.vec_param = 0;
+   ep.N = N;
+   ep.nchw_ohw = 0;
+   ep.n_offset = 0;
    const int8_t *A = d->A, *Bt = d->B;
    char *ws = (char *)workspace;
    size_t ws_left = workspace_bytes;
@@ -142,6 +185,10 @@ static int gemm_i8_with_workspace(sofie_hip_ctx *ctx, const sofie_gemm_i8_desc *
       SOFIE_HIP_REQUIRE(ws != nullptr && ws_left >= need,
                         "sofie_hip_gemm_i8: B is [K,N]; a workspace of %zu bytes is needed to re-lay it out", need);
       SOFIE_HIP_REQUIRE(((uintptr_t)ws & 255) == 0, "sofie_hip_gemm_i8: workspace must be 256-byte aligned");
+      if (!d->transA && mfma8_columns_preferred(launch_cfg_i8(ctx), M, N, K, K % 16 == 0 && lda % 16 == 0 && ((uintptr_t)A & 15) == 0)) {
+         derive_epilogue_fields(ep, N);
+         return launch_mfma8_general<MfmaI8, StagedColumns, I8Epilogue>(launch_cfg_i8(ctx), A, lda, StagedColumns{d->B, ldb, N}, M, N, K, ep);
+      }
       int st = transpose_i8(ctx->stream, (int8_t *)ws, d->B, K, N, ldb, K);
       if (st)
          return st;
@@ -161,21 +208,6 @@ static int gemm_i8_with_workspace(sofie_hip_ctx *ctx, const sofie_gemm_i8_desc *
       lda = K;
    }
 
-   I8Epilogue ep;
-   ep.bias = d->bias;
-   ep.scale = d->scale;
-   ep.scale_scalar = d->scale_scalar;
-   ep.q_scale = d->q_scale;
-   ep.relu_acc = d->relu_acc;
-   ep.relu_out = d->relu_out;
-   ep.out = d->out;
-   ep.Y = d->Y;
-   ep.ldy = ldy;
-   ep.stage_ok = 0;
-   ep.vec_param = 0;
-   ep.N = N;
-   ep.nchw_ohw = 0;
-   ep.n_offset = 0;
    if (K == 0) {
       // empty reduction: acc = 0 everywhere; run the kernel with K = 0 using any valid pointer
       A = (const int8_t *)d->Y;

@@ -1,19 +1,60 @@
 // Kernel choice for the int8 / FP8 GEMM and the int8 convolution: which tile, which pipelined kernel, or the general one.
 #pragma once
 #include "conv_i8_resident.hpp"
+#include "mfma8_staged.hpp"
+#include <algorithm>
+#include <cmath>
 
 namespace sofie_hip {
 
-// Chooses between the pipelined kernels (aligned operands, K a multiple of 64) and the general one.
+// ---- estimates ------------------------------------------------------------------------------------------------------------
+// Below the sizes that fill the matrix cores, all of these kernels are bound by the bytes a CU takes in (37 - 45 KB/us through
+// registers, 67 - 75 KB/us straight into LDS) and by what a tile costs besides (start, store).  Fitted to single launches from
+// 33 x 260 x 100 to 3001 x 3695 x 6991 and to the long, narrow products of small convolutions (200000 x 32 x 224), the estimates hold
+// to about a fifth; they decide between kernels whose times differ by more than that almost everywhere.
+inline double mfma8_time(int M, int N, int K, int bm, int bn, double fixed_us, double tile_us, double bytes_per_us)
+{
+   double rounds = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) / 256.0; // tiles per CU; a CU works on a few at a time
+   rounds = rounds <= 1.0 ? 1.0 : 0.5 * (rounds + std::ceil(rounds));
+   return fixed_us + rounds * (tile_us + (double)(bm + bn) * K / bytes_per_us);
+}
+inline double mfma8_direct16_time(int M, int N, int K) { return mfma8_time(M, N, K, 16, 16, 2.5, 0.4, 41e3); }
+inline double mfma8_direct32_time(int M, int N, int K) { return mfma8_time(M, N, K, 32, 32, 2.5, 0.8, 44e3); }
+inline double mfma8_staged64_time(int M, int N, int K) { return mfma8_time(M, N, K, 64, 64, 3.0, 0.4, 45e3); }
+inline double mfma8_staged128_time(int M, int N, int K) { return mfma8_time(M, N, K, 128, 128, 4.0, 2.5, 39e3); }
+inline double mfma8_ring_time(int M, int N, int K, int tile)
+{
+   return tile >= 128 ? mfma8_time(M, N, K, 128, 128, 3.5, 3.4, 67e3) : mfma8_time(M, N, K, 64, 64, 2.9, 0.6, 75e3);
+}
+
+// The general loop (any alignment, B either way); BSRC says how B is stored.
+template <class MMA, class BSRC, class EPI>
+static int launch_mfma8_general(const LaunchCfg &lc, const int8_t *A, int lda, const BSRC &B, int M, int N, int K, const EPI &ep)
+{
+   const bool wide = lc.tile == 64 ? false : lc.tile >= 128 ? true : mfma8_staged128_time(M, N, K) < mfma8_staged64_time(M, N, K);
+   if (wide)
+      return launch_mfma8_staged<MMA, 128, 128, 128, 4, 2, 2, BSRC, EPI>(lc, A, lda, B, M, N, K, ep);
+   return launch_mfma8_staged<MMA, 64, 64, 128, 2, 2, 2, BSRC, EPI>(lc, A, lda, B, M, N, K, ep);
+}
+
+// Chooses between the direct kernel (few rows or tiles, short rows), the pipelined kernels (aligned operands, K a multiple of 64) and the general one.
 // `variant` selects a tuning alternative of the pipelined kernel (0 = default); -1 forces the general kernel.
 template <class MMA, class EPI>
 static int launch_mfma8_best(const LaunchCfg &lc, const int8_t *A, const int8_t *Bt, int M, int N, int K, int lda, int ldb,
                              const EPI &ep)
 {
    const int force_tile = lc.tile, variant = lc.variant;
+   typedef std::conditional_t<(MMA::KSTEP * 2 <= 64), DirectI8, DirectF8> Direct;
    const bool aligned = (lda % 16 == 0) && (ldb % 16 == 0) && (((uintptr_t)A & 15) == 0) && (((uintptr_t)Bt & 15) == 0);
-   if (variant < 0 || !aligned || K < 64 || K % 64 != 0)
-      return launch_mfma8_auto<MMA, EPI>(lc, A, Bt, M, N, K, lda, ldb, ep);
+   const bool ring = variant >= 0 && aligned && K >= 64 && K % 64 == 0 && (MMA::KSTEP * 2 <= 64 || K % 128 == 0);
+   const double t16 = mfma8_direct16_time(M, N, K), t32 = mfma8_direct32_time(M, N, K);
+   const double others = ring ? mfma8_ring_time(M, N, K, pick_tile(M, N, 0)) : std::min(mfma8_staged64_time(M, N, K), mfma8_staged128_time(M, N, K));
+   if (force_tile == 16 || K < 16 || (!force_tile && variant == 0 && t16 <= t32 && t16 < others))
+      return launch_mfma8_direct<Direct, 1, 1, 8, 4, EPI>(lc, A, Bt, M, N, K, lda, ldb, ep);
+   if (force_tile == 32 || (!force_tile && variant == 0 && t32 < others))
+      return launch_mfma8_direct<Direct, 2, 2, 8, 2, EPI>(lc, A, Bt, M, N, K, lda, ldb, ep);
+   if (!ring)
+      return launch_mfma8_general<MMA, StagedRows, EPI>(lc, A, lda, StagedRows{Bt, ldb, N}, M, N, K, ep);
    const int tile = pick_tile(M, N, force_tile);
    const bool k128 = (K % 128 == 0);
    if constexpr (MMA::KSTEP * 2 <= 64) {
@@ -29,9 +70,7 @@ static int launch_mfma8_best(const LaunchCfg &lc, const int8_t *A, const int8_t 
          return launch_mfma8_dma_src<MMA, 256, 128, 64, 2, 2, 3, EPI, RowMajorRows, 2>(lc, RowMajorRows{A, lda}, Bt, M, N, K, ldb, ep);
    }
    if constexpr (MMA::KSTEP * 2 > 64) {
-      // two K-steps per slab are the minimum: a 64-byte K-step needs 128-byte slabs
-      if (!k128)
-         return launch_mfma8_auto<MMA, EPI>(lc, A, Bt, M, N, K, lda, ldb, ep);
+      // two K-steps per slab are the minimum: a 64-byte K-step needs 128-byte slabs, which `ring` has made sure of
       if ((force_tile == 512 || (!force_tile && variant == 0 && tile == 256)) && mfma8_persist_applies(A, Bt, M, N, K, lda, ldb, ep.elements_per_16_bytes()) &&
           ep.stores_plain_rows())
          return launch_mfma8_persist<MMA, EPI>(lc, A, Bt, M, N, K, lda, ldb, ep);
@@ -61,6 +100,19 @@ static int launch_mfma8_best(const LaunchCfg &lc, const int8_t *A, const int8_t 
       default: return fail(SOFIE_HIP_ERR_INVALID, "gemm: unknown tile %d", tile);
       }
    }
+}
+
+// Whether a product whose B is stored [K,N] is better off with the general loop, which transposes B on its way into LDS, than
+// with a launch that re-lays B out and the kernels above: that launch takes about 2 us and 4.2 TB/s for the bytes it moves.
+static bool mfma8_columns_preferred(const LaunchCfg &lc, int M, int N, int K, bool aligned_behind)
+{
+   if (K < 16 || N < 16 || lc.tile == 16 || lc.tile == 32)
+      return false;
+   const double staged = std::min(mfma8_staged64_time(M, N, K), mfma8_staged128_time(M, N, K));
+   double behind = std::min(std::min(mfma8_direct16_time(M, N, K), mfma8_direct32_time(M, N, K)), staged);
+   if (aligned_behind && K >= 64 && K % 64 == 0)
+      behind = std::min(behind, mfma8_ring_time(M, N, K, pick_tile(M, N, 0)));
+   return lc.tile == 0 && lc.variant <= 0 && staged < 2.0 + 2.0 * K * N / 4.2e6 + behind;
 }
 
 } // namespace sofie_hip

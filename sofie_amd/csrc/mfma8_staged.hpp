@@ -1,0 +1,301 @@
+// General tile loop of the int8 and the FP8 GEMM: any K, any alignment, B stored either way.  The pipelined kernels load straight
+// into LDS, which takes rows that start on 16 bytes and a K of whole slabs; here the slabs go through registers, so that a chunk
+// may be an unaligned 16-byte load (the hardware takes any address), the last chunk of a row is cut off at K, and a B given as
+// [K,N] is transposed on its way into LDS, four bytes by four, instead of by a launch of its own.
+//
+// A workgroup owns a BM x BN tile of Y and walks K in slabs of BK bytes, DEPTH slabs of loads ahead in registers, two slabs of LDS in
+// the swizzled layout of lds_chunk_offset, one barrier per slab.  The Bt rows are the MFMA's first operand, so that a lane ends up
+// with 4 consecutive columns of one row.
+#pragma once
+#include "mfma8_direct.hpp"
+
+namespace sofie_hip {
+
+// The chunk at k of a row of K >= 16 bytes as a load inside the row: where it crosses K, the last 16 bytes of the row instead,
+// which cut_chunk moves down to k, zeros behind them.
+__device__ __forceinline__ v4i fetch_cut(const int8_t *row, int k, int K)
+{
+   return *(const v4i_unaligned *)(row + (k + 16 <= K ? k : K - 16));
+}
+__device__ __forceinline__ v4i cut_chunk(v4i v, int k, int K)
+{
+   union {
+      v4i v;
+      unsigned long long q[2];
+   } u;
+   u.v = v;
+   const int drop = (k + 16 - K) * 8; // bits that lie before k
+   if (drop > 0) {
+      const unsigned long long hi = drop >= 128 ? 0 : u.q[1];
+      u.q[0] = drop >= 64 ? hi >> (drop & 63) : (u.q[0] >> drop) | (u.q[1] << (64 - drop));
+      u.q[1] = drop >= 64 ? 0 : u.q[1] >> drop;
+   }
+   return u.v;
+}
+
+// An operand of `rows` rows that are contiguous in k.
+struct StagedRows {
+   static constexpr bool kTransposed = false;
+   const int8_t *base;
+   int ld, rows;
+};
+// An operand stored [K][rows]: contiguous along the rows.
+struct StagedColumns {
+   static constexpr bool kTransposed = true;
+   const int8_t *base;
+   int ld, rows;
+};
+
+// A slab of R rows x BK bytes on its way from memory to LDS: what one of NTHREADS threads carries.
+template <class SRC, int R, int BK, int NTHREADS>
+struct StagedSlab {
+   static constexpr int CPR = BK / 16;
+   static constexpr int LD = R * CPR / NTHREADS; // 16-byte chunks per thread: chunk t + i * NTHREADS of the slab, row by row
+   static_assert(R * CPR % NTHREADS == 0, "the slab divides over the threads");
+   v4i v[LD];
+   static __device__ __forceinline__ const int8_t *row_of(const SRC &s, int r0, int i, int t)
+   {
+      const int r = r0 + (t + i * NTHREADS) / CPR;
+      return s.base + (size_t)(r < s.rows ? r : s.rows - 1) * (size_t)s.ld; // rows past the edge re-read the last one
+   }
+   static __device__ __forceinline__ int k_of(int k0, int i, int t) { return k0 + (t + i * NTHREADS) % CPR * 16; }
+   // a slab that lies before K
+   __device__ __forceinline__ void load(const SRC &s, int r0, int k0, int, int t)
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i)
+         v[i] = *(const v4i_unaligned *)(row_of(s, r0, i, t) + k_of(k0, i, t));
+   }
+   // the slab that K cuts off: fetched as whole chunks of the row, cut later
+   __device__ __forceinline__ void load_last(const SRC &s, int r0, int k0, int K, int t)
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i)
+         v[i] = fetch_cut(row_of(s, r0, i, t), k_of(k0, i, t), K);
+   }
+   __device__ __forceinline__ void finish_last(int k0, int K, int t)
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i)
+         v[i] = cut_chunk(v[i], k_of(k0, i, t), K);
+   }
+   __device__ __forceinline__ void store(int8_t *lds, int t) const
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i) {
+         const int id = t + i * NTHREADS;
+         *(v4i *)(lds + lds_chunk_offset<BK>(id / CPR, id % CPR)) = v[i];
+      }
+   }
+};
+
+// four bytes each of the k neighbours r0..r3 -> four k bytes of each of four rows
+__device__ __forceinline__ void transpose_4x4_bytes(unsigned r0, unsigned r1, unsigned r2, unsigned r3, unsigned (&out)[4])
+{
+   const unsigned a = __builtin_amdgcn_perm(r1, r0, 0x05010400u), b = __builtin_amdgcn_perm(r1, r0, 0x07030602u);
+   const unsigned c = __builtin_amdgcn_perm(r3, r2, 0x05010400u), d = __builtin_amdgcn_perm(r3, r2, 0x07030602u);
+   out[0] = __builtin_amdgcn_perm(c, a, 0x05040100u);
+   out[1] = __builtin_amdgcn_perm(c, a, 0x07060302u);
+   out[2] = __builtin_amdgcn_perm(d, b, 0x05040100u);
+   out[3] = __builtin_amdgcn_perm(d, b, 0x07060302u);
+}
+
+template <int R, int BK, int NTHREADS>
+struct StagedSlab<StagedColumns, R, BK, NTHREADS> {
+   // a thread carries blocks of 4 k of 8 rows: four 8-byte pieces, one per k
+   static constexpr int RB = R / 8; // blocks along the rows
+   static constexpr int LD = RB * (BK / 4) / NTHREADS;
+   static_assert(RB * (BK / 4) % NTHREADS == 0, "the slab divides over the threads");
+   typedef unsigned long long piece_t;
+   typedef piece_t piece_unaligned_t __attribute__((aligned(1)));
+   piece_t v[LD][4];
+   static __device__ __forceinline__ int row_of(int i, int t) { return (t + i * NTHREADS) % RB * 8; }
+   static __device__ __forceinline__ int k_of(int i, int t) { return (t + i * NTHREADS) / RB * 4; }
+   // pieces past the last column are fetched from the last 8 columns (align_edge moves them), k past K from the last k (finish_last)
+   __device__ __forceinline__ void load_last(const StagedColumns &s, int r0, int k0, int K, int t)
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i) {
+         const int r = r0 + row_of(i, t), k = k0 + k_of(i, t);
+#pragma unroll
+         for (int j = 0; j < 4; ++j)
+            v[i][j] = *(const piece_unaligned_t *)(s.base + (size_t)(k + j < K ? k + j : K - 1) * (size_t)s.ld + (r + 8 <= s.rows ? r : s.rows - 8));
+      }
+   }
+   __device__ __forceinline__ void load(const StagedColumns &s, int r0, int k0, int K, int t)
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i) {
+         const int r = r0 + row_of(i, t);
+         const int8_t *p = s.base + (size_t)(k0 + k_of(i, t)) * (size_t)s.ld + (r + 8 <= s.rows ? r : s.rows - 8);
+#pragma unroll
+         for (int j = 0; j < 4; ++j)
+            v[i][j] = *(const piece_unaligned_t *)(p + (size_t)j * (size_t)s.ld);
+      }
+   }
+   __device__ __forceinline__ void finish_last(int k0, int K, int t)
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i)
+#pragma unroll
+         for (int j = 0; j < 4; ++j)
+            if (k0 + k_of(i, t) + j >= K)
+               v[i][j] = 0;
+   }
+   __device__ __forceinline__ void align_edge(const StagedColumns &s, int r0, int t)
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i) {
+         const int drop = (r0 + row_of(i, t) + 8 - s.rows) * 8; // bits that lie before the piece's first row
+#pragma unroll
+         for (int j = 0; j < 4; ++j)
+            v[i][j] = drop <= 0 ? v[i][j] : drop >= 64 ? 0 : v[i][j] >> drop;
+      }
+   }
+   __device__ __forceinline__ void store(int8_t *lds, int t) const
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i) {
+         const int r = row_of(i, t), k = k_of(i, t);
+#pragma unroll
+         for (int q = 0; q < 2; ++q) {
+            unsigned w[4];
+            transpose_4x4_bytes((unsigned)(v[i][0] >> (32 * q)), (unsigned)(v[i][1] >> (32 * q)), (unsigned)(v[i][2] >> (32 * q)), (unsigned)(v[i][3] >> (32 * q)), w);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+               *(unsigned *)(lds + lds_chunk_offset<BK>(r + 4 * q + e, k / 16) + k % 16) = w[e];
+         }
+      }
+   }
+};
+
+template <class MMA, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int DEPTH, class BSRC, class EPI>
+__global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void mfma8_staged_kernel(StagedRows A, BSRC B, int M, int N, int K, EPI ep, int tiles_m, int tiles_n, int sw)
+{
+   constexpr int NTHREADS = WAVES_M * WAVES_N * 64;
+   constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N, MT = TM / 32, NT = TN / 32;
+   constexpr int STAGE = (BM + BN) * BK;
+   static_assert(TM % 32 == 0 && TN % 32 == 0 && BK % MMA::KSTEP == 0, "wave tile of 32 x 32 blocks, slab of whole steps");
+   static_assert(DEPTH % 2 == 0, "the LDS slot of a slab follows from its place in the unrolled group");
+   typedef typename MMA::acc_t acc_t;
+   typedef typename MMA::frag_t frag_t;
+   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
+
+   int tm, tn;
+   tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, sw, tm, tn);
+   const int m0 = tm * BM, n0 = tn * BN;
+   const int t = threadIdx.x, lane = t & 63;
+   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+   const int lr = lane & 31, lk = lane >> 5;
+
+   acc_t acc[MT][NT];
+#pragma unroll
+   for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+         for (int v = 0; v < 16; ++v)
+            acc[i][j][v] = 0;
+
+   typedef StagedSlab<StagedRows, BM, BK, NTHREADS> SA;
+   typedef StagedSlab<BSRC, BN, BK, NTHREADS> SB;
+   const int whole = K / BK; // slabs that lie before K
+   const bool at_edge = BSRC::kTransposed && n0 + BN > N;
+   auto multiply = [&](const int8_t *cA, const int8_t *cB) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+#pragma unroll
+      for (int ks = 0; ks < BK / MMA::KSTEP; ++ks) {
+         frag_t fa[MT], fb[NT];
+#pragma unroll
+         for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int c = 0; c < MMA::CHUNKS; ++c)
+               fb[j].c[c] = *(const v4i *)(cB + lds_chunk_offset<BK>(wn * TN + j * 32 + lr, (ks * 2 + lk) * MMA::CHUNKS + c));
+#pragma unroll
+         for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int c = 0; c < MMA::CHUNKS; ++c)
+               fa[i].c[c] = *(const v4i *)(cA + lds_chunk_offset<BK>(wm * TM + i * 32 + lr, (ks * 2 + lk) * MMA::CHUNKS + c));
+#pragma unroll
+         for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+               acc[i][j] = MMA::mma(fb[j], fa[i], acc[i][j]);
+      }
+   };
+   // The slab that K cuts off comes first (the order of the slabs does not matter), its chunks fetched ahead of the others.
+   SA last_a;
+   SB last_b;
+   if (whole * BK < K) {
+      last_a.load_last(A, m0, whole * BK, K, t);
+      last_b.load_last(B, n0, whole * BK, K, t);
+   }
+   SA sa[DEPTH];
+   SB sb[DEPTH];
+   // a slab past the end is asked for as the last one again: no branch stands between a load and the wait for it
+   auto load = [&](int kt, auto dc) {
+      constexpr int d = decltype(dc)::value;
+      const int k0 = (kt < whole ? kt : whole - 1) * BK;
+      sa[d].load(A, m0, k0, K, t);
+      sb[d].load(B, n0, k0, K, t);
+   };
+   if (whole > 0)
+      static_for<DEPTH>([&](auto dc) { load(decltype(dc)::value, dc); });
+   if (whole * BK < K) {
+      last_a.finish_last(whole * BK, K, t);
+      if constexpr (BSRC::kTransposed)
+         last_b.align_edge(B, n0, t);
+      last_b.finish_last(whole * BK, K, t);
+      last_a.store(smem + STAGE, t);
+      last_b.store(smem + STAGE + BM * BK, t);
+      multiply(smem + STAGE, smem + STAGE + BM * BK);
+   }
+   auto step = [&](int kt, auto dc, auto more) {
+      constexpr int d = decltype(dc)::value;
+      int8_t *cA = smem + (d & 1) * STAGE, *cB = cA + BM * BK;
+      // this slot was read two slabs ago: the barrier of the slab in between has seen every wave done with it
+      sa[d].store(cA, t);
+      if constexpr (BSRC::kTransposed)
+         if (at_edge)
+            sb[d].align_edge(B, n0, t);
+      sb[d].store(cB, t);
+      if constexpr (decltype(more)::value)
+         load(kt + DEPTH, dc);
+      multiply(cA, cB);
+   };
+   int kt = 0;
+   for (; kt + DEPTH < whole; kt += DEPTH)
+      static_for<DEPTH>([&](auto dc) { step(kt + decltype(dc)::value, dc, std::true_type{}); });
+   static_for<DEPTH>([&](auto dc) {
+      if (kt + decltype(dc)::value < whole)
+         step(kt + decltype(dc)::value, dc, std::false_type{});
+   });
+
+   __syncthreads(); // the slabs are dead: the tile store reuses LDS, one region per wave
+   char *wsm = (char *)smem + wave * tile_store_lds_bytes(TN);
+   ep.dispatch([&](auto mode) {
+      tile_store_via_lds<decltype(mode)::value, MT, NT>(ep, acc, m0 + wm * TM, n0 + wn * TN, M, N, lane, wsm);
+   });
+}
+
+template <class MMA, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int DEPTH, class BSRC, class EPI>
+static int launch_mfma8_staged(const LaunchCfg &lc, const int8_t *A, int lda, const BSRC &B, int M, int N, int K, const EPI &ep)
+{
+   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+   const long long nwg = (long long)tiles_m * tiles_n;
+   if (nwg > 0x7fffffffLL)
+      return fail(SOFIE_HIP_ERR_INVALID, "gemm: too many tiles");
+   constexpr size_t slabs = 2 * (size_t)(BM + BN) * BK, store = (size_t)WAVES_M * WAVES_N * tile_store_lds_bytes(BN / WAVES_N);
+   constexpr size_t smem = slabs > store ? slabs : store;
+   auto kern = mfma8_staged_kernel<MMA, BM, BN, BK, WAVES_M, WAVES_N, DEPTH, BSRC, EPI>;
+   static bool configured[64] = {};
+   if (int st = configure_lds_once(kern, smem, configured))
+      return st;
+   hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(WAVES_M * WAVES_N * 64), smem, lc.stream, StagedRows{A, lda, M}, B, M, N, K, ep, tiles_m, tiles_n, lc.swizzle);
+   return launch_status("mfma8_staged_kernel");
+}
+
+} // namespace sofie_hip
