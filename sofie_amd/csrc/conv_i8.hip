@@ -315,7 +315,7 @@ int sofie_hip_conv_i8(sofie_hip_ctx *ctx, const sofie_conv_desc *d, const sofie_
          ep.nchw_ohw = (a->y_layout == SOFIE_LAYOUT_NHWC || plane_sums) ? 0 : OHW;
          ep.rows_per_plane = plane_sums ? OHW : 0;
          ep.Y = a->Y;
-         if (!nhwc && d->stride_w == 1 && d->dil_w == 1) {
+         if (!nhwc && d->dil_w == 1) {
             FewChannelConv fc;
             fc.X = src.X;
             fc.H = d->H; fc.W = d->W; fc.OH = g.OH; fc.OW = g.OW;
@@ -323,9 +323,17 @@ int sofie_hip_conv_i8(sofie_hip_ctx *ctx, const sofie_conv_desc *d, const sofie_
             fc.kh = d->kh; fc.kw = d->kw; fc.Cg = g.Cg;
             fc.img_stride = src.img_stride;
             bool taken = false;
-            st = conv_i8_few_channels(launch_cfg_i8(ctx), fc, Wp + (size_t)grp * Cout_g * g.Kp, (int)rows, Cout_g, g.Kp, ep, &taken);
-            if (st)
-               return st;
+            const int8_t *Wg = Wp + (size_t)grp * Cout_g * g.Kp;
+            if (d->stride_w == 1) {
+               st = conv_i8_few_channels(launch_cfg_i8(ctx), fc, Wg, (int)rows, Cout_g, g.Kp, ep, &taken);
+               if (st)
+                  return st;
+            }
+            if (!taken) {
+               st = conv_i8_windows(launch_cfg_i8(ctx), fc, d->stride_w, Wg, (int)rows, Cout_g, g.Kp, ep, &taken);
+               if (st)
+                  return st;
+            }
             if (taken)
                continue;
          }
@@ -336,6 +344,43 @@ int sofie_hip_conv_i8(sofie_hip_ctx *ctx, const sofie_conv_desc *d, const sofie_
       return SOFIE_HIP_OK;
    }
    SOFIE_HIP_REQUIRE(!plane_sums, "sofie_hip_conv_i8: plane sums need 16-byte aligned activations and weights");
+   // Other NHWC layers whose channels divide into pieces of 8 or 16 bytes: the general GEMM loop gathers the pieces on their way into
+   // LDS (the column matrix of a 3x3 layer is nine times its input, written and read back).  32-bit offsets as above.
+   {
+      const long long rows = (long long)d->N * OHW;
+      const long long reach = (long long)d->N * d->H * d->W * d->C + (long long)(d->pad_h0 + d->kh * d->dil_h + 1) * d->W * d->C + (long long)(d->pad_w0 + d->kw * d->dil_w + 1) * d->C;
+      const int piece = g.Cg % 16 == 0 ? 16 : 8;
+      if (!column_matrix_by_option && launch_cfg_i8(ctx).variant == 0 && a->x_layout == SOFIE_LAYOUT_NHWC && g.Cg % piece == 0 && d->C % piece == 0 &&
+          ((uintptr_t)a->X % piece) == 0 && reach < (1LL << 31) && rows < (1LL << 31) && g.Kp >= 16 && (g.K + 256LL) * (g.Cg > d->kw ? g.Cg : d->kw) < (1LL << 31)) {
+         for (int grp = 0; grp < d->group; ++grp) {
+            ConvRows src{};
+            src.X = a->X + (size_t)grp * g.Cg;
+            src.H = d->H; src.W = d->W; src.C = d->C; src.OH = g.OH; src.OW = g.OW;
+            src.stride_h = d->stride_h; src.stride_w = d->stride_w; src.pad_h0 = d->pad_h0; src.pad_w0 = d->pad_w0;
+            src.dil_h = d->dil_h; src.dil_w = d->dil_w; src.kw = d->kw;
+            auto recip64 = [](unsigned v) -> unsigned long long { return v <= 1 ? 0ull : (~0ull / v) + 1; };
+            src.ohw_mul = recip64((unsigned)OHW);
+            src.ow_mul = recip64((unsigned)g.OW);
+            I8Epilogue ep;
+            ep.bias = a->bias;
+            ep.scale = a->scale;
+            ep.scale_scalar = 1.0f;
+            ep.q_scale = 1.0f;
+            ep.relu_acc = (out_kind == SOFIE_I8OUT_I32) ? a->relu : 0;
+            ep.relu_out = (out_kind == SOFIE_I8OUT_I32) ? 0 : a->relu;
+            ep.out = out_kind;
+            ep.ldy = d->Cout;
+            ep.N = Cout_g;
+            ep.n_offset = grp * Cout_g;
+            ep.nchw_ohw = a->y_layout == SOFIE_LAYOUT_NHWC ? 0 : OHW;
+            ep.Y = a->Y;
+            st = conv_i8_staged(launch_cfg_i8(ctx), src, g.Cg, Wp + (size_t)grp * Cout_g * g.Kp, (int)rows, Cout_g, g.K, g.Kp, ep);
+            if (st)
+               return st;
+         }
+         return SOFIE_HIP_OK;
+      }
+   }
    const size_t per_image = (size_t)OHW * g.Kp;
    SOFIE_HIP_REQUIRE(ws != nullptr && ws_left >= per_image,
                      "sofie_hip_conv_i8: the activations are not 16-byte aligned; a workspace of %zu bytes is needed for the column matrix",

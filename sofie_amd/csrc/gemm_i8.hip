@@ -1,7 +1,7 @@
 // int8 x int8 -> int32 GEMM on the gfx950 matrix cores (v_mfma_i32_32x32x32_i8) with the
 // requantisation / dequantisation epilogue fused into the store, and the int8 re-layout kernel.
 #include "i8_epilogue.hpp"
-#include "conv_i8_few_channels.hpp"
+#include "conv_i8_windows.hpp"
 #include <cmath>
 #include <mutex>
 
@@ -18,9 +18,9 @@ __global__ __launch_bounds__(256) void transpose_i8_kernel(int8_t *__restrict__ 
    const StagedColumns s{src, ld_src, cols};
    StagedSlab<StagedColumns, 64, 128, 256> slab;
    if (r0 + 128 <= rows)
-      slab.load(s, c0, r0, rows, t);
+      slab.load(s, {}, c0, r0, rows, t);
    else
-      slab.load_last(s, c0, r0, rows, t);
+      slab.load_last(s, {}, c0, r0, rows, t);
    if (c0 + 64 > cols)
       slab.align_edge(s, c0, t);
    slab.store(tile, t);
@@ -81,6 +81,34 @@ int conv_i8_gather(const LaunchCfg &lc, const GatherConvRows &src, const int8_t 
 {
    derive_epilogue_fields(ep, N);
    return launch_mfma8_gather<I8Epilogue>(lc, src, Wp, M, N, Kp, ep);
+}
+
+int conv_i8_staged(const LaunchCfg &lc, const ConvRows &g, int Cg, const int8_t *Wp, int M, int N, int K, int Kp, I8Epilogue ep)
+{
+   derive_epilogue_fields(ep, N);
+   auto go = [&](auto src) {
+      src.X = g.X;
+      src.rows = M;
+      src.H = g.H, src.W = g.W, src.C = g.C, src.OH = g.OH, src.OW = g.OW;
+      src.stride_h = g.stride_h, src.stride_w = g.stride_w, src.pad_h0 = g.pad_h0, src.pad_w0 = g.pad_w0, src.dil_h = g.dil_h, src.dil_w = g.dil_w;
+      src.kw = g.kw;
+      src.Cg = Cg;
+      src.K = K;
+      src.cg_mul = (unsigned)(((1ull << 31) + Cg - 1) / (unsigned)Cg);
+      src.kw_mul = (unsigned)(((1ull << 31) + g.kw - 1) / (unsigned)g.kw);
+      src.ohw_mul = g.ohw_mul, src.ow_mul = g.ow_mul;
+      return launch_mfma8_general<MfmaI8, decltype(src), StagedRows, I8Epilogue>(lc, src, StagedRows{Wp, Kp, N}, M, N, Kp, ep);
+   };
+   if (Cg % 16 == 0)
+      return go(StagedConvRows<16>{});
+   return go(StagedConvRows<8>{});
+}
+
+int conv_i8_windows(const LaunchCfg &lc, const FewChannelConv &src, int stride_w, const int8_t *Wp, int M, int N, int Kp, I8Epilogue ep, bool *taken)
+{
+   derive_epilogue_fields(ep, N);
+   *taken = lc.tile == 0 && lc.variant == 0 && ep.rows_per_plane == 0 && conv_i8_windows_applies(src, N);
+   return *taken ? launch_conv_i8_windows<I8Epilogue>(lc, src, stride_w, Wp, M, N, Kp, ep) : SOFIE_HIP_OK;
 }
 
 int conv_i8_few_channels(const LaunchCfg &lc, const FewChannelConv &src, const int8_t *Wp, int M, int N, int Kp, I8Epilogue ep, bool *taken)
@@ -187,7 +215,7 @@ static int gemm_i8_with_workspace(sofie_hip_ctx *ctx, const sofie_gemm_i8_desc *
       SOFIE_HIP_REQUIRE(((uintptr_t)ws & 255) == 0, "sofie_hip_gemm_i8: workspace must be 256-byte aligned");
       if (!d->transA && mfma8_columns_preferred(launch_cfg_i8(ctx), M, N, K, K % 16 == 0 && lda % 16 == 0 && ((uintptr_t)A & 15) == 0)) {
          derive_epilogue_fields(ep, N);
-         return launch_mfma8_general<MfmaI8, StagedColumns, I8Epilogue>(launch_cfg_i8(ctx), A, lda, StagedColumns{d->B, ldb, N}, M, N, K, ep);
+         return launch_mfma8_general<MfmaI8, StagedRows, StagedColumns, I8Epilogue>(launch_cfg_i8(ctx), StagedRows{A, lda, M}, StagedColumns{d->B, ldb, N}, M, N, K, ep);
       }
       int st = transpose_i8(ctx->stream, (int8_t *)ws, d->B, K, N, ldb, K);
       if (st)

@@ -333,6 +333,11 @@ int conv_i8_gather(const LaunchCfg &lc, const GatherConvRows &src, const int8_t 
 // The same for NCHW input with stride and dilation 1 in x, 64 output channels and rows stored as they are: windows of four
 // bytes instead of single bytes.  *taken tells whether the shape was this kernel's (else nothing was launched).
 int conv_i8_few_channels(const LaunchCfg &lc, const FewChannelConv &src, const int8_t *Wp, int M, int N, int Kp, I8Epilogue ep, bool *taken);
+// The same without those two conditions and without the one on the output; sums of planes excepted.
+int conv_i8_windows(const LaunchCfg &lc, const FewChannelConv &src, int stride_w, const int8_t *Wp, int M, int N, int Kp, I8Epilogue ep, bool *taken);
+// Convolution over NHWC input whose channels per group are a multiple of 8 (and 8- or 16-byte aligned pixels): the general loop
+// reads the activations where they lie.  K = taps * Cg, Kp = the packed weights' row length.
+int conv_i8_staged(const LaunchCfg &lc, const ConvRows &g, int Cg, const int8_t *Wp, int M, int N, int K, int Kp, I8Epilogue ep);
 // Convolution as an implicit GEMM: rows of A come from `src`, Wp is [N][K] with K = taps * Cg.
 int conv_i8_implicit(const LaunchCfg &lc, const ConvRows &src, int Cg, const int8_t *Wp, int M, int N, int K, I8Epilogue ep);
 

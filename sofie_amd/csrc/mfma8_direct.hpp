@@ -43,6 +43,36 @@ __device__ __forceinline__ v4i load_chunk_tail(const int8_t *row, int k, int K)
    return u.v;
 }
 
+// Columns n..n+3 of row m from four accumulators, as a 4-element store where the row allows it.
+template <int MODE, class EPI, class ACC>
+__device__ __forceinline__ void store_four_columns(const EPI &ep, const typename EPI::template col_params<4> &prm, const ACC &v, int m, int n, int N)
+{
+   constexpr int ESZ = EPI::template out_bytes<MODE>();
+   uint32_t w4[4];
+   ep.template pack4<MODE, 4>(prm, 0, v[0], v[1], v[2], v[3], w4);
+   if (ep.rows_vectorizable() && n + 4 <= N) {
+      char *y = ep.out_base() + ep.out_index(m, n) * ESZ;
+      if constexpr (ESZ == 1)
+         *(uint32_t *)y = w4[0];
+      else if constexpr (ESZ == 2)
+         *(uint2 *)y = make_uint2(w4[0], w4[1]);
+      else
+         *(uint4 *)y = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+   } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+         if (n + i < N) {
+            char *y = ep.out_base() + ep.out_index(m, n + i) * ESZ;
+            if constexpr (ESZ == 1)
+               *y = (char)(w4[0] >> (8 * i));
+            else if constexpr (ESZ == 2)
+               *(uint16_t *)y = (uint16_t)(w4[i / 2] >> (16 * (i % 2)));
+            else
+               *(uint32_t *)y = w4[i];
+         }
+   }
+}
+
 // One step of 128 bytes of k on a 16 x 16 block: lane (lk = lane / 16, c = lane % 16) holds bytes 32 lk .. 32 lk + 31 of row c of either
 // operand.  The n side goes first, so that a lane ends up with 4 consecutive columns of one row.
 struct DirectI8 {
@@ -150,7 +180,6 @@ __global__ __launch_bounds__(W * 64) void mfma8_direct_kernel(RowMajorRows A, Ro
    __syncthreads();
    ep.dispatch([&](auto mode) {
       constexpr int MODE = decltype(mode)::value;
-      constexpr int ESZ = EPI::template out_bytes<MODE>();
 #pragma unroll 1
       for (int e = threadIdx.x; e < TM * TN / 4; e += W * 64) {
          const int r = e / (TN / 4), q = e % (TN / 4) * 4;
@@ -163,29 +192,7 @@ __global__ __launch_bounds__(W * 64) void mfma8_direct_kernel(RowMajorRows A, Ro
             continue;
          typename EPI::template col_params<4> prm;
          ep.template load_params<4>(n, prm);
-         uint32_t w4[4];
-         ep.template pack4<MODE, 4>(prm, 0, v[0], v[1], v[2], v[3], w4);
-         if (ep.rows_vectorizable() && n + 4 <= N) {
-            char *y = ep.out_base() + ep.out_index(m, n) * ESZ;
-            if constexpr (ESZ == 1)
-               *(uint32_t *)y = w4[0];
-            else if constexpr (ESZ == 2)
-               *(uint2 *)y = make_uint2(w4[0], w4[1]);
-            else
-               *(uint4 *)y = make_uint4(w4[0], w4[1], w4[2], w4[3]);
-         } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-               if (n + i < N) {
-                  char *y = ep.out_base() + ep.out_index(m, n + i) * ESZ;
-                  if constexpr (ESZ == 1)
-                     *y = (char)(w4[0] >> (8 * i));
-                  else if constexpr (ESZ == 2)
-                     *(uint16_t *)y = (uint16_t)(w4[i / 2] >> (16 * (i % 2)));
-                  else
-                     *(uint32_t *)y = w4[i];
-               }
-         }
+         store_four_columns<MODE>(ep, prm, v, m, n, N);
       }
    });
 }

@@ -27,14 +27,14 @@ inline double mfma8_ring_time(int M, int N, int K, int tile)
    return tile >= 128 ? mfma8_time(M, N, K, 128, 128, 3.5, 3.4, 67e3) : mfma8_time(M, N, K, 64, 64, 2.9, 0.6, 75e3);
 }
 
-// The general loop (any alignment, B either way); BSRC says how B is stored.
-template <class MMA, class BSRC, class EPI>
-static int launch_mfma8_general(const LaunchCfg &lc, const int8_t *A, int lda, const BSRC &B, int M, int N, int K, const EPI &ep)
+// The general loop (any alignment, a convolution's input or plain rows, B either way).
+template <class MMA, class ASRC, class BSRC, class EPI>
+static int launch_mfma8_general(const LaunchCfg &lc, const ASRC &A, const BSRC &B, int M, int N, int K, const EPI &ep)
 {
    const bool wide = lc.tile == 64 ? false : lc.tile >= 128 ? true : mfma8_staged128_time(M, N, K) < mfma8_staged64_time(M, N, K);
    if (wide)
-      return launch_mfma8_staged<MMA, 128, 128, 128, 4, 2, 2, BSRC, EPI>(lc, A, lda, B, M, N, K, ep);
-   return launch_mfma8_staged<MMA, 64, 64, 128, 2, 2, 2, BSRC, EPI>(lc, A, lda, B, M, N, K, ep);
+      return launch_mfma8_staged<MMA, 128, 128, 128, 4, 2, 2, ASRC, BSRC, EPI>(lc, A, B, M, N, K, ep);
+   return launch_mfma8_staged<MMA, 64, 64, 128, 2, 2, 2, ASRC, BSRC, EPI>(lc, A, B, M, N, K, ep);
 }
 
 // Chooses between the direct kernel (few rows or tiles, short rows), the pipelined kernels (aligned operands, K a multiple of 64) and the general one.
@@ -54,7 +54,7 @@ static int launch_mfma8_best(const LaunchCfg &lc, const int8_t *A, const int8_t 
    if (force_tile == 32 || (!force_tile && variant == 0 && t32 < others))
       return launch_mfma8_direct<Direct, 2, 2, 8, 2, EPI>(lc, A, Bt, M, N, K, lda, ldb, ep);
    if (!ring)
-      return launch_mfma8_general<MMA, StagedRows, EPI>(lc, A, lda, StagedRows{Bt, ldb, N}, M, N, K, ep);
+      return launch_mfma8_general<MMA, StagedRows, StagedRows, EPI>(lc, StagedRows{A, lda, M}, StagedRows{Bt, ldb, N}, M, N, K, ep);
    const int tile = pick_tile(M, N, force_tile);
    const bool k128 = (K % 128 == 0);
    if constexpr (MMA::KSTEP * 2 <= 64) {

@@ -46,9 +46,24 @@ struct StagedColumns {
    int ld, rows;
 };
 
+// A convolution input that is never laid out as a matrix: row m is the output pixel (image, oh, ow), k = tap * Cg + channel, read from the
+// NHWC activation tensor in pieces of PIECE bytes that lie inside one tap (PIECE divides the channels per group).  For layers whose
+// channels are no power of two of 64 or more (ConvRows serves those): 16, 24, 32, 48 ...
+template <int PIECE_>
+struct StagedConvRows {
+   static constexpr bool kTransposed = false;
+   static constexpr int PIECE = PIECE_;
+   const int8_t *X; // first channel of the group
+   int rows, H, W, C, OH, OW, stride_h, stride_w, pad_h0, pad_w0, dil_h, dil_w, kw, Cg, K;
+   unsigned cg_mul, kw_mul; // ceil(2^31 / extent): k / extent == umulhi(2 k, mul) while k * extent < 2^31 (checked on the host)
+   unsigned long long ohw_mul, ow_mul; // see ConvRows
+};
+
 // A slab of R rows x BK bytes on its way from memory to LDS: what one of NTHREADS threads carries.
 template <class SRC, int R, int BK, int NTHREADS>
 struct StagedSlab {
+   struct places {}; // what a thread works out once about its rows
+   static __device__ __forceinline__ void find(const SRC &, int, int, places &) {}
    static constexpr int CPR = BK / 16;
    static constexpr int LD = R * CPR / NTHREADS; // 16-byte chunks per thread: chunk t + i * NTHREADS of the slab, row by row
    static_assert(R * CPR % NTHREADS == 0, "the slab divides over the threads");
@@ -60,14 +75,14 @@ struct StagedSlab {
    }
    static __device__ __forceinline__ int k_of(int k0, int i, int t) { return k0 + (t + i * NTHREADS) % CPR * 16; }
    // a slab that lies before K
-   __device__ __forceinline__ void load(const SRC &s, int r0, int k0, int, int t)
+   __device__ __forceinline__ void load(const SRC &s, const places &, int r0, int k0, int, int t)
    {
 #pragma unroll
       for (int i = 0; i < LD; ++i)
          v[i] = *(const v4i_unaligned *)(row_of(s, r0, i, t) + k_of(k0, i, t));
    }
    // the slab that K cuts off: fetched as whole chunks of the row, cut later
-   __device__ __forceinline__ void load_last(const SRC &s, int r0, int k0, int K, int t)
+   __device__ __forceinline__ void load_last(const SRC &s, const places &, int r0, int k0, int K, int t)
    {
 #pragma unroll
       for (int i = 0; i < LD; ++i)
@@ -79,6 +94,64 @@ struct StagedSlab {
       for (int i = 0; i < LD; ++i)
          v[i] = cut_chunk(v[i], k_of(k0, i, t), K);
    }
+   __device__ __forceinline__ void store(int8_t *lds, int t) const
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i) {
+         const int id = t + i * NTHREADS;
+         *(v4i *)(lds + lds_chunk_offset<BK>(id / CPR, id % CPR)) = v[i];
+      }
+   }
+};
+
+template <int PIECE, int R, int BK, int NTHREADS>
+struct StagedSlab<StagedConvRows<PIECE>, R, BK, NTHREADS> {
+   typedef StagedConvRows<PIECE> SRC;
+   static constexpr int CPR = BK / 16, LD = R * CPR / NTHREADS;
+   static_assert(R * CPR % NTHREADS == 0 && NTHREADS % CPR == 0, "the slab divides over the threads");
+   typedef int piece_t __attribute__((ext_vector_type(PIECE / 4), aligned(PIECE)));
+   union chunk_t {
+      v4i v;
+      piece_t p[16 / PIECE];
+   };
+   struct places {
+      int off[LD], ih0[LD], iw0[LD]; // of channel 0 at (ih0, iw0), in bytes from X: may be negative
+   };
+   v4i v[LD];
+   static __device__ __forceinline__ void find(const SRC &s, int r0, int t, places &at)
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i) {
+         const int r = r0 + (t + i * NTHREADS) / CPR, m = r < s.rows ? r : s.rows - 1;
+         const int ohw = s.OH * s.OW;
+         const int n = s.ohw_mul ? (int)__umul64hi((unsigned long long)(unsigned)m, s.ohw_mul) : m, rem = m - n * ohw;
+         const int oh = s.ow_mul ? (int)__umul64hi((unsigned long long)(unsigned)rem, s.ow_mul) : rem, ow = rem - oh * s.OW;
+         at.ih0[i] = oh * s.stride_h - s.pad_h0;
+         at.iw0[i] = ow * s.stride_w - s.pad_w0;
+         at.off[i] = ((n * s.H + at.ih0[i]) * s.W + at.iw0[i]) * s.C;
+      }
+   }
+   __device__ __forceinline__ void load(const SRC &s, const places &at, int, int k0, int, int t)
+   {
+      // the chunk's place in the slab is the same in every load of a thread
+#pragma unroll
+      for (int q = 0; q < 16 / PIECE; ++q) {
+         const int k = k0 + t % CPR * 16 + q * PIECE;
+         const int tap = (int)__umulhi((unsigned)k * 2u, s.cg_mul), ci = k - tap * s.Cg;
+         const int ky = (int)__umulhi((unsigned)tap * 2u, s.kw_mul), kx = tap - ky * s.kw;
+         const int dy = ky * s.dil_h, dx = kx * s.dil_w, off = (dy * s.W + dx) * s.C + ci;
+#pragma unroll
+         for (int i = 0; i < LD; ++i) {
+            const bool inside = k < s.K && (unsigned)(at.ih0[i] + dy) < (unsigned)s.H && (unsigned)(at.iw0[i] + dx) < (unsigned)s.W;
+            chunk_t c;
+            c.v = v[i];
+            c.p[q] = *(const piece_t *)(inside ? s.X + (ptrdiff_t)(at.off[i] + off) : (const int8_t *)conv_zero_page);
+            v[i] = c.v;
+         }
+      }
+   }
+   __device__ __forceinline__ void load_last(const SRC &s, const places &at, int r0, int k0, int K, int t) { load(s, at, r0, k0, K, t); }
+   __device__ __forceinline__ void finish_last(int, int, int) {}
    __device__ __forceinline__ void store(int8_t *lds, int t) const
    {
 #pragma unroll
@@ -109,10 +182,12 @@ struct StagedSlab<StagedColumns, R, BK, NTHREADS> {
    typedef unsigned long long piece_t;
    typedef piece_t piece_unaligned_t __attribute__((aligned(1)));
    piece_t v[LD][4];
+   struct places {};
+   static __device__ __forceinline__ void find(const StagedColumns &, int, int, places &) {}
    static __device__ __forceinline__ int row_of(int i, int t) { return (t + i * NTHREADS) % RB * 8; }
    static __device__ __forceinline__ int k_of(int i, int t) { return (t + i * NTHREADS) / RB * 4; }
    // pieces past the last column are fetched from the last 8 columns (align_edge moves them), k past K from the last k (finish_last)
-   __device__ __forceinline__ void load_last(const StagedColumns &s, int r0, int k0, int K, int t)
+   __device__ __forceinline__ void load_last(const StagedColumns &s, const places &, int r0, int k0, int K, int t)
    {
 #pragma unroll
       for (int i = 0; i < LD; ++i) {
@@ -122,7 +197,7 @@ struct StagedSlab<StagedColumns, R, BK, NTHREADS> {
             v[i][j] = *(const piece_unaligned_t *)(s.base + (size_t)(k + j < K ? k + j : K - 1) * (size_t)s.ld + (r + 8 <= s.rows ? r : s.rows - 8));
       }
    }
-   __device__ __forceinline__ void load(const StagedColumns &s, int r0, int k0, int K, int t)
+   __device__ __forceinline__ void load(const StagedColumns &s, const places &, int r0, int k0, int K, int t)
    {
 #pragma unroll
       for (int i = 0; i < LD; ++i) {
@@ -169,8 +244,8 @@ struct StagedSlab<StagedColumns, R, BK, NTHREADS> {
    }
 };
 
-template <class MMA, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int DEPTH, class BSRC, class EPI>
-__global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void mfma8_staged_kernel(StagedRows A, BSRC B, int M, int N, int K, EPI ep, int tiles_m, int tiles_n, int sw)
+template <class MMA, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int DEPTH, class ASRC, class BSRC, class EPI>
+__global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void mfma8_staged_kernel(ASRC A, BSRC B, int M, int N, int K, EPI ep, int tiles_m, int tiles_n, int sw)
 {
    constexpr int NTHREADS = WAVES_M * WAVES_N * 64;
    constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N, MT = TM / 32, NT = TN / 32;
@@ -198,7 +273,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void mfma8_staged_kernel(
          for (int v = 0; v < 16; ++v)
             acc[i][j][v] = 0;
 
-   typedef StagedSlab<StagedRows, BM, BK, NTHREADS> SA;
+   typedef StagedSlab<ASRC, BM, BK, NTHREADS> SA;
    typedef StagedSlab<BSRC, BN, BK, NTHREADS> SB;
    const int whole = K / BK; // slabs that lie before K
    const bool at_edge = BSRC::kTransposed && n0 + BN > N;
@@ -227,11 +302,15 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void mfma8_staged_kernel(
       }
    };
    // The slab that K cuts off comes first (the order of the slabs does not matter), its chunks fetched ahead of the others.
+   typename SA::places pa;
+   typename SB::places pb;
+   SA::find(A, m0, t, pa);
+   SB::find(B, n0, t, pb);
    SA last_a;
    SB last_b;
    if (whole * BK < K) {
-      last_a.load_last(A, m0, whole * BK, K, t);
-      last_b.load_last(B, n0, whole * BK, K, t);
+      last_a.load_last(A, pa, m0, whole * BK, K, t);
+      last_b.load_last(B, pb, n0, whole * BK, K, t);
    }
    SA sa[DEPTH];
    SB sb[DEPTH];
@@ -239,8 +318,8 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void mfma8_staged_kernel(
    auto load = [&](int kt, auto dc) {
       constexpr int d = decltype(dc)::value;
       const int k0 = (kt < whole ? kt : whole - 1) * BK;
-      sa[d].load(A, m0, k0, K, t);
-      sb[d].load(B, n0, k0, K, t);
+      sa[d].load(A, pa, m0, k0, K, t);
+      sb[d].load(B, pb, n0, k0, K, t);
    };
    if (whole > 0)
       static_for<DEPTH>([&](auto dc) { load(decltype(dc)::value, dc); });
@@ -281,8 +360,8 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void mfma8_staged_kernel(
    });
 }
 
-template <class MMA, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int DEPTH, class BSRC, class EPI>
-static int launch_mfma8_staged(const LaunchCfg &lc, const int8_t *A, int lda, const BSRC &B, int M, int N, int K, const EPI &ep)
+template <class MMA, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int DEPTH, class ASRC, class BSRC, class EPI>
+static int launch_mfma8_staged(const LaunchCfg &lc, const ASRC &A, const BSRC &B, int M, int N, int K, const EPI &ep)
 {
    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
    const long long nwg = (long long)tiles_m * tiles_n;
@@ -290,11 +369,11 @@ static int launch_mfma8_staged(const LaunchCfg &lc, const int8_t *A, int lda, co
       return fail(SOFIE_HIP_ERR_INVALID, "gemm: too many tiles");
    constexpr size_t slabs = 2 * (size_t)(BM + BN) * BK, store = (size_t)WAVES_M * WAVES_N * tile_store_lds_bytes(BN / WAVES_N);
    constexpr size_t smem = slabs > store ? slabs : store;
-   auto kern = mfma8_staged_kernel<MMA, BM, BN, BK, WAVES_M, WAVES_N, DEPTH, BSRC, EPI>;
+   auto kern = mfma8_staged_kernel<MMA, BM, BN, BK, WAVES_M, WAVES_N, DEPTH, ASRC, BSRC, EPI>;
    static bool configured[64] = {};
    if (int st = configure_lds_once(kern, smem, configured))
       return st;
-   hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(WAVES_M * WAVES_N * 64), smem, lc.stream, StagedRows{A, lda, M}, B, M, N, K, ep, tiles_m, tiles_n, lc.swizzle);
+   hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(WAVES_M * WAVES_N * 64), smem, lc.stream, A, B, M, N, K, ep, tiles_m, tiles_n, lc.swizzle);
    return launch_status("mfma8_staged_kernel");
 }
 
