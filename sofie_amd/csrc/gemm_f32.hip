@@ -140,7 +140,7 @@ namespace sofie_hip {
 // need over 256 CUs.  The direct kernel costs a launch and a trip to memory per 512 k (2.0 and 1.35 us), or the 9.4 TB/s at which
 // its fragments, which nothing shares, arrive.
 enum F32Tile { F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
-static int pick_f32_tile(int M, int N, int K, int batch)
+static int pick_f32_tile(int M, int N, int K, int batch, double *time_us = nullptr)
 {
    auto tiles = [&](int bm, int bn) { return (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
    auto tiled = [&](int bm, int bn, double rate, double fixed) {
@@ -158,6 +158,8 @@ static int pick_f32_tile(int M, int N, int K, int batch)
    offer(F32_TILE_64x32, tiled(64, 32, 0.70, 4.6));
    offer(F32_TILE_64, tiled(64, 64, 0.78, 5.0));
    offer(F32_TILE_128, tiled(128, 128, 0.84, 5.5));
+   if (time_us)
+      *time_us = least;
    return best;
 }
 // The same for a convolution, whose tiles carry the arithmetic of the gather: 0.62 of the matrix rate in the loop and 0.7 us per
@@ -166,9 +168,11 @@ static int pick_f32_tile(int M, int N, int K, int batch)
 static int pick_f32_conv_tile(int M, int N, int K, int group)
 {
    auto tiles = [&](int bm, int bn) { return (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * group; };
-   auto tiled = [&](int bm, int bn) {
+   // A 64x32 tile gathers as many image elements as a 64x64 one for half the products: half the matrix rate against 0.64 of it
+   // (64 images of 32x32, 32 -> 64 channels: 46 us with 64x32 tiles, 38 us with 64x64; 74 and 62 us from 64 channels).
+   auto tiled = [&](int bm, int bn, double rate) {
       const double rounds = std::ceil(tiles(bm, bn) / 256.0), blocks = (bm / 32) * (bn / 32), slabs = (K + 31) / 32;
-      return 3.0 + std::max(rounds * blocks * (slabs * 256.0 / (2400.0 * 0.62) + 0.7), 0.75 * slabs + 1.4);
+      return 3.0 + std::max(rounds * blocks * (slabs * 256.0 / (2400.0 * rate) + 0.7), 0.75 * slabs + 1.4);
    };
    int best = F32_DIRECT;
    double least = 5.3 + tiles(16, 16) / 256.0 * (0.9 + 0.17 * ((K + 15) / 16));
@@ -176,10 +180,10 @@ static int pick_f32_conv_tile(int M, int N, int K, int group)
       if (t < least)
          least = t, best = tile;
    };
-   offer(F32_TILE_64x32, tiled(64, 32));
-   offer(F32_TILE_64, tiled(64, 64));
+   offer(F32_TILE_64x32, tiled(64, 32, 0.5));
+   offer(F32_TILE_64, tiled(64, 64, 0.64));
    if (N <= 32 && tiles(128, 32) >= 1024) // a start per 128 rows instead of 64: first convolution of a 64-image network 29.7 -> 27.6 us
-      offer(F32_TILE_128x32, 0.95 * tiled(128, 32));
+      offer(F32_TILE_128x32, 0.95 * tiled(128, 32, 0.5));
    return best;
 }
 
@@ -253,72 +257,12 @@ static int launch_f32_conv(sofie_hip_ctx *ctx, const float *X, F32ConvShape s, c
    return rows(F32ConvRows<false>{});
 }
 
-} // namespace sofie_hip
-
-using namespace sofie_hip;
-
-extern "C" {
-
-int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *d)
+// `count` layers in one launch of the chain kernel, if their shapes, strides and memory allow it (*launched tells).
+static int launch_f32_chain(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *layers, int32_t count, bool *launched)
 {
-   SOFIE_HIP_REQUIRE(ctx && d, "sofie_hip_gemm_f32: NULL argument");
-   SOFIE_HIP_REQUIRE(d->M >= 0 && d->N >= 0 && d->K >= 0, "sofie_hip_gemm_f32: negative dimension");
-   SOFIE_HIP_REQUIRE(d->batch >= 1, "sofie_hip_gemm_f32: batch must be >= 1");
-   SOFIE_HIP_REQUIRE(d->bias_mode >= SOFIE_BIAS_NONE && d->bias_mode <= SOFIE_BIAS_FULL, "sofie_hip_gemm_f32: unknown bias mode %d", d->bias_mode);
-   F32Epilogue ep;
-   int bad = 0;
-   SOFIE_HIP_REQUIRE(make_post_chain(ep.chain, d->act, d->act_alpha, d->post, bad),
-                     "sofie_hip_gemm_f32: unknown activation or post operator %d (or more than %d post operators)", bad, SOFIE_MAX_POST_OPS);
-   if (d->M == 0 || d->N == 0)
-      return SOFIE_HIP_OK;
-   SOFIE_HIP_REQUIRE(d->Y != nullptr, "sofie_hip_gemm_f32: Y is NULL");
-   SOFIE_HIP_REQUIRE(d->K == 0 || (d->A && d->B), "sofie_hip_gemm_f32: A or B is NULL");
-   SOFIE_HIP_REQUIRE(d->bias_mode == SOFIE_BIAS_NONE || d->C != nullptr, "sofie_hip_gemm_f32: bias mode set but C is NULL");
-   const int M = d->M, N = d->N, K = d->K;
-   const long long lda = d->lda ? d->lda : (d->transA ? M : K);
-   const long long ldb = d->ldb ? d->ldb : (d->transB ? K : N);
-   const long long ldy = d->ldy ? d->ldy : N;
-   SOFIE_HIP_REQUIRE(lda >= (d->transA ? M : K) && ldb >= (d->transB ? K : N) && ldy >= N,
-                     "sofie_hip_gemm_f32: leading dimension too small");
-   ep.alpha = d->alpha;
-   ep.beta = d->beta;
-   ep.C = d->bias_mode == SOFIE_BIAS_NONE ? nullptr : d->C;
-   ep.bias_mode = d->bias_mode;
-   ep.ldc = N;
-   ep.R = d->residual;
-   ep.ldr = ldy;
-   SOFIE_HIP_REQUIRE(d->batch <= 65535, "sofie_hip_gemm_f32: batch too large for one launch");
-   auto in_vectors = [](const void *p, long long a, long long b, long long c) { return ((uintptr_t)p & 15) == 0 && a % 4 == 0 && b % 4 == 0 && c % 4 == 0; };
-   F32RowStore out;
-   out.Y = d->Y;
-   out.ldy = ldy;
-   out.ep = ep;
-   out.vec = in_vectors(d->Y, ldy, d->strideY, 0);
-   out.strideC = d->strideC;
-   out.strideY = d->strideY;
-   // 16-byte loads where both operands allow them: address, pitch, and the extent along the contiguous direction
-   const bool vec = in_vectors(d->A, lda, d->strideA, d->transA ? M : K) && in_vectors(d->B, ldb, d->strideB, d->transB ? K : N);
-   auto with_b = [&](const auto &A) {
-      auto go = [&](const auto &B) {
-         return launch_f32_product(ctx, A, B, out, M, N, K, d->batch, d->strideA, d->strideB);
-      };
-      constexpr int VEC = std::remove_reference_t<decltype(A)>::VEC;
-      return d->transB ? go(F32Matrix<true, VEC>{d->B, ldb, N, K}) : go(F32Matrix<false, VEC>{d->B, ldb, N, K});
-   };
-   if (vec)
-      return d->transA ? with_b(F32Matrix<false, 4>{d->A, lda, M, K}) : with_b(F32Matrix<true, 4>{d->A, lda, M, K});
-   return d->transA ? with_b(F32Matrix<false, 1>{d->A, lda, M, K}) : with_b(F32Matrix<true, 1>{d->A, lda, M, K});
-}
-
-int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *layers, int32_t count)
-{
-   SOFIE_HIP_REQUIRE(ctx && layers, "sofie_hip_gemm_chain_f32: NULL argument");
-   SOFIE_HIP_REQUIRE(count >= 1 && count <= SOFIE_MAX_GEMM_CHAIN, "sofie_hip_gemm_chain_f32: %d layers (1..%d allowed)", count, SOFIE_MAX_GEMM_CHAIN);
-   for (int l = 1; l < count; ++l)
-      SOFIE_HIP_REQUIRE(layers[l].A == layers[l - 1].Y && layers[l].A != nullptr, "sofie_hip_gemm_chain_f32: layer %d does not read the output of layer %d", l, l - 1);
-   // One launch when the batch is small enough that launches, not arithmetic, set the time, and the rows fit in LDS.
+   *launched = false;
    const int M = layers[0].M;
-   bool fused = count >= 2 && M >= 1 && (ctx->opt.f32_chain >= 0 ? ctx->opt.f32_chain != 0 : M <= 256);
+   bool fused = count >= 2 && M >= 1;
    int width = layers[0].K;
    ChainArgs a;
    a.count = count;
@@ -401,12 +345,113 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
          hipLaunchKernelGGL(gemm_chain_f32_kernel<2>, grid, dim3(CHAIN_THREADS), lds, ctx->stream, a, width);
       else
          hipLaunchKernelGGL(gemm_chain_f32_kernel<4>, grid, dim3(CHAIN_THREADS), lds, ctx->stream, a, width);
+      *launched = true;
       return launch_status("gemm_chain_f32_kernel");
    }
-   // anything else (and every malformed descriptor, which the single product reports): one launch per layer
-   for (int l = 0; l < count; ++l)
+   return SOFIE_HIP_OK;
+}
+
+} // namespace sofie_hip
+
+using namespace sofie_hip;
+
+extern "C" {
+
+int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *d)
+{
+   SOFIE_HIP_REQUIRE(ctx && d, "sofie_hip_gemm_f32: NULL argument");
+   SOFIE_HIP_REQUIRE(d->M >= 0 && d->N >= 0 && d->K >= 0, "sofie_hip_gemm_f32: negative dimension");
+   SOFIE_HIP_REQUIRE(d->batch >= 1, "sofie_hip_gemm_f32: batch must be >= 1");
+   SOFIE_HIP_REQUIRE(d->bias_mode >= SOFIE_BIAS_NONE && d->bias_mode <= SOFIE_BIAS_FULL, "sofie_hip_gemm_f32: unknown bias mode %d", d->bias_mode);
+   F32Epilogue ep;
+   int bad = 0;
+   SOFIE_HIP_REQUIRE(make_post_chain(ep.chain, d->act, d->act_alpha, d->post, bad),
+                     "sofie_hip_gemm_f32: unknown activation or post operator %d (or more than %d post operators)", bad, SOFIE_MAX_POST_OPS);
+   if (d->M == 0 || d->N == 0)
+      return SOFIE_HIP_OK;
+   SOFIE_HIP_REQUIRE(d->Y != nullptr, "sofie_hip_gemm_f32: Y is NULL");
+   SOFIE_HIP_REQUIRE(d->K == 0 || (d->A && d->B), "sofie_hip_gemm_f32: A or B is NULL");
+   SOFIE_HIP_REQUIRE(d->bias_mode == SOFIE_BIAS_NONE || d->C != nullptr, "sofie_hip_gemm_f32: bias mode set but C is NULL");
+   const int M = d->M, N = d->N, K = d->K;
+   const long long lda = d->lda ? d->lda : (d->transA ? M : K);
+   const long long ldb = d->ldb ? d->ldb : (d->transB ? K : N);
+   const long long ldy = d->ldy ? d->ldy : N;
+   SOFIE_HIP_REQUIRE(lda >= (d->transA ? M : K) && ldb >= (d->transB ? K : N) && ldy >= N,
+                     "sofie_hip_gemm_f32: leading dimension too small");
+   ep.alpha = d->alpha;
+   ep.beta = d->beta;
+   ep.C = d->bias_mode == SOFIE_BIAS_NONE ? nullptr : d->C;
+   ep.bias_mode = d->bias_mode;
+   ep.ldc = N;
+   ep.R = d->residual;
+   ep.ldr = ldy;
+   SOFIE_HIP_REQUIRE(d->batch <= 65535, "sofie_hip_gemm_f32: batch too large for one launch");
+   auto in_vectors = [](const void *p, long long a, long long b, long long c) { return ((uintptr_t)p & 15) == 0 && a % 4 == 0 && b % 4 == 0 && c % 4 == 0; };
+   F32RowStore out;
+   out.Y = d->Y;
+   out.ldy = ldy;
+   out.ep = ep;
+   out.vec = in_vectors(d->Y, ldy, d->strideY, 0);
+   out.strideC = d->strideC;
+   out.strideY = d->strideY;
+   // 16-byte loads where both operands allow them: address, pitch, and the extent along the contiguous direction
+   const bool vec = in_vectors(d->A, lda, d->strideA, d->transA ? M : K) && in_vectors(d->B, ldb, d->strideB, d->transB ? K : N);
+   auto with_b = [&](const auto &A) {
+      auto go = [&](const auto &B) {
+         return launch_f32_product(ctx, A, B, out, M, N, K, d->batch, d->strideA, d->strideB);
+      };
+      constexpr int VEC = std::remove_reference_t<decltype(A)>::VEC;
+      return d->transB ? go(F32Matrix<true, VEC>{d->B, ldb, N, K}) : go(F32Matrix<false, VEC>{d->B, ldb, N, K});
+   };
+   if (vec)
+      return d->transA ? with_b(F32Matrix<false, 4>{d->A, lda, M, K}) : with_b(F32Matrix<true, 4>{d->A, lda, M, K});
+   return d->transA ? with_b(F32Matrix<false, 1>{d->A, lda, M, K}) : with_b(F32Matrix<true, 1>{d->A, lda, M, K});
+}
+
+int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *layers, int32_t count)
+{
+   SOFIE_HIP_REQUIRE(ctx && layers, "sofie_hip_gemm_chain_f32: NULL argument");
+   SOFIE_HIP_REQUIRE(count >= 1 && count <= SOFIE_MAX_GEMM_CHAIN, "sofie_hip_gemm_chain_f32: %d layers (1..%d allowed)", count, SOFIE_MAX_GEMM_CHAIN);
+   for (int l = 1; l < count; ++l)
+      SOFIE_HIP_REQUIRE(layers[l].A == layers[l - 1].Y && layers[l].A != nullptr, "sofie_hip_gemm_chain_f32: layer %d does not read the output of layer %d", l, l - 1);
+   // Which layers share a launch.  A launch of its own spreads a layer over the chip and costs about 3 us (what the host takes for
+   // it); in the chain kernel a workgroup does its rows' share alone: a pass over 64 outputs (W stored [N][K]) or a walk along k
+   // (W stored [K][N]) at a time.  So large layers run one by one, and small ones behind them share a launch.
+   const int M = layers[0].M;
+   int first = count; // first layer of the shared launch
+   if (ctx->opt.f32_chain == 1) {
+      first = 0;
+   } else if (ctx->opt.f32_chain < 0 && M >= 1 && M <= 256) {
+      double before = 0.0, least = 0.0;
+      for (int l = 0; l < count; ++l) {
+         double t = 0.0;
+         pick_f32_tile(M, layers[l].N, layers[l].K, 1, &t);
+         least += std::max(t, 3.0);
+      }
+      for (int s = 0; s + 2 <= count; ++s) {
+         double together = 0.0, t = 0.0;
+         for (int l = s; l < count; ++l) {
+            const double K = layers[l].K, passes = std::ceil(layers[l].N / (layers[l].transB ? 64.0 : 1024.0));
+            together += 0.4 + passes * (layers[l].transB ? 0.9 + 0.002 * K : 0.017 * K);
+         }
+         together = before + 2.3 + together * (M <= 64 ? 1.0 : 1.8);
+         if (together < least)
+            least = together, first = s;
+         pick_f32_tile(M, layers[s].N, layers[s].K, 1, &t);
+         before += std::max(t, 3.0);
+      }
+   }
+   for (int l = 0; l < count; ++l) {
+      if (l == first) {
+         bool launched = false;
+         const int st = launch_f32_chain(ctx, layers + first, count - first, &launched);
+         if (st || launched)
+            return st;
+      }
+      // (and every malformed descriptor, which the single product reports)
       if (int st = sofie_hip_gemm_f32(ctx, &layers[l]))
          return st;
+   }
    return SOFIE_HIP_OK;
 }
 
