@@ -38,6 +38,29 @@ __device__ __forceinline__ void f32_tile_of_block(int tiles_m, int tiles_n, int 
    }
 }
 
+// a value that is the same in all lanes, in scalar registers
+__device__ __forceinline__ long long uniform(long long v)
+{
+   const unsigned lo = __builtin_amdgcn_readfirstlane((int)v), hi = __builtin_amdgcn_readfirstlane((int)(v >> 32));
+   return (long long)(((unsigned long long)hi << 32) | lo);
+}
+
+// Loads into LDS go through a buffer descriptor: its base is scalar and may move, so is a second offset; a lane adds an offset of 31
+// bits, and F32_OUTSIDE, which lies behind the buffer's end, reads as zero.  Vector instructions take their turn on the multipliers of the fp32
+// matrix cores (measured: 2.8 of an MFMA's 64 cycles each, a 64-bit addition 4.6), so what a loop spends on addresses is lost to it:
+// two 64-bit additions and an address in LDS per load took a tenth of it.
+constexpr long long F32_BUFFER_BYTES = 0x7fffff00;
+constexpr int F32_OUTSIDE = -1;
+template <int FLOATS>
+__device__ __forceinline__ void f32_buffer_load(lds_void_t *to, const void *base, int offset, int scalar_offset = 0)
+{
+   const __amdgpu_buffer_rsrc_t buffer = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)F32_BUFFER_BYTES, 0x00020000);
+   if constexpr (FLOATS == 4)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer, to, 16, offset, scalar_offset, 0, 0);
+   else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer, to, 4, offset, scalar_offset, 0, 0);
+}
+
 // ---- operands ---------------------------------------------------------------------------------------------------------------
 // An operand is a matrix of `rows` (m or n) by K.  KC: contiguous in k (a row's k neighbours lie side by side); otherwise
 // contiguous along the rows.  VEC: floats per load; 4 needs 16-byte aligned pieces (the host checks that the address, the
@@ -52,28 +75,46 @@ struct F32Matrix {
    int rows, K;
    __device__ __forceinline__ void shift(long long elements) { p += elements; }
    __device__ __forceinline__ void select_group(int) {}
+   // whether the slabs of any tile lie within a buffer of their own (rows of up to four million floats)
+   bool in_buffers() const { return (KC ? (rows < 128 ? rows : 128) : 32) * ld * 4 + 1024 <= F32_BUFFER_BYTES; }
 
-   // what a lane keeps per load instruction of a slab: the address at k = 0
+   // A slab is loaded through a buffer whose base, in scalar registers, walks along k; what a lane keeps per load instruction of a
+   // slab is its distance from there (32 bits: the host checks that they do).
+   template <int LD>
+   struct walk_state {
+      const char *base; // first row of the tile, first k of the slab to be asked for next
+      long long step;
+      int k0;
+   };
+   template <int LD, class F>
+   __device__ __forceinline__ void walk_start(walk_state<LD> &w, int r0, int, int slab, F &&) const
+   {
+      w.base = (const char *)uniform((long long)(KC ? p + (long long)r0 * ld : p + r0));
+      w.step = (KC ? (long long)slab : slab * ld) * 4;
+      w.k0 = 0;
+   }
+   template <int LD>
+   __device__ __forceinline__ void walk_on(walk_state<LD> &w, int slab) const
+   {
+      w.base += w.step;
+      w.k0 += slab;
+   }
    template <int LD>
    struct lane_state {
-      const float *at[LD];
+      int at[LD];
    };
    template <int LD>
-   __device__ __forceinline__ void init(lane_state<LD> &st, int i, int row, int kk) const
+   __device__ __forceinline__ void init(lane_state<LD> &st, int i, int r0, int row, int kk) const
    {
       // rows past the edge re-read the last piece (their results are not stored)
-      const int r = row < rows ? row : (KC || VEC == 1 ? rows - 1 : rows - VEC);
-      st.at[i] = KC ? p + (long long)r * ld + kk : p + (long long)kk * ld + r;
+      const int last = (KC || VEC == 1 ? rows - 1 : rows - VEC) - r0, r = row < last ? row : last;
+      st.at[i] = (int)(KC ? (long long)r * ld + kk : (long long)kk * ld + r) * 4;
    }
-   struct walk_state {};
-   __device__ __forceinline__ void walk_start(walk_state &, int, int, int) const {}
-   __device__ __forceinline__ void walk_on(walk_state &, int) const {}
-   // address of load i of the slab at k0 (kk: the lane's k within the slab; WHOLE: no k of the slab lies past K)
+   // load i of the slab (kk: the lane's k within the slab; WHOLE: no k of the slab lies past K)
    template <bool WHOLE, int LD>
-   __device__ __forceinline__ const float *load_ptr(const lane_state<LD> &st, const walk_state &, int i, int kk, int k0) const
+   __device__ __forceinline__ void load(lds_void_t *to, const lane_state<LD> &st, const walk_state<LD> &w, int i, int kk) const
    {
-      const float *a = st.at[i] + (KC ? (long long)k0 : (long long)k0 * ld);
-      return WHOLE || k0 + kk < K ? a : f32_zero_page;
+      f32_buffer_load<VEC>(to, w.base, WHOLE || w.k0 + kk < K ? st.at[i] : F32_OUTSIDE);
    }
 
    // direct fetch of row `row`, k..k+3
@@ -113,9 +154,8 @@ struct F32ConvShape {
    unsigned long long ow_mul, oh_mul, od_mul; // ceil(2^64 / extent), 0 for an extent of 1: m / extent == umul64hi(m, mul) for 32-bit m
    unsigned kw_mul, kh_mul, kd_mul, positions_mul; // ceil(2^31 / extent): k / extent == umulhi(2 k, mul) while k * extent < 2^31 (checked on the host)
 };
-// MASKED (at most 31 kernel positions): a lane keeps one bit per kernel position that lies inside the image; lane i walks along the
-// k of load instruction i, from slab to slab, and the instructions take offset and kernel position from there as scalars.
-// About ten instructions per 64 elements, a quarter of what decomposing every k by scalar arithmetic took.
+// MASKED (at most 31 kernel positions, extents that fit a buffer): a lane keeps its row's place and one bit per kernel position that
+// lies outside the image; the walk along k, from slab to slab, is scalar.  Three vector instructions per 64 elements.
 template <bool MASKED>
 struct F32ConvRows {
    static constexpr int kLeastRows = 64; // a load instruction covers one k: what depends on k is scalar
@@ -125,25 +165,32 @@ struct F32ConvRows {
    F32ConvShape s;
    int rows, K;
    long long image, channel; // elements per image and per channel
+   bool in_buffers() const { return true; }
    __device__ __forceinline__ void shift(long long) {}
    __device__ __forceinline__ void select_group(int g) { X += (long long)g * s.Cg * channel; }
 
+   struct position {
+      int image, d, h, w; // of an output
+   };
+   __device__ __forceinline__ position position_of(int row) const
+   {
+      auto quotient = [](int n, unsigned long long mul) { return mul ? (int)__umul64hi((unsigned long long)(unsigned)n, mul) : n; };
+      const int m = row < rows ? row : rows - 1;
+      const int t = quotient(m, s.ow_mul), u = quotient(t, s.oh_mul), image = quotient(u, s.od_mul);
+      return position{image, u - image * s.OD, t - u * s.OH, m - t * s.OW};
+   }
    struct row_state {
       const float *at; // element of channel 0 at (id0, ih0, iw0): dereferenced only inside the image
       int id0, ih0, iw0;
    };
    __device__ __forceinline__ row_state row_of(int row) const
    {
-      auto quotient = [](int n, unsigned long long mul) { return mul ? (int)__umul64hi((unsigned long long)(unsigned)n, mul) : n; };
-      const int m = row < rows ? row : rows - 1;
-      const int t = quotient(m, s.ow_mul), ow = m - t * s.OW;
-      const int u = quotient(t, s.oh_mul), oh = t - u * s.OH;
-      const int img = quotient(u, s.od_mul), od = u - img * s.OD;
+      const position o = position_of(row);
       row_state r;
-      r.id0 = od * s.stride_d - s.pad_d;
-      r.ih0 = oh * s.stride_h - s.pad_h;
-      r.iw0 = ow * s.stride_w - s.pad_w;
-      r.at = X + (long long)img * image + ((long long)r.id0 * s.H + r.ih0) * s.W + r.iw0;
+      r.id0 = o.d * s.stride_d - s.pad_d;
+      r.ih0 = o.h * s.stride_h - s.pad_h;
+      r.iw0 = o.w * s.stride_w - s.pad_w;
+      r.at = X + (long long)o.image * image + ((long long)r.id0 * s.H + r.ih0) * s.W + r.iw0;
       return r;
    }
    static __device__ __forceinline__ int divide(int k, unsigned mul) { return (int)__umulhi((unsigned)k * 2u, mul); }
@@ -162,73 +209,89 @@ struct F32ConvRows {
    template <int LD>
    struct lane_state {
       row_state r;
-      unsigned inside; // bit t: kernel position t of this row lies inside the image
+      int at;           // MASKED: where the window of this row begins in the padded image, from the tile's base, in bytes
+      unsigned outside; // MASKED: bit t: kernel position t of this row lies outside the image; bit 31 is set
    };
    template <int LD>
-   __device__ __forceinline__ void init(lane_state<LD> &st, int i, int row, int) const
+   __device__ __forceinline__ void init(lane_state<LD> &st, int i, int r0, int row, int) const
    {
       if (i != 0)
          return;
-      st.r = row_of(row);
+      st.r = row_of(r0 + row);
       if constexpr (MASKED) {
-         unsigned columns = 0, lines = 0;
+         unsigned columns = 0, lines = 0, inside = 0;
          for (int kx = 0; kx < s.kw; ++kx)
             columns |= ((unsigned)(st.r.iw0 + kx * s.dil_w) < (unsigned)s.W ? 1u : 0u) << kx;
          for (int ky = 0; ky < s.kh; ++ky)
             lines |= ((unsigned)(st.r.ih0 + ky * s.dil_h) < (unsigned)s.H ? columns : 0u) << (ky * s.kw);
-         st.inside = 0;
          for (int kz = 0; kz < s.kd; ++kz)
-            st.inside |= ((unsigned)(st.r.id0 + kz * s.dil_d) < (unsigned)s.D ? lines : 0u) << (kz * s.kh * s.kw);
+            inside |= ((unsigned)(st.r.id0 + kz * s.dil_d) < (unsigned)s.D ? lines : 0u) << (kz * s.kh * s.kw);
+         st.outside = ~inside;
+         st.at = (int)((const char *)st.r.at - base_of(r0));
       }
    }
-   // For MASKED, lane i: the k of load i of the slab to be asked for, its kernel position and the offsets of its channel and position.
+   // the padded image of the first row of a tile: no window of the tile begins before it
+   __device__ __forceinline__ const char *base_of(int r0) const
+   {
+      const long long pad = ((long long)s.pad_d * s.H + s.pad_h) * s.W + s.pad_w;
+      return (const char *)(X + (long long)position_of(r0).image * image - pad);
+   }
+   // For MASKED, scalars: of load i of the slab to be asked for its first k in that slab, its kernel position and the offset of its channel.
+   template <int LD>
    struct walk_state {
-      int k, position, channel_offset;
-      int step_channels, step_rest; // a slab's worth of k in channels (as an offset) and kernel positions: uniform
-      int table;  // lane t: offset of kernel position t
-      int offset; // of k: what load i adds to the address of its row
+      const char *base;
+      int k0;
+      int first[LD], position[LD], channel[LD];
+      int step_channels, step_rest; // a slab's worth of k in channels (as an offset) and kernel positions
+      int table;                    // lane t: offset of kernel position t
    };
-   __device__ __forceinline__ void walk_settle(walk_state &w) const
+   template <int LD, class F>
+   __device__ __forceinline__ void walk_start(walk_state<LD> &w, int r0, int lane, int slab, F &&first_k) const
    {
-      w.offset = w.channel_offset + __builtin_amdgcn_ds_bpermute(w.position << 2, w.table);
-      if (w.k >= K)
-         w.offset = 0;
-   }
-   __device__ __forceinline__ void walk_start(walk_state &w, int k, int lane, int step) const
-   {
+      w.k0 = 0;
       if constexpr (MASKED) {
+         w.base = (const char *)uniform((long long)base_of(r0));
          const int t = divide(lane, s.kw_mul), kx = lane - t * s.kw, kz = divide(t, s.kh_mul), ky = t - kz * s.kh;
-         w.table = (kz * s.dil_d * s.H + ky * s.dil_h) * s.W + kx * s.dil_w; // lanes past the last position are not asked
-         const int ci = divide(k, s.positions_mul), channels = divide(step, s.positions_mul);
-         w.k = k;
-         w.position = k - ci * s.positions;
-         w.channel_offset = ci * (int)channel;
-         w.step_channels = channels * (int)channel;
-         w.step_rest = step - channels * s.positions;
-         walk_settle(w);
+         w.table = ((kz * s.dil_d * s.H + ky * s.dil_h) * s.W + kx * s.dil_w) * 4; // lanes past the last position are not asked
+         const int channels = divide(slab, s.positions_mul);
+         w.step_channels = channels * (int)channel * 4;
+         w.step_rest = slab - channels * s.positions;
+#pragma unroll
+         for (int i = 0; i < LD; ++i) {
+            w.first[i] = first_k(i);
+            const int ci = divide(w.first[i], s.positions_mul);
+            w.position[i] = w.first[i] - ci * s.positions;
+            w.channel[i] = ci * (int)channel * 4;
+         }
       }
    }
-   __device__ __forceinline__ void walk_on(walk_state &w, int step) const // by the `step` of walk_start
+   template <int LD>
+   __device__ __forceinline__ void walk_on(walk_state<LD> &w, int slab) const // by the slab of walk_start
    {
+      w.k0 += slab;
       if constexpr (MASKED) {
-         w.k += step;
-         w.position += w.step_rest;
-         w.channel_offset += w.step_channels;
-         const bool over = w.position >= s.positions;
-         w.position -= over ? s.positions : 0;
-         w.channel_offset += over ? (int)channel : 0;
-         walk_settle(w);
+#pragma unroll
+         for (int i = 0; i < LD; ++i) {
+            const int position = w.position[i] + w.step_rest;
+            const bool over = position >= s.positions;
+            w.position[i] = position - (over ? s.positions : 0);
+            w.channel[i] += w.step_channels + (over ? (int)channel * 4 : 0);
+         }
       }
    }
    template <bool WHOLE, int LD>
-   __device__ __forceinline__ const float *load_ptr(const lane_state<LD> &st, const walk_state &w, int i, int kk, int k0) const
+   __device__ __forceinline__ void load(lds_void_t *to, const lane_state<LD> &st, const walk_state<LD> &w, int i, int kk) const
    {
       if constexpr (MASKED) {
-         const int offset = __builtin_amdgcn_readlane(w.offset, i);
-         const int position = __builtin_amdgcn_readlane(WHOLE || w.k < K ? w.position : 31, i); // no lane has bit 31 set
-         return (st.inside >> position) & 1u ? st.r.at + (long long)offset : f32_zero_page;
+         const bool any = WHOLE || w.k0 + w.first[i] < K;
+         const int position = any ? w.position[i] : 31;
+         const int offset = any ? w.channel[i] + __builtin_amdgcn_readlane(w.table, w.position[i]) : 0;
+         const int outside = __builtin_amdgcn_sbfe(st.outside, position, 1); // all ones, or none
+         f32_buffer_load<1>(to, w.base, st.at | outside, offset);
+      } else {
+         const float *at = element(st.r, w.k0 + __builtin_amdgcn_readfirstlane(kk));
+         __builtin_amdgcn_global_load_lds((global_void_t *)at, to, 4, 0, 0);
       }
-      return element(st.r, k0 + __builtin_amdgcn_readfirstlane(kk));
    }
    __device__ __forceinline__ v4f fetch(const row_state &st, int k) const
    {
@@ -403,7 +466,7 @@ struct F32Slab {
    static constexpr bool KC = SRC::KC;
    static constexpr int FLOATS = f32_slab_floats<SRC::KC, R, BK>();
    typename SRC::template lane_state<LD> st;
-   typename SRC::walk_state walk;
+   typename SRC::template walk_state<LD> walk;
 
    // (row, k) of the slab that load i of this wave brings to this lane's place in LDS
    static __device__ __forceinline__ void place(int i, int wave, int lane, int &row, int &kk)
@@ -424,25 +487,20 @@ struct F32Slab {
       for (int i = 0; i < LD; ++i) {
          int row, kk;
          place(i, wave, lane, row, kk);
-         src.template init<LD>(st, i, r0 + row, kk);
+         src.template init<LD>(st, i, r0, row, kk);
       }
-      src.walk_start(walk, ((lane * NW + wave) % TOTAL) * 64 * VEC / R, lane, BK); // the k of the load whose number is the lane's
+      src.template walk_start<LD>(walk, r0, lane, BK, [&](int i) { return ((i * NW + wave) % TOTAL) * 64 * VEC / R; });
    }
-   // asks for the slab at k0; the slabs are asked for one after the other
+   // asks for the next slab; the slabs are asked for one after the other
    template <bool WHOLE>
-   __device__ __forceinline__ void issue(const SRC &src, float *lds, int k0, int wave, int lane)
+   __device__ __forceinline__ void issue(const SRC &src, float *lds, int wave, int lane)
    {
       static_for<LD>([&](auto ic) {
          constexpr int i = decltype(ic)::value;
          int row, kk;
          place(i, wave, lane, row, kk);
          const int f = ((i * NW + wave) % TOTAL) * 64 * VEC;
-         global_void_t *from = (global_void_t *)src.template load_ptr<WHOLE, LD>(st, walk, i, kk, k0);
-         lds_void_t *to = (lds_void_t *)(lds + f + f32_gap<SRC::KC, R>(f / R));
-         if constexpr (VEC == 4)
-            __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
-         else
-            __builtin_amdgcn_global_load_lds(from, to, 4, 0, 0);
+         src.template load<WHOLE, LD>((lds_void_t *)(lds + f + f32_gap<SRC::KC, R>(f / R)), st, walk, i, kk);
       });
       src.walk_on(walk, BK);
    }
@@ -519,10 +577,17 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_ke
             acc[i][j][e] = 0.0f;
 
    const int KT = (K + BK - 1) / BK;
+   // asks for the next slab, number kt
    auto issue = [&](int kt, int stage, auto whole) {
       float *s = f32_lds + stage * STAGE;
-      sa.template issue<decltype(whole)::value>(A, s, kt * BK, wave, lane);
-      sb.template issue<decltype(whole)::value>(B, s + SA::FLOATS, kt * BK, wave, lane);
+      auto both = [&](auto all) {
+         sa.template issue<decltype(all)::value>(A, s, wave, lane);
+         sb.template issue<decltype(all)::value>(B, s + SA::FLOATS, wave, lane);
+      };
+      if (decltype(whole)::value || kt < K / BK)
+         both(std::true_type{});
+      else
+         both(std::false_type{});
    };
    // until at most `slabs` of the slabs asked for last are still on their way (counts past STAGES - 2 wait for that many)
    auto wait_slabs = [&](int slabs) {
@@ -560,15 +625,15 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_ke
       __builtin_amdgcn_s_barrier();
       read(0, fa[0], fb[0]);
    }
-   int stage = 0;
    // Slab kt: its fragments are in registers.  Behind the barrier slab kt + 1 has landed for every wave and slab kt has been read by
    // every wave: the next fragments are asked for and slab kt + STAGES takes the place of slab kt.  The barrier sits between
    // two halves of the MFMAs, and what is issued behind it is dealt out among those of the second half: a wave that runs alone
    // on its SIMD keeps the matrix core busy.
-   auto step = [&](int kt, auto parity, auto whole) {
-      constexpr int cur = decltype(parity)::value;
+   // Which place of the ring a step reads is known where the code is written, so every address in LDS is a lane's constant plus an
+   // immediate (what computing them took of the multipliers: see F32Matrix).
+   auto step = [&](int kt, auto number, auto whole) {
+      constexpr int cur = decltype(number)::value % 2, stage = decltype(number)::value % STAGES, next = (stage + 1) % STAGES;
       constexpr bool WHOLE = decltype(whole)::value;
-      const int next = stage + 1 == STAGES ? 0 : stage + 1;
       constexpr int QS = GS * 4, HALF = QS / 2;
       auto multiply = [&](auto from, auto to) {
          static_for<decltype(to)::value - decltype(from)::value>([&](auto qc) {
@@ -603,22 +668,18 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_ke
          __builtin_amdgcn_sched_group_barrier(0x020, (LPT + GROUPS - 1) / GROUPS, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
-      stage = next;
    };
-   constexpr std::integral_constant<int, 0> even{};
-   constexpr std::integral_constant<int, 1> odd{};
+   constexpr int ROUND = STAGES % 2 ? 2 * STAGES : STAGES; // steps until ring and register sets are where they were
    int kt = 0;
    // as long as what is asked for is a whole slab, no load looks at its k (the comparison and the selection of an address per load
    // cost 5 - 8 % of the loop)
-   for (; kt + 1 + STAGES < K / BK; kt += 2) {
-      step(kt, even, std::true_type{});
-      step(kt + 1, odd, std::true_type{});
-   }
-   for (; kt < KT; kt += 2) {
-      step(kt, even, any);
-      if (kt + 1 < KT)
-         step(kt + 1, odd, any);
-   }
+   for (; kt + ROUND - 1 + STAGES < K / BK; kt += ROUND)
+      static_for<ROUND>([&](auto u) { step(kt + decltype(u)::value, u, std::true_type{}); });
+   for (; kt < KT; kt += ROUND)
+      static_for<ROUND>([&](auto u) {
+         if (kt + decltype(u)::value < KT)
+            step(kt + decltype(u)::value, u, any);
+      });
 
    // The tile store reuses the ring, one region per wave: the wave's tile is laid out as the result is (rows of columns, or columns
    // of rows), and read back in one rolled loop, so that a wave instruction stores whole lines and the code of the

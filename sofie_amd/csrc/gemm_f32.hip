@@ -135,55 +135,47 @@ __global__ __launch_bounds__(CHAIN_THREADS) void gemm_chain_f32_kernel(ChainArgs
 namespace sofie_hip {
 
 // The kernel for a product of M x N x K, `batch` times: the one whose time, estimated from what each was measured to do, is the
-// shortest.  A CU multiplies a 32 x 32 block by 32 k in 256 cycles at best; the tile kernels reach 0.66 (32 x 32 tiles), 0.78
-// (64 x 64) and 0.84 (128 x 128) of that and take 4.2 / 5 / 5.5 us on top (launch, first loads, store), in as many rounds as the tiles
-// need over 256 CUs.  The direct kernel costs a launch and a trip to memory per 512 k (2.0 and 1.35 us), or the 9.4 TB/s at which
-// its fragments, which nothing shares, arrive.
+// shortest.  A CU multiplies a 32 x 32 block by 32 k in 0.107 us at best.  The tile kernels take 0.128 us (32 x 32 tiles), 0.245
+// (64 x 32: two blocks), 0.452 (64 x 64: four) and 1.765 (128 x 128: sixteen), a start and a store per tile, in as many rounds as
+// the tiles need over 256 CUs, and a launch.  The direct kernel costs a launch, a trip to memory per 512 k or the 10.5 TB/s at which
+// its fragments, which nothing shares, arrive, and 0.45 us per 256 tiles.
 enum F32Tile { F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
 static int pick_f32_tile(int M, int N, int K, int batch, double *time_us = nullptr)
 {
    auto tiles = [&](int bm, int bn) { return (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
-   auto tiled = [&](int bm, int bn, double rate, double fixed) {
-      const double rounds = std::ceil(tiles(bm, bn) / 256.0), blocks = (bm / 32) * (bn / 32);
-      return fixed + rounds * ((K + 31) / 32) * blocks * 256.0 / (2400.0 * rate);
-   };
-   const double steps = (K + 15) / 16;
+   const double slabs = (K + 31) / 32, steps = (K + 15) / 16;
+   auto tiled = [&](int bm, int bn, double launch, double slab, double tile) { return launch + std::ceil(tiles(bm, bn) / 256.0) * (slabs * slab + tile); };
    int best = F32_DIRECT;
-   double least = std::max(2.0 + 1.35 * std::ceil(steps / 32.0), tiles(16, 16) * steps * 2048.0 / 9.4e6 + 2.0);
+   double least = 2.0 + std::max(1.35 * std::ceil(steps / 32.0), tiles(16, 16) * steps * 2048.0 / 10.5e6) + 0.45 * tiles(16, 16) / 256.0;
    auto offer = [&](int tile, double t) {
       if (t < least)
          least = t, best = tile;
    };
-   offer(F32_TILE_32, tiled(32, 32, 0.66, 4.2));
-   offer(F32_TILE_64x32, tiled(64, 32, 0.70, 4.6));
-   offer(F32_TILE_64, tiled(64, 64, 0.78, 5.0));
-   offer(F32_TILE_128, tiled(128, 128, 0.84, 5.5));
+   offer(F32_TILE_32, tiled(32, 32, 3.65, 0.128, 0.25));
+   offer(F32_TILE_64x32, tiled(64, 32, 3.9, 0.245, 0.5));
+   offer(F32_TILE_64, tiled(64, 64, 3.3, 0.452, 1.6));
+   offer(F32_TILE_128, tiled(128, 128, 7.0, 1.765, 4.0));
    if (time_us)
       *time_us = least;
    return best;
 }
-// The same for a convolution, whose tiles carry the arithmetic of the gather: 0.62 of the matrix rate in the loop and 0.7 us per
-// 32 x 32 block of a tile for its start and its store, and not less than 0.75 us per slab where a CU has one tile only.  The direct
-// kernel gathers for every 16 columns anew.
+// The same for a convolution, whose slabs wait for their gather: a load instruction brings 64 floats from three or four lines, and a
+// vector L1 takes four cycles per line.  A slab of 32 k takes 0.42 us (64 x 32 tiles), 0.60 (64 x 64: as many image elements for twice
+// the products) and 0.92 (128 x 32).  The direct kernel decomposes every k by itself: for few tiles only.
 static int pick_f32_conv_tile(int M, int N, int K, int group)
 {
    auto tiles = [&](int bm, int bn) { return (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * group; };
-   // A 64x32 tile gathers as many image elements as a 64x64 one for half the products: half the matrix rate against 0.64 of it
-   // (64 images of 32x32, 32 -> 64 channels: 46 us with 64x32 tiles, 38 us with 64x64; 74 and 62 us from 64 channels).
-   auto tiled = [&](int bm, int bn, double rate) {
-      const double rounds = std::ceil(tiles(bm, bn) / 256.0), blocks = (bm / 32) * (bn / 32), slabs = (K + 31) / 32;
-      return 3.0 + std::max(rounds * blocks * (slabs * 256.0 / (2400.0 * rate) + 0.7), 0.75 * slabs + 1.4);
-   };
+   const double slabs = (K + 31) / 32;
+   auto tiled = [&](int bm, int bn, double launch, double slab, double tile) { return launch + std::ceil(tiles(bm, bn) / 256.0) * (slabs * slab + tile); };
    int best = F32_DIRECT;
    double least = 5.3 + tiles(16, 16) / 256.0 * (0.9 + 0.17 * ((K + 15) / 16));
    auto offer = [&](int tile, double t) {
       if (t < least)
          least = t, best = tile;
    };
-   offer(F32_TILE_64x32, tiled(64, 32, 0.5));
-   offer(F32_TILE_64, tiled(64, 64, 0.64));
-   if (N <= 32 && tiles(128, 32) >= 1024) // a start per 128 rows instead of 64: first convolution of a 64-image network 29.7 -> 27.6 us
-      offer(F32_TILE_128x32, 0.95 * tiled(128, 32, 0.5));
+   offer(F32_TILE_64x32, tiled(64, 32, 6.5, 0.42, 1.15));
+   offer(F32_TILE_64, tiled(64, 64, 6.5, 0.60, 2.4));
+   offer(F32_TILE_128x32, tiled(128, 32, 6.0, 0.92, 1.5));
    return best;
 }
 
@@ -192,7 +184,7 @@ static int launch_f32_product(sofie_hip_ctx *ctx, const ASRC &A, const BSRC &B, 
 {
    hipStream_t s = ctx->stream;
    int tile = ctx->opt.f32_tile;
-   if (ctx->opt.f32_skinny == 1 || K == 0)
+   if (ctx->opt.f32_skinny == 1 || K == 0 || !A.in_buffers() || !B.in_buffers())
       tile = F32_DIRECT;
    else if (ctx->opt.f32_skinny == 0 && !tile)
       tile = F32_TILE_64;
@@ -204,7 +196,7 @@ static int launch_f32_product(sofie_hip_ctx *ctx, const ASRC &A, const BSRC &B, 
    if constexpr (CONV) {
       switch (tile) {
       case F32_TILE_64x32: return launch_f32_tile<ASRC, BSRC, STORE, 64, 32, 32, 2, 1, 2, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
-      case F32_TILE_128x32: return launch_f32_tile<ASRC, BSRC, STORE, 128, 32, 32, 4, 1, 1, 3>(s, A, B, out, M, N, K, batch, strideA, strideB);
+      case F32_TILE_128x32: return launch_f32_tile<ASRC, BSRC, STORE, 128, 32, 16, 4, 1, 1, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
       }
    } else {
       switch (tile) {
@@ -251,8 +243,12 @@ static int launch_f32_conv(sofie_hip_ctx *ctx, const float *X, F32ConvShape s, c
    s.positions = taps;
    auto reciprocal64 = [](unsigned d) -> unsigned long long { return d <= 1 ? 0ull : (~0ull / d) + 1; };
    s.ow_mul = reciprocal64(s.OW), s.oh_mul = reciprocal64(s.OH), s.od_mul = reciprocal64(s.OD);
-   // one bit per kernel position, and offsets inside an image (a few channels past the last one included) in 32 bits
-   if (taps <= 31 && ((long long)s.C + 4096) * s.D * s.H * s.W + ((long long)s.kd * s.dil_d * s.H + (long long)s.kh * s.dil_h) * s.W < (1LL << 31))
+   // one bit per kernel position; the images that the 128 rows of a tile touch within a buffer, and the channels within its scalar offset
+   const long long plane = (long long)s.D * s.H * s.W, window = ((long long)s.kd * s.dil_d * s.H + (long long)s.kh * s.dil_h) * s.W + (long long)s.kw * s.dil_w;
+   const long long images = 127 / ((long long)s.OD * s.OH * s.OW) + 2;
+   const long long padded = ((long long)s.pad_d * s.H + s.pad_h) * s.W + s.pad_w + ((long long)s.D * s.H + s.H) * s.W; // strides step inside it
+   if (taps <= 31 && (images * s.C * plane + 2 * padded) * 4 < F32_BUFFER_BYTES && (s.Cg * plane + window) * 4 < (1LL << 32) &&
+       (s.Cg + 64) * plane * 4 < (1LL << 32))
       return rows(F32ConvRows<true>{});
    return rows(F32ConvRows<false>{});
 }
