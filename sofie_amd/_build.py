@@ -3,11 +3,13 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "sofie_amd", "csrc")
 LIB_DIR = os.path.join(ROOT, "sofie_amd", "lib")
 LIB = os.path.join(LIB_DIR, "libsofie_hip.so")
+CALLS = os.path.join(LIB_DIR, "_calls.so")
 
 HIP_SOURCES = ["runtime.hip", "gemm_i8.hip", "gemm_f32.hip", "gemm_fp8.hip", "conv_i8.hip", "eltwise.hip"]
 
@@ -60,6 +62,13 @@ def build_hip_library(jobs=8):
     return lib
 
 
+def build_python_calls():
+    """The CPython module behind Runtime.call (sofie_amd/lib/_calls.so); host code, bound to the library's entry points when it is loaded."""
+    _run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-Wall", "-I" + sysconfig.get_paths()["include"],
+          "-I" + os.path.join(ROOT, "include"), os.path.join(CSRC, "python_calls.cpp"), "-o", CALLS])
+    return CALLS
+
+
 def build_oracle():
     """Builds the CPU checker (and oracle/_ref when the reference checkout is present)."""
     _run(["make", "-B", "-C", os.path.join(ROOT, "oracle"), "all"])
@@ -67,6 +76,7 @@ def build_oracle():
 
 def build_all():
     lib = build_hip_library()
+    build_python_calls()
     build_oracle()
     _run(["make", "-C", os.path.join(ROOT, "sofie_amd", "emit"), "-B", "-j8", "all"])
     return lib

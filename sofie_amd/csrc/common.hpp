@@ -61,6 +61,18 @@ int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
          return ::sofie_hip::fail(SOFIE_HIP_ERR_INVALID, __VA_ARGS__);                                \
    } while (0)
 
+// A kernel launch with its arguments where they are: the <<<>>> form stores the configuration for the calling thread and fetches
+// it again (0.17 of 2.39 us per launch).  An error is left for launch_status.
+template <class... P, class... A>
+inline void launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds_bytes, hipStream_t stream, A &&...a)
+{
+   static_assert(sizeof...(P) == sizeof...(A), "one argument per parameter of the kernel");
+   [&](P... p) {
+      void *args[] = {(void *)&p...};
+      (void)hipLaunchKernel((const void *)kernel, grid, block, args, lds_bytes, stream);
+   }(std::forward<A>(a)...);
+}
+
 inline int launch_status(const char *what)
 {
    hipError_t e = hipGetLastError();

@@ -133,7 +133,7 @@ int sofie_hip_pack_conv_weight_i8(sofie_hip_ctx *ctx, const sofie_conv_desc *d, 
    size_t blocks = (total + 255) / 256;
    if (blocks > 4096)
       blocks = 4096;
-   hipLaunchKernelGGL(pack_conv_weight_kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, dst, src, d->Cout, g);
+   launch_kernel(pack_conv_weight_kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, dst, src, d->Cout, g);
    return launch_status("pack_conv_weight_kernel");
 }
 
@@ -405,10 +405,10 @@ int sofie_hip_conv_i8(sofie_hip_ctx *ctx, const sofie_conv_desc *d, const sofie_
          if (blocks > 16384)
             blocks = 16384;
          if (fast)
-            hipLaunchKernelGGL(im2col_i8_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, (int8_t *)ws, a->X, g,
+            launch_kernel(im2col_i8_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, (int8_t *)ws, a->X, g,
                                grp * g.Cg, 1, img0 * OHW, rows);
          else
-            hipLaunchKernelGGL(im2col_i8_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, (int8_t *)ws, a->X, g,
+            launch_kernel(im2col_i8_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, (int8_t *)ws, a->X, g,
                                grp * g.Cg, a->x_layout == SOFIE_LAYOUT_NHWC, img0 * OHW, rows);
          st = launch_status("im2col_i8_kernel");
          if (st)

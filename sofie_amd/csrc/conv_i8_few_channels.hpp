@@ -171,7 +171,7 @@ static int launch_conv_i8_few_channels(const LaunchCfg &lc, FewChannelConv g, co
    int grid = (ngroups + 3) / 4;
    if (grid > 2 * ncu)
       grid = 2 * ncu;
-   hipLaunchKernelGGL(conv_i8_few_channels_kernel<EPI>, dim3((unsigned)grid), dim3(256), 0, lc.stream, g, Wp, Kp, ep, ngroups);
+   launch_kernel(conv_i8_few_channels_kernel<EPI>, dim3((unsigned)grid), dim3(256), 0, lc.stream, g, Wp, Kp, ep, ngroups);
    return launch_status("conv_i8_few_channels_kernel");
 }
 

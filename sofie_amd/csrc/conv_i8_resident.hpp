@@ -331,7 +331,7 @@ static int launch_conv_i8_resident(const LaunchCfg &lc, const ConvRows &a, const
    if (int st = cu_count_of_current_device(ncu))
       return st;
    const int grid = ntiles < ncu ? ntiles : ncu;
-   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), smem, lc.stream, g, Wp, ep, ntiles);
+   launch_kernel(kern, dim3((unsigned)grid), dim3(512), smem, lc.stream, g, Wp, ep, ntiles);
    return launch_status("conv_i8_resident_kernel");
 }
 

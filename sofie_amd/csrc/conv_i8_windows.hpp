@@ -121,7 +121,7 @@ static int launch_conv_i8_windows(const LaunchCfg &lc, FewChannelConv g, int str
       grid = 1024;
    auto go = [&](auto nt) {
       constexpr int NT = decltype(nt)::value;
-      hipLaunchKernelGGL((conv_i8_windows_kernel<EPI, NT>), dim3((unsigned)grid), dim3(256), 0, lc.stream, g, stride_w, Wp, Kp, ep, M, N, ngroups);
+      launch_kernel((conv_i8_windows_kernel<EPI, NT>), dim3((unsigned)grid), dim3(256), 0, lc.stream, g, stride_w, Wp, Kp, ep, M, N, ngroups);
       return launch_status("conv_i8_windows_kernel");
    };
    return N <= 16 ? go(std::integral_constant<int, 1>{}) : N <= 32 ? go(std::integral_constant<int, 2>{}) : go(std::integral_constant<int, 4>{});

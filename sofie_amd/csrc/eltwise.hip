@@ -269,9 +269,9 @@ static int launch_transpose(sofie_hip_ctx *ctx, float *Y, const float *X, size_t
          g.sx[k] = sh.sx[k];
       }
       if (vec)
-         hipLaunchKernelGGL((transpose_f32_kernel<f32x4, DIV>), dim3(grid_for(n)), dim3(256), 0, ctx->stream, (f32x4 *)Y, (const f32x4 *)X, n, g);
+         launch_kernel((transpose_f32_kernel<f32x4, DIV>), dim3(grid_for(n)), dim3(256), 0, ctx->stream, (f32x4 *)Y, (const f32x4 *)X, n, g);
       else
-         hipLaunchKernelGGL((transpose_f32_kernel<float, DIV>), dim3(grid_for(n)), dim3(256), 0, ctx->stream, Y, X, n, g);
+         launch_kernel((transpose_f32_kernel<float, DIV>), dim3(grid_for(n)), dim3(256), 0, ctx->stream, Y, X, n, g);
    };
    if (n < (1ull << 31))
       go(Divisor31(1));
@@ -844,7 +844,7 @@ int sofie_hip_quantize_linear(sofie_hip_ctx *ctx, int8_t *dst, const float *src,
    SOFIE_HIP_REQUIRE(dst && src, "sofie_hip_quantize_linear: NULL pointer");
    SOFIE_HIP_REQUIRE(scale > 0.0f, "sofie_hip_quantize_linear: scale must be positive");
    const int vec = (((uintptr_t)src & 15) == 0) && (((uintptr_t)dst & 3) == 0);
-   hipLaunchKernelGGL(quantize_linear_kernel, dim3(grid_for(vec ? (n + 15) / 16 : n)), dim3(256), 0, ctx->stream, dst, src, n, scale, vec);
+   launch_kernel(quantize_linear_kernel, dim3(grid_for(vec ? (n + 15) / 16 : n)), dim3(256), 0, ctx->stream, dst, src, n, scale, vec);
    return launch_status("quantize_linear_kernel");
 }
 
@@ -854,7 +854,7 @@ int sofie_hip_dequantize_linear_i8(sofie_hip_ctx *ctx, float *dst, const int8_t 
    if (n == 0)
       return SOFIE_HIP_OK;
    SOFIE_HIP_REQUIRE(dst && src, "sofie_hip_dequantize_linear_i8: NULL pointer");
-   hipLaunchKernelGGL(dequantize_linear_kernel<int8_t>, dim3(grid_for(n)), dim3(256), 0, ctx->stream, dst, src, n, scale);
+   launch_kernel(dequantize_linear_kernel<int8_t>, dim3(grid_for(n)), dim3(256), 0, ctx->stream, dst, src, n, scale);
    return launch_status("dequantize_linear_kernel");
 }
 
@@ -864,14 +864,14 @@ int sofie_hip_dequantize_linear_i32(sofie_hip_ctx *ctx, float *dst, const int32_
    if (n == 0)
       return SOFIE_HIP_OK;
    SOFIE_HIP_REQUIRE(dst && src, "sofie_hip_dequantize_linear_i32: NULL pointer");
-   hipLaunchKernelGGL(dequantize_linear_kernel<int32_t>, dim3(grid_for(n)), dim3(256), 0, ctx->stream, dst, src, n, scale);
+   launch_kernel(dequantize_linear_kernel<int32_t>, dim3(grid_for(n)), dim3(256), 0, ctx->stream, dst, src, n, scale);
    return launch_status("dequantize_linear_kernel");
 }
 
 static int launch_unary_chain(sofie_hip_ctx *ctx, float *dst, const float *src, size_t n, const PostChain &chain)
 {
    const int vec = (((uintptr_t)src & 15) == 0) && (((uintptr_t)dst & 15) == 0);
-   hipLaunchKernelGGL(unary_f32_kernel, dim3(grid_for(vec ? (n + 3) / 4 : n)), dim3(256), 0, ctx->stream, dst, src, n, chain, vec);
+   launch_kernel(unary_f32_kernel, dim3(grid_for(vec ? (n + 3) / 4 : n)), dim3(256), 0, ctx->stream, dst, src, n, chain, vec);
    return launch_status("unary_f32_kernel");
 }
 
@@ -930,10 +930,10 @@ int sofie_hip_binary_f32(sofie_hip_ctx *ctx, const sofie_add_desc *d, int32_t op
       return SOFIE_HIP_OK;
    SOFIE_HIP_REQUIRE(d->A && d->B && d->Y, "sofie_hip_add_f32: NULL pointer");
    if (op == SOFIE_BINARY_ADD) {
-      hipLaunchKernelGGL(add_f32_kernel, dim3(grid_for(n)), dim3(256), 0, ctx->stream, d->Y, d->A, d->B, n, sh);
+      launch_kernel(add_f32_kernel, dim3(grid_for(n)), dim3(256), 0, ctx->stream, d->Y, d->A, d->B, n, sh);
       return launch_status("add_f32_kernel");
    }
-   hipLaunchKernelGGL(binary_f32_kernel, dim3(grid_for(n)), dim3(256), 0, ctx->stream, d->Y, d->A, d->B, n, sh, op, param);
+   launch_kernel(binary_f32_kernel, dim3(grid_for(n)), dim3(256), 0, ctx->stream, d->Y, d->A, d->B, n, sh, op, param);
    return launch_status("binary_f32_kernel");
 }
 
@@ -950,10 +950,10 @@ int sofie_hip_batchnorm_f32(sofie_hip_ctx *ctx, float *Y, const float *X, const 
    auto go = [&](auto div) {
       typedef decltype(div) DIV;
       if (vec)
-         hipLaunchKernelGGL((batchnorm_f32_kernel<f32x4, DIV>), dim3(grid_for((n / 4 + 3) / 4)), dim3(256), 0, ctx->stream, (f32x4 *)Y, (const f32x4 *)X,
+         launch_kernel((batchnorm_f32_kernel<f32x4, DIV>), dim3(grid_for((n / 4 + 3) / 4)), dim3(256), 0, ctx->stream, (f32x4 *)Y, (const f32x4 *)X,
                             fused_scale, mean, bias, n / 4, DIV(C), DIV(spatial / 4), relu);
       else
-         hipLaunchKernelGGL((batchnorm_f32_kernel<float, DIV>), dim3(grid_for((n + 3) / 4)), dim3(256), 0, ctx->stream, Y, X, fused_scale, mean, bias, n, DIV(C),
+         launch_kernel((batchnorm_f32_kernel<float, DIV>), dim3(grid_for((n + 3) / 4)), dim3(256), 0, ctx->stream, Y, X, fused_scale, mean, bias, n, DIV(C),
                             DIV(spatial), relu);
    };
    if (n < (1ull << 31))
@@ -986,7 +986,7 @@ int sofie_hip_pool3d_f32(sofie_hip_ctx *ctx, const sofie_pool3d_desc *d, float *
    auto window = [&](auto div) {
       typedef decltype(div) DIV;
       const DIV o0(d->out[0]), o1(d->out[1]), o2(d->out[2]);
-      auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid_for((size_t)total)), dim3(256), 0, ctx->stream, Y, X, *d, (size_t)total, o0, o1, o2); };
+      auto go = [&](auto kernel) { launch_kernel(kernel, dim3(grid_for((size_t)total)), dim3(256), 0, ctx->stream, Y, X, *d, (size_t)total, o0, o1, o2); };
       // the flat windows in common use; the first axis has to be one of a single, unpadded slice
       const bool flat = d->in[0] == 1 && d->out[0] == 1 && d->k[0] == 1 && d->pad_begin[0] == 0;
       if (flat && d->k[1] == 3 && d->k[2] == 3)
@@ -1034,7 +1034,7 @@ int sofie_hip_global_avg_pool_f32(sofie_hip_ctx *ctx, float *Y, const float *X, 
    if (NC == 0)
       return SOFIE_HIP_OK;
    SOFIE_HIP_REQUIRE(Y && X, "sofie_hip_global_avg_pool_f32: NULL pointer");
-   hipLaunchKernelGGL((gap_kernel<float, float>), dim3((NC + 3) / 4), dim3(256), 0, ctx->stream, Y, X, NC, HW, 1.0f,
+   launch_kernel((gap_kernel<float, float>), dim3((NC + 3) / 4), dim3(256), 0, ctx->stream, Y, X, NC, HW, 1.0f,
                       (int)(HW % 4 == 0 && ((uintptr_t)X & 15) == 0));
    return launch_status("gap_kernel");
 }
@@ -1056,14 +1056,14 @@ int sofie_hip_global_avg_pool_i8(sofie_hip_ctx *ctx, float *Y, const int8_t *X, 
          auto blocks = [&] { return (C + (16 << chunks_log2) - 1) / (16 << chunks_log2); };
          while (chunks_log2 > 0 && (long long)N * blocks() < 256)
             --chunks_log2;
-         hipLaunchKernelGGL(gap_i8_nhwc_vec_kernel, dim3((unsigned)N, (unsigned)blocks()), dim3(GAP_THREADS), 0, ctx->stream, Y, X, C, HW, scale, chunks_log2);
+         launch_kernel(gap_i8_nhwc_vec_kernel, dim3((unsigned)N, (unsigned)blocks()), dim3(GAP_THREADS), 0, ctx->stream, Y, X, C, HW, scale, chunks_log2);
          return launch_status("gap_i8_nhwc_vec_kernel");
       }
-      hipLaunchKernelGGL(gap_i8_nhwc_kernel, dim3((unsigned)N), dim3(256), 0, ctx->stream, Y, X, C, HW, scale);
+      launch_kernel(gap_i8_nhwc_kernel, dim3((unsigned)N), dim3(256), 0, ctx->stream, Y, X, C, HW, scale);
       return launch_status("gap_i8_nhwc_kernel");
    }
    const int NC = N * C;
-   hipLaunchKernelGGL((gap_kernel<int8_t, int>), dim3((NC + 3) / 4), dim3(256), 0, ctx->stream, Y, X, NC, HW, scale, 0);
+   launch_kernel((gap_kernel<int8_t, int>), dim3((NC + 3) / 4), dim3(256), 0, ctx->stream, Y, X, NC, HW, scale, 0);
    return launch_status("gap_kernel");
 }
 
@@ -1133,7 +1133,7 @@ int sofie_hip_copy_rows(sofie_hip_ctx *ctx, void *dst, size_t dst_pitch_bytes, c
    if (rows == 0 || row_bytes == 0)
       return SOFIE_HIP_OK;
    SOFIE_HIP_REQUIRE(dst && src && (((uintptr_t)dst | (uintptr_t)src) & 3) == 0, "sofie_hip_copy_rows: NULL or misaligned pointer");
-   hipLaunchKernelGGL(copy_rows_kernel, dim3(grid_for(rows * (row_bytes / 4))), dim3(256), 0, ctx->stream, (uint32_t *)dst, dst_pitch_bytes / 4,
+   launch_kernel(copy_rows_kernel, dim3(grid_for(rows * (row_bytes / 4))), dim3(256), 0, ctx->stream, (uint32_t *)dst, dst_pitch_bytes / 4,
                       (const uint32_t *)src, src_pitch_bytes / 4, rows, row_bytes / 4);
    return launch_status("copy_rows_kernel");
 }
@@ -1148,12 +1148,12 @@ int sofie_hip_softmax_f32(sofie_hip_ctx *ctx, float *Y, const float *X, int64_t 
       return SOFIE_HIP_OK;
    SOFIE_HIP_REQUIRE(Y && X, "sofie_hip_softmax_f32: NULL pointer");
    if (inner == 1 && with_line_registers(lines, axis_len, (((uintptr_t)X | (uintptr_t)Y) & 15) == 0, [&](auto vec, auto nv, int G, unsigned blocks) {
-          hipLaunchKernelGGL((softmax_lines_f32_kernel<decltype(vec)::value, decltype(nv)::value>), dim3(blocks), dim3(256), 0, ctx->stream, Y, X, lines, axis_len, G,
+          launch_kernel((softmax_lines_f32_kernel<decltype(vec)::value, decltype(nv)::value>), dim3(blocks), dim3(256), 0, ctx->stream, Y, X, lines, axis_len, G,
                              log_softmax);
        }))
       return launch_status("softmax_lines_f32_kernel");
    const long long blocks = (lines + 3) / 4;
-   hipLaunchKernelGGL(softmax_f32_kernel, dim3((unsigned)(blocks < 256 * 64 ? blocks : 256 * 64)), dim3(256), 0, ctx->stream, Y, X, lines, axis_len,
+   launch_kernel(softmax_f32_kernel, dim3((unsigned)(blocks < 256 * 64 ? blocks : 256 * 64)), dim3(256), 0, ctx->stream, Y, X, lines, axis_len,
                       (long long)inner, log_softmax);
    return launch_status("softmax_f32_kernel");
 }
@@ -1169,10 +1169,10 @@ int sofie_hip_reduce_f32(sofie_hip_ctx *ctx, float *Y, const float *X, int64_t o
       return SOFIE_HIP_OK;
    SOFIE_HIP_REQUIRE(Y && X, "sofie_hip_reduce_f32: NULL pointer");
    if (inner == 1 && A >= 64 && outputs < 16384) {
-      hipLaunchKernelGGL(reduce_lines_f32_kernel, dim3((unsigned)((outputs + 3) / 4)), dim3(256), 0, ctx->stream, Y, X, outputs, A, op);
+      launch_kernel(reduce_lines_f32_kernel, dim3((unsigned)((outputs + 3) / 4)), dim3(256), 0, ctx->stream, Y, X, outputs, A, op);
       return launch_status("reduce_lines_f32_kernel");
    }
-   hipLaunchKernelGGL(reduce_f32_kernel, dim3(grid_for((size_t)outputs)), dim3(256), 0, ctx->stream, Y, X, (size_t)outputs, A, (long long)inner, op);
+   launch_kernel(reduce_f32_kernel, dim3(grid_for((size_t)outputs)), dim3(256), 0, ctx->stream, Y, X, (size_t)outputs, A, (long long)inner, op);
    return launch_status("reduce_f32_kernel");
 }
 
@@ -1187,12 +1187,12 @@ int sofie_hip_layernorm_f32(sofie_hip_ctx *ctx, float *Y, const float *X, const 
    SOFIE_HIP_REQUIRE(Y && X && scale, "sofie_hip_layernorm_f32: NULL pointer");
    const uintptr_t addresses = (uintptr_t)X | (uintptr_t)Y | (uintptr_t)scale | (uintptr_t)bias;
    if (with_line_registers(rows, L, (addresses & 15) == 0, [&](auto vec, auto nv, int G, unsigned blocks) {
-          hipLaunchKernelGGL((layernorm_lines_f32_kernel<decltype(vec)::value, decltype(nv)::value>), dim3(blocks), dim3(256), 0, ctx->stream, Y, X, scale, bias,
+          launch_kernel((layernorm_lines_f32_kernel<decltype(vec)::value, decltype(nv)::value>), dim3(blocks), dim3(256), 0, ctx->stream, Y, X, scale, bias,
                              (long long)rows, L, G, epsilon, mean_out, inv_std_out);
        }))
       return launch_status("layernorm_lines_f32_kernel");
    const long long blocks = (rows + 3) / 4;
-   hipLaunchKernelGGL(layernorm_f32_kernel, dim3((unsigned)(blocks < 256 * 64 ? blocks : 256 * 64)), dim3(256), 0, ctx->stream, Y, X, scale, bias, (long long)rows, L,
+   launch_kernel(layernorm_f32_kernel, dim3((unsigned)(blocks < 256 * 64 ? blocks : 256 * 64)), dim3(256), 0, ctx->stream, Y, X, scale, bias, (long long)rows, L,
                       epsilon, mean_out, inv_std_out);
    return launch_status("layernorm_f32_kernel");
 }
@@ -1204,7 +1204,7 @@ int sofie_hip_plane_sums_to_average(sofie_hip_ctx *ctx, float *Y, const int32_t 
    if (NC == 0)
       return SOFIE_HIP_OK;
    SOFIE_HIP_REQUIRE(Y && sums, "sofie_hip_plane_sums_to_average: NULL pointer");
-   hipLaunchKernelGGL(plane_sums_to_average_kernel, dim3((NC + 255) / 256), dim3(256), 0, ctx->stream, Y, sums, NC, HW, scale);
+   launch_kernel(plane_sums_to_average_kernel, dim3((NC + 255) / 256), dim3(256), 0, ctx->stream, Y, sums, NC, HW, scale);
    return launch_status("plane_sums_to_average_kernel");
 }
 
@@ -1215,7 +1215,7 @@ int sofie_hip_plane_sums_take_average(sofie_hip_ctx *ctx, float *Y, int32_t *sum
    if (NC == 0)
       return SOFIE_HIP_OK;
    SOFIE_HIP_REQUIRE(Y && sums, "sofie_hip_plane_sums_take_average: NULL pointer");
-   hipLaunchKernelGGL(plane_sums_take_average_kernel, dim3((NC + 255) / 256), dim3(256), 0, ctx->stream, Y, sums, NC, HW, scale);
+   launch_kernel(plane_sums_take_average_kernel, dim3((NC + 255) / 256), dim3(256), 0, ctx->stream, Y, sums, NC, HW, scale);
    return launch_status("plane_sums_take_average_kernel");
 }
 

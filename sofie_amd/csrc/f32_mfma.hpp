@@ -842,7 +842,7 @@ static int launch_f32_tile(hipStream_t stream, const ASRC &A, const BSRC &B, con
    static bool configured[64] = {};
    if (int st = configure_lds_once(kern, most, configured))
       return st;
-   hipLaunchKernelGGL(kern, dim3((unsigned)nwg, 1, (unsigned)batch), dim3(WAVES_M * WAVES_N * WAVES_K * 64), smem, stream, A, B, out, M, N, K, tiles_m, tiles_n, strideA,
+   launch_kernel(kern, dim3((unsigned)nwg, 1, (unsigned)batch), dim3(WAVES_M * WAVES_N * WAVES_K * 64), smem, stream, A, B, out, M, N, K, tiles_m, tiles_n, strideA,
                       strideB);
    return launch_status("f32_tile_kernel");
 }
@@ -854,7 +854,7 @@ static int launch_f32_direct(hipStream_t stream, const ASRC &A, const BSRC &B, c
    const long long nwg = (long long)tiles_m * tiles_n;
    if (nwg > 0x7fffffffLL)
       return fail(SOFIE_HIP_ERR_INVALID, "fp32 product: too many tiles");
-   hipLaunchKernelGGL((f32_direct_kernel<ASRC, BSRC, STORE, MB, NB, W, UNROLL>), dim3((unsigned)nwg, 1, (unsigned)batch), dim3(W * 64), 0, stream, A, B, out, M, N, K,
+   launch_kernel((f32_direct_kernel<ASRC, BSRC, STORE, MB, NB, W, UNROLL>), dim3((unsigned)nwg, 1, (unsigned)batch), dim3(W * 64), 0, stream, A, B, out, M, N, K,
                       tiles_m, tiles_n, strideA, strideB);
    return launch_status("f32_direct_kernel");
 }

@@ -336,11 +336,11 @@ static int launch_f32_chain(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *layer
       const size_t lds = (size_t)2 * RB * width * sizeof(float);
       const dim3 grid((unsigned)((M + RB - 1) / RB));
       if (RB == 1)
-         hipLaunchKernelGGL(gemm_chain_f32_kernel<1>, grid, dim3(CHAIN_THREADS), lds, ctx->stream, a, width);
+         launch_kernel(gemm_chain_f32_kernel<1>, grid, dim3(CHAIN_THREADS), lds, ctx->stream, a, width);
       else if (RB == 2)
-         hipLaunchKernelGGL(gemm_chain_f32_kernel<2>, grid, dim3(CHAIN_THREADS), lds, ctx->stream, a, width);
+         launch_kernel(gemm_chain_f32_kernel<2>, grid, dim3(CHAIN_THREADS), lds, ctx->stream, a, width);
       else
-         hipLaunchKernelGGL(gemm_chain_f32_kernel<4>, grid, dim3(CHAIN_THREADS), lds, ctx->stream, a, width);
+         launch_kernel(gemm_chain_f32_kernel<4>, grid, dim3(CHAIN_THREADS), lds, ctx->stream, a, width);
       *launched = true;
       return launch_status("gemm_chain_f32_kernel");
    }

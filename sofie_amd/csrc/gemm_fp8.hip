@@ -211,7 +211,7 @@ int sofie_hip_quantize_fp8(sofie_hip_ctx *ctx, uint8_t *dst, const float *src, s
    size_t blocks = (n + 255) / 256;
    if (blocks > 8192)
       blocks = 8192;
-   hipLaunchKernelGGL(quantize_fp8_kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, dst, src, n, scale);
+   launch_kernel(quantize_fp8_kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, dst, src, n, scale);
    return launch_status("quantize_fp8_kernel");
 }
 

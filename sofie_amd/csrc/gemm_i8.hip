@@ -127,11 +127,11 @@ int conv_i8_few_channels(const LaunchCfg &lc, const FewChannelConv &src, const i
 int transpose_i8(hipStream_t stream, int8_t *dst, const int8_t *src, int rows, int cols, int ld_src, int ld_dst)
 {
    if (cols < 8) {
-      hipLaunchKernelGGL(transpose_few_columns_i8_kernel, dim3((rows + 255) / 256), dim3(256), 0, stream, dst, src, rows, cols, ld_src, ld_dst);
+      launch_kernel(transpose_few_columns_i8_kernel, dim3((rows + 255) / 256), dim3(256), 0, stream, dst, src, rows, cols, ld_src, ld_dst);
       return launch_status("transpose_few_columns_i8_kernel");
    }
    dim3 grid((cols + 63) / 64, (rows + 127) / 128);
-   hipLaunchKernelGGL(transpose_i8_kernel, grid, dim3(256), 0, stream, dst, src, rows, cols, ld_src, ld_dst);
+   launch_kernel(transpose_i8_kernel, grid, dim3(256), 0, stream, dst, src, rows, cols, ld_src, ld_dst);
    return launch_status("transpose_i8_kernel");
 }
 

@@ -204,7 +204,7 @@ static int launch_mfma8_direct(const LaunchCfg &lc, const int8_t *A, const int8_
    const long long nwg = (long long)tiles_m * tiles_n;
    if (nwg > 0x7fffffffLL)
       return fail(SOFIE_HIP_ERR_INVALID, "gemm: too many tiles");
-   hipLaunchKernelGGL((mfma8_direct_kernel<MMA, MB, NB, W, UNROLL, EPI>), dim3((unsigned)nwg), dim3(W * 64), 0, lc.stream, RowMajorRows{A, lda}, RowMajorRows{Bt, ldb}, M, N,
+   launch_kernel((mfma8_direct_kernel<MMA, MB, NB, W, UNROLL, EPI>), dim3((unsigned)nwg), dim3(W * 64), 0, lc.stream, RowMajorRows{A, lda}, RowMajorRows{Bt, ldb}, M, N,
                       K, ep, tiles_m, tiles_n, lc.swizzle);
    return launch_status("mfma8_direct_kernel");
 }

@@ -157,7 +157,7 @@ static int launch_mfma8_gather_kp(const LaunchCfg &lc, const GatherConvRows &a, 
       return st;
    GatherConvRowsT<KP> src;
    static_cast<GatherConvRows &>(src) = a;
-   hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(256), smem, lc.stream, src, RowMajorRows{Wp, KP}, M, N, ep, tiles_m, tiles_n, 0);
+   launch_kernel(kern, dim3((unsigned)nwg), dim3(256), smem, lc.stream, src, RowMajorRows{Wp, KP}, M, N, ep, tiles_m, tiles_n, 0);
    return launch_status("mfma8_gather_kernel");
 }
 

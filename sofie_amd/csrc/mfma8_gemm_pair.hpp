@@ -201,7 +201,7 @@ static int launch_mfma8_pair_src(const LaunchCfg &lc, const ASRC &a, const int8_
    static bool configured[64] = {};
    if (int st = configure_lds_once(kern, smem, configured))
       return st;
-   hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(NTHREADS), smem, lc.stream, a, b, M, N, K, ep, tiles_m, tiles_n, lc.swizzle);
+   launch_kernel(kern, dim3((unsigned)nwg), dim3(NTHREADS), smem, lc.stream, a, b, M, N, K, ep, tiles_m, tiles_n, lc.swizzle);
    return launch_status("mfma8_gemm_pair_kernel");
 }
 

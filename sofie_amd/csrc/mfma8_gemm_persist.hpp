@@ -622,7 +622,7 @@ static int launch_mfma8_persist_src(const LaunchCfg &lc, const ASRC &a, const in
    if (int st = cu_count_of_current_device(ncu))
       return st;
    const int grid = ntiles < ncu ? ntiles : ncu;
-   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), smem, lc.stream, a, Bt, ldb, M, N, K, ep, tiles_m, tiles_n, lc.swizzle);
+   launch_kernel(kern, dim3((unsigned)grid), dim3(512), smem, lc.stream, a, Bt, ldb, M, N, K, ep, tiles_m, tiles_n, lc.swizzle);
    return launch_status("mfma8_gemm_persist_kernel");
 }
 

@@ -373,7 +373,7 @@ static int launch_mfma8_staged(const LaunchCfg &lc, const ASRC &A, const BSRC &B
    static bool configured[64] = {};
    if (int st = configure_lds_once(kern, smem, configured))
       return st;
-   hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(WAVES_M * WAVES_N * 64), smem, lc.stream, A, B, M, N, K, ep, tiles_m, tiles_n, lc.swizzle);
+   launch_kernel(kern, dim3((unsigned)nwg), dim3(WAVES_M * WAVES_N * 64), smem, lc.stream, A, B, M, N, K, ep, tiles_m, tiles_n, lc.swizzle);
    return launch_status("mfma8_staged_kernel");
 }
 

@@ -214,11 +214,11 @@ int sofie_hip_fill_zero(sofie_hip_ctx *ctx, void *dst_device, size_t bytes)
       size_t blocks = (nwords + 255) / 256;
       if (blocks > 65536)
          blocks = 65536;
-      hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, (uint32_t *)dst_device, nwords);
+      launch_kernel(fill_zero_kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, (uint32_t *)dst_device, nwords);
    } else {
       size_t blocks = (bytes + 255) / 256;
       SOFIE_HIP_REQUIRE(blocks < (1ull << 31), "sofie_hip_fill_zero: unaligned region too large");
-      hipLaunchKernelGGL(fill_zero_bytes_kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, (uint8_t *)dst_device, bytes);
+      launch_kernel(fill_zero_bytes_kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, (uint8_t *)dst_device, bytes);
    }
    return launch_status("fill_zero");
 }

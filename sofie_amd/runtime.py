@@ -3,6 +3,7 @@
 There is no fallback: if the library is not built, loading raises.
 """
 import ctypes as C
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -106,6 +107,7 @@ class ConvI8Args(C.Structure):
 
 # every symbol include/sofie_hip.h declares: name -> (restype, argtypes)
 _P = C.c_void_p
+_POINTER_TYPE = type(C.POINTER(C.c_int))
 SYMBOLS = {
     "sofie_hip_ctx_create": (C.c_int, [C.POINTER(_P), C.c_int, _P]),
     "sofie_hip_ctx_destroy": (C.c_int, [_P]),
@@ -184,7 +186,42 @@ def load_library(path=None):
         fn.argtypes = args
     if path is None:
         _lib = lib
+        _bind_calls(lib)
     return lib
+
+
+_calls = None
+
+
+def _bind_calls(lib):
+    """Load the native module that makes the calls of Runtime.call and give it the library's entry points."""
+    global _calls
+    where = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "_calls.so")
+    if not os.path.exists(where):
+        raise SofieHipError("%s is not built: run `python -c 'import __graft_entry__ as g; g.build()'`" % where)
+    spec = importlib.util.spec_from_file_location("_calls", where)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    p, four, sized, real = _P(77), (C.c_int64 * 4)(), C.c_size_t(3), C.c_float(1.5)
+    instances = [(o, C.addressof(o)) for o in (p, four, sized, real)]
+    d, e = GemmF32Desc(), ConvDesc()
+    refs = [(C.byref(o, at), C.addressof(o) + at, o) for o, at in ((d, 0), (e, 0), (d, 8), (four, 16))]
+    module.layout(_P, C.c_size_t, C.c_float, C.Array, type(C.byref(d)), instances, refs)
+    for name, (res, args) in SYMBOLS.items():
+        if res is C.c_int and args and args[0] is _P:
+            module.entry(name, C.cast(getattr(lib, name), _P).value, tuple(getattr(a, "_type_", None) if a.__class__ is _POINTER_TYPE else None for a in args[1:]))
+    _calls = module
+
+
+def _check(lib, status):
+    if status != 0:
+        raise SofieHipError("sofie_hip status %d: %s" % (status, (lib.sofie_hip_last_error() or b"").decode()))
+
+
+def _call_slowly(ctx, status, name, *args):
+    """A call through ctypes, for arguments the native path does not convert; with a status, the report of a native call that failed."""
+    lib = load_library()
+    _check(lib, getattr(lib, name)(ctx, *args) if status is None else status)
 
 
 class Runtime:
@@ -193,26 +230,22 @@ class Runtime:
     def __init__(self, device=0, external_stream=None):
         self.lib = load_library()
         h = C.c_void_p()
-        self._check(self.lib.sofie_hip_ctx_create(C.byref(h), device, external_stream))
+        _check(self.lib, self.lib.sofie_hip_ctx_create(C.byref(h), device, external_stream))
         self.ctx = h
+        # call(name, *args): the entry point of that name on this context
+        self.call = _calls.caller(h.value, _call_slowly)
 
     def close(self):
         if getattr(self, "ctx", None):
             self.lib.sofie_hip_ctx_destroy(self.ctx)
             self.ctx = None
+            self.call = _calls.caller(0, _call_slowly)   # from here on every call is refused
 
     def __del__(self):
         try:
             self.close()
         except Exception:
             pass
-
-    def _check(self, status):
-        if status != 0:
-            raise SofieHipError("sofie_hip status %d: %s" % (status, (self.lib.sofie_hip_last_error() or b"").decode()))
-
-    def call(self, name, *args):
-        self._check(getattr(self.lib, name)(self.ctx, *args))
 
     def set_option(self, name, value):
         """Kernel-choice override of this context (see sofie_hip_ctx_set_option)."""

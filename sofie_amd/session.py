@@ -87,6 +87,9 @@ class Int8MLPSession:
             d.Y = p(dst)
             src = dst
             self.descs.append(d)
+        # one inference, its arguments made once
+        self.calls = [("sofie_hip_quantize_linear", p(self.off_xq), self.x_ptr, M * self.dims[0], C.c_float(float(self.in_scales[0])))]
+        self.calls += [("sofie_hip_gemm_i8", C.byref(d)) for d in self.descs]
 
     @property
     def x_ptr(self):
@@ -103,11 +106,9 @@ class Int8MLPSession:
 
     def infer_nosync(self):
         """Enqueue one inference over the input resident at x_ptr; the result lands at y_ptr."""
-        rt = self.rt
-        rt.call("sofie_hip_quantize_linear", self.p(self.off_xq), self.x_ptr, C.c_size_t(self.batch * self.dims[0]),
-                C.c_float(float(self.in_scales[0])))
-        for d in self.descs:
-            rt.call("sofie_hip_gemm_i8", C.byref(d))
+        call = self.rt.call
+        for c in self.calls:
+            call(*c)
 
     def infer(self, x):
         self.upload_input(x)
@@ -228,6 +229,18 @@ class Int8CNNSession:
         g.A, g.B, g.C, g.Y = p(self.off_pool), p(self.off_fcw), p(self.off_fcb), p(self.off_y)
         g.bias_mode, g.act, g.batch = R.BIAS_ROW, R.ACT_NONE, 1
         self.fc = g
+        # one inference, its arguments made once
+        c, h, w = self.out_shape
+        last_scale = C.c_float(float(self.last_scale))
+        self.calls = [("sofie_hip_quantize_linear", p(self.off_xq), self.x_ptr, N * Cin * H * W, C.c_float(float(self.in_scale)))]
+        if self.pool_in_conv:
+            self.calls.append(("sofie_hip_fill_zero", p(self.off_sums), 4 * N * c))
+        self.calls += [("sofie_hip_conv_i8", C.byref(d), C.byref(a)) for d, a in zip(self.conv_descs, self.conv_args)]
+        if self.pool_in_conv:
+            self.calls.append(("sofie_hip_plane_sums_to_average", p(self.off_pool), p(self.off_sums), N * c, h * w, last_scale))
+        else:
+            self.calls.append(("sofie_hip_global_avg_pool_i8", p(self.off_pool), p(self.off_last), N, c, h * w, R.LAYOUT_NHWC, last_scale))
+        self.calls.append(("sofie_hip_gemm_f32", C.byref(g)))
 
     @property
     def x_ptr(self):
@@ -243,22 +256,9 @@ class Int8CNNSession:
         self.rt.call("sofie_hip_upload", self.x_ptr, x.ctypes.data_as(C.c_void_p), C.c_size_t(x.nbytes))
 
     def infer_nosync(self):
-        rt = self.rt
-        Cin, H, W = self.in_shape
-        rt.call("sofie_hip_quantize_linear", self.p(self.off_xq), self.x_ptr, C.c_size_t(self.batch * Cin * H * W),
-                C.c_float(float(self.in_scale)))
-        c, h, w = self.out_shape
-        if self.pool_in_conv:
-            rt.call("sofie_hip_fill_zero", self.p(self.off_sums), C.c_size_t(4 * self.batch * c))
-        for d, a in zip(self.conv_descs, self.conv_args):
-            rt.call("sofie_hip_conv_i8", C.byref(d), C.byref(a))
-        if self.pool_in_conv:
-            rt.call("sofie_hip_plane_sums_to_average", self.p(self.off_pool), self.p(self.off_sums), self.batch * c, h * w,
-                    C.c_float(float(self.last_scale)))
-        else:
-            rt.call("sofie_hip_global_avg_pool_i8", self.p(self.off_pool), self.p(self.off_last), self.batch, c, h * w, R.LAYOUT_NHWC,
-                    C.c_float(float(self.last_scale)))
-        rt.call("sofie_hip_gemm_f32", C.byref(self.fc))
+        call = self.rt.call
+        for c in self.calls:
+            call(*c)
 
     def infer(self, x):
         self.upload_input(x)
