@@ -1,0 +1,295 @@
+// fp32 3 x 3 convolution (stride 1, no dilation, two spatial axes) with the input patch of a tile in LDS.
+//
+// The implicit product of f32_mfma.hpp gathers every element of the column matrix, nine times the input: a load instruction of 64
+// floats touches three or four lines, and a slab of 32 k of a 64 x 64 tile took 0.60 us where its MFMAs take 0.43.  Here a tile is BM consecutive output pixels
+// (through rows and images) and BN output channels; what it reads of a channel is one run of rows, loaded once, and the nine kernel
+// positions read it from LDS at offsets that are known where the code is written.  64 images, us before -> after: 32 -> 64 channels at
+// 32 x 32 36.7 -> 26.8, 64 -> 64 57.2 -> 43.8 (110 TFLOP/s of the matrix cores' 157), 3 -> 32 at 64 x 64 24.2 -> 17.0; one image, 48 -> 96 at
+// 40 x 40 12.8 -> 8.4.
+//
+// The images are taken as one column of OH + 2 rows each, padding included (row r of image i is row i (OH + 2) + r), and OW + 2 columns:
+// the patch of a tile is the rows from its first pixel's to two below its last pixel's.
+#pragma once
+#include "f32_mfma.hpp"
+#include <algorithm>
+
+namespace sofie_hip {
+
+struct F32Conv3x3 {
+   const float *X, *W; // NCHW; [Cout][C][3][3]
+   int images, C, H, Wd, OH, OW, pad_h, pad_w; // C: channels per group
+   long long image, group;                     // elements per image and per group of channels
+   int M, N, K;                                // output pixels, output channels per group, 9 C
+   int chunks;                                 // of 64 positions that a patch fills
+   unsigned long long ow_mul, oh_mul, vw_mul, vh_mul; // ceil(2^64 / (OW, OH, OW + 2, OH + 2)), 0 for an extent of 1
+};
+
+constexpr int F32_CONV3X3_PATCH = 704; // the largest patch that is taken (a tile across two images of 98 columns: 686)
+
+// Positions of the patch of any tile of `bm` pixels: rows it touches, two more, and two per image that it runs into.
+inline long long f32_conv3x3_patch(int OH, int OW, int bm)
+{
+   const long long plane = (long long)OH * OW;
+   const long long rows = bm % OW == 0 ? bm / OW : (bm - 2 + OW) / OW + 1;
+   const long long images = plane % bm == 0 ? 0 : (bm - 2 + plane) / plane;
+   return (rows + 2 + 2 * images) * (OW + 2);
+}
+
+// CS channels per slab; lane half lk multiplies the channels from lk * CS / 2 on, kernel position by kernel position.
+template <int BM, int BN, int CS, int PLANE, int WVEC>
+struct F32Conv3x3Shape {
+   static constexpr int HALF = CS / 2 * 9;                      // k per lane half and slab
+   static constexpr int PITCH = CS == 8 ? 76 : 38;              // of a weight row in LDS: the rows of a fragment start in different banks
+   static constexpr int READ = CS == 8 ? 4 : 2;                 // floats of a weight row that a lane reads at once
+   static constexpr int PATCH = CS * PLANE + 32;                // the second half of the channels starts 32 banks on
+   static constexpr int WEIGHTS = (BN * PITCH + 64 * WVEC - 1) / (64 * WVEC) * 64 * WVEC;
+   static constexpr int STAGE = (PATCH + WEIGHTS + 3) / 4 * 4;
+   static constexpr int CHUNKS = PLANE / 64;                    // load instructions per channel
+   static constexpr int WLOADS = WEIGHTS / (64 * WVEC);         // load instructions per slab of weights
+   static_assert(PLANE % 64 == 0 && (WVEC == 1 || PITCH % 4 == 0), "whole load instructions");
+};
+
+// Two slabs in LDS, the next on its way while one is multiplied (2304 cycles of MFMAs for 32 x 32 wave tiles), and several workgroups per CU
+// that cover each other's trips to memory and barriers.  WAVES_K waves share a wave tile, each multiplying every WAVES_K-th step of
+// a slab: where there are few tiles, smaller ones keep as many matrix cores busy.
+template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int CS, int PLANE, int WVEC>
+__global__ __launch_bounds__(256, 2) void f32_conv3x3_kernel(F32Conv3x3 a, F32ConvStore out, int tiles_m, int tiles_n)
+{
+   typedef F32Conv3x3Shape<BM, BN, CS, PLANE, WVEC> S;
+   constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N, MT = TM / 32, NT = TN / 32;
+   constexpr int OWN = 16 / WAVES_K; // of a block's 16 elements per lane, those this wave finishes
+   static_assert(WAVES_M * WAVES_N * WAVES_K == 4 && TM % 32 == 0 && TN % 32 == 0, "four waves of 32 x 32 blocks");
+   extern __shared__ __attribute__((aligned(16))) float f32_lds[];
+   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+   const int wk = wave % WAVES_K, wm = wave / WAVES_K / WAVES_N, wn = wave / WAVES_K % WAVES_N, lk = lane >> 5, c = lane & 31;
+   const int z = blockIdx.z;
+   a.X += z * a.group;
+   a.W += (long long)z * a.N * a.K;
+   out.select_batch(z);
+   int tm, tn;
+   f32_tile_of_block(tiles_m, tiles_n, tm, tn);
+   const int m0 = tm * BM, n0 = tn * BN;
+   const int VW = a.OW + 2, VH = a.OH + 2;
+   auto quotient = [](int n, unsigned long long mul) { return mul ? (int)__umul64hi((unsigned long long)(unsigned)n, mul) : n; };
+
+   // where the patch begins
+   const int line0 = quotient(m0, a.ow_mul), image0 = quotient(line0, a.oh_mul);
+   const int row0 = line0 - image0 * a.OH; // of image0, padding row 0 first
+   const char *base = (const char *)uniform((long long)(a.X + image0 * a.image));
+   const int plane_bytes = a.H * a.Wd * 4;
+   int patch_at[S::CHUNKS]; // bytes from `base`, of channel 0
+#pragma unroll
+   for (int q = 0; q < S::CHUNKS; ++q) {
+      const int f = q * 64 + lane, vr = quotient(f, a.vw_mul), ix = f - vr * VW - a.pad_w;
+      const int on = row0 + vr, image = quotient(on, a.vh_mul), iy = on - image * VH - a.pad_h;
+      const bool inside = (unsigned)ix < (unsigned)a.Wd && (unsigned)iy < (unsigned)a.H && image0 + image < a.images;
+      patch_at[q] = inside ? (int)((image * a.image + (long long)iy * a.Wd + ix) * 4) : F32_OUTSIDE;
+   }
+   // the weights of this tile: rows past N and the gaps between rows read as zero
+   constexpr int LDW = (S::WLOADS + 3) / 4;
+   const char *weights = (const char *)uniform((long long)(a.W + (long long)n0 * a.K));
+   int weight_at[LDW];
+   auto weight_place = [&](int i, int &row, int &k) {
+      const int f = ((i * 4 + wave) * 64 + lane) * WVEC;
+      row = f / S::PITCH;
+      k = f - row * S::PITCH;
+   };
+#pragma unroll
+   for (int i = 0; i < LDW; ++i) {
+      int row, k;
+      weight_place(i, row, k);
+      weight_at[i] = n0 + row < a.N && k < 2 * S::HALF ? (row * a.K + k) * 4 : F32_OUTSIDE;
+   }
+
+   const int slabs = (a.C + CS - 1) / CS;
+   auto issue = [&](int s, int stage) {
+      float *lds = f32_lds + stage * S::STAGE;
+      // channels wave, wave + 4
+#pragma unroll
+      for (int h = 0; h < CS; h += 4) {
+         const int ch = h + wave;
+         const bool there = s * CS + ch < a.C;
+         float *to = lds + ch * PLANE + (ch >= CS / 2 ? 32 : 0);
+         const int offset = there ? (s * CS + ch) * plane_bytes : 0;
+#pragma unroll
+         for (int q = 0; q < S::CHUNKS; ++q)
+            if (q < a.chunks)
+               f32_buffer_load<1>((lds_void_t *)(to + q * 64), base, there ? patch_at[q] : F32_OUTSIDE, offset);
+      }
+      const bool whole = (s + 1) * CS <= a.C;
+#pragma unroll
+      for (int i = 0; i < LDW; ++i) {
+         if (i * 4 + wave < S::WLOADS) {
+            int at = weight_at[i];
+            if (!whole) { // k past the last channel are the next row's
+               int row, k;
+               weight_place(i, row, k);
+               at = s * CS * 9 + k < a.K ? at : F32_OUTSIDE;
+            }
+            f32_buffer_load<WVEC>((lds_void_t *)(lds + S::PATCH + (i * 4 + wave) * 64 * WVEC), weights + (long long)s * CS * 9 * 4, at);
+         }
+      }
+   };
+
+   // this lane's pixels in the patch, one address per kernel row, and its weights
+   int pixel[MT][3];
+#pragma unroll
+   for (int i = 0; i < MT; ++i) {
+      const int m = m0 + wm * TM + i * 32 + c, mm = m < a.M ? m : a.M - 1;
+      const int line = quotient(mm, a.ow_mul), image = quotient(line, a.oh_mul);
+      const int vr = (image - image0) * VH + line - image * a.OH - row0;
+#pragma unroll
+      for (int ky = 0; ky < 3; ++ky)
+         pixel[i][ky] = (vr + ky) * VW + mm - line * a.OW + lk * (CS / 2 * PLANE + 32);
+   }
+   const int weight = S::PATCH + (wn * TN + c) * S::PITCH + lk * S::HALF;
+
+   // The sums start at bias and residual, whose loads are on their way with the first slab's (behind the loop they were four
+   // trips to memory in a row).
+   v16f acc[MT][NT];
+#pragma unroll
+   for (int i = 0; i < MT; ++i) {
+      const int m = m0 + wm * TM + i * 32 + c;
+      const auto where = out.row_of(m < a.M ? m : a.M - 1);
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+         for (int e = 0; e < 16; ++e) {
+            const int n = n0 + wn * TN + j * 32 + e / 4 * 8 + lk * 4 + e % 4;
+            acc[i][j][e] = e / OWN == wk ? out.before_sum(where, n < a.N ? n : a.N - 1) : 0.0f;
+         }
+   }
+   // READ k at a time; the fragments of the next ones are read while these are multiplied
+   typedef float part __attribute__((ext_vector_type(S::READ)));
+   part w[2][NT];
+   float x[2][MT][S::READ];
+   auto multiply = [&](auto stage) {
+      const float *lds = f32_lds + decltype(stage)::value * S::STAGE;
+      constexpr int STEPS = S::HALF / S::READ;
+      auto read = [&](auto number, auto set) {
+         constexpr int to = decltype(set)::value, g = decltype(number)::value * S::READ;
+#pragma unroll
+         for (int j = 0; j < NT; ++j)
+            w[to][j] = *(const part *)(lds + weight + j * 32 * S::PITCH + g);
+#pragma unroll
+         for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int u = 0; u < S::READ; ++u)
+               x[to][i][u] = lds[pixel[i][(g + u) % 9 / 3] + (g + u) / 9 * PLANE + (g + u) % 3];
+      };
+      // the steps of wave p of those that share a tile
+      auto steps_of = [&](auto pc) {
+         constexpr int p = decltype(pc)::value, COUNT = (STEPS - p + WAVES_K - 1) / WAVES_K;
+         read(std::integral_constant<int, p>{}, std::integral_constant<int, 0>{});
+         static_for<COUNT>([&](auto gc) {
+            constexpr int g = decltype(gc)::value, set = g % 2;
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (g + 1 < COUNT)
+               read(std::integral_constant<int, p + (g + 1) * WAVES_K>{}, std::integral_constant<int, set ^ 1>{});
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < S::READ; ++u)
+#pragma unroll
+               for (int i = 0; i < MT; ++i)
+#pragma unroll
+                  for (int j = 0; j < NT; ++j)
+                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[set][j][u], x[set][i][u], acc[i][j], 0, 0, 0);
+         });
+      };
+      static_for<WAVES_K>([&](auto pc) {
+         if (WAVES_K == 1 || wk == decltype(pc)::value)
+            steps_of(pc);
+      });
+   };
+
+   issue(0, 0);
+   auto turn = [&](int s, auto stage) {
+      wait_vmcnt<0>();
+      __builtin_amdgcn_s_barrier(); // slab s has landed for every wave, and every wave has read slab s - 1
+      __builtin_amdgcn_sched_barrier(0);
+      if (s + 1 < slabs)
+         issue(s + 1, decltype(stage)::value ^ 1);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(stage);
+      __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0)
+      __builtin_amdgcn_sched_barrier(0);
+   };
+   for (int s = 0; s < slabs; s += 2) {
+      turn(s, std::integral_constant<int, 0>{});
+      if (s + 1 < slabs)
+         turn(s + 1, std::integral_constant<int, 1>{});
+   }
+
+   // Waves that share a tile: each leaves the elements it does not finish in LDS and adds up the others' parts of its own.
+   static_assert(WAVES_K == 1 || (MT == 1 && NT == 1), "one block per wave where waves share it");
+   if constexpr (WAVES_K > 1) {
+      __syncthreads();
+      float *parts = f32_lds + (wave - wk) * 1024;
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+         parts[wk * 1024 + e * 64 + lane] = acc[0][0][e];
+      __syncthreads();
+      static_for<WAVES_K>([&](auto pc) {
+         constexpr int p = decltype(pc)::value;
+         if (wk == p) {
+#pragma unroll
+            for (int e = p * OWN; e < (p + 1) * OWN; ++e)
+#pragma unroll
+               for (int o = 0; o < WAVES_K; ++o)
+                  if (o != p)
+                     acc[0][0][e] += parts[o * 1024 + e * 64 + lane];
+         }
+      });
+   }
+   // 32 neighbouring lanes hold 32 neighbouring pixels of a channel: whole lines, straight from the registers
+#pragma unroll
+   for (int i = 0; i < MT; ++i) {
+      const int m = m0 + wm * TM + i * 32 + c;
+      const auto where = out.row_of(m < a.M ? m : a.M - 1);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+         const int n1 = n0 + wn * TN + j * 32 + lk * 4;
+         auto put = [&](float v, int e) {
+            const int n = n1 + e / 4 * 8 + e % 4;
+            if (m < a.M && n < a.N)
+               out.Y[where.at + (size_t)(out.first + n) * out.positions] = v;
+         };
+         const bool relu = out.chain.count == 1 && out.chain.op0 == SOFIE_ACT_RELU;
+         if (relu || out.chain.count == 0) {
+            static_for<WAVES_K>([&](auto pc) {
+               constexpr int p = decltype(pc)::value;
+               if (WAVES_K == 1 || wk == p) {
+#pragma unroll
+                  for (int e = p * OWN; e < (p + 1) * OWN; ++e)
+                     put(relu ? (acc[i][j][e] > 0.0f ? acc[i][j][e] : 0.0f) : acc[i][j][e], e);
+               }
+            });
+         } else {
+            // one copy of the activations' code for 16 elements
+#pragma unroll 1
+            for (int g = wk * OWN / 4; g < (wk + 1) * OWN / 4; ++g)
+#pragma unroll
+               for (int e = 0; e < 4; ++e)
+                  put(apply_chain(g == 0 ? acc[i][j][e] : g == 1 ? acc[i][j][4 + e] : g == 2 ? acc[i][j][8 + e] : acc[i][j][12 + e], out.chain), g * 4 + e);
+         }
+      }
+   }
+}
+
+template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int CS, int PLANE, int WVEC>
+static int launch_f32_conv3x3_as(hipStream_t stream, const F32Conv3x3 &a, const F32ConvStore &out, int group)
+{
+   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
+   if ((long long)tiles_m * tiles_n > 0x7fffffffLL)
+      return fail(SOFIE_HIP_ERR_INVALID, "fp32 convolution: too many tiles");
+   constexpr size_t stage = sizeof(float) * F32Conv3x3Shape<BM, BN, CS, PLANE, WVEC>::STAGE, parts = WAVES_K > 1 ? 4 * 1024 * sizeof(float) : 0;
+   const size_t smem = std::max(stage * (a.C > CS ? 2 : 1), parts);
+   auto kern = f32_conv3x3_kernel<BM, BN, WAVES_M, WAVES_N, WAVES_K, CS, PLANE, WVEC>;
+   static bool configured[64] = {};
+   if (int st = configure_lds_once(kern, std::max(stage * 2, parts), configured))
+      return st;
+   launch_kernel(kern, dim3((unsigned)(tiles_m * tiles_n), 1, (unsigned)group), dim3(256), smem, stream, a, out, tiles_m, tiles_n);
+   return launch_status("f32_conv3x3_kernel");
+}
+
+} // namespace sofie_hip

@@ -1,6 +1,6 @@
 // fp32 Gemm / MatMul and fp32 convolution (implicit GEMM) with the bias + activation epilogue fused into the store: the entry
 // points and the choice among the kernels of f32_mfma.hpp, and the kernel that runs a chain of small products in one launch.
-#include "f32_mfma.hpp"
+#include "f32_conv3x3.hpp"
 #include <algorithm>
 #include <cmath>
 
@@ -139,7 +139,7 @@ namespace sofie_hip {
 // (64 x 32: two blocks), 0.452 (64 x 64: four) and 1.765 (128 x 128: sixteen), a start and a store per tile, in as many rounds as
 // the tiles need over 256 CUs, and a launch.  The direct kernel costs a launch, a trip to memory per 512 k or the 10.5 TB/s at which
 // its fragments, which nothing shares, arrive, and 0.45 us per 256 tiles.
-enum F32Tile { F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
+enum F32Tile { F32_CONV3X3_32 = 3032, F32_CONV3X3_64 = 3064, F32_CONV3X3_128 = 3128, F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
 static int pick_f32_tile(int M, int N, int K, int batch, double *time_us = nullptr)
 {
    auto tiles = [&](int bm, int bn) { return (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
@@ -191,7 +191,7 @@ static int launch_f32_product(sofie_hip_ctx *ctx, const ASRC &A, const BSRC &B, 
    constexpr bool CONV = ASRC::kLeastRows == 64;
    if (!tile)
       tile = CONV ? pick_f32_conv_tile(M, N, K, batch) : pick_f32_tile(M, N, K, batch);
-   if (CONV ? tile == F32_TILE_32 || tile == F32_TILE_128 : tile == F32_TILE_128x32)
+   if (tile >= F32_CONV3X3_32 || (CONV ? tile == F32_TILE_32 || tile == F32_TILE_128 : tile == F32_TILE_128x32))
       tile = F32_TILE_64; // a request for a tile that the other kind of product has
    if constexpr (CONV) {
       switch (tile) {
@@ -210,6 +210,62 @@ static int launch_f32_product(sofie_hip_ctx *ctx, const ASRC &A, const BSRC &B, 
    case F32_TILE_64: return launch_f32_tile<ASRC, BSRC, STORE, 64, 64, 32, 2, 2, 2, 4>(s, A, B, out, M, N, K, batch, strideA, strideB);
    default: return fail(SOFIE_HIP_ERR_INVALID, "fp32 product: unknown tile %d", tile);
    }
+}
+
+// The kernel of f32_conv3x3.hpp for a convolution it takes (*taken tells): faster than the gathering kernels at every size measured, if only
+// by the launch where a few tiles of one slab are all there is.
+static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvShape &s, const float *W, const F32ConvStore &out, int images, int M, int group, bool *taken)
+{
+   const int K = s.Cg * 9, N = out.Cout_g, force = ctx->opt.f32_tile;
+   *taken = false;
+   if (s.kd != 1 || s.D != 1 || s.kh != 3 || s.kw != 3 || s.stride_h != 1 || s.stride_w != 1 || s.dil_h != 1 || s.dil_w != 1 || ctx->opt.f32_skinny >= 0)
+      return SOFIE_HIP_OK;
+   // the images a patch touches, from the first one's base, within a buffer; channels within its scalar offset
+   const long long plane = (long long)s.H * s.W, most = F32_CONV3X3_PATCH / ((long long)(s.OW + 2) * (s.OH + 2)) + 2;
+   if ((most * s.C + s.Cg) * plane * 4 >= F32_BUFFER_BYTES || 128LL * K * 4 >= F32_BUFFER_BYTES)
+      return SOFIE_HIP_OK;
+   int tile = force;
+   if (!tile) {
+      // A slab of 8 channels takes 1.06 / 0.61 / 0.38 us of a CU with several tiles of 128 / 64 / 32 pixels at work, and 1.42 / 0.95 / 0.70
+      // where a tile is alone and waits for its loads; a tile costs 1.45 / 1.0 / 0.8 us besides, a launch 4.3.  One slab of a few
+      // channels: 1.6 us a tile.  (Fitted to 20 layers from 2 images of 14 x 14 to 64 of 64 x 64; holds to a tenth.)
+      double least = 1e30;
+      auto offer = [&](int which, int bm, double slab, double alone, double each) {
+         const double rounds = std::ceil((double)((M + bm - 1) / bm) * ((N + 31) / 32) * group / 256.0), slabs = std::ceil(s.Cg / 8.0);
+         const double t = std::max(slabs * alone, rounds * (slabs * slab + each));
+         if (f32_conv3x3_patch(s.OH, s.OW, bm) <= F32_CONV3X3_PATCH && t < least)
+            least = t, tile = which;
+      };
+      if (s.Cg <= 4) {
+         offer(F32_CONV3X3_128, 128, 0.3, 0.5, 1.3);
+      } else {
+         offer(F32_CONV3X3_32, 32, 0.383, 0.70, 0.8);
+         offer(F32_CONV3X3_64, 64, 0.606, 0.95, 1.0);
+         offer(F32_CONV3X3_128, 128, 1.06, 1.42, 1.45);
+      }
+   }
+   const long long patch = f32_conv3x3_patch(s.OH, s.OW, tile - 3000);
+   if (tile < F32_CONV3X3_32 || patch > F32_CONV3X3_PATCH)
+      return SOFIE_HIP_OK;
+   auto reciprocal = [](unsigned d) -> unsigned long long { return d <= 1 ? 0ull : (~0ull / d) + 1; };
+   const F32Conv3x3 a{X, W, images, s.Cg, s.H, s.W, s.OH, s.OW, s.pad_h, s.pad_w, plane * s.C, plane * s.Cg, M, N, K, (int)(patch + 63) / 64,
+                      reciprocal(s.OW), reciprocal(s.OH), reciprocal(s.OW + 2), reciprocal(s.OH + 2)};
+   const bool vec = ((uintptr_t)W & 15) == 0 && K % 4 == 0;
+   *taken = true;
+   hipStream_t st = ctx->stream;
+   auto go = [&](auto room, auto wide) {
+      constexpr int P = decltype(room)::value, V = decltype(wide)::value;
+      if (s.Cg <= 4 && tile == F32_CONV3X3_128)
+         return launch_f32_conv3x3_as<128, 32, 4, 1, 1, 4, P, 1>(st, a, out, group);
+      switch (tile) {
+      case F32_CONV3X3_32: return launch_f32_conv3x3_as<32, 32, 1, 1, 4, 8, P, V>(st, a, out, group);
+      case F32_CONV3X3_64: return launch_f32_conv3x3_as<64, 32, 2, 1, 2, 8, P, V>(st, a, out, group);
+      default: return launch_f32_conv3x3_as<128, 32, 4, 1, 1, 8, P, V>(st, a, out, group);
+      }
+   };
+   auto with = [&](auto room) { return vec ? go(room, std::integral_constant<int, 4>{}) : go(room, std::integral_constant<int, 1>{}); };
+   // the places a channel has in LDS: the fewer, the more workgroups share a CU (images of 32, 64 and 96 columns)
+   return patch <= 256 ? with(std::integral_constant<int, 256>{}) : patch <= 448 ? with(std::integral_constant<int, 448>{}) : with(std::integral_constant<int, F32_CONV3X3_PATCH>{});
 }
 
 // A convolution of `group` groups as products of M = images x positions rows and Cout / group columns.
@@ -243,6 +299,9 @@ static int launch_f32_conv(sofie_hip_ctx *ctx, const float *X, F32ConvShape s, c
    s.positions = taps;
    auto reciprocal64 = [](unsigned d) -> unsigned long long { return d <= 1 ? 0ull : (~0ull / d) + 1; };
    s.ow_mul = reciprocal64(s.OW), s.oh_mul = reciprocal64(s.OH), s.od_mul = reciprocal64(s.OD);
+   bool taken = false;
+   if (int st = launch_f32_conv3x3(ctx, X, s, W, out, (int)(M / ((long long)s.OD * s.OH * s.OW)), (int)M, group, &taken); st || taken)
+      return st;
    // one bit per kernel position; the images that the 128 rows of a tile touch within a buffer, and the channels within its scalar offset
    const long long plane = (long long)s.D * s.H * s.W, window = ((long long)s.kd * s.dil_d * s.H + (long long)s.kh * s.dil_h) * s.W + (long long)s.kw * s.dil_w;
    const long long images = 127 / ((long long)s.OD * s.OH * s.OW) + 2;
