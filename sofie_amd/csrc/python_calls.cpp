@@ -1,4 +1,4 @@
-// Calls of the C-ABI from Python: `call(name, *args)` of a Runtime as one vectorcall that converts the arguments and calls the entry
+// Calls of the C-ABI from Python: `call(name, *args)` of a Runtime as one native method that converts the arguments and calls the entry
 // point itself.
 //
 // A launch costs the host about 2.1 us in the HIP runtime; a ctypes call around it took another 0.7 - 1.2 us (one converter object
@@ -8,7 +8,6 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include "sofie_hip.h"
-#include <cstddef>
 #include <cstdint>
 #include <cstring>
 #include <tuple>
@@ -153,39 +152,48 @@ const Known kKnown[] = {
 PyObject *g_entries = nullptr; // name -> index into g_table
 std::vector<Entry> g_table;
 
-// ---- the callable ---------------------------------------------------------------------------------------------------------
-struct Caller {
-   PyObject_HEAD
-   vectorcallfunc vectorcall;
-   sofie_hip_ctx *ctx;
-   PyObject *slow; // slow(ctx address or None, name, *args): converts anything, raises
-};
+// ---- the method -----------------------------------------------------------------------------------------------------------
+// Runtime.call: a method, so that what a caller keeps of it (rt.call, held over a loop) keeps the Runtime, and its context with it, alive;
+// and the context is read from the Runtime at each call, so that one that was closed in between is refused.
+PyObject *g_ctx_name = nullptr; // "ctx"
+PyObject *g_slow = nullptr;     // slow(runtime, status or None, name, *args): converts anything, raises
 
-PyObject *slow_call(Caller *self, PyObject *const *args, Py_ssize_t n, PyObject *kwnames, PyObject *status)
+PyObject *slow_call(PyObject *self, PyObject *const *args, Py_ssize_t n, PyObject *kwnames, PyObject *status)
 {
-   std::vector<PyObject *> all;
-   PyObject *ctx = self->ctx ? PyLong_FromVoidPtr(self->ctx) : Py_NewRef(Py_None);
-   if (!ctx)
+   PyObject *all = PyTuple_New(n + 2), *kw = nullptr, *r = nullptr;
+   if (!all)
       return nullptr;
-   all.push_back(ctx);
-   all.push_back(status);
-   const Py_ssize_t total = n + (kwnames ? PyTuple_GET_SIZE(kwnames) : 0);
-   all.insert(all.end(), args, args + total);
-   PyObject *r = PyObject_Vectorcall(self->slow, all.data(), (size_t)(n + 2), kwnames);
-   Py_DECREF(ctx);
+   PyTuple_SET_ITEM(all, 0, Py_NewRef(self));
+   PyTuple_SET_ITEM(all, 1, Py_NewRef(status));
+   for (Py_ssize_t i = 0; i < n; i++)
+      PyTuple_SET_ITEM(all, i + 2, Py_NewRef(args[i]));
+   bool good = true;
+   if (kwnames) {
+      kw = PyDict_New();
+      good = kw != nullptr;
+      for (Py_ssize_t i = 0; good && i < PyTuple_GET_SIZE(kwnames); i++)
+         good = PyDict_SetItem(kw, PyTuple_GET_ITEM(kwnames, i), args[n + i]) == 0;
+   }
+   if (good)
+      r = PyObject_Call(g_slow, all, kw);
+   Py_XDECREF(kw);
+   Py_DECREF(all);
    return r;
 }
 
-PyObject *caller_call(PyObject *o, PyObject *const *args, size_t nargsf, PyObject *kwnames)
+PyObject *call_method(PyObject *self, PyObject *const *args, Py_ssize_t n, PyObject *kwnames)
 {
-   Caller *self = (Caller *)o;
-   const Py_ssize_t n = PyVectorcall_NARGS(nargsf);
    if (n >= 1 && !kwnames && PyUnicode_CheckExact(args[0])) {
       PyObject *index = PyDict_GetItemWithError(g_entries, args[0]);
       if (index) {
          const Entry &e = g_table[(size_t)PyLong_AsSsize_t(index)];
          if (e.count == n - 1) {
-            const int status = e.thunk(e, self->ctx, args + 1);
+            PyObject *held = PyObject_GetAttr(self, g_ctx_name);
+            if (!held)
+               return nullptr;
+            sofie_hip_ctx *ctx = nullptr;
+            const int status = take(held, nullptr, ctx) ? e.thunk(e, ctx, args + 1) : (int)NOT_TAKEN;
+            Py_DECREF(held);
             if (status == SOFIE_HIP_OK)
                Py_RETURN_NONE;
             if (status != NOT_TAKEN) {
@@ -203,30 +211,18 @@ PyObject *caller_call(PyObject *o, PyObject *const *args, size_t nargsf, PyObjec
    return slow_call(self, args, n, kwnames, Py_None);
 }
 
-void caller_dealloc(PyObject *o)
-{
-   Py_XDECREF(((Caller *)o)->slow);
-   Py_TYPE(o)->tp_free(o);
-}
+PyMethodDef g_call = {"call", (PyCFunction)(void (*)(void))call_method, METH_FASTCALL | METH_KEYWORDS,
+                      "call(name, *args): the entry point of that name on this context; raises SofieHipError where it fails"};
 
-PyTypeObject g_caller_type = {PyVarObject_HEAD_INIT(nullptr, 0) "sofie_amd.Caller", sizeof(Caller)};
-
-// caller(ctx address, slow)
-PyObject *make_caller(PyObject *, PyObject *args)
+// method(type, slow): the method `call` of that type
+PyObject *make_method(PyObject *, PyObject *args)
 {
-   PyObject *address, *slow;
-   if (!PyArg_ParseTuple(args, "OO", &address, &slow))
+   PyObject *type, *slow;
+   if (!PyArg_ParseTuple(args, "O!O", &PyType_Type, &type, &slow))
       return nullptr;
-   void *ctx = PyLong_AsVoidPtr(address);
-   if (!ctx && PyErr_Occurred())
-      return nullptr;
-   Caller *c = PyObject_New(Caller, &g_caller_type);
-   if (!c)
-      return nullptr;
-   c->vectorcall = caller_call;
-   c->ctx = (sofie_hip_ctx *)ctx;
-   c->slow = Py_NewRef(slow);
-   return (PyObject *)c;
+   Py_XDECREF(g_slow);
+   g_slow = Py_NewRef(slow);
+   return PyDescr_NewMethod((PyTypeObject *)type, &g_call);
 }
 
 // entry(name, address of the function, tuple of the structure types its typed pointers ask for (None: any)) -> whether it is taken
@@ -315,7 +311,7 @@ PyObject *learn_layout(PyObject *, PyObject *args)
    return PyBool_FromLong(g_layout.data && g_layout.ref_address);
 }
 
-PyMethodDef g_methods[] = {{"caller", make_caller, METH_VARARGS, "caller(ctx address, slow): what Runtime.call is"},
+PyMethodDef g_methods[] = {{"method", make_method, METH_VARARGS, "method(type, slow): what Runtime.call is"},
                            {"entry", add_entry, METH_VARARGS, "entry(name, address, wanted types): an entry point of the library"},
                            {"layout", learn_layout, METH_VARARGS, "layout(...): where ctypes objects keep their addresses"},
                            {nullptr, nullptr, 0, nullptr}};
@@ -325,14 +321,9 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_calls", "Calls of the C-ABI", -
 
 PyMODINIT_FUNC PyInit__calls(void)
 {
-   g_caller_type.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_VECTORCALL;
-   g_caller_type.tp_vectorcall_offset = offsetof(Caller, vectorcall);
-   g_caller_type.tp_call = PyVectorcall_Call;
-   g_caller_type.tp_dealloc = caller_dealloc;
-   if (PyType_Ready(&g_caller_type) < 0)
-      return nullptr;
    g_entries = PyDict_New();
-   if (!g_entries)
+   g_ctx_name = PyUnicode_InternFromString("ctx");
+   if (!g_entries || !g_ctx_name)
       return nullptr;
    return PyModule_Create(&g_module);
 }

@@ -210,6 +210,7 @@ def _bind_calls(lib):
     for name, (res, args) in SYMBOLS.items():
         if res is C.c_int and args and args[0] is _P:
             module.entry(name, C.cast(getattr(lib, name), _P).value, tuple(getattr(a, "_type_", None) if a.__class__ is _POINTER_TYPE else None for a in args[1:]))
+    Runtime.call = module.method(Runtime, _call_slowly)
     _calls = module
 
 
@@ -218,10 +219,9 @@ def _check(lib, status):
         raise SofieHipError("sofie_hip status %d: %s" % (status, (lib.sofie_hip_last_error() or b"").decode()))
 
 
-def _call_slowly(ctx, status, name, *args):
+def _call_slowly(runtime, status, name, *args):
     """A call through ctypes, for arguments the native path does not convert; with a status, the report of a native call that failed."""
-    lib = load_library()
-    _check(lib, getattr(lib, name)(ctx, *args) if status is None else status)
+    _check(runtime.lib, getattr(runtime.lib, name)(runtime.ctx, *args) if status is None else status)
 
 
 class Runtime:
@@ -232,20 +232,21 @@ class Runtime:
         h = C.c_void_p()
         _check(self.lib, self.lib.sofie_hip_ctx_create(C.byref(h), device, external_stream))
         self.ctx = h
-        # call(name, *args): the entry point of that name on this context
-        self.call = _calls.caller(h.value, _call_slowly)
 
     def close(self):
         if getattr(self, "ctx", None):
-            self.lib.sofie_hip_ctx_destroy(self.ctx)
-            self.ctx = None
-            self.call = _calls.caller(0, _call_slowly)   # from here on every call is refused
+            ctx, self.ctx = self.ctx, None   # from here on every call is refused
+            self.lib.sofie_hip_ctx_destroy(ctx)
 
     def __del__(self):
         try:
             self.close()
         except Exception:
             pass
+
+    def call(self, name, *args):
+        """The entry point of that name on this context (loading the library puts a native method of the same meaning in this place)."""
+        _call_slowly(self, None, name, *args)
 
     def set_option(self, name, value):
         """Kernel-choice override of this context (see sofie_hip_ctx_set_option)."""

@@ -1,17 +1,43 @@
 """Runtime.call's native path: every kind of argument it converts reaches the entry point as ctypes would have passed it, and what it
 does not convert (or a call that fails) takes the ctypes path."""
 import ctypes as C
+import gc
 
 import pytest
 
 from sofie_amd import runtime as R
 
 
-@pytest.fixture(scope="module")
-def caller():
-    lib = R.load_library()
-    room = C.create_string_buffer(4096)          # a context that no launch is made on: every call below ends before one
-    return lib, room, R._calls.caller(C.addressof(room), R._call_slowly)
+class _Library:
+    """The library, its contexts being rooms that no launch is made on: every call below ends before one."""
+
+    def __init__(self):
+        self.real, self.rooms, self.destroyed = R.load_library(), [], []
+
+    def __getattr__(self, name):
+        return getattr(self.real, name)
+
+    def sofie_hip_ctx_create(self, out, device, stream):
+        self.rooms.append(C.create_string_buffer(4096))
+        out._obj.value = C.addressof(self.rooms[-1])
+        return 0
+
+    def sofie_hip_ctx_destroy(self, ctx):
+        self.destroyed.append(ctx.value)
+        return 0
+
+
+@pytest.fixture
+def library(monkeypatch):
+    lib = _Library()
+    monkeypatch.setattr(R, "load_library", lambda: lib)
+    return lib
+
+
+@pytest.fixture
+def caller(library):
+    rt = R.Runtime(0)
+    return library, rt, rt.call
 
 
 @pytest.mark.parametrize("pointer", [C.c_void_p(4096), 4096, (C.c_float * 4)(), C.byref(C.c_float())], ids=["c_void_p", "int", "array", "byref"])
@@ -55,6 +81,30 @@ def test_wrong_arguments_raise(caller):
 
 
 def test_no_context(caller):
-    none = R._calls.caller(0, R._call_slowly)
+    _, rt, none = caller
+    rt.ctx = None
     with pytest.raises(R.SofieHipError, match="NULL argument|ctx is NULL"):
         none("sofie_hip_gemm_f32", C.byref(R.GemmF32Desc()))
+
+
+EMPTY = ("sofie_hip_fill_zero", 4096, 0)
+
+
+def test_a_call_kept_past_close_is_refused(library):
+    rt = R.Runtime(0)
+    call = rt.call
+    assert call(*EMPTY) is None
+    rt.close()
+    assert library.destroyed == [C.addressof(library.rooms[0])]
+    for use in (call, rt.call):
+        with pytest.raises(R.SofieHipError, match="ctx is NULL"):
+            use(*EMPTY)
+
+
+def test_a_call_that_is_kept_keeps_its_context(library):
+    call = R.Runtime(0).call
+    gc.collect()
+    assert not library.destroyed and call(*EMPTY) is None
+    del call
+    gc.collect()
+    assert len(library.destroyed) == 1
