@@ -9,7 +9,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "sofie_amd", "csrc")
 LIB_DIR = os.path.join(ROOT, "sofie_amd", "lib")
 LIB = os.path.join(LIB_DIR, "libsofie_hip.so")
-CALLS = os.path.join(LIB_DIR, "_calls.so")
+CALLS = os.path.join(LIB_DIR, "_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 HIP_SOURCES = ["runtime.hip", "gemm_i8.hip", "gemm_f32.hip", "gemm_fp8.hip", "conv_i8.hip", "eltwise.hip"]
 
@@ -63,8 +63,13 @@ def build_hip_library(jobs=8):
 
 
 def build_python_calls():
-    """The CPython module behind Runtime.call (sofie_amd/lib/_calls.so); host code, bound to the library's entry points when it is loaded."""
-    _run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-Wall", "-I" + sysconfig.get_paths()["include"],
+    """The CPython module behind Runtime.call (sofie_amd/lib/_calls.<interpreter>.so, one per interpreter it was built with); host code, bound to
+    the library's entry points when it is loaded.  Without the interpreter's headers it is left out, and calls go through ctypes."""
+    include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        print("no Python.h in %s: Runtime.call will use ctypes" % include, flush=True)
+        return None
+    _run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-Wall", "-I" + include,
           "-I" + os.path.join(ROOT, "include"), os.path.join(CSRC, "python_calls.cpp"), "-o", CALLS])
     return CALLS
 

@@ -27,6 +27,11 @@ struct CtypesLayout {
    PyTypeObject *void_p = nullptr, *size_t_ = nullptr, *float_ = nullptr, *array = nullptr, *ref = nullptr;
 } g_layout;
 
+PyObject *new_reference(PyObject *o)
+{
+   Py_INCREF(o);
+   return o;
+}
 void *word_at(PyObject *o, Py_ssize_t offset) { return *(void **)((char *)o + offset); }
 
 // ---- one argument ---------------------------------------------------------------------------------------------------------
@@ -163,10 +168,10 @@ PyObject *slow_call(PyObject *self, PyObject *const *args, Py_ssize_t n, PyObjec
    PyObject *all = PyTuple_New(n + 2), *kw = nullptr, *r = nullptr;
    if (!all)
       return nullptr;
-   PyTuple_SET_ITEM(all, 0, Py_NewRef(self));
-   PyTuple_SET_ITEM(all, 1, Py_NewRef(status));
+   PyTuple_SET_ITEM(all, 0, new_reference(self));
+   PyTuple_SET_ITEM(all, 1, new_reference(status));
    for (Py_ssize_t i = 0; i < n; i++)
-      PyTuple_SET_ITEM(all, i + 2, Py_NewRef(args[i]));
+      PyTuple_SET_ITEM(all, i + 2, new_reference(args[i]));
    bool good = true;
    if (kwnames) {
       kw = PyDict_New();
@@ -221,7 +226,7 @@ PyObject *make_method(PyObject *, PyObject *args)
    if (!PyArg_ParseTuple(args, "O!O", &PyType_Type, &type, &slow))
       return nullptr;
    Py_XDECREF(g_slow);
-   g_slow = Py_NewRef(slow);
+   g_slow = new_reference(slow);
    return PyDescr_NewMethod((PyTypeObject *)type, &g_call);
 }
 
@@ -244,7 +249,7 @@ PyObject *add_entry(PyObject *, PyObject *args)
          e.count = k.count;
          for (Py_ssize_t i = 0; i < k.count; i++) {
             PyObject *t = PyTuple_GET_ITEM(want, i);
-            e.want.push_back(PyType_Check(t) ? (PyTypeObject *)Py_NewRef(t) : nullptr);
+            e.want.push_back(PyType_Check(t) ? (PyTypeObject *)new_reference(t) : nullptr);
          }
          PyObject *index = PyLong_FromSize_t(g_table.size());
          if (!index)
@@ -307,7 +312,7 @@ PyObject *learn_layout(PyObject *, PyObject *args)
       return nullptr;
    PyTypeObject **to[5] = {&g_layout.void_p, &g_layout.size_t_, &g_layout.float_, &g_layout.array, &g_layout.ref};
    for (int i = 0; i < 5; i++)
-      *to[i] = (PyTypeObject *)Py_NewRef(types[i]);
+      *to[i] = (PyTypeObject *)new_reference(types[i]);
    return PyBool_FromLong(g_layout.data && g_layout.ref_address);
 }
 

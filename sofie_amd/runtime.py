@@ -1,8 +1,9 @@
 """ctypes view of the C-ABI in include/sofie_hip.h (used by tests/ and bench.py).
 
-There is no fallback: if the library is not built, loading raises.
+There is no fallback for the library: if it is not built, loading raises.
 """
 import ctypes as C
+import importlib.machinery
 import importlib.util
 import os
 
@@ -194,11 +195,12 @@ _calls = None
 
 
 def _bind_calls(lib):
-    """Load the native module that makes the calls of Runtime.call and give it the library's entry points."""
+    """Load the native module that makes the calls of Runtime.call and give it the library's entry points.  Where none was built for this
+    interpreter (its tag is in the file's name), Runtime.call goes through ctypes."""
     global _calls
-    where = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "_calls.so")
+    where = os.path.join(_HERE, "lib", "_calls" + importlib.machinery.EXTENSION_SUFFIXES[0])
     if not os.path.exists(where):
-        raise SofieHipError("%s is not built: run `python -c 'import __graft_entry__ as g; g.build()'`" % where)
+        return
     spec = importlib.util.spec_from_file_location("_calls", where)
     module = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(module)
@@ -245,7 +247,7 @@ class Runtime:
             pass
 
     def call(self, name, *args):
-        """The entry point of that name on this context (loading the library puts a native method of the same meaning in this place)."""
+        """The entry point of that name on this context (where it was built, a native method of the same meaning takes this place)."""
         _call_slowly(self, None, name, *args)
 
     def set_option(self, name, value):

@@ -2,10 +2,15 @@
 does not convert (or a call that fails) takes the ctypes path."""
 import ctypes as C
 import gc
+import os
+import subprocess
+import sys
 
 import pytest
 
 from sofie_amd import runtime as R
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 class _Library:
@@ -108,3 +113,25 @@ def test_a_call_that_is_kept_keeps_its_context(library):
     del call
     gc.collect()
     assert len(library.destroyed) == 1
+
+
+def test_another_interpreter_calls_through_ctypes():
+    """A build for one interpreter is none for another: the calls work, by the slower way."""
+    assert R.load_library() and R._calls is not None
+    code = """
+import ctypes as C, importlib.machinery as machinery
+machinery.EXTENSION_SUFFIXES[:] = [".another.so"]
+from sofie_amd import runtime as R
+rt = R.Runtime.__new__(R.Runtime)
+rt.lib, room = R.load_library(), C.create_string_buffer(4096)
+rt.ctx = C.c_void_p(C.addressof(room))
+rt.call("sofie_hip_fill_zero", C.c_void_p(4096), 0)
+try:
+    rt.call("sofie_hip_gemm_f32", C.byref(R.GemmF32Desc()))
+except R.SofieHipError as e:
+    assert "batch" in str(e)
+    print("refused")
+rt.ctx = None
+assert R._calls is None
+"""
+    assert subprocess.run([sys.executable, "-c", code], cwd=ROOT, stdout=subprocess.PIPE, check=True).stdout == b"refused\n"
