@@ -24,6 +24,10 @@ namespace {
 struct CtypesLayout {
    Py_ssize_t data = 0;                    // instance -> void * of its value
    Py_ssize_t ref_address = 0, ref_obj = 0; // byref() object -> void *, PyObject *
+   // Other parameters that ctypes has already converted (c_int.from_param) have the same type as a byref() object.  The two words behind the
+   // object's head, the second of which begins with a letter, tell them apart.
+   void *ref_kind = nullptr;
+   char ref_letter = 0;
    PyTypeObject *void_p = nullptr, *size_t_ = nullptr, *float_ = nullptr, *array = nullptr, *ref = nullptr;
 } g_layout;
 
@@ -33,6 +37,8 @@ PyObject *new_reference(PyObject *o)
    return o;
 }
 void *word_at(PyObject *o, Py_ssize_t offset) { return *(void **)((char *)o + offset); }
+constexpr Py_ssize_t REF_KIND = sizeof(PyObject), REF_LETTER = REF_KIND + (Py_ssize_t)sizeof(void *);
+bool is_reference(PyObject *o) { return word_at(o, REF_KIND) == g_layout.ref_kind && ((const char *)o)[REF_LETTER] == g_layout.ref_letter; }
 
 // ---- one argument ---------------------------------------------------------------------------------------------------------
 // `want`: the structure type a typed pointer asks for, or null.  False: not an argument this file converts.
@@ -44,7 +50,10 @@ bool take(PyObject *o, PyTypeObject *want, T &out)
          return out = nullptr, true;
       PyTypeObject *t = Py_TYPE(o);
       if (t == g_layout.ref && g_layout.ref_address) {
-         if (want && Py_TYPE((PyObject *)word_at(o, g_layout.ref_obj)) != want)
+         if (!is_reference(o))
+            return false;
+         PyObject *of = (PyObject *)word_at(o, g_layout.ref_obj);
+         if (want && (!of || Py_TYPE(of) != want))
             return false;
          return out = (T)word_at(o, g_layout.ref_address), true;
       }
@@ -68,7 +77,8 @@ bool take(PyObject *o, PyTypeObject *want, T &out)
          const long long v = PyLong_AsLongLongAndOverflow(o, &overflow);
          return out = (T)v, !overflow;
       }
-      if (sizeof(T) == sizeof(size_t) && Py_TYPE(o) == g_layout.size_t_ && g_layout.data)
+      // a parameter of another type, of the same size though it be, refuses a c_size_t
+      if (std::is_same_v<T, size_t> && Py_TYPE(o) == g_layout.size_t_ && g_layout.data)
          return out = (T) * (size_t *)word_at(o, g_layout.data), true;
       return false;
    }
@@ -306,7 +316,14 @@ PyObject *learn_layout(PyObject *, PyObject *args)
    }
    g_layout.ref_address = objects.size() >= 2 ? offset_of(objects, words) : 0;
    g_layout.ref_obj = objects.size() >= 2 ? offset_of(objects, owners) : 0;
-   if (!g_layout.ref_obj)
+   if (!objects.empty()) {
+      g_layout.ref_kind = word_at(objects[0], REF_KIND);
+      g_layout.ref_letter = ((const char *)objects[0])[REF_LETTER];
+   }
+   bool alike = g_layout.ref_address > REF_LETTER && g_layout.ref_obj > REF_LETTER;
+   for (PyObject *o : objects)
+      alike = alike && is_reference(o);
+   if (!alike)
       g_layout.ref_address = 0;
    if (PyErr_Occurred())
       return nullptr;

@@ -115,6 +115,36 @@ def test_a_call_that_is_kept_keeps_its_context(library):
     assert len(library.destroyed) == 1
 
 
+_D = R.GemmF32Desc()
+POINTERS = [C.c_void_p(4096), C.c_void_p(), 4096, None, (C.c_float * 4)(), C.byref(_D), C.byref(_D, 8), _D, C.pointer(_D), C.c_void_p.from_param(5),
+            C.c_int.from_param(5), C.c_int64.from_param(5), C.c_double.from_param(2.0), C.c_char_p.from_param(b"x"), C.c_char_p(b"x"), C.c_int(5), b"x", "x", 1.5]
+INTEGERS = [0, 1, -1, True, 1 << 40, (1 << 63) + 5, 1.0, None, C.c_int32(1), C.c_int64(1), C.c_size_t(1), C.c_uint64(1), C.c_float(1), C.c_int.from_param(5), "1"]
+REALS = [0.5, 0, True, C.c_float(0.5), C.c_double(0.5), C.c_int(1), C.c_float.from_param(0.5), None, "0.5"]
+
+
+@pytest.mark.parametrize("name, before, kind, behind", [("sofie_hip_fill_zero", (), POINTERS, (0,)), ("sofie_hip_gemm_f32", (), POINTERS + [(R.GemmF32Desc * 2)(), C.byref(R.GemmI8Desc())], ()),
+                                                        ("sofie_hip_softmax_f32", (None, None, 0, 4), INTEGERS, (0,)), ("sofie_hip_softmax_f32", (None, None, 0), INTEGERS, (1, 0)),
+                                                        ("sofie_hip_fill_zero", (None,), INTEGERS, ()), ("sofie_hip_layernorm_f32", (None, None, None, None, 0, 8), REALS, (None, None))],
+                         ids=["pointer", "structure", "int64", "int32", "size_t", "float"])
+def test_what_ctypes_refuses_is_refused(caller, name, before, kind, behind):
+    """Every kind of argument has the outcome of the plain ctypes call (which, as these calls do, ends before a launch)."""
+    library, rt, call = caller
+
+    def outcome(f):
+        try:
+            return f()
+        except R.SofieHipError as e:
+            return str(e)
+        except Exception as e:
+            return type(e)
+
+    def plainly(*args):
+        R._check(library, getattr(library, name)(rt.ctx, *args))
+    for value in kind:
+        args = before + (value,) + behind
+        assert outcome(lambda: call(name, *args)) == outcome(lambda: plainly(*args)), value
+
+
 def test_another_interpreter_calls_through_ctypes():
     """A build for one interpreter is none for another: the calls work, by the slower way."""
     assert R.load_library() and R._calls is not None
