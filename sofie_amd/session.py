@@ -87,9 +87,8 @@ class Int8MLPSession:
             d.Y = p(dst)
             src = dst
             self.descs.append(d)
-        # one inference, its arguments made once
-        self.calls = [("sofie_hip_quantize_linear", p(self.off_xq), self.x_ptr, M * self.dims[0], C.c_float(float(self.in_scales[0])))]
-        self.calls += [("sofie_hip_gemm_i8", C.byref(d)) for d in self.descs]
+        # the addresses of the plan hold as long as the arena; what a pass takes from the attributes it reads at each pass
+        self._quantize = p(self.off_xq), p(self.off_x)
 
     @property
     def x_ptr(self):
@@ -106,9 +105,10 @@ class Int8MLPSession:
 
     def infer_nosync(self):
         """Enqueue one inference over the input resident at x_ptr; the result lands at y_ptr."""
-        call = self.rt.call
-        for c in self.calls:
-            call(*c)
+        call, byref = self.rt.call, C.byref
+        call("sofie_hip_quantize_linear", *self._quantize, self.batch * self.dims[0], float(self.in_scales[0]))
+        for d in self.descs:
+            call("sofie_hip_gemm_i8", byref(d))
 
     def infer(self, x):
         self.upload_input(x)
@@ -229,18 +229,8 @@ class Int8CNNSession:
         g.A, g.B, g.C, g.Y = p(self.off_pool), p(self.off_fcw), p(self.off_fcb), p(self.off_y)
         g.bias_mode, g.act, g.batch = R.BIAS_ROW, R.ACT_NONE, 1
         self.fc = g
-        # one inference, its arguments made once
-        c, h, w = self.out_shape
-        last_scale = C.c_float(float(self.last_scale))
-        self.calls = [("sofie_hip_quantize_linear", p(self.off_xq), self.x_ptr, N * Cin * H * W, C.c_float(float(self.in_scale)))]
-        if self.pool_in_conv:
-            self.calls.append(("sofie_hip_fill_zero", p(self.off_sums), 4 * N * c))
-        self.calls += [("sofie_hip_conv_i8", C.byref(d), C.byref(a)) for d, a in zip(self.conv_descs, self.conv_args)]
-        if self.pool_in_conv:
-            self.calls.append(("sofie_hip_plane_sums_to_average", p(self.off_pool), p(self.off_sums), N * c, h * w, last_scale))
-        else:
-            self.calls.append(("sofie_hip_global_avg_pool_i8", p(self.off_pool), p(self.off_last), N, c, h * w, R.LAYOUT_NHWC, last_scale))
-        self.calls.append(("sofie_hip_gemm_f32", C.byref(g)))
+        # the addresses of the plan hold as long as the arena; what a pass takes from the attributes it reads at each pass
+        self._quantize, self._last, self._pool, self._sums = (p(self.off_xq), p(self.off_x)), p(self.off_last), p(self.off_pool), p(self.off_sums)
 
     @property
     def x_ptr(self):
@@ -256,9 +246,19 @@ class Int8CNNSession:
         self.rt.call("sofie_hip_upload", self.x_ptr, x.ctypes.data_as(C.c_void_p), C.c_size_t(x.nbytes))
 
     def infer_nosync(self):
-        call = self.rt.call
-        for c in self.calls:
-            call(*c)
+        call, byref, N = self.rt.call, C.byref, self.batch
+        Cin, H, W = self.in_shape
+        call("sofie_hip_quantize_linear", *self._quantize, N * Cin * H * W, float(self.in_scale))
+        c, h, w = self.out_shape
+        if self.pool_in_conv:
+            call("sofie_hip_fill_zero", self._sums, 4 * N * c)
+        for d, a in zip(self.conv_descs, self.conv_args):
+            call("sofie_hip_conv_i8", byref(d), byref(a))
+        if self.pool_in_conv:
+            call("sofie_hip_plane_sums_to_average", self._pool, self._sums, N * c, h * w, float(self.last_scale))
+        else:
+            call("sofie_hip_global_avg_pool_i8", self._pool, self._last, N, c, h * w, R.LAYOUT_NHWC, float(self.last_scale))
+        call("sofie_hip_gemm_f32", byref(self.fc))
 
     def infer(self, x):
         self.upload_input(x)
