@@ -81,6 +81,24 @@ inline int launch_status(const char *what)
    return SOFIE_HIP_OK;
 }
 
+// ---- index arithmetic ---------------------------------------------------------------------------
+
+// Index arithmetic by an extent that the launch knows: a multiplication while every index fits 31 bits (a 64-bit division by a
+// run-time value is some hundred instructions per element, several times what the memory traffic of most kernels leaves room for).
+struct Divisor31 {
+   // with s = ceil(log2 d) and mul = ceil(2^(31 + s) / d), mul d - 2^(31 + s) < 2^s: below 2^31 the error of n mul / 2^(31 + s) is
+   // smaller than 1 / d, and mul < 2^32
+   unsigned d, mul, shift;
+   explicit Divisor31(long long extent) : d((unsigned)extent), shift(0)
+   {
+      while ((1ull << shift) < d)
+         ++shift;
+      mul = (unsigned)(((1ull << (31 + shift)) + d - 1) / d);
+   }
+   typedef unsigned index;
+   __device__ __forceinline__ index over(index n) const { return __umulhi(2 * n, mul) >> shift; }
+};
+
 // ---- scalar formulas shared by every epilogue --------------------------------------------------
 
 // Activation on fp32, the reference's CPU formulas (see sofie_hip.h for the citations).

@@ -17,21 +17,7 @@ static inline unsigned grid_for(size_t work_items, unsigned block = 256, unsigne
    return (unsigned)b;
 }
 
-// Index arithmetic by an extent that the launch knows: a multiplication while every index fits 31 bits (a 64-bit division by a
-// run-time value is some hundred instructions per element, several times what the memory traffic of these kernels leaves room for).
-struct Divisor31 {
-   // with s = ceil(log2 d) and mul = ceil(2^(31 + s) / d), mul d - 2^(31 + s) < 2^s: below 2^31 the error of n mul / 2^(31 + s) is
-   // smaller than 1 / d, and mul < 2^32
-   unsigned d, mul, shift;
-   explicit Divisor31(long long extent) : d((unsigned)extent), shift(0)
-   {
-      while ((1ull << shift) < d)
-         ++shift;
-      mul = (unsigned)(((1ull << (31 + shift)) + d - 1) / d);
-   }
-   typedef unsigned index;
-   __device__ __forceinline__ index over(index n) const { return __umulhi(2 * n, mul) >> shift; }
-};
+// Divisor31 of common.hpp for indices of any size.
 struct Divisor64 {
    unsigned long long d;
    explicit Divisor64(long long extent) : d((unsigned long long)extent) {}

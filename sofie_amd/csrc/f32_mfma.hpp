@@ -152,7 +152,7 @@ struct F32ConvShape {
    int Cg;                                 // channels per group
    int positions;                          // kd * kh * kw
    unsigned long long ow_mul, oh_mul, od_mul; // ceil(2^64 / extent), 0 for an extent of 1: m / extent == umul64hi(m, mul) for 32-bit m
-   unsigned kw_mul, kh_mul, kd_mul, positions_mul; // ceil(2^31 / extent): k / extent == umulhi(2 k, mul) while k * extent < 2^31 (checked on the host)
+   Divisor31 by_kw{1}, by_kh{1}, by_kd{1}, by_positions{1};
 };
 // MASKED (at most 31 kernel positions, extents that fit a buffer): a lane keeps its row's place and one bit per kernel position that
 // lies outside the image; the walk along k, from slab to slab, is scalar.  Three vector instructions per 64 elements.
@@ -193,13 +193,13 @@ struct F32ConvRows {
       r.at = X + (long long)o.image * image + ((long long)r.id0 * s.H + r.ih0) * s.W + r.iw0;
       return r;
    }
-   static __device__ __forceinline__ int divide(int k, unsigned mul) { return (int)__umulhi((unsigned)k * 2u, mul); }
+   static __device__ __forceinline__ int divide(int k, const Divisor31 &by) { return (int)by.over((unsigned)k); }
    // address of column k of a row, or of a zero
    __device__ __forceinline__ const float *element(const row_state &r, int k) const
    {
-      const int t = divide(k, s.kw_mul), kx = k - t * s.kw;
-      const int u = divide(t, s.kh_mul), ky = t - u * s.kh;
-      const int ci = divide(u, s.kd_mul), kz = u - ci * s.kd;
+      const int t = divide(k, s.by_kw), kx = k - t * s.kw;
+      const int u = divide(t, s.by_kh), ky = t - u * s.kh;
+      const int ci = divide(u, s.by_kd), kz = u - ci * s.kd;
       const int dz = kz * s.dil_d, dy = ky * s.dil_h, dx = kx * s.dil_w;
       const bool inside = k < K && (unsigned)(r.id0 + dz) < (unsigned)s.D && (unsigned)(r.ih0 + dy) < (unsigned)s.H && (unsigned)(r.iw0 + dx) < (unsigned)s.W;
       const float *p = r.at + ((long long)ci * channel + ((long long)dz * s.H + dy) * s.W + dx);
@@ -251,15 +251,15 @@ struct F32ConvRows {
       w.k0 = 0;
       if constexpr (MASKED) {
          w.base = (const char *)uniform((long long)base_of(r0));
-         const int t = divide(lane, s.kw_mul), kx = lane - t * s.kw, kz = divide(t, s.kh_mul), ky = t - kz * s.kh;
+         const int t = divide(lane, s.by_kw), kx = lane - t * s.kw, kz = divide(t, s.by_kh), ky = t - kz * s.kh;
          w.table = ((kz * s.dil_d * s.H + ky * s.dil_h) * s.W + kx * s.dil_w) * 4; // lanes past the last position are not asked
-         const int channels = divide(slab, s.positions_mul);
+         const int channels = divide(slab, s.by_positions);
          w.step_channels = channels * (int)channel * 4;
          w.step_rest = slab - channels * s.positions;
 #pragma unroll
          for (int i = 0; i < LD; ++i) {
             w.first[i] = first_k(i);
-            const int ci = divide(w.first[i], s.positions_mul);
+            const int ci = divide(w.first[i], s.by_positions);
             w.position[i] = w.first[i] - ci * s.positions;
             w.channel[i] = ci * (int)channel * 4;
          }

@@ -281,11 +281,7 @@ static int launch_f32_conv_rows(sofie_hip_ctx *ctx, const F32ConvRows<MASKED> &A
 static int launch_f32_conv(sofie_hip_ctx *ctx, const float *X, F32ConvShape s, const float *W, const F32ConvStore &out, long long M, int group, const char *who)
 {
    const int taps = s.kd * s.kh * s.kw, K = s.Cg * taps;
-   auto reciprocal = [](int d) { return (unsigned)(((1ull << 31) + d - 1) / (unsigned)d); };
-   s.kw_mul = reciprocal(s.kw), s.kh_mul = reciprocal(s.kh), s.kd_mul = reciprocal(s.kd), s.positions_mul = reciprocal(taps);
-   // umulhi(2 k, ceil(2^31 / d)) is k / d while k * d < 2^31; a few slabs past K are divided as well
-   const long long longest = taps;
-   SOFIE_HIP_REQUIRE((K + 4096LL) * longest < (1LL << 31), "%s: reduction too long", who);
+   s.by_kw = Divisor31(s.kw), s.by_kh = Divisor31(s.kh), s.by_kd = Divisor31(s.kd), s.by_positions = Divisor31(taps);
    SOFIE_HIP_REQUIRE(group <= 65535, "%s: too many groups for one launch", who);
    auto rows = [&](auto A) {
       A.X = X;
@@ -538,7 +534,7 @@ int sofie_hip_conv_f32(sofie_hip_ctx *ctx, const sofie_conv_desc *d, const float
    SOFIE_HIP_REQUIRE(M < (1LL << 31), "sofie_hip_conv_f32: too many output pixels");
    SOFIE_HIP_REQUIRE((long long)(d->C / d->group) * d->kh * d->kw < (1LL << 31), "sofie_hip_conv_f32: reduction too long");
    const F32ConvShape s{d->C, 1, d->H, d->W, 1, d->kh, d->kw, 1, OH, OW, 0, d->pad_h0, d->pad_w0, 1, d->stride_h, d->stride_w, 1, d->dil_h, d->dil_w,
-                        d->C / d->group, 0, 0, 0, 0, 0, 0, 0, 0};
+                        d->C / d->group, 0, 0, 0, 0};
    const F32ConvStore out{Y, bias, residual, chain, d->Cout, d->Cout / d->group, OH * OW, 0};
    return launch_f32_conv(ctx, X, s, W, out, M, d->group, "sofie_hip_conv_f32");
 }
@@ -573,7 +569,7 @@ int sofie_hip_conv3d_f32(sofie_hip_ctx *ctx, const sofie_conv3d_desc *d, const f
    const long long Kg64 = (long long)(d->C / d->group) * d->kd * d->kh * d->kw;
    SOFIE_HIP_REQUIRE(Kg64 < (1LL << 31), "sofie_hip_conv3d_f32: reduction too long");
    const F32ConvShape s{d->C, d->D, d->H, d->W, d->kd, d->kh, d->kw, outd[0], outd[1], outd[2], d->pad[0], d->pad[1], d->pad[2],
-                        d->stride[0], d->stride[1], d->stride[2], d->dil[0], d->dil[1], d->dil[2], d->C / d->group, 0, 0, 0, 0, 0, 0, 0, 0};
+                        d->stride[0], d->stride[1], d->stride[2], d->dil[0], d->dil[1], d->dil[2], d->C / d->group, 0, 0, 0, 0};
    const F32ConvStore out{Y, bias, residual, chain, d->Cout, d->Cout / d->group, (int)plane, 0};
    return launch_f32_conv(ctx, X, s, W, out, M, d->group, "sofie_hip_conv3d_f32");
 }

@@ -53,3 +53,30 @@ def test_convolutions_around_tile_edges(rt, tile, case):
     rt.sync()
     want = ob.conv_f32(X, Wt, b, pads=pads, strides=strides, dils=dils, group=group, act=1)
     assert np.abs(util.to_host(dY) - want).max() <= 1e-5 * max(1.0, float(np.abs(want).max()))
+
+
+def conv2d_f64(X, Wt, pads):
+    """Stride 1, one group; also the sum of the products' magnitudes, which bounds what rounding can do."""
+    x = np.pad(X.astype(np.float64), ((0, 0), (0, 0), (pads[0], pads[2]), (pads[1], pads[3])))
+    w = Wt.astype(np.float64).reshape(len(Wt), -1)
+    windows = np.lib.stride_tricks.sliding_window_view(x, Wt.shape[2:], axis=(2, 3)).transpose(0, 2, 3, 1, 4, 5)
+    columns = windows.reshape(*windows.shape[:3], -1)
+    return [(c @ v.T).transpose(0, 3, 1, 2) for c, v in ((columns, w), (np.abs(columns), np.abs(w)))]
+
+
+@pytest.mark.parametrize("tile", [0] + TILES, indirect=True)
+@pytest.mark.parametrize("case", [(1, 1, 218, 219, 3, 216, 216, (0, 1, 1, 0)), (1, 3, 225, 224, 2, 224, 224, (0, 0, 0, 0)), (2, 1, 1, 50003, 4, 1, 50000, (0, 2, 0, 0)),
+                                  (1, 2, 40000, 1, 5, 39998, 1, (0, 0, 0, 0))])
+def test_convolutions_with_windows_of_any_length(rt, tile, case):
+    """Reductions times window extents far beyond 2^31, which the index arithmetic of the gather has to divide exactly."""
+    N, Cc, H, W, Cout, kh, kw, pads = case
+    X = util.normal(33, N * Cc * H * W).reshape(N, Cc, H, W)
+    Wt = util.normal(34, Cout * Cc * kh * kw, 0.1).reshape(Cout, Cc, kh, kw)
+    d = conv_desc(N, Cc, H, W, Cout, kh, kw, pads, (1, 1), (1, 1), 1)
+    dX, dW, dY = util.to_dev(X), util.to_dev(Wt), util.dev_empty((N, Cout, d.OH, d.OW), np.float32)
+    torch.cuda.synchronize()
+    print("conv", tile, case, flush=True)
+    rt.call("sofie_hip_conv_f32", C.byref(d), util.ptr(dX), util.ptr(dW), None, R.ACT_NONE, C.c_float(0), util.ptr(dY), None, None)
+    rt.sync()
+    want, most = conv2d_f64(X, Wt, pads)
+    assert np.all(np.abs(util.to_host(dY) - want) <= 1e-5 * most)
