@@ -83,6 +83,9 @@ inline int launch_status(const char *what)
 
 // ---- index arithmetic ---------------------------------------------------------------------------
 
+// The longest M or N of a product: rows are counted in 32 bits up to the end of the last tile, of at most 256.
+constexpr long long MOST_ROWS = 0x7fffffffLL - 255;
+
 // Index arithmetic by an extent that the launch knows: a multiplication while every index fits 31 bits (a 64-bit division by a
 // run-time value is some hundred instructions per element, several times what the memory traffic of most kernels leaves room for).
 struct Divisor31 {

@@ -153,7 +153,7 @@ static bool conv_i8_implicit_shape(const sofie_conv_desc *d, int x_layout)
       if (((t * kw_recip) >> 16) != t / d->kw)
          return false;
    return x_layout == SOFIE_LAYOUT_NHWC && (Cg & (Cg - 1)) == 0 && Cg >= 64 && ntaps <= 32 &&
-          d->C % 16 == 0 && reach < (1LL << 31) && rows < (1LL << 31);
+          d->C % 16 == 0 && reach < (1LL << 31) && rows <= MOST_ROWS;
 }
 
 // The whole reduction (taps x channels per group) fits one 64-byte slab: the rows are gathered inside the GEMM kernel.
@@ -163,7 +163,7 @@ static bool conv_i8_gather_shape(const sofie_conv_desc *d)
       return false;
    const long long K = (long long)(d->C / d->group) * d->kh * d->kw;
    return K <= 64 && (long long)(d->kh - 1) * d->dil_h <= 127 && (long long)(d->kw - 1) * d->dil_w <= 127 &&
-          (long long)d->C * d->H * d->W < (1LL << 31) && (long long)d->N * d->OH * d->OW < (1LL << 31);
+          (long long)d->C * d->H * d->W < (1LL << 31) && (long long)d->N * d->OH * d->OW <= MOST_ROWS;
 }
 
 size_t sofie_hip_conv_i8_workspace(const sofie_conv_desc *d, const sofie_conv_i8_args *a)
@@ -210,6 +210,7 @@ int sofie_hip_conv_i8(sofie_hip_ctx *ctx, const sofie_conv_desc *d, const sofie_
    if (d->N == 0)
       return SOFIE_HIP_OK;
    SOFIE_HIP_REQUIRE(a->X && a->W && a->Y, "sofie_hip_conv_i8: NULL tensor pointer");
+   SOFIE_HIP_REQUIRE((long long)g.OH * g.OW <= MOST_ROWS && d->Cout <= MOST_ROWS, "sofie_hip_conv_i8: too many output pixels or channels");
    const size_t need = sofie_hip_conv_i8_workspace(d, a);
    SOFIE_HIP_REQUIRE(need == 0 || (a->workspace != nullptr && a->workspace_bytes >= need),
                      "sofie_hip_conv_i8: a workspace of at least %zu bytes is needed", need);
@@ -351,7 +352,7 @@ int sofie_hip_conv_i8(sofie_hip_ctx *ctx, const sofie_conv_desc *d, const sofie_
       const long long reach = (long long)d->N * d->H * d->W * d->C + (long long)(d->pad_h0 + d->kh * d->dil_h + 1) * d->W * d->C + (long long)(d->pad_w0 + d->kw * d->dil_w + 1) * d->C;
       const int piece = g.Cg % 16 == 0 ? 16 : 8;
       if (!column_matrix_by_option && launch_cfg_i8(ctx).variant == 0 && a->x_layout == SOFIE_LAYOUT_NHWC && g.Cg % piece == 0 && d->C % piece == 0 &&
-          ((uintptr_t)a->X % piece) == 0 && reach < (1LL << 31) && rows < (1LL << 31) && g.Kp >= 16 && (g.K + 256LL) * (g.Cg > d->kw ? g.Cg : d->kw) < (1LL << 31)) {
+          ((uintptr_t)a->X % piece) == 0 && reach < (1LL << 31) && rows <= MOST_ROWS && g.Kp >= 16 && (g.K + 256LL) * (g.Cg > d->kw ? g.Cg : d->kw) < (1LL << 31)) {
          for (int grp = 0; grp < d->group; ++grp) {
             ConvRows src{};
             src.X = a->X + (size_t)grp * g.Cg;
@@ -393,7 +394,7 @@ int sofie_hip_conv_i8(sofie_hip_ctx *ctx, const sofie_conv_desc *d, const sofie_
    if (imgs_per_chunk > d->N)
       imgs_per_chunk = d->N;
    SOFIE_HIP_REQUIRE(imgs_per_chunk >= 1, "sofie_hip_conv_i8: workspace too small for one image");
-   SOFIE_HIP_REQUIRE(imgs_per_chunk * OHW < (1LL << 31), "sofie_hip_conv_i8: too many rows per chunk");
+   SOFIE_HIP_REQUIRE(imgs_per_chunk * OHW <= MOST_ROWS, "sofie_hip_conv_i8: too many rows per chunk");
    const bool fast = a->x_layout == SOFIE_LAYOUT_NHWC && (g.Cg % 16 == 0) && (d->C % 16 == 0) && (((uintptr_t)a->X & 15) == 0);
 
    for (long long img0 = 0; img0 < d->N; img0 += imgs_per_chunk) {

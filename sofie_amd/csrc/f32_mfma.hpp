@@ -84,7 +84,7 @@ struct F32Matrix {
    struct walk_state {
       const char *base; // first row of the tile, first k of the slab to be asked for next
       long long step;
-      int k0;
+      unsigned k0; // up to a slab past K
    };
    template <int LD, class F>
    __device__ __forceinline__ void walk_start(walk_state<LD> &w, int r0, int, int slab, F &&) const
@@ -114,7 +114,7 @@ struct F32Matrix {
    template <bool WHOLE, int LD>
    __device__ __forceinline__ void load(lds_void_t *to, const lane_state<LD> &st, const walk_state<LD> &w, int i, int kk) const
    {
-      f32_buffer_load<VEC>(to, w.base, WHOLE || w.k0 + kk < K ? st.at[i] : F32_OUTSIDE);
+      f32_buffer_load<VEC>(to, w.base, WHOLE || w.k0 + (unsigned)kk < (unsigned)K ? st.at[i] : F32_OUTSIDE);
    }
 
    // direct fetch of row `row`, k..k+3
@@ -126,16 +126,17 @@ struct F32Matrix {
       const int r = row < rows ? row : rows - 1;
       return row_state{KC ? p + (long long)r * ld : p + r};
    }
-   __device__ __forceinline__ v4f fetch(const row_state &st, int k) const
+   // `left`: how many k there are from k on, negative past K
+   __device__ __forceinline__ v4f fetch(const row_state &st, int k, int left) const
    {
       v4f v = {0.f, 0.f, 0.f, 0.f};
       if (KC && VEC == 4) {
-         if (k < K)
+         if (left > 0)
             v = *(const v4f *)(st.at + k);
       } else {
 #pragma unroll
          for (int j = 0; j < 4; ++j)
-            if (k + j < K)
+            if (j < left)
                v[j] = st.at[KC ? (long long)(k + j) : (long long)(k + j) * ld];
       }
       return v;
@@ -193,15 +194,15 @@ struct F32ConvRows {
       r.at = X + (long long)o.image * image + ((long long)r.id0 * s.H + r.ih0) * s.W + r.iw0;
       return r;
    }
-   static __device__ __forceinline__ int divide(int k, const Divisor31 &by) { return (int)by.over((unsigned)k); }
+   static __device__ __forceinline__ int divide(unsigned k, const Divisor31 &by) { return (int)by.over(k); }
    // address of column k of a row, or of a zero
-   __device__ __forceinline__ const float *element(const row_state &r, int k) const
+   __device__ __forceinline__ const float *element(const row_state &r, unsigned k) const
    {
-      const int t = divide(k, s.by_kw), kx = k - t * s.kw;
+      const int t = divide(k, s.by_kw), kx = (int)k - t * s.kw;
       const int u = divide(t, s.by_kh), ky = t - u * s.kh;
       const int ci = divide(u, s.by_kd), kz = u - ci * s.kd;
       const int dz = kz * s.dil_d, dy = ky * s.dil_h, dx = kx * s.dil_w;
-      const bool inside = k < K && (unsigned)(r.id0 + dz) < (unsigned)s.D && (unsigned)(r.ih0 + dy) < (unsigned)s.H && (unsigned)(r.iw0 + dx) < (unsigned)s.W;
+      const bool inside = k < (unsigned)K && (unsigned)(r.id0 + dz) < (unsigned)s.D && (unsigned)(r.ih0 + dy) < (unsigned)s.H && (unsigned)(r.iw0 + dx) < (unsigned)s.W;
       const float *p = r.at + ((long long)ci * channel + ((long long)dz * s.H + dy) * s.W + dx);
       return inside ? p : f32_zero_page;
    }
@@ -240,7 +241,7 @@ struct F32ConvRows {
    template <int LD>
    struct walk_state {
       const char *base;
-      int k0;
+      unsigned k0;
       int first[LD], position[LD], channel[LD];
       int step_channels, step_rest; // a slab's worth of k in channels (as an offset) and kernel positions
       int table;                    // lane t: offset of kernel position t
@@ -283,22 +284,22 @@ struct F32ConvRows {
    __device__ __forceinline__ void load(lds_void_t *to, const lane_state<LD> &st, const walk_state<LD> &w, int i, int kk) const
    {
       if constexpr (MASKED) {
-         const bool any = WHOLE || w.k0 + w.first[i] < K;
+         const bool any = WHOLE || w.k0 + (unsigned)w.first[i] < (unsigned)K;
          const int position = any ? w.position[i] : 31;
          const int offset = any ? w.channel[i] + __builtin_amdgcn_readlane(w.table, w.position[i]) : 0;
          const int outside = __builtin_amdgcn_sbfe(st.outside, position, 1); // all ones, or none
          f32_buffer_load<1>(to, w.base, st.at | outside, offset);
       } else {
-         const float *at = element(st.r, w.k0 + __builtin_amdgcn_readfirstlane(kk));
+         const float *at = element(st.r, w.k0 + (unsigned)__builtin_amdgcn_readfirstlane(kk));
          __builtin_amdgcn_global_load_lds((global_void_t *)at, to, 4, 0, 0);
       }
    }
-   __device__ __forceinline__ v4f fetch(const row_state &st, int k) const
+   __device__ __forceinline__ v4f fetch(const row_state &st, int k, int) const
    {
       v4f v;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-         v[j] = *element(st, k + j);
+         v[j] = *element(st, (unsigned)k + j);
       return v;
    }
 };
@@ -584,7 +585,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_ke
          for (int e = 0; e < 16; ++e)
             acc[i][j][e] = 0.0f;
 
-   const int KT = (K + BK - 1) / BK;
+   const int KT = (int)(((unsigned)K + BK - 1) / BK);
    // asks for the next slab, number kt
    auto issue = [&](int kt, int stage, auto whole) {
       float *s = f32_lds + stage * STAGE;
@@ -791,18 +792,20 @@ __global__ __launch_bounds__(W * 64) void f32_direct_kernel(ASRC A, BSRC B, STOR
 #pragma unroll
       for (int j = 0; j < NB; ++j)
          acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-   const int KS = (K + 15) / 16;
+   const int KS = (int)(((unsigned)K + 15) / 16);
    for (int s0 = wave; s0 < KS; s0 += W * UNROLL) {
       v4f fa[UNROLL][MB], fb[UNROLL][NB];
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
-         const int k = (s0 + u * W) * 16 + lk * 4; // steps past the end fetch zeros
+         // steps past the end, whose k may leave 31 bits, fetch zeros
+         const unsigned first = (unsigned)(s0 + u * W) * 16;
+         const int k = (int)(first + lk * 4), left = (int)((unsigned)K - first) - lk * 4;
 #pragma unroll
          for (int i = 0; i < MB; ++i)
-            fa[u][i] = A.fetch(ra[i], k);
+            fa[u][i] = A.fetch(ra[i], k, left);
 #pragma unroll
          for (int j = 0; j < NB; ++j)
-            fb[u][j] = B.fetch(rb[j], k);
+            fb[u][j] = B.fetch(rb[j], k, left);
       }
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u)

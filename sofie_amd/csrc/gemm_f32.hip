@@ -142,8 +142,8 @@ namespace sofie_hip {
 enum F32Tile { F32_CONV3X3_32 = 3032, F32_CONV3X3_64 = 3064, F32_CONV3X3_128 = 3128, F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
 static int pick_f32_tile(int M, int N, int K, int batch, double *time_us = nullptr)
 {
-   auto tiles = [&](int bm, int bn) { return (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
-   const double slabs = (K + 31) / 32, steps = (K + 15) / 16;
+   auto tiles = [&](int bm, int bn) { return std::ceil((double)M / bm) * std::ceil((double)N / bn) * batch; };
+   const double slabs = std::ceil(K / 32.0), steps = std::ceil(K / 16.0);
    auto tiled = [&](int bm, int bn, double launch, double slab, double tile) { return launch + std::ceil(tiles(bm, bn) / 256.0) * (slabs * slab + tile); };
    int best = F32_DIRECT;
    double least = 2.0 + std::max(1.35 * std::ceil(steps / 32.0), tiles(16, 16) * steps * 2048.0 / 10.5e6) + 0.45 * tiles(16, 16) / 256.0;
@@ -164,11 +164,11 @@ static int pick_f32_tile(int M, int N, int K, int batch, double *time_us = nullp
 // the products) and 0.92 (128 x 32).  The direct kernel decomposes every k by itself: for few tiles only.
 static int pick_f32_conv_tile(int M, int N, int K, int group)
 {
-   auto tiles = [&](int bm, int bn) { return (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * group; };
-   const double slabs = (K + 31) / 32;
+   auto tiles = [&](int bm, int bn) { return std::ceil((double)M / bm) * std::ceil((double)N / bn) * group; };
+   const double slabs = std::ceil(K / 32.0);
    auto tiled = [&](int bm, int bn, double launch, double slab, double tile) { return launch + std::ceil(tiles(bm, bn) / 256.0) * (slabs * slab + tile); };
    int best = F32_DIRECT;
-   double least = 5.3 + tiles(16, 16) / 256.0 * (0.9 + 0.17 * ((K + 15) / 16));
+   double least = 5.3 + tiles(16, 16) / 256.0 * (0.9 + 0.17 * std::ceil(K / 16.0));
    auto offer = [&](int tile, double t) {
       if (t < least)
          least = t, best = tile;
@@ -283,6 +283,7 @@ static int launch_f32_conv(sofie_hip_ctx *ctx, const float *X, F32ConvShape s, c
    const int taps = s.kd * s.kh * s.kw, K = s.Cg * taps;
    s.by_kw = Divisor31(s.kw), s.by_kh = Divisor31(s.kh), s.by_kd = Divisor31(s.kd), s.by_positions = Divisor31(taps);
    SOFIE_HIP_REQUIRE(group <= 65535, "%s: too many groups for one launch", who);
+   SOFIE_HIP_REQUIRE(M <= MOST_ROWS && out.Cout_g <= MOST_ROWS, "%s: too many output pixels or channels", who);
    auto rows = [&](auto A) {
       A.X = X;
       A.s = s;
@@ -313,7 +314,7 @@ static int launch_f32_chain(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *layer
 {
    *launched = false;
    const int M = layers[0].M;
-   bool fused = count >= 2 && M >= 1;
+   bool fused = count >= 2 && M >= 1 && M <= MOST_ROWS;
    int width = layers[0].K;
    ChainArgs a;
    a.count = count;
@@ -323,7 +324,7 @@ static int launch_f32_chain(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *layer
    for (int l = 0; l < count && fused; ++l) {
       const sofie_gemm_f32_desc &d = layers[l];
       const long long ldb = d.ldb ? d.ldb : (d.transB ? d.K : d.N), ldy = d.ldy ? d.ldy : d.N;
-      fused = d.M == M && d.N >= 1 && d.K >= 1 && !d.transA && d.batch == 1 && d.A && d.B && d.Y && ldb >= (d.transB ? d.K : d.N) && ldy >= d.N &&
+      fused = d.M == M && d.N >= 1 && d.N <= 8192 && d.K >= 1 && d.K <= 8192 && !d.transA && d.batch == 1 && d.A && d.B && d.Y && ldb >= (d.transB ? d.K : d.N) && ldy >= d.N &&
               d.bias_mode >= SOFIE_BIAS_NONE && d.bias_mode <= SOFIE_BIAS_FULL && (d.bias_mode == SOFIE_BIAS_NONE || d.C != nullptr) &&
               (l == 0 ? a.lda >= d.K : (d.K == layers[l - 1].N && (d.lda ? d.lda : d.K) == (layers[l - 1].ldy ? layers[l - 1].ldy : layers[l - 1].N)));
       if (!fused)
@@ -429,6 +430,7 @@ int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *d)
    const long long ldy = d->ldy ? d->ldy : N;
    SOFIE_HIP_REQUIRE(lda >= (d->transA ? M : K) && ldb >= (d->transB ? K : N) && ldy >= N,
                      "sofie_hip_gemm_f32: leading dimension too small");
+   SOFIE_HIP_REQUIRE(M <= MOST_ROWS && N <= MOST_ROWS, "sofie_hip_gemm_f32: M or N too long");
    ep.alpha = d->alpha;
    ep.beta = d->beta;
    ep.C = d->bias_mode == SOFIE_BIAS_NONE ? nullptr : d->C;

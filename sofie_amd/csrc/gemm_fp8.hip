@@ -231,6 +231,7 @@ int sofie_hip_gemm_fp8(sofie_hip_ctx *ctx, const sofie_gemm_fp8_desc *d)
    int ldb = d->ldb ? d->ldb : (d->transB ? K : N);
    int ldy = d->ldy ? d->ldy : N;
    SOFIE_HIP_REQUIRE(lda >= K && ldb >= (d->transB ? K : N) && ldy >= N, "sofie_hip_gemm_fp8: leading dimension too small");
+   SOFIE_HIP_REQUIRE(M <= MOST_ROWS && N <= MOST_ROWS, "sofie_hip_gemm_fp8: M or N too long");
    F8Epilogue ep;
    ep.bias = d->bias;
    ep.scale = d->scale;

@@ -166,7 +166,7 @@ int sofie_hip_transpose_i8(sofie_hip_ctx *ctx, int8_t *dst, const int8_t *src, i
    if (ld_dst == 0)
       ld_dst = rows;
    SOFIE_HIP_REQUIRE(ld_src >= cols && ld_dst >= rows, "sofie_hip_transpose_i8: leading dimension too small");
-   SOFIE_HIP_REQUIRE((rows + 63) / 64 <= 65535, "sofie_hip_transpose_i8: too many rows");
+   SOFIE_HIP_REQUIRE(rows <= 65535 * 64 && cols <= MOST_ROWS, "sofie_hip_transpose_i8: too many rows or columns");
    return transpose_i8(ctx->stream, dst, src, rows, cols, ld_src, ld_dst);
 }
 
@@ -188,6 +188,7 @@ static int gemm_i8_with_workspace(sofie_hip_ctx *ctx, const sofie_gemm_i8_desc *
    int ldy = d->ldy ? d->ldy : N;
    SOFIE_HIP_REQUIRE(lda >= (d->transA ? M : K) && ldb >= (d->transB ? K : N) && ldy >= N,
                      "sofie_hip_gemm_i8: leading dimension too small");
+   SOFIE_HIP_REQUIRE(M <= MOST_ROWS && N <= MOST_ROWS, "sofie_hip_gemm_i8: M or N too long");
 
    I8Epilogue ep;
    ep.bias = d->bias;

@@ -13,7 +13,7 @@ typedef int v4i_unaligned __attribute__((ext_vector_type(4), aligned(1)));
 // The 16 bytes of a row from k on, zero from K on.  Never reads outside the row's K bytes.
 __device__ __forceinline__ v4i load_chunk_tail(const int8_t *row, int k, int K)
 {
-   if (k + 16 <= K)
+   if (k <= K - 16)
       return *(const v4i_unaligned *)(row + k);
    union {
       v4i v;
@@ -26,7 +26,7 @@ __device__ __forceinline__ v4i load_chunk_tail(const int8_t *row, int k, int K)
    if (K >= 16) {
       // the last 16 bytes of the row, shifted down to where k lies
       u.v = *(const v4i_unaligned *)(row + K - 16);
-      const int drop = (k + 16 - K) * 8; // bits; 8 .. 120
+      const int drop = (k - K + 16) * 8; // bits; 8 .. 120
       if (drop >= 64) {
          u.q[0] = u.q[1] >> (drop - 64);
          u.q[1] = 0;

@@ -15,7 +15,7 @@ namespace sofie_hip {
 // which cut_chunk moves down to k, zeros behind them.
 __device__ __forceinline__ v4i fetch_cut(const int8_t *row, int k, int K)
 {
-   return *(const v4i_unaligned *)(row + (k + 16 <= K ? k : K - 16));
+   return *(const v4i_unaligned *)(row + (k <= K - 16 ? k : K - 16));
 }
 __device__ __forceinline__ v4i cut_chunk(v4i v, int k, int K)
 {
@@ -24,7 +24,7 @@ __device__ __forceinline__ v4i cut_chunk(v4i v, int k, int K)
       unsigned long long q[2];
    } u;
    u.v = v;
-   const int drop = (k + 16 - K) * 8; // bits that lie before k
+   const int drop = (k - K + 16) * 8; // bits that lie before k
    if (drop > 0) {
       const unsigned long long hi = drop >= 128 ? 0 : u.q[1];
       u.q[0] = drop >= 64 ? hi >> (drop & 63) : (u.q[0] >> drop) | (u.q[1] << (64 - drop));
