@@ -73,6 +73,16 @@ inline void launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t ld
    }(std::forward<A>(a)...);
 }
 
+// A launch takes fewer than 2^32 threads: a longer list of workgroups goes out in several, f(first workgroup, how many).  All but the last
+// are of a multiple of eight, so that a workgroup's XCD follows from its place in the list.
+template <class F>
+inline void in_launches(long long workgroups, int threads, F &&f)
+{
+   const long long most = 0xffffffffLL / threads / 8 * 8;
+   for (long long first = 0; first < workgroups; first += most)
+      f((int)first, (unsigned)(workgroups - first < most ? workgroups - first : most));
+}
+
 inline int launch_status(const char *what)
 {
    hipError_t e = hipGetLastError();

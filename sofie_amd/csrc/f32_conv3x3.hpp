@@ -53,7 +53,7 @@ struct F32Conv3x3Shape {
 // that cover each other's trips to memory and barriers.  WAVES_K waves share a wave tile, each multiplying every WAVES_K-th step of
 // a slab: where there are few tiles, smaller ones keep as many matrix cores busy.
 template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int CS, int PLANE, int WVEC>
-__global__ __launch_bounds__(256, 2) void f32_conv3x3_kernel(F32Conv3x3 a, F32ConvStore out, int tiles_m, int tiles_n)
+__global__ __launch_bounds__(256, 2) void f32_conv3x3_kernel(F32Conv3x3 a, F32ConvStore out, int tiles_m, int tiles_n, int first_tile)
 {
    typedef F32Conv3x3Shape<BM, BN, CS, PLANE, WVEC> S;
    constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N, MT = TM / 32, NT = TN / 32;
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_kernel(F32Conv3x3 a, F32Co
    a.W += (long long)z * a.N * a.K;
    out.select_batch(z);
    int tm, tn;
-   f32_tile_of_block(tiles_m, tiles_n, tm, tn);
+   f32_tile_of_block(first_tile, tiles_m, tiles_n, tm, tn);
    const int m0 = tm * BM, n0 = tn * BN;
    const int VW = a.OW + 2, VH = a.OH + 2;
    auto quotient = [](int n, unsigned long long mul) { return mul ? (int)__umul64hi((unsigned long long)(unsigned)n, mul) : n; };
@@ -288,7 +288,9 @@ static int launch_f32_conv3x3_as(hipStream_t stream, const F32Conv3x3 &a, const 
    static bool configured[64] = {};
    if (int st = configure_lds_once(kern, std::max(stage * 2, parts), configured))
       return st;
-   launch_kernel(kern, dim3((unsigned)(tiles_m * tiles_n), 1, (unsigned)group), dim3(256), smem, stream, a, out, tiles_m, tiles_n);
+   in_launches((long long)tiles_m * tiles_n, 256, [&](int first, unsigned count) {
+      launch_kernel(kern, dim3(count, 1, (unsigned)group), dim3(256), smem, stream, a, out, tiles_m, tiles_n, first);
+   });
    return launch_status("f32_conv3x3_kernel");
 }
 

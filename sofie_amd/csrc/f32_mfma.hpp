@@ -26,15 +26,16 @@ __device__ __forceinline__ v4f mfma_f32_step(const v4f &n_side, const v4f &m_sid
    return acc;
 }
 
-// tile_of_block; a single column of tiles (the usual convolution) needs none of its divisions
-__device__ __forceinline__ void f32_tile_of_block(int tiles_m, int tiles_n, int &tm, int &tn)
+// tile_of_block for a launch of in_launches; a single column of tiles (the usual convolution) needs none of its divisions
+__device__ __forceinline__ void f32_tile_of_block(int first, int tiles_m, int tiles_n, int &tm, int &tn)
 {
+   const int bid = first + blockIdx.x;
    if (tiles_n == 1) {
-      const int bid = blockIdx.x, per = tiles_m / 8, rem = tiles_m % 8, xcd = bid % 8;
+      const int per = tiles_m / 8, rem = tiles_m % 8, xcd = bid % 8;
       tm = xcd * per + (xcd < rem ? xcd : rem) + bid / 8;
       tn = 0;
    } else {
-      tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, 4, tm, tn);
+      tile_of_block(bid, tiles_m * tiles_n, tiles_m, tiles_n, 4, tm, tn);
    }
 }
 
@@ -547,7 +548,7 @@ constexpr size_t f32_tile_lds_bytes(int stages)
 // which puts all four SIMDs of a CU to work on tiles smaller than four blocks of 32 x 32.
 template <class ASRC, class BSRC, class STORE, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int WAVES_K, int STAGES>
 __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_kernel(ASRC A, BSRC B, STORE out, int M, int N, int K, int tiles_m,
-                                                                                   int tiles_n, long long strideA, long long strideB)
+                                                                                   int tiles_n, int first_tile, long long strideA, long long strideB)
 {
    constexpr int NW = WAVES_M * WAVES_N * WAVES_K;
    constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N, MT = TM / 32, NT = TN / 32;
@@ -566,7 +567,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_ke
    A.select_group(z);
    out.select_batch(z);
    int tm, tn;
-   f32_tile_of_block(tiles_m, tiles_n, tm, tn);
+   f32_tile_of_block(first_tile, tiles_m, tiles_n, tm, tn);
    const int m0 = tm * BM, n0 = tn * BN;
    const int lane = threadIdx.x & 63;
    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -762,8 +763,8 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_ke
 // % 16) supplies k = 4 lk + j of row c to MFMA j); the partial tiles meet in LDS.  What such a product
 // costs is one trip to memory for its operands: every wave has UNROLL steps of loads in flight at once.
 template <class ASRC, class BSRC, class STORE, int MB, int NB, int W, int UNROLL>
-__global__ __launch_bounds__(W * 64) void f32_direct_kernel(ASRC A, BSRC B, STORE out, int M, int N, int K, int tiles_m, int tiles_n, long long strideA,
-                                                            long long strideB)
+__global__ __launch_bounds__(W * 64) void f32_direct_kernel(ASRC A, BSRC B, STORE out, int M, int N, int K, int tiles_m, int tiles_n, int first_tile,
+                                                            long long strideA, long long strideB)
 {
    constexpr int TM = MB * 16, TN = NB * 16, PITCH = TN + 4;
    __shared__ __attribute__((aligned(16))) float part[W][TM][PITCH];
@@ -773,7 +774,7 @@ __global__ __launch_bounds__(W * 64) void f32_direct_kernel(ASRC A, BSRC B, STOR
    A.select_group(z);
    out.select_batch(z);
    int tm, tn;
-   f32_tile_of_block(tiles_m, tiles_n, tm, tn);
+   f32_tile_of_block(first_tile, tiles_m, tiles_n, tm, tn);
    const int m0 = tm * TM, n0 = tn * TN;
    const int lane = threadIdx.x & 63;
    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -853,8 +854,10 @@ static int launch_f32_tile(hipStream_t stream, const ASRC &A, const BSRC &B, con
    static bool configured[64] = {};
    if (int st = configure_lds_once(kern, most, configured))
       return st;
-   launch_kernel(kern, dim3((unsigned)nwg, 1, (unsigned)batch), dim3(WAVES_M * WAVES_N * WAVES_K * 64), smem, stream, A, B, out, M, N, K, tiles_m, tiles_n, strideA,
-                      strideB);
+   constexpr int NTHREADS = WAVES_M * WAVES_N * WAVES_K * 64;
+   in_launches(nwg, NTHREADS, [&](int first, unsigned count) {
+      launch_kernel(kern, dim3(count, 1, (unsigned)batch), dim3(NTHREADS), smem, stream, A, B, out, M, N, K, tiles_m, tiles_n, first, strideA, strideB);
+   });
    return launch_status("f32_tile_kernel");
 }
 
@@ -865,8 +868,10 @@ static int launch_f32_direct(hipStream_t stream, const ASRC &A, const BSRC &B, c
    const long long nwg = (long long)tiles_m * tiles_n;
    if (nwg > 0x7fffffffLL)
       return fail(SOFIE_HIP_ERR_INVALID, "fp32 product: too many tiles");
-   launch_kernel((f32_direct_kernel<ASRC, BSRC, STORE, MB, NB, W, UNROLL>), dim3((unsigned)nwg, 1, (unsigned)batch), dim3(W * 64), 0, stream, A, B, out, M, N, K,
-                      tiles_m, tiles_n, strideA, strideB);
+   in_launches(nwg, W * 64, [&](int first, unsigned count) {
+      launch_kernel((f32_direct_kernel<ASRC, BSRC, STORE, MB, NB, W, UNROLL>), dim3(count, 1, (unsigned)batch), dim3(W * 64), 0, stream, A, B, out, M, N, K, tiles_m,
+                    tiles_n, first, strideA, strideB);
+   });
    return launch_status("f32_direct_kernel");
 }
 

@@ -97,14 +97,15 @@ struct DirectF8 {
 };
 
 template <class MMA, int MB, int NB, int W, int UNROLL, class EPI>
-__global__ __launch_bounds__(W * 64) void mfma8_direct_kernel(RowMajorRows A, RowMajorRows Bt, int M, int N, int K, EPI ep, int tiles_m, int tiles_n, int sw)
+__global__ __launch_bounds__(W * 64) void mfma8_direct_kernel(RowMajorRows A, RowMajorRows Bt, int M, int N, int K, EPI ep, int tiles_m, int tiles_n, int sw,
+                                                              int first_tile)
 {
    constexpr int STEP = 128, TM = MB * 16, TN = NB * 16, PITCH = TN + 4;
    typedef typename MMA::acc_t acc_t;
    typedef typename MMA::elem_t elem_t;
    __shared__ __attribute__((aligned(16))) elem_t part[W][TM][PITCH];
    int tm, tn;
-   tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, sw, tm, tn);
+   tile_of_block(first_tile + blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, sw, tm, tn);
    const int m0 = tm * TM, n0 = tn * TN;
    const int lane = threadIdx.x & 63;
    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -204,8 +205,10 @@ static int launch_mfma8_direct(const LaunchCfg &lc, const int8_t *A, const int8_
    const long long nwg = (long long)tiles_m * tiles_n;
    if (nwg > 0x7fffffffLL)
       return fail(SOFIE_HIP_ERR_INVALID, "gemm: too many tiles");
-   launch_kernel((mfma8_direct_kernel<MMA, MB, NB, W, UNROLL, EPI>), dim3((unsigned)nwg), dim3(W * 64), 0, lc.stream, RowMajorRows{A, lda}, RowMajorRows{Bt, ldb}, M, N,
-                      K, ep, tiles_m, tiles_n, lc.swizzle);
+   in_launches(nwg, W * 64, [&](int first, unsigned count) {
+      launch_kernel((mfma8_direct_kernel<MMA, MB, NB, W, UNROLL, EPI>), dim3(count), dim3(W * 64), 0, lc.stream, RowMajorRows{A, lda}, RowMajorRows{Bt, ldb}, M, N, K, ep,
+                    tiles_m, tiles_n, lc.swizzle, first);
+   });
    return launch_status("mfma8_direct_kernel");
 }
 

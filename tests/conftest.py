@@ -27,7 +27,7 @@ def rt():
 def opt(rt):
     """opt(name, value) sets a kernel-choice override on the shared context (sofie_hip_ctx_set_option); the defaults are put
     back when the test ends."""
-    defaults = {"swizzle": 4, "i8_tile": 0, "f8_tile": 0, "gemm_variant": 0, "conv_explicit": 0, "f32_skinny": -1, "f32_chain": -1}
+    defaults = {"swizzle": 4, "i8_tile": 0, "f8_tile": 0, "gemm_variant": 0, "conv_explicit": 0, "f32_skinny": -1, "f32_chain": -1, "f32_tile": 0}
     touched = []
 
     def set_option(name, value):
