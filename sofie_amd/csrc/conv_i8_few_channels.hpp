@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256) void conv_i8_few_channels_kernel(FewChannelCon
       const int pair = lk * 4 + q;
       const int c = g.pair_c[pair], ky = g.pair_ky[pair];
       pair_off[q] = (c * g.H + ky * g.dil_h) * g.W;
-      pair_dy[q] = pair < npairs ? ky * g.dil_h : (1 << 24);
+      pair_dy[q] = pair < npairs ? ky * g.dil_h : -(1 << 30); // above any image (rows of 8 bytes or more: at most 2^28 of them)
    }
 
    // ---- epilogue constants of the lane's column, and the accumulators' start values (bias or zero), per column block

@@ -42,7 +42,7 @@ __global__ __launch_bounds__(256) void conv_i8_windows_kernel(FewChannelConv g, 
       const int pair = lk * 4 + q;
       const int ch = g.pair_c[pair], ky = g.pair_ky[pair];
       pair_off[q] = (ch * g.H + ky * g.dil_h) * g.W;
-      pair_dy[q] = pair < npairs ? ky * g.dil_h : (1 << 24);
+      pair_dy[q] = pair < npairs ? ky * g.dil_h : -(1 << 30); // above any image (rows of 8 bytes or more: at most 2^28 of them)
    }
    typename EPI::template col_params<4> prm[NT];
 #pragma unroll

@@ -86,3 +86,27 @@ def test_fp32_convolutions_of_many_pixels(rt, opt, images, hw, kernel, tile):
             want[:, rows, columns] += w[i, j] * x[:, max(0, i - h):hw[0] - max(0, h - i), max(0, j - h):hw[1] - max(0, h - j)]
     # nine products of values below one, added in either order
     assert float(want.sub_(y).abs_().max()) <= 2 * 9 * 9 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("Cout", [3, 64])
+def test_int8_convolution_of_a_tall_image(rt, Cout):
+    """More rows than 2^24: the unused places of a window kernel's reduction still lie outside the image."""
+    H, W = (1 << 24) + 40, 8
+    print("conv_i8", H, W, Cout, flush=True)
+    x, w = torch.randint(-3, 4, (H, W), device="cuda", dtype=torch.int8), torch.randint(-2, 3, (Cout, 3, 3), device="cuda", dtype=torch.int8)
+    y, scale = torch.empty((H, W, Cout), device="cuda", dtype=torch.int8), torch.ones(Cout, device="cuda")
+    d, a = R.ConvDesc(), R.ConvI8Args()
+    d.N, d.C, d.Cout, d.group, d.H, d.OH, d.W, d.OW, d.kh, d.kw = 1, 1, Cout, 1, H, H, W, W, 3, 3
+    d.pad_h0 = d.pad_w0 = d.pad_h1 = d.pad_w1 = d.stride_h = d.stride_w = d.dil_h = d.dil_w = 1
+    packed = torch.zeros(rt.lib.sofie_hip_conv_weight_i8_packed_bytes(C.byref(d)), device="cuda", dtype=torch.int8)
+    torch.cuda.synchronize()
+    rt.call("sofie_hip_pack_conv_weight_i8", C.byref(d), p(packed), p(w))
+    a.X, a.W, a.scale, a.Y, a.out, a.w_is_packed = p(x), p(packed), p(scale), p(y), R.I8OUT_I8, 1
+    a.x_layout, a.y_layout = R.LAYOUT_NCHW, R.LAYOUT_NHWC
+    rt.call("sofie_hip_conv_i8", C.byref(d), C.byref(a))
+    rt.sync()
+    padded = torch.zeros((H + 2, W + 2), device="cuda", dtype=torch.int8)
+    padded[1:-1, 1:-1] = x
+    for c in (0, 1, Cout - 1):          # sums of at most 54: exact in 8 bits
+        want = sum(w[c, i, j] * padded[i:i + H, j:j + W] for i in range(3) for j in range(3))
+        assert torch.equal(y[:, :, c], want), c
