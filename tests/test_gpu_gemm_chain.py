@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 def run_chain(rt, X, layers, alias=None):
     """layers: dicts with W (stored as given), transB, bias (or None), bias_mode, act, act_alpha, alpha, post (list or None),
-    residual (array of the output's shape or None).  alias = {l: m}: layer l writes into the buffer of layer m < l (same
+    residual (array of the output's shape or None), residual_of (number of an earlier layer whose output is the residual).  alias = {l: m}: layer l writes into the buffer of layer m < l (same
     size, or the first floats of it when the shapes differ).  Returns the device results of every layer."""
     n = len(layers)
     descs = (R.GemmF32Desc * n)()
@@ -26,7 +26,7 @@ def run_chain(rt, X, layers, alias=None):
         N = L["W"].shape[0] if L["transB"] else L["W"].shape[1]
         dW = util.to_dev(L["W"])
         dC = None if L.get("bias") is None else util.to_dev(L["bias"])
-        dR = None if L.get("residual") is None else util.to_dev(L["residual"])
+        dR = outs[L["residual_of"]] if "residual_of" in L else None if L.get("residual") is None else util.to_dev(L["residual"])
         if alias and l in alias:
             dY = outs[alias[l]]
             if tuple(dY.shape) != (M, N):      # another shape: the first M * N floats of that buffer
@@ -63,6 +63,8 @@ def oracle_chain(X, layers):
         N = W.shape[0] if L["transB"] else W.shape[1]
         bm = L.get("bias_mode", R.BIAS_NONE if L.get("bias") is None else R.BIAS_ROW)
         y = ob.gemm_f32(A, W, L.get("bias"), M=M, N=N, K=K, transB=int(L["transB"]), alpha=L.get("alpha", 1.0), beta=L.get("beta", 1.0), bias_mode=bm, act=0)
+        if "residual_of" in L:
+            y = (y + outs[L["residual_of"]]).astype(np.float32)
         if L.get("residual") is not None:
             y = (y + L["residual"]).astype(np.float32)
         ops = ([(L["act"], L.get("act_alpha", 0.0), 0.0)] if L.get("act", 0) else []) + list(L.get("post") or [])
@@ -179,3 +181,18 @@ def test_chain_of_one_wide_rows_and_refusals(rt):
         rt.call("sofie_hip_gemm_chain_f32", descs, 2)
     with pytest.raises(R.SofieHipError, match="layers"):
         rt.call("sofie_hip_gemm_chain_f32", descs, 17)
+
+
+@pytest.mark.parametrize("dims, to, of", [([784, 128, 128, 128, 10], 2, 0), ([2048, 64, 64, 64, 64, 7], 3, 0), ([2048, 64, 64, 64, 64, 64, 7], 4, 1), ([40, 600, 48, 48, 600], 3, 0)])
+@pytest.mark.parametrize("M", [1, 64, 200])
+@pytest.mark.parametrize("transB", [True, False])
+def test_a_chain_whose_residual_is_an_earlier_layers_output(rt, dims, to, of, M, transB):
+    """Wide first layers run by themselves and the layers behind them share a launch: the residual then comes from before the split, or from
+    within the layers that would share one, which run one by one."""
+    layers = mlp_layers(dims, 970, transB)
+    layers[to]["residual_of"] = of
+    X = util.uniform01(971 + M, M * dims[0]).reshape(M, dims[0])
+    print("gemm chain with a residual", dims, to, of, M, transB, flush=True)
+    got = run_chain(rt, X, layers)
+    want, mags = oracle_chain(X, layers)
+    check(got, want, mags)
