@@ -48,12 +48,21 @@ enum {
 int sofie_hip_ctx_create(sofie_hip_ctx **out, int device, void *external_stream);
 int sofie_hip_ctx_destroy(sofie_hip_ctx *ctx);
 /* Kernel-choice overrides of one context, for tuning and for tests that must reach a particular kernel (no counterpart in the
- * reference, whose GPU path has no such choice): "i8_tile" / "f8_tile" (64, 128, 256; 258 and 512 ask for the two-per-CU and the
- * persistent kernel; 0 = heuristic), "gemm_variant" (1: alternative pipelined kernel, -1: general kernel only), "swizzle"
- * (tile order), "conv_explicit" (1: int8 convolutions through a column matrix whenever the workspace holds one), "f32_skinny",
- * "f32_chain" (0 / 1, -1 = heuristic), "f32_tile" (fp32 products and convolutions: 16 the direct kernel; 32, 62, 64, 126, 128 the tile
- * kernel with tiles of 32 x 32, 64 x 32, 64 x 64, 128 x 32 (convolutions), 128 x 128 (products); 0 = heuristic).  Each is also read once, at sofie_hip_ctx_create, from the environment variable
- * SOFIE_HIP_<NAME IN CAPITALS>; nothing reads the environment after that. */
+ * reference, whose GPU path has no such choice).  A kernel that does not take a call's shape leaves it to the others.
+ *   "i8_tile" / "f8_tile"  0 = heuristic; 64, 128, 256 the tile of the pipelined or general kernel; 258 and 512 the two-per-CU and the
+ *                          persistent kernel; 16 and 32 the direct kernel with tiles of 16 x 16 and 32 x 32 (products only: an int8
+ *                          convolution that reads its input directly refuses them); for int8 convolutions also 27 the window kernel of
+ *                          few input channels, 257 the 256 x 128 tile with a ring of five, 576 the kernel with resident weights
+ *   "gemm_variant"         1: alternative pipelined kernel, -1: general kernel only
+ *   "swizzle"              tile order
+ *   "conv_explicit"        1: int8 convolutions through a column matrix whenever the workspace holds one
+ *   "f32_tile"             0 = heuristic; 16 the direct kernel; 32, 62, 64, 126, 128 the tile kernel with tiles of 32 x 32, 64 x 32,
+ *                          64 x 64, 128 x 32 (convolutions), 128 x 128 (products); 3032, 3064, 3128 the kernel of 3 x 3 convolutions with
+ *                          tiles of 32, 64, 128 pixels (64 x 64 tiles for what it does not take)
+ *   "f32_skinny"           -1 = heuristic; 1 the direct kernel, 0 the 64 x 64 tiles where "f32_tile" is 0
+ *   "f32_chain"            -1 = heuristic; 1 all layers of sofie_hip_gemm_chain_f32 in one launch if they allow it, 0 each by itself
+ * Each is also read once, at sofie_hip_ctx_create, from the environment variable SOFIE_HIP_<NAME IN CAPITALS>; nothing reads the
+ * environment after that. */
 int sofie_hip_ctx_set_option(sofie_hip_ctx *ctx, const char *name, int32_t value);
 const char *sofie_hip_last_error(void);
 int sofie_hip_abi_version(void);
@@ -210,9 +219,13 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
  *                              next layer's QuantizeLinear, same fp32 operations in the same order)
  * One fp32 multiply (no fused multiply-add), round-half-to-even, saturation to [-128,127].
  * A is [M,K] int8 row-major (lda), B is [K,N] row-major (ldb) or, with transB, stored [N,K].
- * The MFMA kernel wants both operands K-contiguous; a B given as [K,N] is transposed into
- * `workspace` (K*N bytes, 256-B aligned) on every call.  A constant B (a weight) is better re-laid
- * out once at Session construction with sofie_hip_transpose_i8 and then passed with transB = 1. */
+ * The MFMA kernel wants both operands K-contiguous; a B given as [K,N] is transposed on its way
+ * through the kernel or into `workspace` (K*N bytes, 256-B aligned) on every call: which of the two
+ * depends on sizes, alignment and the context's options, so the workspace is asked for in either case.
+ * A constant B (a weight) is better re-laid out once at Session construction with
+ * sofie_hip_transpose_i8 and then passed with transB = 1.
+ * M and N of a product are at most 2^31 - 256 (here and in the fp32 and FP8 products, and for the output
+ * pixels and channels of a convolution); longer ones are refused. */
 enum { SOFIE_I8OUT_I32 = 0, SOFIE_I8OUT_F32 = 1, SOFIE_I8OUT_I8 = 2, SOFIE_I8OUT_I8_DQQ = 3,
        SOFIE_I8OUT_I8_PLANE_SUMS = 4 /* sofie_hip_conv_i8 only, see there */ };
 typedef struct sofie_gemm_i8_desc {
@@ -232,7 +245,8 @@ typedef struct sofie_gemm_i8_desc {
    size_t workspace_bytes;
 } sofie_gemm_i8_desc;
 int sofie_hip_gemm_i8(sofie_hip_ctx *ctx, const sofie_gemm_i8_desc *d);
-/* Bytes of workspace sofie_hip_gemm_i8 needs for this descriptor (0 if none). */
+/* Bytes of workspace sofie_hip_gemm_i8 asks for with this descriptor (0 if none): enough for every kernel that a context may choose, so
+ * some calls leave it unused. */
 size_t sofie_hip_gemm_i8_workspace(const sofie_gemm_i8_desc *d);
 /* sofie_hip_gemm_i8 for callers that cannot allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  It has no counterpart in the reference.  The scratch for the operand re-layout (B given
@@ -377,9 +391,13 @@ int sofie_hip_conv3d_f32(sofie_hip_ctx *ctx, const sofie_conv3d_desc *d, const f
  * w_is_packed, the re-laid-out form sofie_hip_pack_conv_weight_i8 writes once at Session construction
  * (the role of tensor_<Y>_f in the reference, ROperator_Conv.hxx:456-476).  NHWC input whose channels
  * per group are a power of two >= 64 (and at most 32 filter taps) is read directly by the GEMM kernel
- * (implicit GEMM, no column matrix); any other case gathers a column matrix first.  The workspace holds
- * the packed weights (unless w_is_packed) and, when a column matrix is needed, that of as many images as
- * fit (at least one); sofie_hip_conv_i8_workspace returns the minimum, which may be 0. */
+ * (implicit GEMM, no column matrix), a reduction of at most 64 bytes is gathered in it, and NHWC input whose
+ * channels per group are a multiple of 8 is gathered on its way into LDS; any other case gathers a column
+ * matrix first.  The workspace holds the packed weights (unless w_is_packed) and, when a column matrix is
+ * needed, that of as many images as fit (at least one); sofie_hip_conv_i8_workspace returns the minimum,
+ * which may be 0.  It knows neither addresses nor the context's options, so for the channels that are a
+ * multiple of 8 it still asks for one image's column matrix: what the call falls back to where the input is
+ * not aligned or an option asks for it. */
 enum { SOFIE_LAYOUT_NCHW = 0, SOFIE_LAYOUT_NHWC = 1 };
 typedef struct sofie_conv_i8_args {
    const int8_t *X;

@@ -4,8 +4,9 @@
 // floats touches three or four lines, and a slab of 32 k of a 64 x 64 tile took 0.60 us where its MFMAs take 0.43.  Here a tile is BM consecutive output pixels
 // (through rows and images) and BN output channels; what it reads of a channel is one run of rows, loaded once, and the nine kernel
 // positions read it from LDS at offsets that are known where the code is written.  64 images, us before -> after: 32 -> 64 channels at
-// 32 x 32 36.7 -> 26.8, 64 -> 64 57.2 -> 43.8 (110 TFLOP/s of the matrix cores' 157), 3 -> 32 at 64 x 64 24.2 -> 17.0; one image, 48 -> 96 at
-// 40 x 40 12.8 -> 8.4.
+// 32 x 32 36.7 -> 26.8, 64 -> 64 57.2 -> 43.8 (110 TFLOP/s of the matrix cores' 157; on another box 46.1, with a residual 48.1), 3 -> 32 at
+// 64 x 64 24.2 -> 17.0; one image, 48 -> 96 at 40 x 40 12.8 -> 8.4.  On 64 -> 64 the matrix cores work in 0.66 of the cycles and no bank conflicts are
+// counted; what is left is a patch that is loaded once per 32 output channels and one MFMA per value read from LDS.
 //
 // The images are taken as one column of OH + 2 rows each, padding included (row r of image i is row i (OH + 2) + r), and OW + 2 columns:
 // the patch of a tile is the rows from its first pixel's to two below its last pixel's.
@@ -24,7 +25,10 @@ struct F32Conv3x3 {
    unsigned long long ow_mul, oh_mul, vw_mul, vh_mul; // ceil(2^64 / (OW, OH, OW + 2, OH + 2)), 0 for an extent of 1
 };
 
-constexpr int F32_CONV3X3_PATCH = 704; // the largest patch that is taken (a tile across two images of 98 columns: 686)
+// The largest patch that is taken: square images of up to 115 columns at every tile but the largest, and wider ones up to 168 whose columns a
+// tile divides.  No image wider than 96 was timed when the line was drawn (a tile across two of those: 686 places); beyond it the gathering
+// kernels run.  It is not a limit of LDS: 904 places, for any image of 224 columns, would be 80 KB for two slabs, twice on a CU.
+constexpr int F32_CONV3X3_PATCH = 704;
 
 // Positions of the patch of any tile of `bm` pixels: rows it touches, two more, and two per image that it runs into.
 inline long long f32_conv3x3_patch(int OH, int OW, int bm)

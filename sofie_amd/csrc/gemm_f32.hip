@@ -264,7 +264,8 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
       }
    };
    auto with = [&](auto room) { return vec ? go(room, std::integral_constant<int, 4>{}) : go(room, std::integral_constant<int, 1>{}); };
-   // the places a channel has in LDS: the fewer, the more workgroups share a CU (images of 32, 64 and 96 columns)
+   // the places a channel has in LDS: the fewer, the more workgroups share a CU (with 128 pixels, images of up to 17, 54 and 98 columns, and
+   // those that such a tile divides: 32, 64, 80, 112, 128 ...)
    return patch <= 256 ? with(std::integral_constant<int, 256>{}) : patch <= 448 ? with(std::integral_constant<int, 448>{}) : with(std::integral_constant<int, F32_CONV3X3_PATCH>{});
 }
 

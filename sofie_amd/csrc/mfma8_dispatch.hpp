@@ -11,7 +11,9 @@ namespace sofie_hip {
 // Below the sizes that fill the matrix cores, all of these kernels are bound by the bytes a CU takes in (37 - 45 KB/us through
 // registers, 67 - 75 KB/us straight into LDS) and by what a tile costs besides (start, store).  Fitted to single launches from
 // 33 x 260 x 100 to 3001 x 3695 x 6991 and to the long, narrow products of small convolutions (200000 x 32 x 224), the estimates hold
-// to about a fifth; they decide between kernels whose times differ by more than that almost everywhere.
+// to about a fifth where both operands are rows; they decide between kernels whose times differ by more than that almost everywhere.
+// The loader that transposes B (mfma8_columns_preferred) has no term of its own and takes up to half as long again: 1537 x 1000 x 777 7.6 us
+// estimated and 11.4 measured, 300 x 300 x 300 4.3 and 6.2.
 inline double mfma8_time(int M, int N, int K, int bm, int bn, double fixed_us, double tile_us, double bytes_per_us)
 {
    double rounds = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) / 256.0; // tiles per CU; a CU works on a few at a time
@@ -103,7 +105,10 @@ static int launch_mfma8_best(const LaunchCfg &lc, const int8_t *A, const int8_t 
 }
 
 // Whether a product whose B is stored [K,N] is better off with the general loop, which transposes B on its way into LDS, than
-// with a launch that re-lays B out and the kernels above: that launch takes about 2 us and 4.2 TB/s for the bytes it moves.
+// with a launch that re-lays B out and the kernels above: that launch takes about 2 us and 4.2 TB/s for the bytes it moves.  Both sides come out
+// low (above; two launches in a row take 4.0 us for B of 0.8 MB, 6.9 for 4.2 MB), so the line lies near the right place up to about
+// 2048^3: in the loop / re-laid out 1537 x 1000 x 777 11.4 / 14.1 us, 1000 x 2000 x 500 8.0 / 9.8, 100 x 4000 x 4000 17.5 / 21.8, 2048^3 19.3 / 19.3.
+// Past them the loop is taken although it is slower: 4096 x 4096 x 1000 42.8 / 37.4, 3001 x 3695 x 1999 68.8 / 60.5.
 static bool mfma8_columns_preferred(const LaunchCfg &lc, int M, int N, int K, bool aligned_behind)
 {
    if (K < 16 || N < 16 || lc.tile == 16 || lc.tile == 32)
