@@ -48,7 +48,7 @@ __device__ __forceinline__ long long uniform(long long v)
 
 // Loads into LDS go through a buffer descriptor: its base is scalar and may move, so is a second offset; a lane adds an offset of 31
 // bits, and F32_OUTSIDE, which lies behind the buffer's end, reads as zero.  Vector instructions take their turn on the multipliers of the fp32
-// matrix cores (two waves per SIMD, eight additions per MFMA of 64 cycles: 2.8 cycles each, 64-bit ones 5.2; one wave alone: 4 to 6), so
+// matrix cores (two waves per SIMD, eight additions per MFMA of 64 cycles: 3.0 cycles each, 64-bit ones 5.2; one wave alone: 6), so
 // what a loop spends on addresses is lost to it: two 64-bit additions and an address in LDS per load took a tenth of it.
 constexpr long long F32_BUFFER_BYTES = 0x7fffff00;
 constexpr int F32_OUTSIDE = -1;
