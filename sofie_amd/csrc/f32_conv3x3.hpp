@@ -148,20 +148,32 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_kernel(F32Conv3x3 a, F32Co
    }
    const int weight = S::PATCH + (wn * TN + c) * S::PITCH + lk * S::HALF;
 
-   // The sums start at bias and residual, whose loads are on their way with the first slab's (behind the loop they were four
-   // trips to memory in a row).
+   // Bias and residual are on their way with the first slab's loads (behind the loop they were four trips to memory in a row) and wait in
+   // registers: as the start of the sums they would be rounded with every product (bias of 100, 64 channels: 4.2e-7 of the result against 2.4e-8).
    v16f acc[MT][NT];
+   float bias[NT][OWN], residual[MT][NT][OWN]; // of the elements that this wave finishes
+   auto column = [&](int j, int o) {
+      const int e = wk * OWN + o, n = n0 + wn * TN + j * 32 + e / 4 * 8 + lk * 4 + e % 4;
+      return n < a.N ? n : a.N - 1;
+   };
+#pragma unroll
+   for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int o = 0; o < OWN; ++o)
+         bias[j][o] = out.bias_of(column(j, o));
 #pragma unroll
    for (int i = 0; i < MT; ++i) {
       const int m = m0 + wm * TM + i * 32 + c;
       const auto where = out.row_of(m < a.M ? m : a.M - 1);
 #pragma unroll
-      for (int j = 0; j < NT; ++j)
+      for (int j = 0; j < NT; ++j) {
 #pragma unroll
-         for (int e = 0; e < 16; ++e) {
-            const int n = n0 + wn * TN + j * 32 + e / 4 * 8 + lk * 4 + e % 4;
-            acc[i][j][e] = e / OWN == wk ? out.before_sum(where, n < a.N ? n : a.N - 1) : 0.0f;
-         }
+         for (int e = 0; e < 16; ++e)
+            acc[i][j][e] = 0.0f;
+#pragma unroll
+         for (int o = 0; o < OWN; ++o)
+            residual[i][j][o] = out.residual_of(where, column(j, o));
+      }
    }
    // READ k at a time; the fragments of the next ones are read while these are multiplied
    typedef float part __attribute__((ext_vector_type(S::READ)));
@@ -245,6 +257,18 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_kernel(F32Conv3x3 a, F32Co
          }
       });
    }
+   static_for<WAVES_K>([&](auto pc) {
+      constexpr int p = decltype(pc)::value;
+      if (WAVES_K == 1 || wk == p) {
+#pragma unroll
+         for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+               for (int o = 0; o < OWN; ++o)
+                  acc[i][j][p * OWN + o] = (acc[i][j][p * OWN + o] + bias[j][o]) + residual[i][j][o];
+      }
+   });
    // 32 neighbouring lanes hold 32 neighbouring pixels of a channel: whole lines, straight from the registers
 #pragma unroll
    for (int i = 0; i < MT; ++i) {

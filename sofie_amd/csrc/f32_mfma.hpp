@@ -404,14 +404,9 @@ struct F32ConvStore {
       const int img = m / positions;
       return row_state{(size_t)img * Cout * positions + (m - img * positions)};
    }
-   // what is added to column n of a row before the activation
-   __device__ __forceinline__ float before_sum(const row_state &r, int n) const
-   {
-      float v = bias ? bias[first + n] : 0.0f;
-      if (R)
-         v += R[r.at + (size_t)(first + n) * positions];
-      return v;
-   }
+   // what is added to the sum of column n of a row before the activation, one after the other
+   __device__ __forceinline__ float bias_of(int n) const { return bias ? bias[first + n] : 0.0f; }
+   __device__ __forceinline__ float residual_of(const row_state &r, int n) const { return R ? R[r.at + (size_t)(first + n) * positions] : 0.0f; }
    // C columns of one row; those from N on are left out
    template <int C>
    __device__ __forceinline__ void put_columns(float (&v)[C], const row_state &r, const int (&n)[C], int N) const

@@ -12,6 +12,7 @@ from oracle import binding as ob
 from sofie_amd import runtime as R
 from tests import util
 from tests.test_gpu_f32 import conv_desc
+from tests.test_gpu_f32_tiles import conv2d_f64
 
 pytestmark = pytest.mark.gpu
 
@@ -53,3 +54,24 @@ def test_conv3x3(rt, tile, case):
             assert np.abs(util.to_host(dY) - want).max() <= 1e-5 * max(1.0, float(np.abs(want).max()))
     finally:
         rt.set_option("f32_tile", 0)
+
+
+@pytest.mark.parametrize("tile", [0, 3032, 3064, 3128, 16, 62, 64, 126])
+@pytest.mark.parametrize("channels", [3, 16, 200])
+@pytest.mark.parametrize("bias, residual", [(1000.0, 0.0), (0.1, 1000.0), (700.0, 700.0)])
+def test_bias_and_residual_are_rounded_once(rt, opt, tile, channels, bias, residual):
+    """Beside a large bias or residual the products' sum keeps its own precision: the result is that sum plus two additions, each rounded once."""
+    N, H, W, Cout = 2, 12, 17, 34
+    X = util.uniform01(44, N * channels * H * W).reshape(N, channels, H, W)
+    Wt = util.normal(45, Cout * channels * 9, 0.1).reshape(Cout, channels, 3, 3)
+    b, r = util.normal(46, Cout, bias), util.normal(47, N * Cout * H * W, residual or 1.0).reshape(N, Cout, H, W) * np.float32(residual != 0)
+    d = conv_desc(N, channels, H, W, Cout, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), 1)
+    dX, dW, db, dR, dY = util.to_dev(X), util.to_dev(Wt), util.to_dev(b), util.to_dev(r), util.dev_empty(r.shape, np.float32)
+    torch.cuda.synchronize()
+    opt("f32_tile", tile)
+    rt.call("sofie_hip_conv_f32", C.byref(d), util.ptr(dX), util.ptr(dW), util.ptr(db), R.ACT_NONE, C.c_float(0), util.ptr(dY), None, util.ptr(dR))
+    rt.sync()
+    products, most = conv2d_f64(X, Wt, (1, 1, 1, 1))
+    beside = np.abs(b.astype(np.float64))[None, :, None, None] + np.abs(r)
+    # two additions of values below `beside` + most; 1800 products summed in any order stay far within 1e-6 of their magnitudes
+    assert np.all(np.abs(util.to_host(dY) - (products + b[None, :, None, None] + r)) <= 2 * 2.0 ** -24 * (beside + most) + 1e-6 * most)
