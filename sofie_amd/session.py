@@ -105,8 +105,8 @@ class Int8MLPSession:
 
     def infer_nosync(self):
         """Enqueue one inference over the input resident at x_ptr; the result lands at y_ptr."""
-        call, byref = self.rt.call, C.byref
-        call("sofie_hip_quantize_linear", *self._quantize, self.batch * self.dims[0], float(self.in_scales[0]))
+        call, byref, (quantized, x) = self.rt.call, C.byref, self._quantize
+        call("sofie_hip_quantize_linear", quantized, x, self.batch * self.dims[0], float(self.in_scales[0]))
         for d in self.descs:
             call("sofie_hip_gemm_i8", byref(d))
 
@@ -246,9 +246,9 @@ class Int8CNNSession:
         self.rt.call("sofie_hip_upload", self.x_ptr, x.ctypes.data_as(C.c_void_p), C.c_size_t(x.nbytes))
 
     def infer_nosync(self):
-        call, byref, N = self.rt.call, C.byref, self.batch
+        call, byref, N, (quantized, x) = self.rt.call, C.byref, self.batch, self._quantize
         Cin, H, W = self.in_shape
-        call("sofie_hip_quantize_linear", *self._quantize, N * Cin * H * W, float(self.in_scale))
+        call("sofie_hip_quantize_linear", quantized, x, N * Cin * H * W, float(self.in_scale))
         c, h, w = self.out_shape
         if self.pool_in_conv:
             call("sofie_hip_fill_zero", self._sums, 4 * N * c)
