@@ -1,0 +1,337 @@
+// fp32 3 x 3 convolution (stride 1, no dilation, two spatial axes) on the bf16 matrix cores.
+//
+// Every fp32 value is the sum of three bf16 values, x = h + m + l (h = bf16(x), m = bf16(x - h), l = bf16(x - h - m): the remainders are exact, and what is
+// left behind l is at most 2^-26 of x), and a product of two such sums is taken as the six terms down to 2^-17 of it:
+//   a b = ah bh + (ah bm + am bh) + (ah bl + am bm + al bh),       left out: am bl + al bm + al bl < 2^-24 a b.
+// bf16 products are exact in the fp32 accumulators, and v_mfma_f32_32x32x16_bf16 multiplies 16 k in 32 cycles where v_mfma_f32_32x32x2_f32 needs
+// 512: the six terms cost 0.375 of the fp32 instructions.  The leading products and the other terms are summed apart, so that an accumulator is rounded
+// once per 16 k.
+//
+// What the pieces cost is vector instructions (5.5 per value) and LDS (6 bytes written per value, at 79 B/clk): a 3 x 3 convolution uses every value of its
+// input patch nine times, which pays for both.  (A plain product of 64 x 64 tiles uses a value twice per wave: 20 - 27 us where fp32 takes 20 - 32.)
+// 64 images of 32 x 32, us, the fp32 kernel -> this one: 32 -> 64 channels 29.4 -> 22.1, 64 -> 64 50 -> 34.5 (with a residual 50 -> 37); 128 -> 128 at
+// 16 x 16 48.3 -> 38.  Error of 64 -> 64 against 64 bits: 4.2e-7 -> 1.4e-7 of the result.  On 64 -> 64 the matrix cores are busy in 0.47 of the cycles at
+// 1.9 GHz of 2.4 (power); 10 us of the launch are the first slab's load, the store and the launch itself, which nothing overlaps.
+//
+// Exceptions: bf16 has the exponents of fp32, so nothing overflows or vanishes that would not in fp32, except that a value within 2^-8 of the largest
+// rounds to an infinity, and that the remainders of an infinity are NaN.  Both end in a sum that is not finite; a wave that finds one among its sums
+// computes them again with fp32 instructions straight from memory, which gives IEEE's infinities and NaN.
+#pragma once
+#include "f32_conv3x3.hpp"
+
+namespace sofie_hip {
+
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+
+// The next piece of eight values, and what is left of them.  (v_dot2_f32_bf16 takes a remainder in one instruction instead of two, but not beside the
+// matrix cores: an MFMA and four of them take 58 cycles, an MFMA and four subtractions 34.)
+template <int P>
+__device__ __forceinline__ v4u f32_next_piece(float (&x)[8])
+{
+   v4u words;
+#pragma unroll
+   for (int e = 0; e < 4; ++e) {
+      const unsigned both = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f{x[2 * e], x[2 * e + 1]}), v2bf));
+      words[e] = both;
+      if constexpr (P < 2) {
+         x[2 * e] -= __builtin_bit_cast(float, both << 16);
+         x[2 * e + 1] -= __builtin_bit_cast(float, both & 0xffff0000u);
+      }
+   }
+   return words;
+}
+
+// A float of a buffer of which `base` is the (scalar) start; F32_OUTSIDE reads as zero.
+__device__ __forceinline__ float f32_buffer_read(const void *base, int offset, int scalar_offset)
+{
+   const __amdgpu_buffer_rsrc_t buffer = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)F32_BUFFER_BYTES, 0x00020000);
+   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buffer, offset, scalar_offset, 0));
+}
+
+// The largest patch that is taken: with it two workgroups fit a CU (81 KB each); one alone takes 1.9 times as long (32 images, 64 -> 128 at 56 x 56: 206 us
+// against the fp32 kernel's 165).
+constexpr int F32_CONV3X3_SPLIT_PATCH = 360;
+
+// LDS of a workgroup.  A slab is 16 channels.  Pieces lie in columns of 16 bytes, eight channels each: of a patch, [piece][half of the channels][position]; of the
+// weights, [piece][kernel position][half][output channel], columns 16 bytes apart beside their 32 rows (the 18 columns of a row, which are written
+// side by side, start in different banks).  The weights come as they are in memory, a row of 144 floats per output channel, and are split from there.
+template <int PLANE, int WVEC>
+struct F32Conv3x3SplitShape {
+   static constexpr int CS = 16, BN = 32;
+   static constexpr int PITCH = CS * 9;                                                    // of a row of weights, in floats
+   static constexpr int WLOADS = (BN * PITCH + 64 * WVEC - 1) / (64 * WVEC);               // load instructions per slab of weights
+   static constexpr int HALF = PLANE * 16, PATCH = 2 * HALF;                               // bytes of a piece of a patch
+   static constexpr int COLUMN = BN * 16 + 16, WEIGHTS = 18 * COLUMN;                      // bytes of a piece of the weights
+   static constexpr int RAW_AT = 3 * (PATCH + WEIGHTS), BYTES = RAW_AT + WLOADS * 64 * WVEC * 4;
+};
+
+// Four waves, each with BM / 4 pixels and 32 output channels.  One slab lies in LDS in pieces, the next one as raw weights and, in registers, as raw patch; two
+// workgroups per CU, one of which splits while the other multiplies.  (One workgroup whose other four waves split for it, through two slabs of pieces, is no
+// faster: 36 us, bound by LDS.)
+template <int BM, int PLANE, int WVEC>
+__global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a, F32ConvStore out, int tiles_m, int tiles_n, int first_tile)
+{
+   typedef F32Conv3x3SplitShape<PLANE, WVEC> S;
+   constexpr int CS = S::CS, BN = S::BN, TM = BM / 4, MT = TM / 32;
+   static_assert(TM % 32 == 0 && PLANE % 8 == 0, "wave tiles of 32 x 32 blocks");
+   extern __shared__ __attribute__((aligned(16))) char split_lds[];
+   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lk = lane >> 5, c = lane & 31;
+   const int z = blockIdx.z;
+   a.X += z * a.group;
+   a.W += (long long)z * a.N * a.K;
+   out.select_batch(z);
+   int tm, tn;
+   f32_tile_of_block(first_tile, tiles_m, tiles_n, tm, tn);
+   const int m0 = tm * BM, n0 = tn * BN;
+   const int VW = a.OW + 2, VH = a.OH + 2;
+   auto quotient = [](int n, unsigned long long mul) { return mul ? (int)__umul64hi((unsigned long long)(unsigned)n, mul) : n; };
+
+   // where the patch begins; a wave splits every other 64 positions of one half of a slab's channels
+   const int line0 = quotient(m0, a.ow_mul), image0 = quotient(line0, a.oh_mul);
+   const int row0 = line0 - image0 * a.OH; // of image0, padding row 0 first
+   const char *base = (const char *)uniform((long long)(a.X + image0 * a.image));
+   const int plane_bytes = a.H * a.Wd * 4;
+   constexpr int CHUNKS = (PLANE + 127) / 128; // of 64 positions per wave
+   const int half = wave & 1;
+   int patch_at[CHUNKS]; // bytes from `base`, of channel 0
+   auto position = [&](int q) { return (2 * q + (wave >> 1)) * 64 + lane; };
+#pragma unroll
+   for (int q = 0; q < CHUNKS; ++q) {
+      const int f = position(q), vr = quotient(f, a.vw_mul), ix = f - vr * VW - a.pad_w;
+      const int on = row0 + vr, image = quotient(on, a.vh_mul), iy = on - image * VH - a.pad_h;
+      const bool inside = (unsigned)ix < (unsigned)a.Wd && (unsigned)iy < (unsigned)a.H && image0 + image < a.images;
+      patch_at[q] = inside ? (int)((image * a.image + (long long)iy * a.Wd + ix) * 4) : F32_OUTSIDE;
+   }
+   // the weights of this tile: rows past N and the gaps between rows read as zero
+   constexpr int LDW = (S::WLOADS + 3) / 4;
+   const char *weights = (const char *)uniform((long long)(a.W + (long long)n0 * a.K));
+   auto weight_place = [&](int i, int &row, int &k) {
+      const int f = ((i * 4 + wave) * 64 + lane) * WVEC;
+      row = f / S::PITCH;
+      k = f - row * S::PITCH;
+   };
+   // eight weights that a thread splits: an output channel, half the channels of a slab, a kernel position
+   constexpr int TASKS = BN * 18, PER = (TASKS + 255) / 256;
+   int from[PER], to[PER];
+#pragma unroll
+   for (int t = 0; t < PER; ++t) {
+      const int f = t * 256 + threadIdx.x, n = f / 18, r = f - n * 18, h = r / 9, pos = r - h * 9;
+      from[t] = S::RAW_AT + (n * S::PITCH + h * 72 + pos) * 4;
+      to[t] = 3 * S::PATCH + (pos * 2 + h) * S::COLUMN + n * 16;
+   }
+
+   const int slabs = (a.C + CS - 1) / CS;
+   float raw[CHUNKS][8];
+   auto issue = [&](int s) {
+      const int first = s * CS + half * 8;
+#pragma unroll
+      for (int q = 0; q < CHUNKS; ++q)
+#pragma unroll
+         for (int e = 0; e < 8; ++e) {
+            const bool there = first + e < a.C;
+            raw[q][e] = f32_buffer_read(base, there ? patch_at[q] : F32_OUTSIDE, there ? (first + e) * plane_bytes : 0);
+         }
+#pragma unroll
+      for (int i = 0; i < LDW; ++i) {
+         if (i * 4 + wave < S::WLOADS) {
+            int row, k;
+            weight_place(i, row, k);
+            // k past the last channel are the next row's
+            const int at = n0 + row < a.N && s * CS * 9 + k < a.K ? (row * a.K + k) * 4 : F32_OUTSIDE;
+            f32_buffer_load<WVEC>((lds_void_t *)(split_lds + S::RAW_AT + (i * 4 + wave) * 64 * WVEC * 4), weights + (long long)s * CS * 9 * 4, at);
+         }
+      }
+   };
+   auto split = [&]() {
+      auto pieces = [&](float (&x)[8], char *at, int step) {
+         *(v4u *)at = f32_next_piece<0>(x);
+         *(v4u *)(at + step) = f32_next_piece<1>(x);
+         *(v4u *)(at + 2 * step) = f32_next_piece<2>(x);
+      };
+#pragma unroll
+      for (int t = 0; t < PER; ++t) {
+         if ((t + 1) * 256 <= TASKS || t * 256 + (int)threadIdx.x < TASKS) {
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+               x[e] = *(const float *)(split_lds + from[t] + e * 36);
+            pieces(x, split_lds + to[t], S::WEIGHTS);
+         }
+      }
+#pragma unroll
+      for (int q = 0; q < CHUNKS; ++q)
+         if (position(q) < PLANE)
+            pieces(raw[q], split_lds + half * S::HALF + position(q) * 16, S::PATCH);
+   };
+
+   // this lane's pixels in the patch, one address per kernel row, and its weights
+   int pixel[MT][3];
+#pragma unroll
+   for (int i = 0; i < MT; ++i) {
+      const int m = m0 + wave * TM + i * 32 + c, mm = m < a.M ? m : a.M - 1;
+      const int line = quotient(mm, a.ow_mul), image = quotient(line, a.oh_mul);
+      const int vr = (image - image0) * VH + line - image * a.OH - row0;
+#pragma unroll
+      for (int ky = 0; ky < 3; ++ky)
+         pixel[i][ky] = ((vr + ky) * VW + mm - line * a.OW) * 16 + lk * S::HALF;
+   }
+   const int weight = 3 * S::PATCH + lk * S::COLUMN + c * 16;
+
+   v16f acc[MT], low[MT];
+   auto clear = [](v16f(&sums)[MT]) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+         for (int e = 0; e < 16; ++e)
+            sums[i][e] = 0.0f;
+   };
+   clear(acc);
+   clear(low);
+   // kernel position by kernel position; the fragments of the next one are read while these are multiplied
+   v8bf w[2][3], x[2][MT][3];
+   auto multiply = [&]() {
+      auto read = [&](auto number) {
+         constexpr int t = decltype(number)::value, set = t % 2;
+#pragma unroll
+         for (int p = 0; p < 3; ++p) {
+            w[set][p] = *(const v8bf *)(split_lds + weight + p * S::WEIGHTS + t * 2 * S::COLUMN);
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+               x[set][i][p] = *(const v8bf *)(split_lds + pixel[i][t / 3] + p * S::PATCH + t % 3 * 16);
+         }
+      };
+      read(std::integral_constant<int, 0>{});
+      static_for<9>([&](auto tc) {
+         constexpr int t = decltype(tc)::value, set = t % 2;
+         __builtin_amdgcn_sched_barrier(0);
+         if constexpr (t < 8)
+            read(std::integral_constant<int, t + 1>{});
+         __builtin_amdgcn_sched_barrier(0);
+         constexpr int TERM[6][2] = {{0, 0}, {1, 0}, {0, 1}, {1, 1}, {2, 0}, {0, 2}};
+         static_for<6>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            auto &sums = q == 0 ? acc : low;
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+               sums[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[set][TERM[q][1]], x[set][i][TERM[q][0]], sums[i], 0, 0, 0);
+         });
+      });
+   };
+   auto meet = []() {
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0)
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+   };
+
+   issue(0);
+#pragma unroll 1
+   for (int s = 0; s < slabs; ++s) {
+      wait_vmcnt<0>();
+      meet(); // the raw weights have landed for every wave, and every wave has read the pieces of slab s - 1
+      split();
+      meet();
+      if (s + 1 < slabs)
+         issue(s + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply();
+   }
+
+   float finite = 0.0f;
+#pragma unroll
+   for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+         acc[i][e] += low[i][e];
+         finite = __builtin_fmaf(acc[i][e], 0.0f, finite);
+      }
+   const int n1 = n0 + lk * 4; // this lane's columns: n1 + e / 4 * 8 + e % 4
+   if (__builtin_amdgcn_ballot_w64(finite != 0.0f) != 0) {
+      clear(acc);
+      const float *row = a.W + (long long)(n0 + c < a.N ? n0 + c : a.N - 1) * a.K;
+#pragma unroll 1
+      for (int k0 = 0; k0 < a.K; k0 += 8) {
+         float u[4], v[MT][4];
+#pragma unroll
+         for (int j = 0; j < 4; ++j) {
+            const int k = k0 + lk * 4 + j, ch = k / 9, r = k - ch * 9, ky = r / 3, kx = r - ky * 3;
+            u[j] = k < a.K ? row[k] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+               const int m = m0 + wave * TM + i * 32 + c, mm = m < a.M ? m : a.M - 1;
+               const int line = quotient(mm, a.ow_mul), image = quotient(line, a.oh_mul);
+               const int iy = line - image * a.OH + ky - a.pad_h, ix = mm - line * a.OW + kx - a.pad_w;
+               v[i][j] = k < a.K && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.Wd ? a.X[image * a.image + ((long long)ch * a.H + iy) * a.Wd + ix] : 0.0f;
+            }
+         }
+#pragma unroll
+         for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+               acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(u[j], v[i][j], acc[i], 0, 0, 0);
+      }
+   }
+
+   // 32 neighbouring lanes hold 32 neighbouring pixels of a channel: whole lines, straight from the registers
+   auto column = [&](int e) { return n1 + e / 4 * 8 + e % 4; };
+   float bias[16], residual[MT][16];
+#pragma unroll
+   for (int e = 0; e < 16; ++e) {
+      const int n = column(e) < a.N ? column(e) : a.N - 1;
+      bias[e] = out.bias_of(n);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+         const int m = m0 + wave * TM + i * 32 + c;
+         residual[i][e] = out.residual_of(out.row_of(m < a.M ? m : a.M - 1), n);
+      }
+   }
+#pragma unroll
+   for (int i = 0; i < MT; ++i) {
+      const int m = m0 + wave * TM + i * 32 + c;
+      const auto where = out.row_of(m < a.M ? m : a.M - 1);
+      auto put = [&](float v, int e) {
+         if (m < a.M && column(e) < a.N)
+            out.Y[where.at + (size_t)(out.first + column(e)) * out.positions] = v;
+      };
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+         acc[i][e] = (acc[i][e] + bias[e]) + residual[i][e];
+      const bool relu = out.chain.count == 1 && out.chain.op0 == SOFIE_ACT_RELU;
+      if (relu || out.chain.count == 0) {
+#pragma unroll
+         for (int e = 0; e < 16; ++e)
+            put(relu ? (acc[i][e] > 0.0f ? acc[i][e] : 0.0f) : acc[i][e], e);
+      } else {
+         // one copy of the activations' code for 16 elements
+#pragma unroll 1
+         for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+               put(apply_chain(g == 0 ? acc[i][e] : g == 1 ? acc[i][4 + e] : g == 2 ? acc[i][8 + e] : acc[i][12 + e], out.chain), g * 4 + e);
+      }
+   }
+}
+
+template <int BM, int PLANE, int WVEC>
+static int launch_f32_conv3x3_split_as(hipStream_t stream, const F32Conv3x3 &a, const F32ConvStore &out, int group)
+{
+   constexpr int BN = F32Conv3x3SplitShape<PLANE, WVEC>::BN;
+   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
+   if ((long long)tiles_m * tiles_n > 0x7fffffffLL)
+      return fail(SOFIE_HIP_ERR_INVALID, "fp32 convolution: too many tiles");
+   constexpr size_t smem = F32Conv3x3SplitShape<PLANE, WVEC>::BYTES;
+   static_assert(smem <= 160 * 1024, "LDS of a CU");
+   auto kern = f32_conv3x3_split_kernel<BM, PLANE, WVEC>;
+   static bool configured[64] = {};
+   if (int st = configure_lds_once(kern, smem, configured))
+      return st;
+   in_launches((long long)tiles_m * tiles_n, 256, [&](int first, unsigned count) {
+      launch_kernel(kern, dim3(count, 1, (unsigned)group), dim3(256), smem, stream, a, out, tiles_m, tiles_n, first);
+   });
+   return launch_status("f32_conv3x3_split_kernel");
+}
+
+} // namespace sofie_hip

@@ -1,6 +1,6 @@
 // fp32 Gemm / MatMul and fp32 convolution (implicit GEMM) with the bias + activation epilogue fused into the store: the entry
 // points and the choice among the kernels of f32_mfma.hpp, and the kernel that runs a chain of small products in one launch.
-#include "f32_conv3x3.hpp"
+#include "f32_conv3x3_split.hpp"
 #include <algorithm>
 #include <cmath>
 
@@ -139,7 +139,7 @@ namespace sofie_hip {
 // (64 x 32: two blocks), 0.452 (64 x 64: four) and 1.765 (128 x 128: sixteen), a start and a store per tile, in as many rounds as
 // the tiles need over 256 CUs, and a launch.  The direct kernel costs a launch, a trip to memory per 512 k or the 10.5 TB/s at which
 // its fragments, which nothing shares, arrive, and 0.45 us per 256 tiles.
-enum F32Tile { F32_CONV3X3_32 = 3032, F32_CONV3X3_64 = 3064, F32_CONV3X3_128 = 3128, F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
+enum F32Tile { F32_CONV3X3_32 = 3032, F32_CONV3X3_64 = 3064, F32_CONV3X3_128 = 3128, F32_CONV3X3_SPLIT_128 = 4128, F32_CONV3X3_SPLIT_256 = 4256, F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
 static int pick_f32_tile(int M, int N, int K, int batch, double *time_us = nullptr)
 {
    auto tiles = [&](int bm, int bn) { return std::ceil((double)M / bm) * std::ceil((double)N / bn) * batch; };
@@ -224,6 +224,7 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
    const long long plane = (long long)s.H * s.W, most = F32_CONV3X3_PATCH / ((long long)(s.OW + 2) * (s.OH + 2)) + 2;
    if ((most * s.C + s.Cg) * plane * 4 >= F32_BUFFER_BYTES || 128LL * K * 4 >= F32_BUFFER_BYTES)
       return SOFIE_HIP_OK;
+   const bool vec = ((uintptr_t)W & 15) == 0 && K % 4 == 0;
    int tile = force;
    if (!tile) {
       // A slab of 8 channels takes 1.06 / 0.61 / 0.38 us of a CU with several tiles of 128 / 64 / 32 pixels at work, and 1.42 / 0.95 / 0.70
@@ -243,16 +244,35 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
          offer(F32_CONV3X3_64, 64, 0.606, 0.95, 1.0);
          offer(F32_CONV3X3_128, 128, 1.06, 1.42, 1.45);
       }
+      // The kernel of f32_conv3x3_split.hpp takes slabs of 16 channels, two tiles to a CU: 1.75 us of a CU a slab (128 pixels; 2.4 us where the weights come
+      // float by float) and 2.95 (256 pixels), 2.3 and 3.5 us a tile; alone 2.4, 3.6 and 3.2 us a slab.  (Fitted to 34 layers as above; holds to a tenth.)
+      auto offer_split = [&](int which, int bm, double slab, double alone, double each) {
+         const double rounds = std::ceil((double)((M + bm - 1) / bm) * ((N + 31) / 32) * group / 256.0), slabs = std::ceil(s.Cg / 16.0);
+         const double t = std::max(slabs * alone + each, rounds * (slabs * slab + each));
+         if (f32_conv3x3_patch(s.OH, s.OW, bm) <= F32_CONV3X3_SPLIT_PATCH && t < least)
+            least = t, tile = which;
+      };
+      offer_split(F32_CONV3X3_SPLIT_128, 128, vec ? 1.75 : 2.4, vec ? 2.4 : 3.6, 2.3);
+      if (vec)
+         offer_split(F32_CONV3X3_SPLIT_256, 256, 2.95, 3.2, 3.5);
    }
-   const long long patch = f32_conv3x3_patch(s.OH, s.OW, tile - 3000);
-   if (tile < F32_CONV3X3_32 || patch > F32_CONV3X3_PATCH)
+   const bool split = tile >= F32_CONV3X3_SPLIT_128;
+   const long long patch = f32_conv3x3_patch(s.OH, s.OW, tile - (split ? 4000 : 3000));
+   if (tile < F32_CONV3X3_32 || patch > (split ? F32_CONV3X3_SPLIT_PATCH : F32_CONV3X3_PATCH))
       return SOFIE_HIP_OK;
    auto reciprocal = [](unsigned d) -> unsigned long long { return d <= 1 ? 0ull : (~0ull / d) + 1; };
    const F32Conv3x3 a{X, W, images, s.Cg, s.H, s.W, s.OH, s.OW, s.pad_h, s.pad_w, plane * s.C, plane * s.Cg, M, N, K, (int)(patch + 63) / 64,
                       reciprocal(s.OW), reciprocal(s.OH), reciprocal(s.OW + 2), reciprocal(s.OH + 2)};
-   const bool vec = ((uintptr_t)W & 15) == 0 && K % 4 == 0;
    *taken = true;
    hipStream_t st = ctx->stream;
+   if (split) {
+      auto go = [&](auto pixels, auto wide) {
+         constexpr int BM = decltype(pixels)::value, V = decltype(wide)::value;
+         return patch <= 256 ? launch_f32_conv3x3_split_as<BM, 256, V>(st, a, out, group) : launch_f32_conv3x3_split_as<BM, F32_CONV3X3_SPLIT_PATCH, V>(st, a, out, group);
+      };
+      auto with = [&](auto pixels) { return vec ? go(pixels, std::integral_constant<int, 4>{}) : go(pixels, std::integral_constant<int, 1>{}); };
+      return tile == F32_CONV3X3_SPLIT_128 ? with(std::integral_constant<int, 128>{}) : with(std::integral_constant<int, 256>{});
+   }
    auto go = [&](auto room, auto wide) {
       constexpr int P = decltype(room)::value, V = decltype(wide)::value;
       if (s.Cg <= 4 && tile == F32_CONV3X3_128)

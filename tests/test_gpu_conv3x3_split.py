@@ -1,0 +1,85 @@
+"""The fp32 3 x 3 convolution that multiplies bf16 pieces (f32_conv3x3_split.hpp), forced by the context option "f32_tile", at the edges of its tiles (128 or 256
+pixels, 32 output channels), of its slabs (16 channels) and of its patch (360 places), against sums in 64 bits: the error is that of fp32 sums, at any
+scale of the inputs, and infinities and NaN are where IEEE arithmetic has them."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from sofie_amd import runtime as R
+from tests import util
+from tests.test_gpu_f32 import conv_desc
+from tests.test_gpu_f32_tiles import same_as_ieee, with_nonfinite
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def tile(rt, request):
+    rt.set_option("f32_tile", request.param)
+    yield request.param
+    rt.set_option("f32_tile", 0)
+
+
+def run(rt, X, Wt, b, pads, group=1, act=R.ACT_NONE, residual=None):
+    N, Cc, H, W = X.shape
+    d = conv_desc(N, Cc, H, W, len(Wt), 3, 3, pads, (1, 1), (1, 1), group)
+    dX, dW, dY = util.to_dev(X), util.to_dev(Wt), util.dev_empty((N, len(Wt), d.OH, d.OW), np.float32)
+    db, dR = (util.to_dev(t) if t is not None else None for t in (b, residual))
+    torch.cuda.synchronize()
+    ptr = lambda t: util.ptr(t) if t is not None else None
+    rt.call("sofie_hip_conv_f32", C.byref(d), ptr(dX), ptr(dW), ptr(db), act, C.c_float(0.1), ptr(dY), None, ptr(dR))
+    rt.sync()
+    return util.to_host(dY)
+
+
+def products(X, Wt, pads, group=1):
+    """Every product of every sum, in 64 bits: [image, output channel, row, column, k]."""
+    x = np.pad(X.astype(np.float64), ((0, 0), (0, 0), (pads[0], pads[2]), (pads[1], pads[3])))
+    win = np.lib.stride_tricks.sliding_window_view(x, (3, 3), axis=(2, 3)).transpose(0, 2, 3, 1, 4, 5)
+    Cg, Ng = Wt.shape[1], len(Wt) // group
+    parts = [win[:, None, :, :, g * Cg:(g + 1) * Cg] * Wt[g * Ng:(g + 1) * Ng].astype(np.float64)[None, :, None, None] for g in range(group)]
+    whole = np.concatenate(parts, axis=1)
+    return whole.reshape(*whole.shape[:4], -1)
+
+
+CASES = [(1, 1, 3, 3, 1, (1, 1, 1, 1), 1), (3, 15, 9, 7, 31, (0, 0, 0, 0), 1), (2, 17, 13, 11, 33, (1, 0, 2, 1), 1), (1, 32, 16, 16, 64, (1, 1, 1, 1), 1), (5, 36, 8, 33, 20, (1, 1, 1, 1), 1),
+         (2, 20, 10, 12, 66, (2, 2, 2, 2), 2), (17, 16, 4, 4, 32, (1, 1, 1, 1), 1), (1, 33, 5, 118, 3, (1, 1, 1, 1), 1)]
+
+
+@pytest.mark.parametrize("tile", [4128, 4256], indirect=True)
+@pytest.mark.parametrize("scale", [1.0, 1e-30, 1e30])
+@pytest.mark.parametrize("case", CASES)
+def test_convolutions_around_tile_edges(rt, tile, case, scale):
+    N, Cc, H, W, Cout, pads, group = case
+    X = (util.normal(70, N * Cc * H * W).reshape(N, Cc, H, W) * np.float32(scale)).astype(np.float32)
+    Wt = util.normal(71, Cout * Cc // group * 9, 0.3).reshape(Cout, Cc // group, 3, 3)
+    b = (util.normal(72, Cout) * np.float32(scale)).astype(np.float32)
+    p = products(X, Wt, pads, group)
+    r = (util.normal(73, p[..., 0].size) * np.float32(scale)).reshape(p.shape[:4]).astype(np.float32)
+    got = run(rt, X, Wt, b, pads, group, R.ACT_LEAKYRELU, r)
+    # Sums of n terms, the products exact and the six-term form of a product within 2^-23 of it, every addition within 2^-24 of the magnitudes so far:
+    # (n + 2) 2^-24 of the sum of magnitudes, n = one addition per 16 channels and kernel position in each of five chains, bias, residual and their join
+    n = 5 * 9 * -(-Cc // group // 16) + 4
+    want = p.sum(4) + b.reshape(1, -1, 1, 1) + r
+    most = np.abs(p).sum(4) + np.abs(b).reshape(1, -1, 1, 1) + np.abs(r)
+    want = np.where(want >= 0, want, np.float64(np.float32(0.1)) * want)
+    assert np.all(np.abs(got - want) <= (n + 2) * 2.0 ** -24 * most)
+
+
+@pytest.mark.parametrize("tile", [4128, 4256], indirect=True)
+@pytest.mark.parametrize("case", [(2, 18, 13, 11, 35), (1, 3, 40, 41, 5)])
+def test_nan_infinity_and_the_largest_numbers(rt, tile, case):
+    N, Cc, H, W, Cout = case
+    X = with_nonfinite(util.normal(74, N * Cc * H * W), 75).reshape(N, Cc, H, W)
+    X.reshape(-1)[7] = np.finfo(np.float32).max            # rounds to an infinity in bf16
+    Wt = util.normal(76, Cout * Cc * 9, 0.2).reshape(Cout, Cc, 3, 3)
+    Wt[1, 0, 0, 0] = np.inf
+    Wt[2] = np.clip(Wt[2], -0.9, 0.9)
+    with np.errstate(invalid="ignore", over="ignore"):
+        p = products(X, Wt, (1, 1, 1, 1))
+        want, most = p.sum(4), np.abs(p).sum(4)
+    got = run(rt, X, Wt, None, (1, 1, 1, 1))
+    assert np.all(np.abs(want[np.isfinite(want)]) < np.finfo(np.float32).max)
+    same_as_ieee(got, want, most)
