@@ -5,6 +5,7 @@
 // as 16 rows, where theirs have 64.  Rows may start at any byte: a chunk is one unaligned 16-byte load.
 #pragma once
 #include "mfma8_gemm_dma.hpp"
+#include <algorithm>
 
 namespace sofie_hip {
 
@@ -73,6 +74,14 @@ __device__ __forceinline__ void store_four_columns(const EPI &ep, const typename
    }
 }
 
+// 16 bytes per lane into LDS, from a buffer that starts at `base`; an offset past its end (-1) reads as zero.
+constexpr int DIRECT_BUFFER_BYTES = 0x7fffff00;
+__device__ __forceinline__ void direct_buffer_load(lds_void_t *to, const void *base, int offset)
+{
+   const __amdgpu_buffer_rsrc_t buffer = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, DIRECT_BUFFER_BYTES, 0x00020000);
+   __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer, to, 16, offset, 0, 0, 0);
+}
+
 // One step of 128 bytes of k on a 16 x 16 block: lane (lk = lane / 16, c = lane % 16) holds bytes 32 lk .. 32 lk + 31 of row c of either
 // operand.  The n side goes first, so that a lane ends up with 4 consecutive columns of one row.
 struct DirectI8 {
@@ -95,6 +104,39 @@ struct DirectF8 {
       return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
    }
 };
+
+// The partial tiles of W waves meet in LDS and are stored.
+template <class MMA, int MB, int NB, int W, class EPI>
+__device__ __forceinline__ void direct_store(const EPI &ep, const typename MMA::acc_t (&acc)[MB][NB], typename MMA::elem_t (*part)[MB * 16][NB * 16 + 4], int m0, int n0,
+                                             int M, int N, int wave, int lane)
+{
+   constexpr int TM = MB * 16, TN = NB * 16;
+   typedef typename MMA::acc_t acc_t;
+   const int lk = lane >> 4, c = lane & 15;
+#pragma unroll
+   for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+         *(acc_t *)&part[wave][i * 16 + c][j * 16 + lk * 4] = acc[i][j];
+   __syncthreads();
+   ep.dispatch([&](auto mode) {
+      constexpr int MODE = decltype(mode)::value;
+#pragma unroll 1
+      for (int e = threadIdx.x; e < TM * TN / 4; e += W * 64) {
+         const int r = e / (TN / 4), q = e % (TN / 4) * 4;
+         acc_t v = *(const acc_t *)&part[0][r][q];
+#pragma unroll
+         for (int w = 1; w < W; ++w)
+            v += *(const acc_t *)&part[w][r][q];
+         const int m = m0 + r, n = n0 + q;
+         if (m >= M || n >= N)
+            continue;
+         typename EPI::template col_params<4> prm;
+         ep.template load_params<4>(n, prm);
+         store_four_columns<MODE>(ep, prm, v, m, n, N);
+      }
+   });
+}
 
 template <class MMA, int MB, int NB, int W, int UNROLL, class EPI>
 __global__ __launch_bounds__(W * 64) void mfma8_direct_kernel(RowMajorRows A, RowMajorRows Bt, int M, int N, int K, EPI ep, int tiles_m, int tiles_n, int sw,
@@ -173,29 +215,89 @@ __global__ __launch_bounds__(W * 64) void mfma8_direct_kernel(RowMajorRows A, Ro
             acc[i][j] = MMA::mma(fb[j], fa[i], acc[i][j]);
    }
 
+   direct_store<MMA, MB, NB, W>(ep, acc, part, m0, n0, M, N, wave, lane);
+}
+
+// The same with the operands going through LDS, for rows that start on 16 bytes.  A vector L1 takes four cycles per line that a load instruction touches: fragments
+// in the layout of the MFMA come from 16 rows, 64 bytes of a line each, at 16 B/clk, which bounds the kernel above (its 16 rows of 4096 bytes and as
+// many of B: 128 KB, 3.5 us of 6.8).  Loaded line by line, 128 bytes of eight rows per instruction, straight into LDS, they come at twice that.  A wave's steps
+// pass through a ring of its own of `depth` places: no barrier in the loop.
+template <class MMA, int MB, int NB, int W, class EPI>
+__global__ __launch_bounds__(W * 64) void mfma8_direct_ring_kernel(RowMajorRows A, RowMajorRows Bt, int M, int N, int K, EPI ep, int tiles_m, int tiles_n, int sw,
+                                                                   int first_tile, int depth)
+{
+   constexpr int STEP = 128, LA = MB * 2, LB = NB * 2, LOADS = LA + LB, PLACE = (MB + NB) * 16 * STEP;
+   typedef typename MMA::acc_t acc_t;
+   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
+   int tm, tn;
+   tile_of_block(first_tile + blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, sw, tm, tn);
+   const int m0 = tm * MB * 16, n0 = tn * NB * 16;
+   const int lane = threadIdx.x & 63;
+   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+   const int lk = lane >> 4, c = lane & 15;
+   // load i brings rows 8 i .. 8 i + 7 of the tile's B, then A, in the order of lds_chunk_offset; rows past the edge re-read the last one
+   int at[LOADS], chunk[LOADS];
+#pragma unroll
+   for (int i = 0; i < LOADS; ++i) {
+      const int row = i * 8 + lane / 8, r = i < LB ? row : row - NB * 16, last = i < LB ? N - 1 - n0 : M - 1 - m0;
+      chunk[i] = ((lane & 7) ^ (row >> 1 & 7)) * 16;
+      at[i] = (r < last ? r : last) * (i < LB ? Bt.ld : A.ld) + chunk[i];
+   }
+   int8_t *const mine = smem + wave * depth * PLACE;
+   const int8_t *const base_a = A.row(m0), *const base_b = Bt.row(n0);
+   const int steps = (int)(((unsigned)K + STEP - 1) / STEP), own = wave < steps ? (steps - wave + W - 1) / W : 0;
+   auto issue = [&](int i, int place) {
+      const int k = (wave + i * W) * STEP;
+#pragma unroll
+      for (int l = 0; l < LOADS; ++l) {
+         direct_buffer_load((lds_void_t *)(mine + place * PLACE + l * 1024), (l < LB ? base_b : base_a) + k, chunk[l] < K - k ? at[l] : -1);
+      }
+   };
+   acc_t acc[MB][NB];
 #pragma unroll
    for (int i = 0; i < MB; ++i)
 #pragma unroll
       for (int j = 0; j < NB; ++j)
-         *(acc_t *)&part[wave][i * 16 + c][j * 16 + lk * 4] = acc[i][j];
-   __syncthreads();
-   ep.dispatch([&](auto mode) {
-      constexpr int MODE = decltype(mode)::value;
+         acc[i][j] = acc_t{0, 0, 0, 0};
+   for (int i = 0; i < depth && i < own; ++i)
+      issue(i, i);
+   int place = 0;
 #pragma unroll 1
-      for (int e = threadIdx.x; e < TM * TN / 4; e += W * 64) {
-         const int r = e / (TN / 4), q = e % (TN / 4) * 4;
-         acc_t v = *(const acc_t *)&part[0][r][q];
+   for (int i = 0; i < own; ++i) {
+      const int ahead = own - 1 - i < depth - 1 ? own - 1 - i : depth - 1; // steps that may still be on their way
+      if (ahead >= 3)
+         wait_vmcnt<3 * LOADS>();
+      else if (ahead == 2)
+         wait_vmcnt<2 * LOADS>();
+      else if (ahead == 1)
+         wait_vmcnt<LOADS>();
+      else
+         wait_vmcnt<0>();
+      __builtin_amdgcn_sched_barrier(0);
+      v4i fa[MB][2], fb[NB][2];
+      const int8_t *const from = mine + place * PLACE;
 #pragma unroll
-         for (int w = 1; w < W; ++w)
-            v += *(const acc_t *)&part[w][r][q];
-         const int m = m0 + r, n = n0 + q;
-         if (m >= M || n >= N)
-            continue;
-         typename EPI::template col_params<4> prm;
-         ep.template load_params<4>(n, prm);
-         store_four_columns<MODE>(ep, prm, v, m, n, N);
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+         for (int j = 0; j < NB; ++j)
+            fb[j][h] = *(const v4i *)(from + lds_chunk_offset<STEP>(j * 16 + c, lk * 2 + h));
+#pragma unroll
+         for (int m = 0; m < MB; ++m)
+            fa[m][h] = *(const v4i *)(from + lds_chunk_offset<STEP>((NB + m) * 16 + c, lk * 2 + h));
       }
-   });
+      __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0): the place may be filled again
+      __builtin_amdgcn_sched_barrier(0);
+      if (i + depth < own)
+         issue(i + depth, place);
+      place = place + 1 == depth ? 0 : place + 1;
+#pragma unroll
+      for (int m = 0; m < MB; ++m)
+#pragma unroll
+         for (int j = 0; j < NB; ++j)
+            acc[m][j] = MMA::mma(fb[j], fa[m], acc[m][j]);
+   }
+   __syncthreads();
+   direct_store<MMA, MB, NB, W>(ep, acc, (typename MMA::elem_t(*)[MB * 16][NB * 16 + 4])smem, m0, n0, M, N, wave, lane);
 }
 
 template <class MMA, int MB, int NB, int W, int UNROLL, class EPI>
@@ -205,6 +307,21 @@ static int launch_mfma8_direct(const LaunchCfg &lc, const int8_t *A, const int8_
    const long long nwg = (long long)tiles_m * tiles_n;
    if (nwg > 0x7fffffffLL)
       return fail(SOFIE_HIP_ERR_INVALID, "gemm: too many tiles");
+   // rows on 16 bytes, and a tile's rows within a buffer
+   const long long pitch = lda > ldb ? lda : ldb;
+   if (((uintptr_t)A & 15) == 0 && ((uintptr_t)Bt & 15) == 0 && lda % 16 == 0 && ldb % 16 == 0 && K % 16 == 0 && K > 0 && MB * 16 * pitch + 256 < DIRECT_BUFFER_BYTES) {
+      constexpr int PLACES = W * (MB + NB) * 16 * 128, most = 128 * 1024 / PLACES;
+      const int depth = std::max(1, nwg > 256 ? most / 2 : most);
+      const size_t part = (size_t)W * MB * 16 * (NB * 16 + 4) * 4, smem = std::max((size_t)depth * PLACES, part);
+      auto kern = mfma8_direct_ring_kernel<MMA, MB, NB, W, EPI>;
+      static bool configured[64] = {};
+      if (int st = configure_lds_once(kern, (size_t)most * PLACES, configured))
+         return st;
+      in_launches(nwg, W * 64, [&](int first, unsigned count) {
+         launch_kernel(kern, dim3(count), dim3(W * 64), smem, lc.stream, RowMajorRows{A, lda}, RowMajorRows{Bt, ldb}, M, N, K, ep, tiles_m, tiles_n, lc.swizzle, first, depth);
+      });
+      return launch_status("mfma8_direct_ring_kernel");
+   }
    in_launches(nwg, W * 64, [&](int first, unsigned count) {
       launch_kernel((mfma8_direct_kernel<MMA, MB, NB, W, UNROLL, EPI>), dim3(count), dim3(W * 64), 0, lc.stream, RowMajorRows{A, lda}, RowMajorRows{Bt, ldb}, M, N, K, ep,
                     tiles_m, tiles_n, lc.swizzle, first);

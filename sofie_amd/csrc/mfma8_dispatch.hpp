@@ -20,8 +20,15 @@ inline double mfma8_time(int M, int N, int K, int bm, int bn, double fixed_us, d
    rounds = rounds <= 1.0 ? 1.0 : 0.5 * (rounds + std::ceil(rounds));
    return fixed_us + rounds * (tile_us + (double)(bm + bn) * K / bytes_per_us);
 }
-inline double mfma8_direct16_time(int M, int N, int K) { return mfma8_time(M, N, K, 16, 16, 2.5, 0.4, 41e3); }
-inline double mfma8_direct32_time(int M, int N, int K) { return mfma8_time(M, N, K, 32, 32, 2.5, 0.8, 44e3); }
+// `lines`: rows start on 16 bytes, so that the direct kernel loads line by line through its ring: 115 KB/us a CU while few CUs are at work, and 21 TB/s
+// from L2 over all of them (us, us estimated / measured: 16 x 4096 x 4096 4.4 / 4.0, 609 x 377 x 5728 7.5 / 7.5, 108 x 4816 x 1392 6.8 / 6.8).
+inline double mfma8_direct_time(int M, int N, int K, int b, bool lines)
+{
+   if (!lines)
+      return b == 16 ? mfma8_time(M, N, K, 16, 16, 2.5, 0.4, 41e3) : mfma8_time(M, N, K, 32, 32, 2.5, 0.8, 44e3);
+   const double tiles = (double)((M + b - 1) / b) * ((N + b - 1) / b);
+   return mfma8_time(M, N, K, b, b, 2.5, b == 16 ? 0.3 : 0.5, std::min(115e3, 21e6 / std::min(tiles, 256.0)));
+}
 inline double mfma8_staged64_time(int M, int N, int K) { return mfma8_time(M, N, K, 64, 64, 3.0, 0.4, 45e3); }
 inline double mfma8_staged128_time(int M, int N, int K) { return mfma8_time(M, N, K, 128, 128, 4.0, 2.5, 39e3); }
 inline double mfma8_ring_time(int M, int N, int K, int tile)
@@ -49,7 +56,8 @@ static int launch_mfma8_best(const LaunchCfg &lc, const int8_t *A, const int8_t 
    typedef std::conditional_t<(MMA::KSTEP * 2 <= 64), DirectI8, DirectF8> Direct;
    const bool aligned = (lda % 16 == 0) && (ldb % 16 == 0) && (((uintptr_t)A & 15) == 0) && (((uintptr_t)Bt & 15) == 0);
    const bool ring = variant >= 0 && aligned && K >= 64 && K % 64 == 0 && (MMA::KSTEP * 2 <= 64 || K % 128 == 0);
-   const double t16 = mfma8_direct16_time(M, N, K), t32 = mfma8_direct32_time(M, N, K);
+   const bool lines = aligned && K % 16 == 0;
+   const double t16 = mfma8_direct_time(M, N, K, 16, lines), t32 = mfma8_direct_time(M, N, K, 32, lines);
    const double others = ring ? mfma8_ring_time(M, N, K, pick_tile(M, N, 0)) : std::min(mfma8_staged64_time(M, N, K), mfma8_staged128_time(M, N, K));
    if (force_tile == 16 || K < 16 || (!force_tile && variant == 0 && t16 <= t32 && t16 < others))
       return launch_mfma8_direct<Direct, 1, 1, 8, 4, EPI>(lc, A, Bt, M, N, K, lda, ldb, ep);
@@ -114,7 +122,7 @@ static bool mfma8_columns_preferred(const LaunchCfg &lc, int M, int N, int K, bo
    if (K < 16 || N < 16 || lc.tile == 16 || lc.tile == 32)
       return false;
    const double staged = std::min(mfma8_staged64_time(M, N, K), mfma8_staged128_time(M, N, K));
-   double behind = std::min(std::min(mfma8_direct16_time(M, N, K), mfma8_direct32_time(M, N, K)), staged);
+   double behind = std::min(std::min(mfma8_direct_time(M, N, K, 16, aligned_behind), mfma8_direct_time(M, N, K, 32, aligned_behind)), staged);
    if (aligned_behind && K >= 64 && K % 64 == 0)
       behind = std::min(behind, mfma8_ring_time(M, N, K, pick_tile(M, N, 0)));
    return lc.tile == 0 && lc.variant <= 0 && staged < 2.0 + 2.0 * K * N / 4.2e6 + behind;
