@@ -138,15 +138,20 @@ namespace sofie_hip {
 // shortest.  A CU multiplies a 32 x 32 block by 32 k in 0.107 us at best.  The tile kernels take 0.128 us (32 x 32 tiles), 0.245
 // (64 x 32: two blocks), 0.452 (64 x 64: four) and 1.765 (128 x 128: sixteen), a start and a store per tile, in as many rounds as
 // the tiles need over 256 CUs, and a launch.  The direct kernel costs a launch, a trip to memory per 512 k or the 10.5 TB/s at which
-// its fragments, which nothing shares, arrive, and 0.45 us per 256 tiles.
+// its fragments, which nothing shares, arrive, and 0.45 us per 256 tiles; `lines`: where both operands come line by line through its ring, 82 KB/us a CU and 0.35 us
+// for the first 256 tiles, 66 and 0.55 a tile where there are more (estimated / measured: 16 x 1024 x 1024 4.2 / 4.5, 1157 x 189 x 116 5.1 / 4.8).
 enum F32Tile { F32_CONV3X3_32 = 3032, F32_CONV3X3_64 = 3064, F32_CONV3X3_128 = 3128, F32_CONV3X3_SPLIT_128 = 4128, F32_CONV3X3_SPLIT_256 = 4256, F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
-static int pick_f32_tile(int M, int N, int K, int batch, double *time_us = nullptr)
+static int pick_f32_tile(int M, int N, int K, int batch, bool lines, double *time_us = nullptr)
 {
    auto tiles = [&](int bm, int bn) { return std::ceil((double)M / bm) * std::ceil((double)N / bn) * batch; };
    const double slabs = std::ceil(K / 32.0), steps = std::ceil(K / 16.0);
    auto tiled = [&](int bm, int bn, double launch, double slab, double tile) { return launch + std::ceil(tiles(bm, bn) / 256.0) * (slabs * slab + tile); };
    int best = F32_DIRECT;
    double least = 2.0 + std::max(1.35 * std::ceil(steps / 32.0), tiles(16, 16) * steps * 2048.0 / 10.5e6) + 0.45 * tiles(16, 16) / 256.0;
+   if (lines) {
+      const double each = tiles(16, 16) / 256.0, rounds = each <= 1.0 ? 1.0 : 0.5 * (each + std::ceil(each));
+      least = 2.3 + rounds * (each <= 1.0 ? 0.35 + 128.0 * K / 82e3 : 0.55 + 128.0 * K / 66e3);
+   }
    auto offer = [&](int tile, double t) {
       if (t < least)
          least = t, best = tile;
@@ -190,7 +195,7 @@ static int launch_f32_product(sofie_hip_ctx *ctx, const ASRC &A, const BSRC &B, 
       tile = F32_TILE_64;
    constexpr bool CONV = ASRC::kLeastRows == 64;
    if (!tile)
-      tile = CONV ? pick_f32_conv_tile(M, N, K, batch) : pick_f32_tile(M, N, K, batch);
+      tile = CONV ? pick_f32_conv_tile(M, N, K, batch) : pick_f32_tile(M, N, K, batch, ASRC::KC && BSRC::KC && ASRC::VEC == 4 && BSRC::VEC == 4);
    if (tile >= F32_CONV3X3_32 || (CONV ? tile == F32_TILE_32 || tile == F32_TILE_128 : tile == F32_TILE_128x32))
       tile = F32_TILE_64; // a request for a tile that the other kind of product has
    if constexpr (CONV) {
@@ -496,10 +501,11 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
    if (ctx->opt.f32_chain == 1) {
       first = 0;
    } else if (ctx->opt.f32_chain < 0 && M >= 1 && M <= 256) {
+      auto lines = [&](int l) { return layers[l].transB && !layers[l].transA && layers[l].K % 4 == 0; };
       double before = 0.0, least = 0.0;
       for (int l = 0; l < count; ++l) {
          double t = 0.0;
-         pick_f32_tile(M, layers[l].N, layers[l].K, 1, &t);
+         pick_f32_tile(M, layers[l].N, layers[l].K, 1, lines(l), &t);
          least += std::max(t, 3.0);
       }
       for (int s = 0; s + 2 <= count; ++s) {
@@ -511,7 +517,7 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
          together = before + 2.3 + together * (M <= 64 ? 1.0 : 1.8);
          if (together < least)
             least = together, first = s;
-         pick_f32_tile(M, layers[s].N, layers[s].K, 1, &t);
+         pick_f32_tile(M, layers[s].N, layers[s].K, 1, lines(s), &t);
          before += std::max(t, 3.0);
       }
    }

@@ -222,18 +222,12 @@ __global__ __launch_bounds__(W * 64) void mfma8_direct_kernel(RowMajorRows A, Ro
 // in the layout of the MFMA come from 16 rows, 64 bytes of a line each, at 16 B/clk, which bounds the kernel above (its 16 rows of 4096 bytes and as
 // many of B: 128 KB, 3.5 us of 6.8).  Loaded line by line, 128 bytes of eight rows per instruction, straight into LDS, they come at twice that.  A wave's steps
 // pass through a ring of its own of `depth` places: no barrier in the loop.
-template <class MMA, int MB, int NB, int W, class EPI>
-__global__ __launch_bounds__(W * 64) void mfma8_direct_ring_kernel(RowMajorRows A, RowMajorRows Bt, int M, int N, int K, EPI ep, int tiles_m, int tiles_n, int sw,
-                                                                   int first_tile, int depth)
+// (Pitches and K are in bytes: the fp32 products use it too.)
+template <class MMA, int MB, int NB, int W>
+__device__ __forceinline__ void direct_ring_sums(typename MMA::acc_t (&acc)[MB][NB], const RowMajorRows &A, const RowMajorRows &Bt, int M, int N, int K, int m0, int n0,
+                                                 int8_t *smem, int depth, int wave, int lane)
 {
    constexpr int STEP = 128, LA = MB * 2, LB = NB * 2, LOADS = LA + LB, PLACE = (MB + NB) * 16 * STEP;
-   typedef typename MMA::acc_t acc_t;
-   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
-   int tm, tn;
-   tile_of_block(first_tile + blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, sw, tm, tn);
-   const int m0 = tm * MB * 16, n0 = tn * NB * 16;
-   const int lane = threadIdx.x & 63;
-   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
    const int lk = lane >> 4, c = lane & 15;
    // load i brings rows 8 i .. 8 i + 7 of the tile's B, then A, in the order of lds_chunk_offset; rows past the edge re-read the last one
    int at[LOADS], chunk[LOADS];
@@ -253,12 +247,11 @@ __global__ __launch_bounds__(W * 64) void mfma8_direct_ring_kernel(RowMajorRows 
          direct_buffer_load((lds_void_t *)(mine + place * PLACE + l * 1024), (l < LB ? base_b : base_a) + k, chunk[l] < K - k ? at[l] : -1);
       }
    };
-   acc_t acc[MB][NB];
 #pragma unroll
    for (int i = 0; i < MB; ++i)
 #pragma unroll
       for (int j = 0; j < NB; ++j)
-         acc[i][j] = acc_t{0, 0, 0, 0};
+         acc[i][j] = typename MMA::acc_t{0};
    for (int i = 0; i < depth && i < own; ++i)
       issue(i, i);
    int place = 0;
@@ -296,9 +289,45 @@ __global__ __launch_bounds__(W * 64) void mfma8_direct_ring_kernel(RowMajorRows 
          for (int j = 0; j < NB; ++j)
             acc[m][j] = MMA::mma(fb[j], fa[m], acc[m][j]);
    }
+}
+
+template <class MMA, int MB, int NB, int W, class EPI>
+__global__ __launch_bounds__(W * 64) void mfma8_direct_ring_kernel(RowMajorRows A, RowMajorRows Bt, int M, int N, int K, EPI ep, int tiles_m, int tiles_n, int sw,
+                                                                   int first_tile, int depth)
+{
+   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
+   int tm, tn;
+   tile_of_block(first_tile + blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, sw, tm, tn);
+   const int m0 = tm * MB * 16, n0 = tn * NB * 16;
+   const int lane = threadIdx.x & 63;
+   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+   typename MMA::acc_t acc[MB][NB];
+   direct_ring_sums<MMA, MB, NB, W>(acc, A, Bt, M, N, K, m0, n0, smem, depth, wave, lane);
    __syncthreads();
    direct_store<MMA, MB, NB, W>(ep, acc, (typename MMA::elem_t(*)[MB * 16][NB * 16 + 4])smem, m0, n0, M, N, wave, lane);
 }
+
+// The ring of a launch: places per wave (as many as fit and are used; half of them where a CU has several tiles), and bytes of LDS, in which the partial tiles
+// meet too.  K in bytes.
+template <int MB, int NB, int W>
+struct DirectRing {
+   static constexpr int PLACE = (MB + NB) * 16 * 128, MOST = 128 * 1024 / (W * PLACE);
+   static constexpr size_t PART = (size_t)W * MB * 16 * (NB * 16 + 4) * 4;
+   int depth;
+   size_t bytes;
+   DirectRing(long long workgroups, int K)
+   {
+      const int steps = (int)(((unsigned)K + 127) / 128);
+      depth = std::max(1, std::min(workgroups > 256 ? MOST / 2 : MOST, (steps + W - 1) / W));
+      bytes = std::max((size_t)std::min(steps, W) * depth * PLACE, PART);
+   }
+   // rows on 16 bytes, and a tile's rows within a buffer
+   static bool takes(const void *A, const void *Bt, long long lda, long long ldb, long long K)
+   {
+      return ((uintptr_t)A & 15) == 0 && ((uintptr_t)Bt & 15) == 0 && lda % 16 == 0 && ldb % 16 == 0 && K % 16 == 0 && K > 0 && K <= 0x7fffffff &&
+             (MB > NB ? MB : NB) * 16 * (lda > ldb ? lda : ldb) + 256 < DIRECT_BUFFER_BYTES;
+   }
+};
 
 template <class MMA, int MB, int NB, int W, int UNROLL, class EPI>
 static int launch_mfma8_direct(const LaunchCfg &lc, const int8_t *A, const int8_t *Bt, int M, int N, int K, int lda, int ldb, const EPI &ep)
@@ -307,18 +336,16 @@ static int launch_mfma8_direct(const LaunchCfg &lc, const int8_t *A, const int8_
    const long long nwg = (long long)tiles_m * tiles_n;
    if (nwg > 0x7fffffffLL)
       return fail(SOFIE_HIP_ERR_INVALID, "gemm: too many tiles");
-   // rows on 16 bytes, and a tile's rows within a buffer
-   const long long pitch = lda > ldb ? lda : ldb;
-   if (((uintptr_t)A & 15) == 0 && ((uintptr_t)Bt & 15) == 0 && lda % 16 == 0 && ldb % 16 == 0 && K % 16 == 0 && K > 0 && MB * 16 * pitch + 256 < DIRECT_BUFFER_BYTES) {
-      constexpr int PLACES = W * (MB + NB) * 16 * 128, most = 128 * 1024 / PLACES;
-      const int depth = std::max(1, nwg > 256 ? most / 2 : most);
-      const size_t part = (size_t)W * MB * 16 * (NB * 16 + 4) * 4, smem = std::max((size_t)depth * PLACES, part);
+   typedef DirectRing<MB, NB, W> Ring;
+   if (Ring::takes(A, Bt, lda, ldb, K)) {
+      const Ring ring(nwg, K);
       auto kern = mfma8_direct_ring_kernel<MMA, MB, NB, W, EPI>;
       static bool configured[64] = {};
-      if (int st = configure_lds_once(kern, (size_t)most * PLACES, configured))
+      if (int st = configure_lds_once(kern, 128 * 1024, configured))
          return st;
       in_launches(nwg, W * 64, [&](int first, unsigned count) {
-         launch_kernel(kern, dim3(count), dim3(W * 64), smem, lc.stream, RowMajorRows{A, lda}, RowMajorRows{Bt, ldb}, M, N, K, ep, tiles_m, tiles_n, lc.swizzle, first, depth);
+         launch_kernel(kern, dim3(count), dim3(W * 64), ring.bytes, lc.stream, RowMajorRows{A, lda}, RowMajorRows{Bt, ldb}, M, N, K, ep, tiles_m, tiles_n,
+                       lc.swizzle, first, ring.depth);
       });
       return launch_status("mfma8_direct_ring_kernel");
    }
