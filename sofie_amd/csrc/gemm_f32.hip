@@ -11,7 +11,7 @@ namespace sofie_hip {
 // workgroup takes RB rows through every layer, the rows of activations staying in LDS between layers (each layer's
 // output is also written to its Y, as separate launches would).  The weights stream from L2 once per workgroup:
 //   transB (W stored [N][K], the ONNX export of a Linear layer): a wave takes 4 outputs at a time, its lanes stride over k
-//     (coalesced 256-byte reads of each weight row), then the 64 partial sums are folded with shuffles;
+//     (coalesced 256-byte reads of each weight row), then the 64 partial sums are folded across the lanes;
 //   else (W stored [K][N]): a thread owns output n and walks k (lanes read consecutive n of one weight row).
 struct ChainLayerArgs {
    const float *B;
@@ -80,12 +80,10 @@ __global__ __launch_bounds__(CHAIN_THREADS) void gemm_chain_f32_kernel(ChainArgs
                }
             }
 #pragma unroll
-            for (int off = 32; off >= 1; off >>= 1)
+            for (int j = 0; j < 4; ++j)
 #pragma unroll
-               for (int j = 0; j < 4; ++j)
-#pragma unroll
-                  for (int r = 0; r < RB; ++r)
-                     acc[j][r] += __shfl_xor(acc[j][r], off, 64);
+               for (int r = 0; r < RB; ++r)
+                  acc[j][r] = sum_over_lanes(acc[j][r]);
             // every lane now holds the 4 x RB sums: lane j finishes output n0 + j
             const int n = n0 + lane;
             if (lane < 4 && n < N) {
