@@ -12,7 +12,10 @@ namespace sofie_hip {
 // output is also written to its Y, as separate launches would).  The weights stream from L2 once per workgroup:
 //   transB (W stored [N][K], the ONNX export of a Linear layer): a wave takes 4 outputs at a time, its lanes stride over k
 //     (coalesced 256-byte reads of each weight row), then the 64 partial sums are folded across the lanes;
-//   else (W stored [K][N]): a thread owns output n and walks k (lanes read consecutive n of one weight row).
+//   else (W stored [K][N]): a thread owns output n and walks k (lanes read consecutive n of one weight row); up to 512 outputs, whose threads alone
+//     would leave the others idle, k is dealt out over groups of threads, and their sums are added up through LDS (39 rows through
+//     256-137-1800-17: 28.6 -> 19.9 us, most of it by taking the first layer into the chain, whose waves were one in eight before; 4 rows through
+//     128-112-32-9 9.3 -> 8.1).
 struct ChainLayerArgs {
    const float *B;
    long long ldb;
@@ -31,10 +34,39 @@ struct ChainArgs {
 // 16 waves per workgroup: what a layer costs is the round trips to L2 for its weights, and the waves' loads overlap
 constexpr int CHAIN_THREADS = 1024;
 
+// A thread's column of W (its floats `ldb` apart) times RB rows in LDS, for k0 <= k < k1, sixteen loads in flight.
+template <int RB>
+__device__ __forceinline__ void chain_walk(float (&acc)[RB], const float *column, long long ldb, const float *in, int width, int k0, int k1)
+{
+   int k = k0;
+   const float *w = column + k * ldb;
+   auto some = [&](auto count) {
+      constexpr int U = decltype(count)::value;
+      for (; k + U <= k1; k += U) {
+         float v[U];
+#pragma unroll
+         for (int u = 0; u < U; ++u) {
+            v[u] = *w;
+            w += ldb;
+         }
+         if constexpr (U > 1)
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+         for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+               acc[r] = fmaf(v[u], in[r * width + k + u], acc[r]);
+      }
+   };
+   some(std::integral_constant<int, 16>{});
+   some(std::integral_constant<int, 4>{});
+   some(std::integral_constant<int, 1>{});
+}
+
 template <int RB>
 __global__ __launch_bounds__(CHAIN_THREADS) void gemm_chain_f32_kernel(ChainArgs a, int width)
 {
-   extern __shared__ float chain_lds[]; // two buffers of RB rows x width
+   extern __shared__ float chain_lds[]; // two buffers of RB rows x width, RB sums per thread
    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
    const int m0 = blockIdx.x * RB;
    const int rows = (a.M - m0) < RB ? (a.M - m0) : RB;
@@ -98,19 +130,38 @@ __global__ __launch_bounds__(CHAIN_THREADS) void gemm_chain_f32_kernel(ChainArgs
                }
             }
          }
+      } else if (N <= CHAIN_THREADS / 2) {
+         const int shift = N <= 64 ? 6 : N <= 128 ? 7 : N <= 256 ? 8 : 9, span = 1 << shift, parts = CHAIN_THREADS >> shift;
+         const int n = t & (span - 1), part = t >> shift, per = (K + parts - 1) / parts, k1 = (part + 1) * per < K ? (part + 1) * per : K;
+         float acc[RB];
+#pragma unroll
+         for (int r = 0; r < RB; ++r)
+            acc[r] = 0.0f;
+         chain_walk<RB>(acc, B + (n < N ? n : N - 1), L.ldb, in, width, part * per, k1); // columns past N are the last one's, and their sums dropped
+         float *sums = chain_lds + 2 * RB * width;
+#pragma unroll
+         for (int r = 0; r < RB; ++r)
+            sums[r * CHAIN_THREADS + t] = acc[r];
+         __syncthreads();
+#pragma unroll
+         for (int r = 0; r < RB; ++r) {
+            // row r is finished by the threads of group r % parts
+            if (part == r % parts && r < rows && n < N) {
+               float s = sums[r * CHAIN_THREADS + n];
+               for (int p = 1; p < parts; ++p)
+                  s += sums[r * CHAIN_THREADS + (p << shift) + n];
+               const float v = f32_epilogue(L.ep, s, m0 + r, n);
+               out[r * width + n] = v;
+               L.Y[(long long)(m0 + r) * L.ldy + n] = v;
+            }
+         }
       } else {
          for (int n = t; n < N; n += CHAIN_THREADS) {
             float acc[RB];
 #pragma unroll
             for (int r = 0; r < RB; ++r)
                acc[r] = 0.0f;
-#pragma unroll 8
-            for (int k = 0; k < K; ++k) {
-               const float w = B[(long long)k * L.ldb + n];
-#pragma unroll
-               for (int r = 0; r < RB; ++r)
-                  acc[r] = fmaf(w, in[r * width + k], acc[r]);
-            }
+            chain_walk<RB>(acc, B + n, L.ldb, in, width, 0, K);
 #pragma unroll
             for (int r = 0; r < RB; ++r) {
                if (r < rows) {
@@ -413,14 +464,18 @@ static int launch_f32_chain(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *layer
    const int RB = M <= 64 ? 1 : M <= 128 ? 2 : 4;
    width = (width + 3) / 4 * 4;
    if (fused && (long long)RB * width <= 8192) {
-      const size_t lds = (size_t)2 * RB * width * sizeof(float);
+      const size_t lds = ((size_t)2 * RB * width + RB * CHAIN_THREADS) * sizeof(float);
       const dim3 grid((unsigned)((M + RB - 1) / RB));
-      if (RB == 1)
-         launch_kernel(gemm_chain_f32_kernel<1>, grid, dim3(CHAIN_THREADS), lds, ctx->stream, a, width);
-      else if (RB == 2)
-         launch_kernel(gemm_chain_f32_kernel<2>, grid, dim3(CHAIN_THREADS), lds, ctx->stream, a, width);
-      else
-         launch_kernel(gemm_chain_f32_kernel<4>, grid, dim3(CHAIN_THREADS), lds, ctx->stream, a, width);
+      auto launch = [&](auto rows) -> int {
+         auto kern = gemm_chain_f32_kernel<decltype(rows)::value>;
+         static bool configured[64] = {};
+         if (int st = configure_lds_once(kern, (2 * 8192 + decltype(rows)::value * CHAIN_THREADS) * sizeof(float), configured))
+            return st;
+         launch_kernel(kern, grid, dim3(CHAIN_THREADS), lds, ctx->stream, a, width);
+         return SOFIE_HIP_OK;
+      };
+      if (int st = RB == 1 ? launch(std::integral_constant<int, 1>{}) : RB == 2 ? launch(std::integral_constant<int, 2>{}) : launch(std::integral_constant<int, 4>{}))
+         return st;
       *launched = true;
       return launch_status("gemm_chain_f32_kernel");
    }
@@ -493,7 +548,8 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
       SOFIE_HIP_REQUIRE(layers[l].A == layers[l - 1].Y && layers[l].A != nullptr, "sofie_hip_gemm_chain_f32: layer %d does not read the output of layer %d", l, l - 1);
    // Which layers share a launch.  A launch of its own spreads a layer over the chip and costs about 3 us (what the host takes for
    // it); in the chain kernel a workgroup does its rows' share alone: a pass over 64 outputs (W stored [N][K]) or a walk along k
-   // (W stored [K][N]) at a time.  So large layers run one by one, and small ones behind them share a launch.
+   // (W stored [K][N]) at a time.  So large layers run one by one, and small ones behind them share a launch.  (Fitted to 60 networks of two to four
+   // layers; of 40 others one is 1.5 us slower than the best split.)
    const int M = layers[0].M;
    int first = count; // first layer of the shared launch
    if (ctx->opt.f32_chain == 1) {
@@ -509,8 +565,9 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
       for (int s = 0; s + 2 <= count; ++s) {
          double together = 0.0, t = 0.0;
          for (int l = s; l < count; ++l) {
-            const double K = layers[l].K, passes = std::ceil(layers[l].N / (layers[l].transB ? 64.0 : 1024.0));
-            together += 0.4 + passes * (layers[l].transB ? 0.9 + 0.002 * K : 0.017 * K);
+            const double K = layers[l].K, N = layers[l].N, passes = std::ceil(N / (layers[l].transB ? 64.0 : 1024.0));
+            const double groups = N <= 64 ? 16.0 : N <= 128 ? 8.0 : N <= 256 ? 4.0 : N <= 512 ? 2.0 : 1.0; // that deal out k
+            together += 0.4 + passes * (layers[l].transB ? 0.7 + 0.002 * K : 1.3 + 0.023 * K / groups);
          }
          together = before + 2.3 + together * (M <= 64 ? 1.0 : 1.8);
          if (together < least)
