@@ -9,9 +9,10 @@
 //
 // What the pieces cost is vector instructions (5.5 per value) and LDS (6 bytes written per value, at 79 B/clk): a 3 x 3 convolution uses every value of its
 // input patch nine times, which pays for both.  (A plain product of 64 x 64 tiles uses a value twice per wave: 20 - 27 us where fp32 takes 20 - 32.)
-// 64 images of 32 x 32, us, the fp32 kernel -> this one: 32 -> 64 channels 29.4 -> 22.1, 64 -> 64 50 -> 34.5 (with a residual 50 -> 37); 128 -> 128 at
-// 16 x 16 48.3 -> 38.  Error of 64 -> 64 against 64 bits: 4.2e-7 -> 1.4e-7 of the result.  On 64 -> 64 the matrix cores are busy in 0.47 of the cycles at
-// 1.9 GHz of 2.4 (power); 10 us of the launch are the first slab's load, the store and the launch itself, which nothing overlaps.
+// 64 images of 32 x 32, us, the fp32 kernel (with the stores it had) -> this one: 32 -> 64 channels 29.1 -> 20.1, 64 -> 64 49.7 -> 31.5 (with a residual 51.1 ->
+// 32.1); 128 -> 128 at 16 x 16 49.2 -> 36.9; 48 images of 37 x 37, 32 -> 96 48.9 -> 38.9.  Error of 64 -> 64 against 64 bits: 4.2e-7 -> 1.4e-7 of the result.  On
+// 64 -> 64 the matrix cores are busy in half of the cycles at 1.75 GHz of 2.4 (power); 8 us of the launch are the first slab's load, the store and the launch
+// itself, which nothing overlaps.
 //
 // Exceptions: bf16 has the exponents of fp32, so nothing overflows or vanishes that would not in fp32, except that a value within 2^-8 of the largest
 // rounds to an infinity, and that the remainders of an infinity are NaN.  Both end in a sum that is not finite; a wave that finds one among its sums
@@ -44,13 +45,6 @@ __device__ __forceinline__ v4u f32_next_piece(float (&x)[8])
    return words;
 }
 
-// A float of a buffer of which `base` is the (scalar) start; F32_OUTSIDE reads as zero.
-__device__ __forceinline__ float f32_buffer_read(const void *base, int offset, int scalar_offset)
-{
-   const __amdgpu_buffer_rsrc_t buffer = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)F32_BUFFER_BYTES, 0x00020000);
-   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buffer, offset, scalar_offset, 0));
-}
-
 // The largest patch that is taken: with it two workgroups fit a CU (81 KB each); one alone takes 1.9 times as long (32 images, 64 -> 128 at 56 x 56: 206 us
 // against the fp32 kernel's 165).
 constexpr int F32_CONV3X3_SPLIT_PATCH = 360;
@@ -71,7 +65,7 @@ struct F32Conv3x3SplitShape {
 // Four waves, each with BM / 4 pixels and 32 output channels.  One slab lies in LDS in pieces, the next one as raw weights and, in registers, as raw patch; two
 // workgroups per CU, one of which splits while the other multiplies.  (One workgroup whose other four waves split for it, through two slabs of pieces, is no
 // faster: 36 us, bound by LDS.)
-template <int BM, int PLANE, int WVEC>
+template <int BM, int PLANE, int WVEC, bool PLAIN>
 __global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a, F32ConvStore out, int tiles_m, int tiles_n, int first_tile)
 {
    typedef F32Conv3x3SplitShape<PLANE, WVEC> S;
@@ -79,7 +73,7 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a,
    static_assert(TM % 32 == 0 && PLANE % 8 == 0, "wave tiles of 32 x 32 blocks");
    extern __shared__ __attribute__((aligned(16))) char split_lds[];
    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lk = lane >> 5, c = lane & 31;
-   const int z = blockIdx.z;
+   const int wave_id = wave, z = blockIdx.z;
    a.X += z * a.group;
    a.W += (long long)z * a.N * a.K;
    out.select_batch(z);
@@ -87,10 +81,10 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a,
    f32_tile_of_block(first_tile, tiles_m, tiles_n, tm, tn);
    const int m0 = tm * BM, n0 = tn * BN;
    const int VW = a.OW + 2, VH = a.OH + 2;
-   auto quotient = [](int n, unsigned long long mul) { return mul ? (int)__umul64hi((unsigned long long)(unsigned)n, mul) : n; };
+   auto quotient = [](int n, const Divisor31 &by) { return (int)by.over((unsigned)n); };
 
    // where the patch begins; a wave splits every other 64 positions of one half of a slab's channels
-   const int line0 = quotient(m0, a.ow_mul), image0 = quotient(line0, a.oh_mul);
+   const int line0 = quotient(m0, a.by_ow), image0 = quotient(line0, a.by_oh);
    const int row0 = line0 - image0 * a.OH; // of image0, padding row 0 first
    const char *base = (const char *)uniform((long long)(a.X + image0 * a.image));
    const int plane_bytes = a.H * a.Wd * 4;
@@ -100,8 +94,8 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a,
    auto position = [&](int q) { return (2 * q + (wave >> 1)) * 64 + lane; };
 #pragma unroll
    for (int q = 0; q < CHUNKS; ++q) {
-      const int f = position(q), vr = quotient(f, a.vw_mul), ix = f - vr * VW - a.pad_w;
-      const int on = row0 + vr, image = quotient(on, a.vh_mul), iy = on - image * VH - a.pad_h;
+      const int f = position(q), vr = quotient(f, a.by_vw), ix = f - vr * VW - a.pad_w;
+      const int on = row0 + vr, image = quotient(on, a.by_vh), iy = on - image * VH - a.pad_h;
       const bool inside = (unsigned)ix < (unsigned)a.Wd && (unsigned)iy < (unsigned)a.H && image0 + image < a.images;
       patch_at[q] = inside ? (int)((image * a.image + (long long)iy * a.Wd + ix) * 4) : F32_OUTSIDE;
    }
@@ -126,12 +120,14 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a,
    const int slabs = (a.C + CS - 1) / CS;
    float raw[CHUNKS][8];
    auto issue = [&](int s) {
-      const int first = s * CS + half * 8;
+      int wave = wave_id, C = a.C, K = a.K, N = a.N;
+      forget(wave), forget(C), forget(K), forget(N);
+      const int first = s * CS + (wave & 1) * 8;
 #pragma unroll
       for (int q = 0; q < CHUNKS; ++q)
 #pragma unroll
          for (int e = 0; e < 8; ++e) {
-            const bool there = first + e < a.C;
+            const bool there = first + e < C;
             raw[q][e] = f32_buffer_read(base, there ? patch_at[q] : F32_OUTSIDE, there ? (first + e) * plane_bytes : 0);
          }
 #pragma unroll
@@ -140,7 +136,7 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a,
             int row, k;
             weight_place(i, row, k);
             // k past the last channel are the next row's
-            const int at = n0 + row < a.N && s * CS * 9 + k < a.K ? (row * a.K + k) * 4 : F32_OUTSIDE;
+            const int at = n0 + row < N && s * CS * 9 + k < K ? (row * K + k) * 4 : F32_OUTSIDE;
             f32_buffer_load<WVEC>((lds_void_t *)(split_lds + S::RAW_AT + (i * 4 + wave) * 64 * WVEC * 4), weights + (long long)s * CS * 9 * 4, at);
          }
       }
@@ -172,7 +168,7 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a,
 #pragma unroll
    for (int i = 0; i < MT; ++i) {
       const int m = m0 + wave * TM + i * 32 + c, mm = m < a.M ? m : a.M - 1;
-      const int line = quotient(mm, a.ow_mul), image = quotient(line, a.oh_mul);
+      const int line = quotient(mm, a.by_ow), image = quotient(line, a.by_oh);
       const int vr = (image - image0) * VH + line - image * a.OH - row0;
 #pragma unroll
       for (int ky = 0; ky < 3; ++ky)
@@ -248,7 +244,6 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a,
          acc[i][e] += low[i][e];
          finite = __builtin_fmaf(acc[i][e], 0.0f, finite);
       }
-   const int n1 = n0 + lk * 4; // this lane's columns: n1 + e / 4 * 8 + e % 4
    if (__builtin_amdgcn_ballot_w64(finite != 0.0f) != 0) {
       clear(acc);
       const float *row = a.W + (long long)(n0 + c < a.N ? n0 + c : a.N - 1) * a.K;
@@ -262,7 +257,7 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a,
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
                const int m = m0 + wave * TM + i * 32 + c, mm = m < a.M ? m : a.M - 1;
-               const int line = quotient(mm, a.ow_mul), image = quotient(line, a.oh_mul);
+               const int line = quotient(mm, a.by_ow), image = quotient(line, a.by_oh);
                const int iy = line - image * a.OH + ky - a.pad_h, ix = mm - line * a.OW + kx - a.pad_w;
                v[i][j] = k < a.K && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.Wd ? a.X[image * a.image + ((long long)ch * a.H + iy) * a.Wd + ix] : 0.0f;
             }
@@ -275,43 +270,16 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a,
       }
    }
 
-   // 32 neighbouring lanes hold 32 neighbouring pixels of a channel: whole lines, straight from the registers
-   auto column = [&](int e) { return n1 + e / 4 * 8 + e % 4; };
-   float bias[16], residual[MT][16];
-#pragma unroll
-   for (int e = 0; e < 16; ++e) {
-      const int n = column(e) < a.N ? column(e) : a.N - 1;
-      bias[e] = out.bias_of(n);
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-         const int m = m0 + wave * TM + i * 32 + c;
-         residual[i][e] = out.residual_of(out.row_of(m < a.M ? m : a.M - 1), n);
-      }
-   }
 #pragma unroll
    for (int i = 0; i < MT; ++i) {
-      const int m = m0 + wave * TM + i * 32 + c;
-      const auto where = out.row_of(m < a.M ? m : a.M - 1);
-      auto put = [&](float v, int e) {
-         if (m < a.M && column(e) < a.N)
-            out.Y[where.at + (size_t)(out.first + column(e)) * out.positions] = v;
-      };
+      const int m = m0 + wave * TM + i * 32 + c, mm = m < a.M ? m : a.M - 1, image = quotient(quotient(mm, a.by_ow), a.by_oh);
+      const Conv3x3Block<16> block(out, image0, image, mm - image * out.positions, n0, a.N, lk, 0, m < a.M, a.near);
+      float bias[16], residual[16], v[16];
+      block.load(bias, residual);
 #pragma unroll
       for (int e = 0; e < 16; ++e)
-         acc[i][e] = (acc[i][e] + bias[e]) + residual[i][e];
-      const bool relu = out.chain.count == 1 && out.chain.op0 == SOFIE_ACT_RELU;
-      if (relu || out.chain.count == 0) {
-#pragma unroll
-         for (int e = 0; e < 16; ++e)
-            put(relu ? (acc[i][e] > 0.0f ? acc[i][e] : 0.0f) : acc[i][e], e);
-      } else {
-         // one copy of the activations' code for 16 elements
-#pragma unroll 1
-         for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-               put(apply_chain(g == 0 ? acc[i][e] : g == 1 ? acc[i][4 + e] : g == 2 ? acc[i][8 + e] : acc[i][12 + e], out.chain), g * 4 + e);
-      }
+         v[e] = (acc[i][e] + bias[e]) + residual[e];
+      block.store<PLAIN>(v, out.chain);
    }
 }
 
@@ -324,14 +292,17 @@ static int launch_f32_conv3x3_split_as(hipStream_t stream, const F32Conv3x3 &a, 
       return fail(SOFIE_HIP_ERR_INVALID, "fp32 convolution: too many tiles");
    constexpr size_t smem = F32Conv3x3SplitShape<PLANE, WVEC>::BYTES;
    static_assert(smem <= 160 * 1024, "LDS of a CU");
-   auto kern = f32_conv3x3_split_kernel<BM, PLANE, WVEC>;
-   static bool configured[64] = {};
-   if (int st = configure_lds_once(kern, smem, configured))
-      return st;
-   in_launches((long long)tiles_m * tiles_n, 256, [&](int first, unsigned count) {
-      launch_kernel(kern, dim3(count, 1, (unsigned)group), dim3(256), smem, stream, a, out, tiles_m, tiles_n, first);
-   });
-   return launch_status("f32_conv3x3_split_kernel");
+   auto go = [&](auto plain) {
+      auto kern = f32_conv3x3_split_kernel<BM, PLANE, WVEC, decltype(plain)::value>;
+      static bool configured[64] = {};
+      if (int st = configure_lds_once(kern, smem, configured))
+         return st;
+      in_launches((long long)tiles_m * tiles_n, 256, [&](int first, unsigned count) {
+         launch_kernel(kern, dim3(count, 1, (unsigned)group), dim3(256), smem, stream, a, out, tiles_m, tiles_n, first);
+      });
+      return launch_status("f32_conv3x3_split_kernel");
+   };
+   return conv3x3_plain(out.chain) ? go(std::true_type{}) : go(std::false_type{});
 }
 
 } // namespace sofie_hip

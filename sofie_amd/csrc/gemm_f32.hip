@@ -280,43 +280,37 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
       return SOFIE_HIP_OK;
    const bool vec = ((uintptr_t)W & 15) == 0 && K % 4 == 0;
    int tile = force;
-   if (!tile) {
-      // A slab of 8 channels takes 1.06 / 0.61 / 0.38 us of a CU with several tiles of 128 / 64 / 32 pixels at work, and 1.42 / 0.95 / 0.70
-      // where a tile is alone and waits for its loads; a tile costs 1.45 / 1.0 / 0.8 us besides, a launch 4.3.  One slab of a few
-      // channels: 1.6 us a tile.  (Fitted to 20 layers from 2 images of 14 x 14 to 64 of 64 x 64; holds to a tenth.)
+   if (!tile && s.Cg <= 4) {
+      tile = F32_CONV3X3_128; // slabs of four channels; half of any other kernel's slab would be zeros
+   } else if (!tile) {
+      // us: a launch; a slab (8 channels, 16 of the split kernel) of a CU whose tiles wait for their loads, and of one with several tiles at work; a tile.  The
+      // second set is for weights that come float by float.  Fitted to 156 layers from 1 image of 6 x 6 to 64 of 64 x 64, 6 to 130 channels; holds to a sixth, and
+      // costs 1 % of the best kernel's time on average over those layers, 4 % the most but for three.
       double least = 1e30;
-      auto offer = [&](int which, int bm, double slab, double alone, double each) {
-         const double rounds = std::ceil((double)((M + bm - 1) / bm) * ((N + 31) / 32) * group / 256.0), slabs = std::ceil(s.Cg / 8.0);
-         const double t = std::max(slabs * alone, rounds * (slabs * slab + each));
-         if (f32_conv3x3_patch(s.OH, s.OW, bm) <= F32_CONV3X3_PATCH && t < least)
+      struct Cost {
+         double launch, alone, slab, each;
+      };
+      auto offer = [&](int which, int bm, int channels, long long room, Cost wide, Cost narrow) {
+         const Cost cost = vec ? wide : narrow;
+         const double rounds = std::ceil((double)((M + bm - 1) / bm) * ((N + 31) / 32) * group / 256.0), slabs = (s.Cg + channels - 1) / channels;
+         const double t = cost.launch + std::max(slabs * cost.alone, rounds * (slabs * cost.slab + cost.each));
+         if (f32_conv3x3_patch(s.OH, s.OW, bm) <= room && t < least)
             least = t, tile = which;
       };
-      if (s.Cg <= 4) {
-         offer(F32_CONV3X3_128, 128, 0.3, 0.5, 1.3);
-      } else {
-         offer(F32_CONV3X3_32, 32, 0.383, 0.70, 0.8);
-         offer(F32_CONV3X3_64, 64, 0.606, 0.95, 1.0);
-         offer(F32_CONV3X3_128, 128, 1.06, 1.42, 1.45);
-      }
-      // The kernel of f32_conv3x3_split.hpp takes slabs of 16 channels, two tiles to a CU: 1.75 us of a CU a slab (128 pixels; 2.4 us where the weights come
-      // float by float) and 2.95 (256 pixels), 2.3 and 3.5 us a tile; alone 2.4, 3.6 and 3.2 us a slab.  (Fitted to 34 layers as above; holds to a tenth.)
-      auto offer_split = [&](int which, int bm, double slab, double alone, double each) {
-         const double rounds = std::ceil((double)((M + bm - 1) / bm) * ((N + 31) / 32) * group / 256.0), slabs = std::ceil(s.Cg / 16.0);
-         const double t = std::max(slabs * alone + each, rounds * (slabs * slab + each));
-         if (f32_conv3x3_patch(s.OH, s.OW, bm) <= F32_CONV3X3_SPLIT_PATCH && t < least)
-            least = t, tile = which;
-      };
-      offer_split(F32_CONV3X3_SPLIT_128, 128, vec ? 1.75 : 2.4, vec ? 2.4 : 3.6, 2.3);
-      if (vec)
-         offer_split(F32_CONV3X3_SPLIT_256, 256, 2.95, 3.2, 3.5);
+      offer(F32_CONV3X3_32, 32, 8, F32_CONV3X3_PATCH, {3.21, 0.82, 0.49, 0.40}, {3.56, 1.09, 0.58, 0.68});
+      offer(F32_CONV3X3_64, 64, 8, F32_CONV3X3_PATCH, {3.10, 1.09, 0.69, 0.72}, {3.67, 1.35, 0.84, 0.68});
+      offer(F32_CONV3X3_128, 128, 8, F32_CONV3X3_PATCH, {3.32, 1.59, 1.26, 0.84}, {3.75, 1.89, 1.47, 0.63});
+      offer(F32_CONV3X3_SPLIT_128, 128, 16, F32_CONV3X3_SPLIT_PATCH, {3.32, 2.61, 1.66, 1.27}, {4.32, 3.25, 2.05, 1.14});
+      offer(F32_CONV3X3_SPLIT_256, 256, 16, F32_CONV3X3_SPLIT_PATCH, {3.60, 3.70, 1.75, 4.32}, {5.38, 4.07, 2.34, 1.81});
    }
    const bool split = tile >= F32_CONV3X3_SPLIT_128;
    const long long patch = f32_conv3x3_patch(s.OH, s.OW, tile - (split ? 4000 : 3000));
    if (tile < F32_CONV3X3_32 || patch > (split ? F32_CONV3X3_SPLIT_PATCH : F32_CONV3X3_PATCH))
       return SOFIE_HIP_OK;
-   auto reciprocal = [](unsigned d) -> unsigned long long { return d <= 1 ? 0ull : (~0ull / d) + 1; };
-   const F32Conv3x3 a{X, W, images, s.Cg, s.H, s.W, s.OH, s.OW, s.pad_h, s.pad_w, plane * s.C, plane * s.Cg, M, N, K, (int)(patch + 63) / 64,
-                      reciprocal(s.OW), reciprocal(s.OH), reciprocal(s.OW + 2), reciprocal(s.OH + 2)};
+   // the images that 256 pixels touch, all their channels
+   const int near = (255 / ((long long)s.OH * s.OW) + 2) * (long long)out.Cout * out.positions * 4 < F32_BUFFER_BYTES - (1 << 20);
+   const F32Conv3x3 a{X, W, images, s.Cg, s.H, s.W, s.OH, s.OW, s.pad_h, s.pad_w, plane * s.C, plane * s.Cg, M, N, K, (int)(patch + 63) / 64, near,
+                      Divisor31(s.OW), Divisor31(s.OH), Divisor31(s.OW + 2LL), Divisor31(s.OH + 2LL)};
    *taken = true;
    hipStream_t st = ctx->stream;
    if (split) {
