@@ -136,17 +136,14 @@ struct Conv3x3Block {
          // one copy of the activations' code for four elements
 #pragma unroll 1
          for (int g = 0; g < E; g += 4) {
+            float four[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-               float one = v[e];
+            for (int e = 0; e < E; ++e)
+               four[e % 4] = e < 4 || g == e / 4 * 4 ? v[e] : four[e % 4];
+            f32_activate_all<4>(four, chain);
 #pragma unroll
-               for (int h = 4; h < E; h += 4)
-                  one = g == h ? v[h + e] : one;
-               one = apply_chain(one, chain);
-#pragma unroll
-               for (int h = 0; h < E; h += 4)
-                  v[h + e] = g == h ? one : v[h + e];
-            }
+            for (int e = 0; e < E; ++e)
+               v[e] = g == e / 4 * 4 ? four[e % 4] : v[e];
          }
       }
       if (near) {
