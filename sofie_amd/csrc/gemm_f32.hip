@@ -184,31 +184,41 @@ __global__ __launch_bounds__(CHAIN_THREADS) void gemm_chain_f32_kernel(ChainArgs
 namespace sofie_hip {
 
 // The kernel for a product of M x N x K, `batch` times: the one whose time, estimated from what each was measured to do, is the
-// shortest.  A CU multiplies a 32 x 32 block by 32 k in 0.107 us at best.  The tile kernels take 0.128 us (32 x 32 tiles), 0.245
-// (64 x 32: two blocks), 0.452 (64 x 64: four) and 1.765 (128 x 128: sixteen), a start and a store per tile, in as many rounds as
-// the tiles need over 256 CUs, and a launch.  The direct kernel costs a launch, a trip to memory per 512 k or the 10.5 TB/s at which
-// its fragments, which nothing shares, arrive, and 0.45 us per 256 tiles; `lines`: where both operands come line by line through its ring, 82 KB/us a CU and 0.35 us
-// for the first 256 tiles, 66 and 0.55 a tile where there are more (estimated / measured: 16 x 1024 x 1024 4.2 / 4.5, 1157 x 189 x 116 5.1 / 4.8).
+// shortest.  A CU multiplies a 32 x 32 block by 32 k in 0.107 us at best.  A tile kernel takes a launch, `alone` per slab of 32 k where its tiles wait for their
+// loads, and `slab` and `tile` in as many rounds as the tiles need over 256 CUs; operands that come float by float (ragged) take longer.  The direct
+// kernel takes a launch, `alone` per 128 k (16 of each wave) or, where there are many tiles, `slab` per 16 k and 256 tiles, and `tile` per 256 tiles; where both operands
+// come line by line through its ring, 82 KB/us a CU and 0.35 us for the first 256 tiles, 66 and 0.55 a tile where there are more.
+// Fitted to 490 products of 1 MFLOP to 8 GFLOP, 3 .. 4096 rows: on average 1.1 % above the best kernel's time, where one set of costs for every operand was 5.7 %
+// (571 x 170 x 1317: 28.8 us, now 10.2; 216 x 384 x 905 14.7, now 8.0).
 enum F32Tile { F32_CONV3X3_32 = 3032, F32_CONV3X3_64 = 3064, F32_CONV3X3_128 = 3128, F32_CONV3X3_SPLIT_128 = 4128, F32_CONV3X3_SPLIT_256 = 4256, F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
-static int pick_f32_tile(int M, int N, int K, int batch, bool lines, double *time_us = nullptr)
+enum F32Loads { F32_LOADS_RAGGED, F32_LOADS_RAGGED_LINES, F32_LOADS_WIDE, F32_LOADS_LINES }; // float by float, 16 bytes; lines: along k of both operands
+static F32Loads f32_loads(bool wide, bool lines) { return wide ? lines ? F32_LOADS_LINES : F32_LOADS_WIDE : lines ? F32_LOADS_RAGGED_LINES : F32_LOADS_RAGGED; }
+static int pick_f32_tile(int M, int N, int K, int batch, F32Loads loads, double *time_us = nullptr)
 {
+   struct Cost {
+      double launch, alone, slab, tile;
+   };
    auto tiles = [&](int bm, int bn) { return std::ceil((double)M / bm) * std::ceil((double)N / bn) * batch; };
-   const double slabs = std::ceil(K / 32.0), steps = std::ceil(K / 16.0);
-   auto tiled = [&](int bm, int bn, double launch, double slab, double tile) { return launch + std::ceil(tiles(bm, bn) / 256.0) * (slabs * slab + tile); };
+   const double slabs = std::ceil(K / 32.0), steps = std::ceil(K / 16.0), each = tiles(16, 16) / 256.0;
    int best = F32_DIRECT;
-   double least = 2.0 + std::max(1.35 * std::ceil(steps / 32.0), tiles(16, 16) * steps * 2048.0 / 10.5e6) + 0.45 * tiles(16, 16) / 256.0;
-   if (lines) {
-      const double each = tiles(16, 16) / 256.0, rounds = each <= 1.0 ? 1.0 : 0.5 * (each + std::ceil(each));
+   double least;
+   if (loads == F32_LOADS_LINES) {
+      const double rounds = each <= 1.0 ? 1.0 : 0.5 * (each + std::ceil(each));
       least = 2.3 + rounds * (each <= 1.0 ? 0.35 + 128.0 * K / 82e3 : 0.55 + 128.0 * K / 66e3);
+   } else {
+      const Cost c = loads == F32_LOADS_WIDE ? Cost{3.16, 0.34, 0.048, 0.514} : loads == F32_LOADS_RAGGED ? Cost{3.2, 0.72, 0.110, 0.45} : Cost{2.91, 1.09, 0.160, 0.37};
+      least = c.launch + std::max(c.alone * std::ceil(steps / 8.0), c.slab * each * steps) + c.tile * each;
    }
-   auto offer = [&](int tile, double t) {
+   auto offer = [&](int tile, int bm, int bn, Cost whole, Cost ragged) {
+      const Cost c = loads <= F32_LOADS_RAGGED_LINES ? ragged : whole;
+      const double t = c.launch + std::max(slabs * c.alone, std::ceil(tiles(bm, bn) / 256.0) * (slabs * c.slab + c.tile));
       if (t < least)
          least = t, best = tile;
    };
-   offer(F32_TILE_32, tiled(32, 32, 3.65, 0.128, 0.25));
-   offer(F32_TILE_64x32, tiled(64, 32, 3.9, 0.245, 0.5));
-   offer(F32_TILE_64, tiled(64, 64, 3.3, 0.452, 1.6));
-   offer(F32_TILE_128, tiled(128, 128, 7.0, 1.765, 4.0));
+   offer(F32_TILE_32, 32, 32, {3.04, 0.11, 0.120, 0.49}, {3.59, 0.033, 0.138, 0.55});
+   offer(F32_TILE_64x32, 64, 32, {3.36, 0.22, 0.232, 0.72}, {4.37, 0.255, 0.285, 0.84});
+   offer(F32_TILE_64, 64, 64, {3.13, 0.35, 0.457, 1.2}, {3.88, 0.10, 0.467, 1.65});
+   offer(F32_TILE_128, 128, 128, {5.6, 0.05, 1.78, 2.2}, {5.1, 0.23, 1.94, 6.1});
    if (time_us)
       *time_us = least;
    return best;
@@ -244,7 +254,7 @@ static int launch_f32_product(sofie_hip_ctx *ctx, const ASRC &A, const BSRC &B, 
       tile = F32_TILE_64;
    constexpr bool CONV = ASRC::kLeastRows == 64;
    if (!tile)
-      tile = CONV ? pick_f32_conv_tile(M, N, K, batch) : pick_f32_tile(M, N, K, batch, ASRC::KC && BSRC::KC && ASRC::VEC == 4 && BSRC::VEC == 4);
+      tile = CONV ? pick_f32_conv_tile(M, N, K, batch) : pick_f32_tile(M, N, K, batch, f32_loads(ASRC::VEC == 4 && BSRC::VEC == 4, ASRC::KC && BSRC::KC));
    if (tile >= F32_CONV3X3_32 || (CONV ? tile == F32_TILE_32 || tile == F32_TILE_128 : tile == F32_TILE_128x32))
       tile = F32_TILE_64; // a request for a tile that the other kind of product has
    if constexpr (CONV) {
@@ -549,11 +559,14 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
    if (ctx->opt.f32_chain == 1) {
       first = 0;
    } else if (ctx->opt.f32_chain < 0 && M >= 1 && M <= 256) {
-      auto lines = [&](int l) { return layers[l].transB && !layers[l].transA && layers[l].K % 4 == 0; };
+      auto loads = [&](int l) {
+         const auto &d = layers[l];
+         return f32_loads((d.transA ? d.M : d.K) % 4 == 0 && (d.transB ? d.K : d.N) % 4 == 0, d.transB && !d.transA);
+      };
       double before = 0.0, least = 0.0;
       for (int l = 0; l < count; ++l) {
          double t = 0.0;
-         pick_f32_tile(M, layers[l].N, layers[l].K, 1, lines(l), &t);
+         pick_f32_tile(M, layers[l].N, layers[l].K, 1, loads(l), &t);
          least += std::max(t, 3.0);
       }
       for (int s = 0; s + 2 <= count; ++s) {
@@ -566,7 +579,7 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
          together = before + 2.3 + together * (M <= 64 ? 1.0 : 1.8);
          if (together < least)
             least = together, first = s;
-         pick_f32_tile(M, layers[s].N, layers[s].K, 1, lines(s), &t);
+         pick_f32_tile(M, layers[s].N, layers[s].K, 1, loads(s), &t);
          before += std::max(t, 3.0);
       }
    }
