@@ -1,8 +1,9 @@
 // fp32 products on the matrix cores (v_mfma_f32_32x32x2_f32, v_mfma_f32_16x16x4_f32: full fp32 multiply-adds at twice the rate of the unpacked vector
-// instructions), for Gemm / MatMul and for convolutions as implicit GEMM.  Two kernels:
-//   f32_tile_kernel     a workgroup of four waves owns a BM x BN tile; slabs of k go straight from memory into a ring in LDS
-//   f32_direct_kernel   small products: a workgroup owns one small tile and its waves split the reduction; every fragment is
-//                       loaded from memory into the registers the MFMA reads, with many loads in flight and no LDS in the loop
+// instructions), for Gemm / MatMul and for convolutions as implicit GEMM.  Three kernels:
+//   f32_tile_kernel          a workgroup of four or eight waves owns a BM x BN tile; slabs of k go straight from memory into a ring in LDS
+//   f32_direct_kernel        small products: a workgroup owns one small tile and its waves split the reduction; every fragment is
+//                            loaded from memory into the registers the MFMA reads, with many loads in flight and no LDS in the loop
+//   f32_direct_ring_kernel   the same where both operands have 16-byte rows along k: whole lines through a ring in LDS per wave
 //
 // Both feed an MFMA the n side as first operand and the m side as second, so a lane ends up with 4 consecutive columns n of one
 // row m.  Four MFMAs take four consecutive k from every lane: which k a lane supplies to which MFMA only has to agree between the
