@@ -1,7 +1,7 @@
 // fp32 3 x 3 convolution (stride 1, no dilation, two spatial axes) on the bf16 matrix cores.
 //
-// Every fp32 value is the sum of three bf16 values, x = h + m + l (h = bf16(x), m = bf16(x - h), l = bf16(x - h - m): the remainders are exact, and what is
-// left behind l is at most 2^-26 of x), and a product of two such sums is taken as the six terms down to 2^-17 of it:
+// Every fp32 value from 2^-110 on is the sum of three bf16 values, x = h + m + l (h = bf16(x), m = bf16(x - h), l = x - h - m; |m| <= 2^-8 |x|, |l| <= 2^-17 |x|;
+// Henry, Tang, Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations", ARITH 2019), and a product of two such sums is taken as the six terms down to 2^-17 of it:
 //   a b = ah bh + (ah bm + am bh) + (ah bl + am bm + al bh),       left out: am bl + al bm + al bl < 2^-24 a b.
 // bf16 products are exact in the fp32 accumulators, and v_mfma_f32_32x32x16_bf16 multiplies 16 k in 32 cycles where v_mfma_f32_32x32x2_f32 needs
 // 512: the six terms cost 0.375 of the fp32 instructions.  The leading products and the other terms are summed apart, so that an accumulator is rounded
@@ -14,9 +14,13 @@
 // 64 -> 64 the matrix cores are busy in half of the cycles at 1.75 GHz of 2.4 (power); 8 us of the launch are the first slab's load, the store and the launch
 // itself, which nothing overlaps.
 //
-// Exceptions: bf16 has the exponents of fp32, so nothing overflows or vanishes that would not in fp32, except that a value within 2^-8 of the largest
-// rounds to an infinity, and that the remainders of an infinity are NaN.  Both end in a sum that is not finite; a wave that finds one among its sums
-// computes them again with fp32 instructions straight from memory, which gives IEEE's infinities and NaN.
+// Exceptions: bf16 has the exponents of fp32, and the matrix cores keep subnormal numbers, so pieces hold every multiple of 2^-133.  Three things do not fit:
+// a value within 2^-8 of the largest rounds to an infinity, the remainders of an infinity are NaN, and the last bits of a value below 2^-110 are lost.  The first two
+// end in a sum that is not finite; the last shows where a value is split, as a subnormal third piece.  A wave whose sums are not finite, and a workgroup that met
+// such a piece, compute their sums again with fp32 instructions straight from memory.  (The matrix cores' treatment of subnormals was measured: subnormal
+// operands, products and sums of v_mfma_f32_32x32x16_bf16 come out exact.)  Telling costs an instruction per value: 64 -> 64 at 32 x 32 takes 1.3 us longer.  Summing
+// again, for every tile of 64 images of 32 x 32: 32 -> 64 channels 20.6 -> 57 us, 64 -> 64 31 -> 105 (the fp32 kernel takes 43); two channels at a time with their
+// loads in flight, where eight k with their index arithmetic took 132.
 #pragma once
 #include "f32_conv3x3.hpp"
 
@@ -141,10 +145,14 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a,
          }
       }
    };
+   bool small = false; // a remainder was met that the third piece may not hold
    auto split = [&]() {
       auto pieces = [&](float (&x)[8], char *at, int step) {
          *(v4u *)at = f32_next_piece<0>(x);
          *(v4u *)(at + step) = f32_next_piece<1>(x);
+#pragma unroll
+         for (int e = 0; e < 8; ++e)
+            small |= __builtin_amdgcn_classf(x[e], 0x90); // a subnormal number of either sign
          *(v4u *)(at + 2 * step) = f32_next_piece<2>(x);
       };
 #pragma unroll
@@ -244,29 +252,45 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a,
          acc[i][e] += low[i][e];
          finite = __builtin_fmaf(acc[i][e], 0.0f, finite);
       }
-   if (__builtin_amdgcn_ballot_w64(finite != 0.0f) != 0) {
+   // the raw weights of the last slab have been split by every wave: their place takes a word per wave
+   int *const cut = (int *)(split_lds + S::RAW_AT);
+   const bool mine = __builtin_amdgcn_ballot_w64(small) != 0;
+   if (lane == 0)
+      cut[wave] = mine;
+   meet();
+   const bool any = __builtin_amdgcn_readfirstlane(cut[0] | cut[1] | cut[2] | cut[3]) != 0;
+   if (any || __builtin_amdgcn_ballot_w64(finite != 0.0f) != 0) {
       clear(acc);
-      const float *row = a.W + (long long)(n0 + c < a.N ? n0 + c : a.N - 1) * a.K;
-#pragma unroll 1
-      for (int k0 = 0; k0 < a.K; k0 += 8) {
-         float u[4], v[MT][4];
+      int at[MT][9]; // bytes from `base` of this lane's pixels at the nine positions, of channel lk
 #pragma unroll
-         for (int j = 0; j < 4; ++j) {
-            const int k = k0 + lk * 4 + j, ch = k / 9, r = k - ch * 9, ky = r / 3, kx = r - ky * 3;
-            u[j] = k < a.K ? row[k] : 0.0f;
+      for (int i = 0; i < MT; ++i) {
+         const int m = m0 + wave * TM + i * 32 + c, mm = m < a.M ? m : a.M - 1;
+         const int line = quotient(mm, a.by_ow), image = quotient(line, a.by_oh);
 #pragma unroll
-            for (int i = 0; i < MT; ++i) {
-               const int m = m0 + wave * TM + i * 32 + c, mm = m < a.M ? m : a.M - 1;
-               const int line = quotient(mm, a.by_ow), image = quotient(line, a.by_oh);
-               const int iy = line - image * a.OH + ky - a.pad_h, ix = mm - line * a.OW + kx - a.pad_w;
-               v[i][j] = k < a.K && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.Wd ? a.X[image * a.image + ((long long)ch * a.H + iy) * a.Wd + ix] : 0.0f;
-            }
+         for (int t = 0; t < 9; ++t) {
+            const int iy = line - image * a.OH + t / 3 - a.pad_h, ix = mm - line * a.OW + t % 3 - a.pad_w;
+            const bool inside = (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.Wd;
+            at[i][t] = inside ? (int)(((image - image0) * a.image + (long long)iy * a.Wd + ix) * 4) + lk * plane_bytes : F32_OUTSIDE;
          }
+      }
+      const int row = n0 + c < a.N ? (c * a.K + lk * 9) * 4 : F32_OUTSIDE;
+#pragma unroll 1
+      for (int ch = 0; ch < a.C; ch += 2) { // lane half lk multiplies channel ch + lk
+         const bool there = ch + lk < a.C;
+         float u[9], v[MT][9];
 #pragma unroll
-         for (int j = 0; j < 4; ++j)
+         for (int t = 0; t < 9; ++t) {
+            u[t] = f32_buffer_read(weights, there && row != F32_OUTSIDE ? row + t * 4 : F32_OUTSIDE, ch * 36);
 #pragma unroll
             for (int i = 0; i < MT; ++i)
-               acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(u[j], v[i][j], acc[i], 0, 0, 0);
+               v[i][t] = f32_buffer_read(base, there ? at[i][t] : F32_OUTSIDE, ch * plane_bytes);
+         }
+         __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+         for (int t = 0; t < 9; ++t)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+               acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(u[t], v[i][t], acc[i], 0, 0, 0);
       }
    }
 

@@ -1,6 +1,6 @@
 """The fp32 3 x 3 convolution that multiplies bf16 pieces (f32_conv3x3_split.hpp), forced by the context option "f32_tile", at the edges of its tiles (128 or 256
 pixels, 32 output channels), of its slabs (16 channels) and of its patch (360 places), against sums in 64 bits: the error is that of fp32 sums, at any
-scale of the inputs, and infinities and NaN are where IEEE arithmetic has them."""
+scale of the inputs down to the smallest subnormal number, and infinities and NaN are where IEEE arithmetic has them."""
 import ctypes as C
 
 import numpy as np
@@ -83,3 +83,36 @@ def test_nan_infinity_and_the_largest_numbers(rt, tile, case):
     got = run(rt, X, Wt, None, (1, 1, 1, 1))
     assert np.all(np.abs(want[np.isfinite(want)]) < np.finfo(np.float32).max)
     same_as_ieee(got, want, most)
+
+
+SMALL = [(1e-33, 1e9), (1e-36, 1e12), (1e37, 1e-37), (3e-42, 1e30)]    # of the inputs, of the weights: results are normal numbers
+
+
+@pytest.mark.parametrize("tile", [4128, 4256], indirect=True)
+@pytest.mark.parametrize("scales", SMALL)
+@pytest.mark.parametrize("case", [(3, 15, 9, 7, 31, (0, 0, 0, 0), 1), (2, 17, 13, 11, 33, (1, 0, 2, 1), 1), (2, 20, 10, 12, 66, (2, 2, 2, 2), 2), (17, 16, 4, 4, 32, (1, 1, 1, 1), 1)])
+def test_numbers_that_pieces_do_not_hold(rt, tile, case, scales):
+    """bf16 holds multiples of 2^-133: the last bits of values below 2^-110 (7.7e-34) are in no piece."""
+    N, Cc, H, W, Cout, pads, group = case
+    X = (util.normal(77, N * Cc * H * W).astype(np.float64) * scales[0]).astype(np.float32).reshape(N, Cc, H, W)
+    Wt = (util.normal(78, Cout * Cc // group * 9, 0.3).astype(np.float64) * scales[1]).astype(np.float32).reshape(Cout, Cc // group, 3, 3)
+    p = products(X, Wt, pads, group)
+    got = run(rt, X, Wt, None, pads, group)
+    # fp32 multiply-adds, two products at a time, each within 2^-23 of the magnitudes so far
+    n = 9 * (Cc // group)
+    assert np.all(np.abs(got - p.sum(4)) <= n * 2.0 ** -23 * np.abs(p).sum(4))
+    # rounding errors cancel in part: a sequential fp32 sum comes to 0.45 of this, pieces cut at 2^-133 to 50 and more from 1e-36 on
+    assert np.linalg.norm(got - p.sum(4)) <= 2.0 ** -21 * np.linalg.norm(p.sum(4))
+
+
+@pytest.mark.parametrize("tile", [4128, 4256], indirect=True)
+def test_one_small_number_that_counts(rt, tile):
+    """Among ordinary numbers, one input and one weight that pieces cut, each the only thing in its sums."""
+    X, Wt = util.normal(79, 2 * 18 * 81).reshape(2, 18, 9, 9), np.zeros((34, 18, 3, 3), np.float32)
+    X[0, 17, 4, 4], X[:, 3] = np.float32(1.2345678e-37), 0
+    Wt[33, 17, 1, 1] = np.float32(7.654321e35)             # 9.4e-2 at the one pixel, large numbers elsewhere
+    Wt[5, 2, 0, 2] = np.float32(1.2345678e-38)
+    X[1, 2] *= np.float32(1e37)
+    p = products(X, Wt, (1, 1, 1, 1))
+    got = run(rt, X, Wt, None, (1, 1, 1, 1))
+    assert np.all(np.abs(got - p.sum(4)) <= 2.0 ** -23 * np.abs(p).sum(4) + 2.0 ** -149)
