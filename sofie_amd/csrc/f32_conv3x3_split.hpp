@@ -1,18 +1,18 @@
 // fp32 3 x 3 convolution (stride 1, no dilation, two spatial axes) on the bf16 matrix cores.
 //
 // Every fp32 value from 2^-110 on is the sum of three bf16 values, x = h + m + l (h = bf16(x), m = bf16(x - h), l = x - h - m; |m| <= 2^-8 |x|, |l| <= 2^-17 |x|;
-// Henry, Tang, Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations", ARITH 2019), and a product of two such sums is taken as the six terms down to 2^-17 of it:
-//   a b = ah bh + (ah bm + am bh) + (ah bl + am bm + al bh),       left out: am bl + al bm + al bl < 2^-24 a b.
+// Henry, Tang, Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations", ARITH 2019), and a product of two such sums is taken as eight terms:
+//   a b = ah bh + (ah bm + am bh) + (ah bl + am bm + al bh) + (am bl + al bm),       left out: al bl <= 2^-34 a b.
+// (Without the last two, each up to 2^-25 of the product, a sum with one product that counts would be known to 2^-23 only, where fp32 gives 2^-24.)
 // bf16 products are exact in the fp32 accumulators, and v_mfma_f32_32x32x16_bf16 multiplies 16 k in 32 cycles where v_mfma_f32_32x32x2_f32 needs
-// 512: the six terms cost 0.375 of the fp32 instructions.  The leading products and the other terms are summed apart, so that an accumulator is rounded
-// once per 16 k.
+// 512: the eight terms cost half of the fp32 instructions.  The leading products and the other terms are summed apart: an accumulator of leading products is
+// rounded once per 16 k and instruction, by up to 1.6 2^-24 of the magnitudes in it (measured; 1.9 per 2 k for the fp32 instruction).
 //
 // What the pieces cost is vector instructions (5.5 per value) and LDS (6 bytes written per value, at 79 B/clk): a 3 x 3 convolution uses every value of its
 // input patch nine times, which pays for both.  (A plain product of 64 x 64 tiles uses a value twice per wave: 20 - 27 us where fp32 takes 20 - 32.)
-// 64 images of 32 x 32, us, the fp32 kernel (with the stores it had) -> this one: 32 -> 64 channels 29.1 -> 20.1, 64 -> 64 49.7 -> 31.5 (with a residual 51.1 ->
-// 32.1); 128 -> 128 at 16 x 16 49.2 -> 36.9; 48 images of 37 x 37, 32 -> 96 48.9 -> 38.9.  Error of 64 -> 64 against 64 bits: 4.2e-7 -> 1.4e-7 of the result.  On
-// 64 -> 64 the matrix cores are busy in half of the cycles at 1.75 GHz of 2.4 (power); 8 us of the launch are the first slab's load, the store and the launch
-// itself, which nothing overlaps.
+// 64 images of 32 x 32, us, the fp32 kernel's best tile -> this one: 32 -> 64 channels 26.1 -> 22.8, 64 -> 64 43.4 -> 37.0 (with a residual 47.0 -> 37.7); 128 -> 128
+// at 16 x 16 45.2 -> 40.2; 48 images of 37 x 37, 32 -> 96 44.3 -> 42.9.  With six terms 20.6, 31.0 (32.3), 35.7, 39.4.  Error of 64 -> 64 against 64 bits: 2.4e-7 to
+// 3.4e-7 -> 1.0e-7 of the result.
 //
 // Exceptions: bf16 has the exponents of fp32, and the matrix cores keep subnormal numbers, so pieces hold every multiple of 2^-133.  Three things do not fit:
 // a value within 2^-8 of the largest rounds to an infinity, the remainders of an infinity are NaN, and the last bits of a value below 2^-110 are lost.  The first two
@@ -214,8 +214,8 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a,
          if constexpr (t < 8)
             read(std::integral_constant<int, t + 1>{});
          __builtin_amdgcn_sched_barrier(0);
-         constexpr int TERM[6][2] = {{0, 0}, {1, 0}, {0, 1}, {1, 1}, {2, 0}, {0, 2}};
-         static_for<6>([&](auto qc) {
+         constexpr int TERM[8][2] = {{0, 0}, {2, 1}, {1, 2}, {2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}};
+         static_for<8>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
             auto &sums = q == 0 ? acc : low;
 #pragma unroll

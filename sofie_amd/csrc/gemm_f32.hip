@@ -294,8 +294,8 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
       tile = F32_CONV3X3_128; // slabs of four channels; half of any other kernel's slab would be zeros
    } else if (!tile) {
       // us: a launch; a slab (8 channels, 16 of the split kernel) of a CU whose tiles wait for their loads, and of one with several tiles at work; a tile.  The
-      // second set is for weights that come float by float.  Fitted to 156 layers from 1 image of 6 x 6 to 64 of 64 x 64, 6 to 130 channels; holds to a sixth, and
-      // costs 1 % of the best kernel's time on average over those layers, 4 % the most but for three.
+      // second set is for weights that come float by float.  Fitted to 156 layers (the split kernel's to 230 others) from 1 image of 6 x 6 to 64 of 64 x 64, 5 to 130
+      // channels; holds to a sixth, the split kernel's to a quarter, and costs 0.8 % of the best of these kernels on average over the 260 layers, 14 % the most.
       double least = 1e30;
       struct Cost {
          double launch, alone, slab, each;
@@ -310,8 +310,8 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
       offer(F32_CONV3X3_32, 32, 8, F32_CONV3X3_PATCH, {3.21, 0.82, 0.49, 0.40}, {3.56, 1.09, 0.58, 0.68});
       offer(F32_CONV3X3_64, 64, 8, F32_CONV3X3_PATCH, {3.10, 1.09, 0.69, 0.72}, {3.67, 1.35, 0.84, 0.68});
       offer(F32_CONV3X3_128, 128, 8, F32_CONV3X3_PATCH, {3.32, 1.59, 1.26, 0.84}, {3.75, 1.89, 1.47, 0.63});
-      offer(F32_CONV3X3_SPLIT_128, 128, 16, F32_CONV3X3_SPLIT_PATCH, {3.32, 2.61, 1.66, 1.27}, {4.32, 3.25, 2.05, 1.14});
-      offer(F32_CONV3X3_SPLIT_256, 256, 16, F32_CONV3X3_SPLIT_PATCH, {3.60, 3.70, 1.75, 4.32}, {5.38, 4.07, 2.34, 1.81});
+      offer(F32_CONV3X3_SPLIT_128, 128, 16, F32_CONV3X3_SPLIT_PATCH, {4.08, 3.00, 2.14, 0.95}, {4.91, 3.79, 2.36, 1.11});
+      offer(F32_CONV3X3_SPLIT_256, 256, 16, F32_CONV3X3_SPLIT_PATCH, {5.04, 1.84, 4.24, 0.16}, {6.41, 4.74, 4.16, 0.73});
    }
    const bool split = tile >= F32_CONV3X3_SPLIT_128;
    const long long patch = f32_conv3x3_patch(s.OH, s.OW, tile - (split ? 4000 : 3000));

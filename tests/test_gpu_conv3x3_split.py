@@ -44,8 +44,25 @@ def products(X, Wt, pads, group=1):
     return whole.reshape(*whole.shape[:4], -1)
 
 
+def in_pieces(tile, OH, OW):
+    """Whether the kernel takes images of OH x OW results at this tile: its patch, the rows a tile touches, two more and two per image that it runs into, is at most
+    360 places.  256 pixels: of 8, 16 or 32 columns."""
+    bm, plane = tile - 4000, OH * OW
+    rows = bm // OW if bm % OW == 0 else (bm - 2 + OW) // OW + 1
+    images = 0 if plane % bm == 0 else (bm - 2 + plane) // plane
+    return (rows + 2 + 2 * images) * (OW + 2) <= 360
+
+
+def roundings(tile, Cg, OH, OW):
+    """Errors of a sum, in 2^-24 of the sum of magnitudes.  In pieces: an instruction per 16 channels and kernel position for the leading products, each within 2 (1.6
+    measured) of the magnitudes so far, seven for terms of at most 2^-7 of them together (2 2^-8 + 3 2^-16 + ...), and the join.  In fp32: one per two products."""
+    return 2 * 9 * -(-Cg // 16) * (1 + 7 * 2.0 ** -7 * 1.02) + 1 if in_pieces(tile, OH, OW) else 2 * (9 * Cg // 2 + 4)
+
+
 CASES = [(1, 1, 3, 3, 1, (1, 1, 1, 1), 1), (3, 15, 9, 7, 31, (0, 0, 0, 0), 1), (2, 17, 13, 11, 33, (1, 0, 2, 1), 1), (1, 32, 16, 16, 64, (1, 1, 1, 1), 1), (5, 36, 8, 33, 20, (1, 1, 1, 1), 1),
-         (2, 20, 10, 12, 66, (2, 2, 2, 2), 2), (17, 16, 4, 4, 32, (1, 1, 1, 1), 1), (1, 33, 5, 118, 3, (1, 1, 1, 1), 1)]
+         (2, 20, 10, 12, 66, (2, 2, 2, 2), 2), (17, 16, 4, 4, 32, (1, 1, 1, 1), 1), (1, 33, 5, 118, 3, (1, 1, 1, 1), 1),
+         # taken at 256 pixels: tiles across images, a last one that is not filled, odd channels, groups
+         (3, 15, 17, 16, 31, (1, 1, 1, 1), 1), (1, 33, 18, 18, 20, (0, 0, 0, 0), 1), (2, 17, 24, 32, 33, (1, 1, 1, 1), 1), (2, 20, 34, 9, 66, (1, 0, 1, 1), 2)]
 
 
 @pytest.mark.parametrize("tile", [4128, 4256], indirect=True)
@@ -59,17 +76,15 @@ def test_convolutions_around_tile_edges(rt, tile, case, scale):
     p = products(X, Wt, pads, group)
     r = (util.normal(73, p[..., 0].size) * np.float32(scale)).reshape(p.shape[:4]).astype(np.float32)
     got = run(rt, X, Wt, b, pads, group, R.ACT_LEAKYRELU, r)
-    # Sums of n terms, the products exact and the six-term form of a product within 2^-23 of it, every addition within 2^-24 of the magnitudes so far:
-    # (n + 2) 2^-24 of the sum of magnitudes, n = one addition per 16 channels and kernel position in each of five chains, bias, residual and their join
-    n = 5 * 9 * -(-Cc // group // 16) + 4
     want = p.sum(4) + b.reshape(1, -1, 1, 1) + r
     most = np.abs(p).sum(4) + np.abs(b).reshape(1, -1, 1, 1) + np.abs(r)
     want = np.where(want >= 0, want, np.float64(np.float32(0.1)) * want)
-    assert np.all(np.abs(got - want) <= (n + 2) * 2.0 ** -24 * most)
+    # bias, residual and activation: another rounding each
+    assert np.all(np.abs(got - want) <= (roundings(tile, Cc // group, *p.shape[2:4]) + 3) * 2.0 ** -24 * most)
 
 
 @pytest.mark.parametrize("tile", [4128, 4256], indirect=True)
-@pytest.mark.parametrize("case", [(2, 18, 13, 11, 35), (1, 3, 40, 41, 5)])
+@pytest.mark.parametrize("case", [(2, 18, 13, 11, 35), (1, 3, 40, 41, 5), (2, 19, 17, 16, 35)])
 def test_nan_infinity_and_the_largest_numbers(rt, tile, case):
     N, Cc, H, W, Cout = case
     X = with_nonfinite(util.normal(74, N * Cc * H * W), 75).reshape(N, Cc, H, W)
@@ -90,7 +105,8 @@ SMALL = [(1e-33, 1e9), (1e-36, 1e12), (1e37, 1e-37), (3e-42, 1e30)]    # of the 
 
 @pytest.mark.parametrize("tile", [4128, 4256], indirect=True)
 @pytest.mark.parametrize("scales", SMALL)
-@pytest.mark.parametrize("case", [(3, 15, 9, 7, 31, (0, 0, 0, 0), 1), (2, 17, 13, 11, 33, (1, 0, 2, 1), 1), (2, 20, 10, 12, 66, (2, 2, 2, 2), 2), (17, 16, 4, 4, 32, (1, 1, 1, 1), 1)])
+@pytest.mark.parametrize("case", [(3, 15, 9, 7, 31, (0, 0, 0, 0), 1), (2, 17, 13, 11, 33, (1, 0, 2, 1), 1), (2, 20, 10, 12, 66, (2, 2, 2, 2), 2), (17, 16, 4, 4, 32, (1, 1, 1, 1), 1),
+                                  (3, 15, 17, 16, 31, (1, 1, 1, 1), 1), (2, 20, 34, 9, 66, (1, 0, 1, 1), 2)])
 def test_numbers_that_pieces_do_not_hold(rt, tile, case, scales):
     """bf16 holds multiples of 2^-133: the last bits of values below 2^-110 (7.7e-34) are in no piece."""
     N, Cc, H, W, Cout, pads, group = case
@@ -105,10 +121,33 @@ def test_numbers_that_pieces_do_not_hold(rt, tile, case, scales):
     assert np.linalg.norm(got - p.sum(4)) <= 2.0 ** -21 * np.linalg.norm(p.sum(4))
 
 
+def piece_rich(seed, n):
+    """Numbers from 1 on whose second and third bf16 pieces are near their largest, 2^-8 and 2^-17 (and of either sign)."""
+    sign = np.where(util.normal(seed, n) < 0, -1.0, 1.0)
+    rest = 1 - np.abs(util.normal(seed + 1, n)) % 0.1, 1 - np.abs(util.normal(seed + 2, n)) % 0.1
+    whole = 1 + np.floor(np.abs(util.normal(seed + 3, n)) % 1 * 8) / 128
+    return (whole + 2.0 ** -8 * rest[0] * sign + 2.0 ** -17 * rest[1]).astype(np.float32)
+
+
+@pytest.mark.parametrize("tile", [4128, 4256], indirect=True)
+@pytest.mark.parametrize("channels", [16, 36])
+def test_single_products(rt, tile, channels):
+    """One nonzero weight per output channel, at every kernel position and in every slab: each result is one product, within 2^-24 of itself but for what the
+    matrix cores lose of the small terms (seven sums of at most 2^-7 of it, 2^-23 of each) and the one left out (2^-34).  On the CPU, leaving out any one of the
+    eight terms misses this by a quarter and more."""
+    out = 9 * -(-channels // 4)
+    X = piece_rich(90, 2 * channels * 342).reshape(2, channels, 19, 18)
+    Wt, n = np.zeros((out, channels, 3, 3), np.float32), np.arange(out)
+    Wt[n, (n // 9 * 4 + n % 4) % channels, n % 9 // 3, n % 3] = piece_rich(94, out)
+    want = products(X, Wt, (0, 0, 0, 0)).sum(4)
+    got = run(rt, X, Wt, None, (0, 0, 0, 0))
+    assert np.all(np.abs(got - want) <= 2.0 ** -24 * (1 + 7 * 2.0 ** -6 + 2.0 ** -10) * np.abs(want))
+
+
 @pytest.mark.parametrize("tile", [4128, 4256], indirect=True)
 def test_one_small_number_that_counts(rt, tile):
     """Among ordinary numbers, one input and one weight that pieces cut, each the only thing in its sums."""
-    X, Wt = util.normal(79, 2 * 18 * 81).reshape(2, 18, 9, 9), np.zeros((34, 18, 3, 3), np.float32)
+    X, Wt = util.normal(79, 2 * 18 * 272).reshape(2, 18, 17, 16), np.zeros((34, 18, 3, 3), np.float32)
     X[0, 17, 4, 4], X[:, 3] = np.float32(1.2345678e-37), 0
     Wt[33, 17, 1, 1] = np.float32(7.654321e35)             # 9.4e-2 at the one pixel, large numbers elsewhere
     Wt[5, 2, 0, 2] = np.float32(1.2345678e-38)
