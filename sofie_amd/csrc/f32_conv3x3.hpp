@@ -40,11 +40,17 @@ inline long long f32_conv3x3_patch(int OH, int OW, int bm)
    return (rows + 2 + 2 * images) * (OW + 2);
 }
 
-// A float of a buffer of which `base` is the (scalar) start; from `bytes` on, and at F32_OUTSIDE, it reads as zero.
-__device__ __forceinline__ float f32_buffer_read(const void *base, int offset, int scalar_offset, int bytes = (int)F32_BUFFER_BYTES)
+// A float of a buffer of which `base` is the (scalar) start; F32_OUTSIDE reads as zero.
+__device__ __forceinline__ float f32_buffer_read(const void *base, int offset, int scalar_offset)
+{
+   const __amdgpu_buffer_rsrc_t buffer = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)F32_BUFFER_BYTES, 0x00020000);
+   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buffer, offset, scalar_offset, 0));
+}
+// A float of a buffer of `bytes`, zero from its end on.  No scalar offset: the check against the end leaves it out.
+__device__ __forceinline__ float f32_bounded_read(const void *base, int offset, int bytes)
 {
    const __amdgpu_buffer_rsrc_t buffer = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, bytes, 0x00020000);
-   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buffer, offset, scalar_offset, 0));
+   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buffer, offset, 0, 0));
 }
 __device__ __forceinline__ void f32_buffer_store(float v, const void *base, int offset, int scalar_offset)
 {
@@ -110,7 +116,7 @@ struct Conv3x3Block {
       if (B) {
 #pragma unroll
          for (int e = 0; e < E; ++e)
-            bias[e] = f32_buffer_read(B, lk * 16 + (channel(e) - e0 * 2) * 4, e0 * 8, N * 4);
+            bias[e] = f32_bounded_read(B, lk * 16 + channel(e) * 4, N * 4);
       }
       if (R) {
          if (near) {
