@@ -191,6 +191,18 @@ namespace sofie_hip {
 // Fitted to 490 products of 1 MFLOP to 8 GFLOP, 3 .. 4096 rows: on average 1.1 % above the best kernel's time, where one set of costs for every operand was 5.7 %
 // (571 x 170 x 1317: 28.8 us, now 10.2; 216 x 384 x 905 14.7, now 8.0).
 enum F32Tile { F32_CONV3X3_32 = 3032, F32_CONV3X3_64 = 3064, F32_CONV3X3_128 = 3128, F32_CONV3X3_SPLIT_128 = 4128, F32_CONV3X3_SPLIT_256 = 4256, F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
+// Pixels of a tile of the 3 x 3 convolution kernels; 0 for any other kernel.
+static int conv3x3_pixels(int tile)
+{
+   switch (tile) {
+   case F32_CONV3X3_32: return 32;
+   case F32_CONV3X3_64: return 64;
+   case F32_CONV3X3_128:
+   case F32_CONV3X3_SPLIT_128: return 128;
+   case F32_CONV3X3_SPLIT_256: return 256;
+   default: return 0;
+   }
+}
 enum F32Loads { F32_LOADS_RAGGED, F32_LOADS_RAGGED_LINES, F32_LOADS_WIDE, F32_LOADS_LINES }; // float by float, 16 bytes; lines: along k of both operands
 static F32Loads f32_loads(bool wide, bool lines) { return wide ? lines ? F32_LOADS_LINES : F32_LOADS_WIDE : lines ? F32_LOADS_RAGGED_LINES : F32_LOADS_RAGGED; }
 static int pick_f32_tile(int M, int N, int K, int batch, F32Loads loads, double *time_us = nullptr)
@@ -255,7 +267,7 @@ static int launch_f32_product(sofie_hip_ctx *ctx, const ASRC &A, const BSRC &B, 
    constexpr bool CONV = ASRC::kLeastRows == 64;
    if (!tile)
       tile = CONV ? pick_f32_conv_tile(M, N, K, batch) : pick_f32_tile(M, N, K, batch, f32_loads(ASRC::VEC == 4 && BSRC::VEC == 4, ASRC::KC && BSRC::KC));
-   if (tile >= F32_CONV3X3_32 || (CONV ? tile == F32_TILE_32 || tile == F32_TILE_128 : tile == F32_TILE_128x32))
+   if (conv3x3_pixels(tile) || (CONV ? tile == F32_TILE_32 || tile == F32_TILE_128 : tile == F32_TILE_128x32))
       tile = F32_TILE_64; // a request for a tile that the other kind of product has
    if constexpr (CONV) {
       switch (tile) {
@@ -300,22 +312,26 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
       struct Cost {
          double launch, alone, slab, each;
       };
-      auto offer = [&](int which, int bm, int channels, long long room, Cost wide, Cost narrow) {
+      auto offer = [&](int which, int channels, long long room, Cost wide, Cost narrow) {
+         const int bm = conv3x3_pixels(which);
          const Cost cost = vec ? wide : narrow;
          const double rounds = std::ceil((double)((M + bm - 1) / bm) * ((N + 31) / 32) * group / 256.0), slabs = (s.Cg + channels - 1) / channels;
          const double t = cost.launch + std::max(slabs * cost.alone, rounds * (slabs * cost.slab + cost.each));
          if (f32_conv3x3_patch(s.OH, s.OW, bm) <= room && t < least)
             least = t, tile = which;
       };
-      offer(F32_CONV3X3_32, 32, 8, F32_CONV3X3_PATCH, {3.21, 0.82, 0.49, 0.40}, {3.56, 1.09, 0.58, 0.68});
-      offer(F32_CONV3X3_64, 64, 8, F32_CONV3X3_PATCH, {3.10, 1.09, 0.69, 0.72}, {3.67, 1.35, 0.84, 0.68});
-      offer(F32_CONV3X3_128, 128, 8, F32_CONV3X3_PATCH, {3.32, 1.59, 1.26, 0.84}, {3.75, 1.89, 1.47, 0.63});
-      offer(F32_CONV3X3_SPLIT_128, 128, 16, F32_CONV3X3_SPLIT_PATCH, {4.08, 3.00, 2.14, 0.95}, {4.91, 3.79, 2.36, 1.11});
-      offer(F32_CONV3X3_SPLIT_256, 256, 16, F32_CONV3X3_SPLIT_PATCH, {5.04, 1.84, 4.24, 0.16}, {6.41, 4.74, 4.16, 0.73});
+      offer(F32_CONV3X3_32, 8, F32_CONV3X3_PATCH, {3.21, 0.82, 0.49, 0.40}, {3.56, 1.09, 0.58, 0.68});
+      offer(F32_CONV3X3_64, 8, F32_CONV3X3_PATCH, {3.10, 1.09, 0.69, 0.72}, {3.67, 1.35, 0.84, 0.68});
+      offer(F32_CONV3X3_128, 8, F32_CONV3X3_PATCH, {3.32, 1.59, 1.26, 0.84}, {3.75, 1.89, 1.47, 0.63});
+      offer(F32_CONV3X3_SPLIT_128, 16, F32_CONV3X3_SPLIT_PATCH, {4.08, 3.00, 2.14, 0.95}, {4.91, 3.79, 2.36, 1.11});
+      offer(F32_CONV3X3_SPLIT_256, 16, F32_CONV3X3_SPLIT_PATCH, {5.04, 1.84, 4.24, 0.16}, {6.41, 4.74, 4.16, 0.73});
    }
-   const bool split = tile >= F32_CONV3X3_SPLIT_128;
-   const long long patch = f32_conv3x3_patch(s.OH, s.OW, tile - (split ? 4000 : 3000));
-   if (tile < F32_CONV3X3_32 || patch > (split ? F32_CONV3X3_SPLIT_PATCH : F32_CONV3X3_PATCH))
+   const int pixels = conv3x3_pixels(tile);
+   if (!pixels)
+      return SOFIE_HIP_OK; // another kernel, or a request for one that there is not: launch_f32_product's
+   const bool split = tile == F32_CONV3X3_SPLIT_128 || tile == F32_CONV3X3_SPLIT_256;
+   const long long patch = f32_conv3x3_patch(s.OH, s.OW, pixels);
+   if (patch > (split ? F32_CONV3X3_SPLIT_PATCH : F32_CONV3X3_PATCH))
       return SOFIE_HIP_OK;
    // the images that 256 pixels touch, all their channels
    const int near = (255 / ((long long)s.OH * s.OW) + 2) * (long long)out.Cout * out.positions * 4 < F32_BUFFER_BYTES - (1 << 20);

@@ -81,3 +81,28 @@ def test_elementwise_and_arena_argument_checks(rt):
     finally:
         own.close()
     rt.sync()
+
+
+@pytest.mark.parametrize("tile", [8, 48, 3000, 3031, 3033, 3100, 4127, 4200, 4257, 1 << 30])
+def test_f32_tiles_that_there_are_not(rt, tile):
+    """A request for a kernel that does not exist is refused, by products and by convolutions, 3 x 3 and others."""
+    A, Y = util.to_dev(np.zeros(4096, np.float32)), util.dev_empty((64, 64), np.float32)
+    g = R.GemmF32Desc()
+    g.M, g.N, g.K, g.alpha, g.batch = 8, 8, 8, 1.0, 1
+    g.A = g.B = util.ptr(A)
+    g.Y = util.ptr(Y)
+    rt.set_option("f32_tile", tile)
+    try:
+        with pytest.raises(SofieHipError, match="unknown tile"):
+            rt.call("sofie_hip_gemm_f32", C.byref(g))
+        for k in (3, 1):
+            d = R.ConvDesc()
+            d.N, d.C, d.H, d.W, d.Cout, d.kh, d.kw = 1, 4, 8, 8, 6, k, k
+            d.stride_h = d.stride_w = d.dil_h = d.dil_w = d.group = 1
+            d.OH = d.OW = 9 - k
+            with pytest.raises(SofieHipError, match="unknown tile"):
+                rt.call("sofie_hip_conv_f32", C.byref(d), util.ptr(A), util.ptr(A), None, 0, C.c_float(0), util.ptr(Y), None, None)
+    finally:
+        rt.set_option("f32_tile", 0)
+    rt.call("sofie_hip_gemm_f32", C.byref(g))
+    rt.sync()
