@@ -340,12 +340,14 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
    *taken = true;
    hipStream_t st = ctx->stream;
    if (split) {
-      auto go = [&](auto pixels, auto wide) {
-         constexpr int BM = decltype(pixels)::value, V = decltype(wide)::value;
-         return patch <= 256 ? launch_f32_conv3x3_split_as<BM, 256, V>(st, a, out, group) : launch_f32_conv3x3_split_as<BM, F32_CONV3X3_SPLIT_PATCH, V>(st, a, out, group);
+      // (a patch of 256 pixels has 324 places and more)
+      auto go = [&](auto wide) {
+         constexpr int V = decltype(wide)::value;
+         if (tile == F32_CONV3X3_SPLIT_256)
+            return launch_f32_conv3x3_split_as<256, F32_CONV3X3_SPLIT_PATCH, V>(st, a, out, group);
+         return patch <= 256 ? launch_f32_conv3x3_split_as<128, 256, V>(st, a, out, group) : launch_f32_conv3x3_split_as<128, F32_CONV3X3_SPLIT_PATCH, V>(st, a, out, group);
       };
-      auto with = [&](auto pixels) { return vec ? go(pixels, std::integral_constant<int, 4>{}) : go(pixels, std::integral_constant<int, 1>{}); };
-      return tile == F32_CONV3X3_SPLIT_128 ? with(std::integral_constant<int, 128>{}) : with(std::integral_constant<int, 256>{});
+      return vec ? go(std::integral_constant<int, 4>{}) : go(std::integral_constant<int, 1>{});
    }
    auto go = [&](auto room, auto wide) {
       constexpr int P = decltype(room)::value, V = decltype(wide)::value;
