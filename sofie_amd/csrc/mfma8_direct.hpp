@@ -329,6 +329,19 @@ struct DirectRing {
    }
 };
 
+// Whether an int8 / FP8 product of 16-byte rows in tiles of b x b comes line by line.  A wave with a single step has nothing to pipeline, and the trip through LDS is
+// what the ring adds: K = 128 in 16 x 16 tiles 2.49 us, 2.62 through the ring, in 32 x 32 tiles 2.85 and 3.08; K = 256 2.60 and 2.63, 3.02 and 3.09.  With more than
+// two tiles of 32 x 32 a CU, lines count again (500 x 1500 x 256 5.3 us, 4.4).  Up to four rows are as many lines less for the registers: 1 x 1000 x 640 2.81 us and
+// 2.97, even at K = 896.  A last step that is not whole is loaded chunk by chunk into the registers, which costs more than the ring (16 rows of 112 bytes 2.7, 2.5).
+inline bool mfma8_direct_by_lines(int b, int M, int N, int K)
+{
+   if (K % 128 != 0)
+      return true;
+   if (K <= 256)
+      return b > 16 && (long long)((M + b - 1) / b) * ((N + b - 1) / b) > 512;
+   return !(b == 16 && M <= 4 && K <= 768);
+}
+
 template <class MMA, int MB, int NB, int W, int UNROLL, class EPI>
 static int launch_mfma8_direct(const LaunchCfg &lc, const int8_t *A, const int8_t *Bt, int M, int N, int K, int lda, int ldb, const EPI &ep)
 {
@@ -337,7 +350,7 @@ static int launch_mfma8_direct(const LaunchCfg &lc, const int8_t *A, const int8_
    if (nwg > 0x7fffffffLL)
       return fail(SOFIE_HIP_ERR_INVALID, "gemm: too many tiles");
    typedef DirectRing<MB, NB, W> Ring;
-   if (Ring::takes(A, Bt, lda, ldb, K)) {
+   if (mfma8_direct_by_lines(MB * 16, M, N, K) && Ring::takes(A, Bt, lda, ldb, K)) {
       const Ring ring(nwg, K);
       auto kern = mfma8_direct_ring_kernel<MMA, MB, NB, W, EPI>;
       static bool configured[64] = {};

@@ -14,20 +14,27 @@ namespace sofie_hip {
 // to about a fifth where both operands are rows; they decide between kernels whose times differ by more than that almost everywhere.
 // The loader that transposes B (mfma8_columns_preferred) has no term of its own and takes up to half as long again: 1537 x 1000 x 777 7.6 us
 // estimated and 11.4 measured, 300 x 300 x 300 4.3 and 6.2.
+inline double mfma8_rounds(int M, int N, int bm, int bn)
+{
+   const double rounds = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) / 256.0; // tiles per CU; a CU works on a few at a time
+   return rounds <= 1.0 ? 1.0 : 0.5 * (rounds + std::ceil(rounds));
+}
 inline double mfma8_time(int M, int N, int K, int bm, int bn, double fixed_us, double tile_us, double bytes_per_us)
 {
-   double rounds = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) / 256.0; // tiles per CU; a CU works on a few at a time
-   rounds = rounds <= 1.0 ? 1.0 : 0.5 * (rounds + std::ceil(rounds));
-   return fixed_us + rounds * (tile_us + (double)(bm + bn) * K / bytes_per_us);
+   return fixed_us + mfma8_rounds(M, N, bm, bn) * (tile_us + (double)(bm + bn) * K / bytes_per_us);
 }
-// `lines`: rows start on 16 bytes, so that the direct kernel loads line by line through its ring: 115 KB/us a CU while few CUs are at work, and 21 TB/s
-// from L2 over all of them (us, us estimated / measured: 16 x 4096 x 4096 4.4 / 4.0, 609 x 377 x 5728 7.5 / 7.5, 108 x 4816 x 1392 6.8 / 6.8).
+// `lines`: rows start on 16 bytes, so that the direct kernel loads line by line through its ring where that pays: 120 KB/us a CU for the first 2048 of a row, which
+// are asked for at once, and as much behind them while few CUs are at work, 20 TB/s from L2 over all of them (us, estimated / measured: 16 x 4096 x 4096
+// 4.4 / 4.2, 600 x 320 x 6144 6.7 / 6.4, 108 x 4096 x 8192 16.0 / 14.4); whole steps of a short K through registers at the rates below.  Fitted, int8 and FP8, to 1900
+// products of 1 .. 800 rows by 32 .. 4096 columns, K = 32 .. 8192, with what the 64 x 64 tiles took: the choice is 0.05 % above the fastest on average, 7 % the most.
 inline double mfma8_direct_time(int M, int N, int K, int b, bool lines)
 {
    if (!lines)
       return b == 16 ? mfma8_time(M, N, K, 16, 16, 2.5, 0.4, 41e3) : mfma8_time(M, N, K, 32, 32, 2.5, 0.8, 44e3);
-   const double tiles = (double)((M + b - 1) / b) * ((N + b - 1) / b);
-   return mfma8_time(M, N, K, b, b, 2.5, b == 16 ? 0.3 : 0.5, std::min(115e3, 21e6 / std::min(tiles, 256.0)));
+   if (!mfma8_direct_by_lines(b, M, N, K))
+      return b == 16 ? mfma8_time(M, N, K, 16, 16, 2.5, 0.3, 41e3) : mfma8_time(M, N, K, 32, 32, 2.5, 0.45, 80e3);
+   const double tiles = (double)((M + b - 1) / b) * ((N + b - 1) / b), ahead = std::min(K, 2048);
+   return 2.5 + mfma8_rounds(M, N, b, b) * ((b == 16 ? 0.5 : 0.62) + 2.0 * b * (ahead / 120e3 + (K - ahead) / std::min(120e3, 20e6 / std::min(tiles, 256.0))));
 }
 inline double mfma8_staged64_time(int M, int N, int K) { return mfma8_time(M, N, K, 64, 64, 3.0, 0.4, 45e3); }
 inline double mfma8_staged128_time(int M, int N, int K) { return mfma8_time(M, N, K, 128, 128, 4.0, 2.5, 39e3); }
@@ -58,7 +65,9 @@ static int launch_mfma8_best(const LaunchCfg &lc, const int8_t *A, const int8_t 
    const bool ring = variant >= 0 && aligned && K >= 64 && K % 64 == 0 && (MMA::KSTEP * 2 <= 64 || K % 128 == 0);
    const bool lines = aligned && K % 16 == 0;
    const double t16 = mfma8_direct_time(M, N, K, 16, lines), t32 = mfma8_direct_time(M, N, K, 32, lines);
-   const double others = ring ? mfma8_ring_time(M, N, K, pick_tile(M, N, 0)) : std::min(mfma8_staged64_time(M, N, K), mfma8_staged128_time(M, N, K));
+   // (the general loop takes 0.4 - 0.7 us longer than estimated where few tiles of aligned rows are all there is: 300 x 1000 x 32 3.9 int8, 4.2 FP8, the direct kernel 3.8)
+   const double others = ring ? mfma8_ring_time(M, N, K, pick_tile(M, N, 0))
+                              : std::min(mfma8_staged64_time(M, N, K), mfma8_staged128_time(M, N, K)) + (lines ? 0.5 : 0.0);
    if (force_tile == 16 || K < 16 || (!force_tile && variant == 0 && t16 <= t32 && t16 < others))
       return launch_mfma8_direct<Direct, 1, 1, 8, 4, EPI>(lc, A, Bt, M, N, K, lda, ldb, ep);
    if (force_tile == 32 || (!force_tile && variant == 0 && t32 < others))

@@ -13,7 +13,9 @@ from tests import util
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(1, 1, 16, 0), (16, 17, 112, 16), (31, 33, 128, 0), (17, 15, 144, 48), (33, 64, 1040, 0), (5, 40, 4096, 16), (48, 20, 4240, 0), (16, 16, 9200, 0), (300, 600, 400, 0), (270, 530, 2064, 16)]
+SHAPES = [(1, 1, 16, 0), (16, 17, 112, 16), (31, 33, 128, 0), (17, 15, 144, 48), (33, 64, 1040, 0), (5, 40, 4096, 16), (48, 20, 4240, 0), (16, 16, 9200, 0), (300, 600, 400, 0), (270, 530, 2064, 16),
+          # by registers: whole steps up to 256 bytes (of 32 x 32 tiles two a CU, and more than that by lines), four rows up to 768
+          (33, 70, 256, 16), (16, 16, 128, 0), (500, 1040, 128, 0), (530, 1040, 256, 16), (4, 48, 768, 0), (5, 48, 768, 16), (3, 33, 896, 0), (2, 20, 384, 0)]
 
 
 @pytest.fixture
