@@ -979,7 +979,10 @@ static int launch_f32_direct(hipStream_t stream, const ASRC &A, const BSRC &B, c
       return fail(SOFIE_HIP_ERR_INVALID, "fp32 product: too many tiles");
    if constexpr (ASRC::KC && BSRC::KC && ASRC::VEC == 4 && BSRC::VEC == 4) {
       typedef DirectRing<MB, NB, W> Ring;
-      if (Ring::takes(A.p, B.p, A.ld * 4, B.ld * 4, K * 4LL)) {
+      // A single step has nothing to pipeline: 64 x 640 x 32 2.83 us, 2.89 through the ring, 130 x 1500 x 32 9 % longer.  Few rows that do not start on lines take two
+      // lines a step, which the registers' finer steps hide up to K = 512: 4 x 97 x 436 3.84 us, 4.10 through the ring.
+      const bool by_lines = K > 32 && (M > 8 || K <= 128 || K >= 512 || (A.ld % 32 == 0 && B.ld % 32 == 0));
+      if (by_lines && Ring::takes(A.p, B.p, A.ld * 4, B.ld * 4, K * 4LL)) {
          const Ring ring(nwg * batch, K * 4);
          auto kern = f32_direct_ring_kernel<STORE, MB, NB, W>;
          static bool configured[64] = {};

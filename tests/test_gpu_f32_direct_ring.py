@@ -1,5 +1,5 @@
 """The fp32 kernel for small products whose operands pass through a ring in LDS (both contiguous in k, rows on 16 bytes), at the edges of its tile (16), of its
-steps of 32 k over eight waves and of its ring: less than a step, four k more or less than whole steps, more steps than the ring holds, more tiles than CUs,
+steps of 32 k over eight waves and of its ring: up to a step (by registers), four k more or less than whole steps, more steps than the ring holds, more tiles than CUs,
 batches, and rows that lie further apart than they are long."""
 import ctypes as C
 
