@@ -62,14 +62,16 @@ __device__ __forceinline__ void f32_buffer_store(float v, const void *base, int 
 // mask each) it fills the scalar registers, and a spilled one costs a vector instruction where it is written and one where it is read.
 __device__ __forceinline__ void forget(int &v) { asm volatile("" : "+s"(v)); }
 
-// Activations that take no call: the registers that a call keeps free are spilled where the tile begins.
+// Activations that take no call.  Kernels apart for those that do, whose calls keep registers free: they spill 17 - 70 scalars where most of the plain ones spill fewer.
 inline bool conv3x3_plain(const PostChain &chain) { return chain.count == 0 || (chain.count == 1 && chain.op0 == SOFIE_ACT_RELU); }
 
 // The results that a lane holds of a block: E of the 16 channels first + 4 lk + e / 4 * 8 + e % 4, from element e0 (a multiple of 4) on, of one pixel.  32 neighbouring
 // lanes hold 32 neighbouring pixels of a channel: whole lines, loaded and stored straight from the registers.  Addresses are an offset per lane, one for all
 // channels, and a scalar per channel.  A tile of few input channels is bound by the instructions around its MFMAs: with an address, a bound and a branch per
-// channel, places of the patch worked out by every wave and scalars spilled, 3 -> 32 channels had 18 MFMAs a wave among 573 vector and 357 scalar instructions, now
-// 303 and 298.  64 images of 64 x 64, us before -> after: 3 -> 32 channels 19.3 -> 14.9; 40 of 90 x 90, 3 -> 12 23.2 -> 16.7; 1 of 64 x 64 5.5 -> 4.0.
+// channel, places of the patch worked out by every wave and more scalars spilled, 3 -> 32 channels had 18 MFMAs a wave among 573 vector and 357 scalar instructions, now
+// 303 and 298.  64 images of 64 x 64, us before -> after, for all of these together: 3 -> 32 channels 19.3 -> 14.9; 40 of 90 x 90, 3 -> 12 23.2 -> 16.7; 1 of 64 x 64
+// 5.5 -> 4.0.  Still spilled, in plain kernels: 6 scalars with few channels, 20 - 32 at 128 pixels, up to 66 where waves share a tile (none at 256 places with wide
+// weights).
 template <int E>
 struct Conv3x3Block {
    float *Y;         // result of channel `first`, pixel 0 of the tile's first image (scalar)

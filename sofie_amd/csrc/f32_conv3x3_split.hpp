@@ -19,8 +19,8 @@
 // end in a sum that is not finite; the last shows where a value is split, as a subnormal third piece.  A wave whose sums are not finite, and a workgroup that met
 // such a piece, compute their sums again with fp32 instructions straight from memory.  (The matrix cores' treatment of subnormals was measured: subnormal
 // operands, products and sums of v_mfma_f32_32x32x16_bf16 come out exact.)  Telling costs an instruction per value: 64 -> 64 at 32 x 32 takes 1.3 us longer.  Summing
-// again, for every tile of 64 images of 32 x 32: 32 -> 64 channels 20.6 -> 57 us, 64 -> 64 31 -> 105 (the fp32 kernel takes 43); two channels at a time with their
-// loads in flight, where eight k with their index arithmetic took 132.
+// again, in every tile of 64 images of 32 x 32, has its price: 32 -> 64 channels 22.8 -> 59 us, 64 -> 64 37 -> 109, 128 -> 128 at 16 x 16 40 -> 180.  It takes two channels at a
+// time with their loads in flight; eight k at a time with their index arithmetic were 132 for the second.
 #pragma once
 #include "f32_conv3x3.hpp"
 
@@ -68,7 +68,7 @@ struct F32Conv3x3SplitShape {
 
 // Four waves, each with BM / 4 pixels and 32 output channels.  One slab lies in LDS in pieces, the next one as raw weights and, in registers, as raw patch; two
 // workgroups per CU, one of which splits while the other multiplies.  (One workgroup whose other four waves split for it, through two slabs of pieces, is no
-// faster: 36 us, bound by LDS.)
+// faster: 36 us, bound by LDS.)  8 - 14 scalars are spilled, 48 - 70 in the kernels of activations with calls; 256 pixels with narrow weights fill the 256 vector registers.
 template <int BM, int PLANE, int WVEC, bool PLAIN>
 __global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a, F32ConvStore out, int tiles_m, int tiles_n, int first_tile)
 {

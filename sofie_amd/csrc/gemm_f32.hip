@@ -317,7 +317,7 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
    } else if (!tile) {
       // us: a launch; a slab (8 channels, 16 of the split kernel) of a CU whose tiles wait for their loads, and of one with several tiles at work; a tile.  The
       // second set is for weights that come float by float.  Fitted to 156 layers (the split kernel's to 230 others) from 1 image of 6 x 6 to 64 of 64 x 64, 5 to 130
-      // channels; holds to a sixth, the split kernel's to a quarter, and costs 0.8 % of the best of these kernels on average over the 260 layers, 14 % the most.
+      // channels; holds to a sixth, and costs 0.4 % of the best of these kernels on average over the 260 layers, 14 % the most, 10 % but for that one.
       double least = 1e30;
       struct Cost {
          double launch, alone, slab, each;
@@ -325,7 +325,9 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
       auto offer = [&](int which, int channels, long long room, Cost wide, Cost narrow) {
          const int bm = conv3x3_pixels(which);
          const Cost cost = vec ? wide : narrow;
-         const double rounds = std::ceil((double)((M + bm - 1) / bm) * ((N + 31) / 32) * group / 256.0), slabs = (s.Cg + channels - 1) / channels;
+         const double tiles = (double)((M + bm - 1) / bm) * ((N + 31) / 32) * group / 256.0, slabs = (s.Cg + channels - 1) / channels;
+         // (two workgroups of the split kernel share a CU, and one's odd tile runs beside the other's)
+         const double rounds = channels == 8 || tiles <= 1.0 ? std::ceil(tiles) : 0.5 * (tiles + std::ceil(tiles));
          const double t = cost.launch + std::max(slabs * cost.alone, rounds * (slabs * cost.slab + cost.each));
          if (f32_conv3x3_patch(s.OH, s.OW, bm) <= room && t < least)
             least = t, tile = which;
@@ -333,8 +335,8 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
       offer(F32_CONV3X3_32, 8, F32_CONV3X3_PATCH, {3.21, 0.82, 0.49, 0.40}, {3.56, 1.09, 0.58, 0.68});
       offer(F32_CONV3X3_64, 8, F32_CONV3X3_PATCH, {3.10, 1.09, 0.69, 0.72}, {3.67, 1.35, 0.84, 0.68});
       offer(F32_CONV3X3_128, 8, F32_CONV3X3_PATCH, {3.32, 1.59, 1.26, 0.84}, {3.75, 1.89, 1.47, 0.63});
-      offer(F32_CONV3X3_SPLIT_128, 16, F32_CONV3X3_SPLIT_PATCH, {4.08, 3.00, 2.14, 0.95}, {4.91, 3.79, 2.36, 1.11});
-      offer(F32_CONV3X3_SPLIT_256, 16, F32_CONV3X3_SPLIT_PATCH, {5.04, 1.84, 4.24, 0.16}, {6.41, 4.74, 4.16, 0.73});
+      offer(F32_CONV3X3_SPLIT_128, 16, F32_CONV3X3_SPLIT_PATCH, {3.95, 3.25, 2.20, 1.06}, {5.12, 3.65, 2.82, 0.65});
+      offer(F32_CONV3X3_SPLIT_256, 16, F32_CONV3X3_SPLIT_PATCH, {5.17, 4.60, 3.75, 0.65}, {6.95, 4.60, 4.19, 0.30});
    }
    const int pixels = conv3x3_pixels(tile);
    if (!pixels)
