@@ -187,9 +187,9 @@ namespace sofie_hip {
 // shortest.  A CU multiplies a 32 x 32 block by 32 k in 0.107 us at best.  A tile kernel takes a launch, `alone` per slab of 32 k where its tiles wait for their
 // loads, and `slab` and `tile` in as many rounds as the tiles need over 256 CUs; operands that come float by float (ragged) take longer.  The direct
 // kernel takes a launch, `alone` per 128 k (16 of each wave) and `row` for every sixteenth of its 16 rows or, where there are many tiles, `slab` per 16 k and 256
-// tiles, and `tile` per 256 tiles; where both operands come line by line through its ring, 110 KB/us a CU and 0.34 us for the first 256 tiles, 72 and 0.49 a tile where
-// there are more.  Fitted to 1120 products of each kind of loads, 20 kFLOP to 30 GFLOP, 1 .. 4096 rows, K = 8 .. 2048: on average 0.6 % (float by float), 0.3 % (float by float along
-// k), 0.13 % and 0.15 % (16 bytes, along k) above the best kernel's time.  Costs without the rows were 2.1, 1.6, 0.55 and 0.47 % above, and a third on a few rows of long k
+// tiles, and `tile` per 256 tiles; where both operands come line by line through its ring, 78 KB/us a CU and 0.48 us for the first 256 tiles, 73 and 0.49 a tile where
+// there are more.  Fitted to 1220 products of each kind of loads, 20 kFLOP to 30 GFLOP, 1 .. 4096 rows, K = 8 .. 2048: on average 0.5 % (float by float), 0.25 % (float by float
+// along k), 0.2 % and 0.2 % (16 bytes, along k) above the best kernel's time.  Costs without the rows were 2.1, 1.6, 0.7 and 0.7 % above, and a third on a few rows of long k
 // (4 x 3545 x 468, float by float: 6.6 us, now 4.9; 4 x 4096 x 192, 16 bytes: 4.2, now 3.7).  (Launches take 0.4 us more or less from box to box; these are of
 // the shorter kind, as the chain's costs below are.)
 enum F32Tile { F32_CONV3X3_32 = 3032, F32_CONV3X3_64 = 3064, F32_CONV3X3_128 = 3128, F32_CONV3X3_SPLIT_128 = 4128, F32_CONV3X3_SPLIT_256 = 4256, F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
@@ -216,10 +216,10 @@ static int pick_f32_tile(int M, int N, int K, int batch, F32Loads loads, double 
       Cost direct, tile32, tile64x32, tile64, tile128;
    };
    static constexpr Costs COSTS[] = { // by F32Loads
-      {{3.09, 0.39, 0.125, 0.38, 0.365}, {3.86, 0.03, 0.133, 0.55}, {4.07, 0.34, 0.286, 0.91}, {3.86, 0.04, 0.519, 1.62}, {7.86, 0.08, 2.05, 3.29}},
-      {{2.65, 0.71, 0.241, 0.41, 0.193}, {3.66, 0.02, 0.134, 0.59}, {3.89, 0.21, 0.290, 0.97}, {3.81, 0.16, 0.529, 1.51}, {5.30, 0.44, 2.27, 4.92}},
-      {{3.00, 0.33, 0.073, 0.42, 0.043}, {3.05, 0.12, 0.142, 0.49}, {3.66, 0.20, 0.276, 0.78}, {2.81, 0.40, 0.514, 1.70}, {5.26, 0.02, 2.23, 4.14}},
-      {{}, {2.78, 0.09, 0.124, 0.49}, {3.39, 0.10, 0.248, 0.70}, {2.66, 0.23, 0.468, 1.56}, {5.92, 0.03, 1.66, 4.97}}};
+      {{2.77, 0.49, 0.096, 0.63, 0.336}, {3.80, 0.03, 0.136, 0.54}, {4.06, 0.26, 0.291, 0.86}, {4.17, 0.09, 0.526, 1.51}, {7.85, 0.37, 2.08, 3.06}},
+      {{2.11, 0.85, 0.284, 0.57, 0.210}, {3.62, 0.03, 0.140, 0.56}, {3.80, 0.39, 0.298, 0.92}, {3.73, 0.11, 0.545, 1.47}, {5.41, 0.39, 2.34, 4.67}},
+      {{3.09, 0.31, 0.068, 0.38, 0.038}, {3.06, 0.09, 0.134, 0.53}, {3.64, 0.14, 0.262, 0.78}, {3.14, 0.34, 0.504, 1.53}, {5.94, 0.03, 2.01, 3.56}},
+      {{}, {2.78, 0.10, 0.125, 0.49}, {3.45, 0.18, 0.251, 0.66}, {2.68, 0.48, 0.478, 1.47}, {5.36, 0.03, 1.80, 3.55}}};
    auto tiles = [&](int bm, int bn) { return std::ceil((double)M / bm) * std::ceil((double)N / bn) * batch; };
    const double slabs = std::ceil(K / 32.0), steps = std::ceil(K / 16.0), each = tiles(16, 16) / 256.0;
    const Costs &costs = COSTS[loads];
@@ -227,7 +227,7 @@ static int pick_f32_tile(int M, int N, int K, int batch, F32Loads loads, double 
    double least;
    if (loads == F32_LOADS_LINES) {
       const double rounds = each <= 1.0 ? 1.0 : 0.5 * (each + std::ceil(each));
-      least = 2.36 + rounds * (each <= 1.0 ? 0.34 + 128.0 * K / 110e3 : 0.49 + 128.0 * K / 72e3);
+      least = 2.36 + rounds * (each <= 1.0 ? 0.48 + 128.0 * K / 78e3 : 0.49 + 128.0 * K / 73e3);
    } else {
       const Cost &c = costs.direct;
       least = c.launch + std::max((c.alone + c.row * std::min(M, 16) / 16.0) * std::ceil(steps / 8.0), c.slab * each * steps) + c.tile * each;
