@@ -190,7 +190,7 @@ namespace sofie_hip {
 // tiles, and `tile` per 256 tiles; where both operands come line by line through its ring, 78 KB/us a CU and 0.48 us for the first 256 tiles, 73 and 0.49 a tile where
 // there are more.  Fitted to 1220 products of each kind of loads, 20 kFLOP to 30 GFLOP, 1 .. 4096 rows, K = 8 .. 2048: on average 0.5 % (float by float), 0.25 % (float by float
 // along k), 0.2 % and 0.2 % (16 bytes, along k) above the best kernel's time.  Costs without the rows were 2.1, 1.6, 0.7 and 0.7 % above, and a third on a few rows of long k
-// (4 x 3545 x 468, float by float: 6.6 us, now 4.9; 4 x 4096 x 192, 16 bytes: 4.2, now 3.7).  (Launches take 0.4 us more or less from box to box; these are of
+// (4 x 3545 x 468, float by float: 6.6 us, now 4.9; 4 x 4096 x 192, 16 bytes: 4.2, now 3.7).  (Launches take 0.4 us more or less from one card to another; these are of
 // the shorter kind, as the chain's costs below are.)
 enum F32Tile { F32_CONV3X3_32 = 3032, F32_CONV3X3_64 = 3064, F32_CONV3X3_128 = 3128, F32_CONV3X3_SPLIT_128 = 4128, F32_CONV3X3_SPLIT_256 = 4256, F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
 // Pixels of a tile of the 3 x 3 convolution kernels; 0 for any other kernel.
