@@ -28,34 +28,24 @@ struct Divisor64 {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // q = sat8(rne(x / scale)), fp32 division (ONNX QuantizeLinear, zero point 0)
+// A load per thread: the divisions of four values take a wave that is alone on its SIMD as long as the trip to memory, and sixteen of them, with four loads in flight,
+// three times as long.  us with sixteen -> four: 16 K values 2.35 -> 1.83, 1 M 2.65 -> 2.13, 3 M 3.76 -> 3.41.
 __global__ __launch_bounds__(256) void quantize_linear_kernel(int8_t *__restrict__ dst, const float *__restrict__ src,
                                                                size_t n, float scale, int vec)
 {
    const size_t stride = (size_t)gridDim.x * blockDim.x;
    size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
    if (vec) {
-      // four 16-byte loads per lane are issued before the first is used (a lane's pieces lie a workgroup's width apart, so every
-      // wave instruction reads and writes whole lines): the kernel is a single round trip to memory, and a quarter of the waves run it
       const size_t n4 = n / 4;
-      for (size_t base = blockIdx.x * (size_t)blockDim.x * 4 + threadIdx.x; base < n4; base += stride * 4) {
-         float4 v[4];
-#pragma unroll
-         for (int j = 0; j < 4; ++j) {
-            const size_t k = base + (size_t)j * blockDim.x;
-            v[j] = k < n4 ? ((const float4 *)src)[k] : make_float4(0.f, 0.f, 0.f, 0.f);
-         }
-#pragma unroll
-         for (int j = 0; j < 4; ++j) {
-            const size_t k = base + (size_t)j * blockDim.x;
-            int q0 = quantize_rne_sat8(__fdiv_rn(v[j].x, scale));
-            int q1 = quantize_rne_sat8(__fdiv_rn(v[j].y, scale));
-            int q2 = quantize_rne_sat8(__fdiv_rn(v[j].z, scale));
-            int q3 = quantize_rne_sat8(__fdiv_rn(v[j].w, scale));
-            if (k < n4)
-               ((uint32_t *)dst)[k] = (uint32_t)(q0 & 0xff) | ((uint32_t)(q1 & 0xff) << 8) | ((uint32_t)(q2 & 0xff) << 16) | ((uint32_t)(q3 & 0xff) << 24);
-         }
+      for (size_t k = i; k < n4; k += stride) {
+         const float4 v = ((const float4 *)src)[k];
+         const int q0 = quantize_rne_sat8(__fdiv_rn(v.x, scale));
+         const int q1 = quantize_rne_sat8(__fdiv_rn(v.y, scale));
+         const int q2 = quantize_rne_sat8(__fdiv_rn(v.z, scale));
+         const int q3 = quantize_rne_sat8(__fdiv_rn(v.w, scale));
+         ((uint32_t *)dst)[k] = (uint32_t)(q0 & 0xff) | ((uint32_t)(q1 & 0xff) << 8) | ((uint32_t)(q2 & 0xff) << 16) | ((uint32_t)(q3 & 0xff) << 24);
       }
-      i = n4 * 4 + (blockIdx.x * (size_t)blockDim.x + threadIdx.x);
+      i += n4 * 4;
       if (i < n)
          dst[i] = (int8_t)quantize_rne_sat8(__fdiv_rn(src[i], scale));
    } else {
@@ -772,13 +762,13 @@ __global__ __launch_bounds__(256) void plane_sums_take_average_kernel(float *__r
 
 // NHWC int8 input with C a multiple of 16 (and 16-byte aligned): one workgroup per (image, block of 16 << chunks_log2 channels).
 // A thread owns 16 consecutive channels and every (512 >> chunks_log2)-th pixel, reads 16 bytes per pixel, and the
-// per-thread int32 sums are added up through LDS (integer sums: exact in any order), by all threads first and then by one per
-// channel.  5 images of 28x28x64: 5.2 us with one workgroup per image, whose last threads each read 64 sums, 4.6 us now.
+// per-thread int32 sums are added up (integer sums: exact in any order) across a wave's lanes in registers, and over the eight waves through LDS.  us, with all of it through
+// LDS -> now: 5 images of 28 x 28 x 64 3.60 -> 2.79, one of 8 x 8 x 256 2.81 -> 1.97, 100 of 50 x 50 x 32 3.79 -> 3.03, 256 of 64 x 64 x 256 (read from memory) 38.5 -> 38.2.
 constexpr int GAP_THREADS = 512;
 __global__ __launch_bounds__(GAP_THREADS) void gap_i8_nhwc_vec_kernel(float *__restrict__ Y, const int8_t *__restrict__ X, int C, int HW,
                                                                float scale, int chunks_log2)
 {
-   __shared__ int part[GAP_THREADS][17];
+   __shared__ int part[GAP_THREADS / 64][256];
    const int img = blockIdx.x, c_first = blockIdx.y << (4 + chunks_log2);
    const int groups = GAP_THREADS >> chunks_log2;
    const int chunk = threadIdx.x & ((1 << chunks_log2) - 1), group = threadIdx.x >> chunks_log2;
@@ -807,24 +797,44 @@ __global__ __launch_bounds__(GAP_THREADS) void gap_i8_nhwc_vec_kernel(float *__r
             }
       }
    }
+   // Over the pixels of a wave: halves of the wave, then of either half, keep the sums of half of the channels each; lanes of a row of 16 that differ in their pixels alone
+   // add up in place.  Lane l then holds channels l / 16 * 4 .. + 3 of its 16.
 #pragma unroll
-   for (int k = 0; k < 16; ++k)
-      part[threadIdx.x][k] = s[k];
+   for (int k = 0; k < 8; ++k) {
+      const auto both = __builtin_amdgcn_permlane32_swap((unsigned)s[k], (unsigned)s[k + 8], false, false);
+      s[k] = (int)((unsigned)both[0] + (unsigned)both[1]);
+   }
+#pragma unroll
+   for (int k = 0; k < 4; ++k) {
+      const auto both = __builtin_amdgcn_permlane16_swap((unsigned)s[k], (unsigned)s[k + 4], false, false);
+      s[k] = (int)((unsigned)both[0] + (unsigned)both[1]);
+   }
+   auto fold = [&](auto control) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+         s[k] += __builtin_amdgcn_update_dpp(0, s[k], decltype(control)::value, 0xf, 0xf, false);
+   };
+   if (chunks_log2 < 4)
+      fold(std::integral_constant<int, 0x128>{}); // row_ror:8
+   if (chunks_log2 < 3)
+      fold(std::integral_constant<int, 0x124>{}); // row_ror:4, the same as lane ^ 4 now
+   if (chunks_log2 < 2)
+      fold(std::integral_constant<int, 0x122>{});
+   if (chunks_log2 < 1)
+      fold(std::integral_constant<int, 0x121>{});
+   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+   if ((lane & 15) >> chunks_log2 == 0) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+         part[wave][chunk * 16 + (lane >> 4) * 4 + k] = s[k];
+   }
    __syncthreads();
-   // channel c_first + of: `slices` threads add every slices-th partial sum, one of them the rest
-   const int here_log2 = 4 + chunks_log2, slices = GAP_THREADS >> here_log2, of = threadIdx.x & ((1 << here_log2) - 1), slice = threadIdx.x >> here_log2;
-   int tot = 0;
-#pragma unroll 8
-   for (int g = slice; g < groups; g += slices)
-      tot += part[(g << chunks_log2) + (of >> 4)][of & 15];
-   __syncthreads();
-   int *sums = &part[0][0];
-   sums[threadIdx.x] = tot;
-   __syncthreads();
-   if (slice == 0 && c_first + of < C) {
-#pragma unroll 8
-      for (int q = 1; q < slices; ++q)
-         tot += sums[(q << here_log2) + of];
+   const int of = threadIdx.x;
+   if (of < 16 << chunks_log2 && c_first + of < C) {
+      int tot = 0;
+#pragma unroll
+      for (int w = 0; w < GAP_THREADS / 64; ++w)
+         tot += part[w][of];
       Y[(size_t)img * C + c_first + of] = __fdiv_rn(mul_nofma((float)tot, scale), (float)HW);
    }
 }
@@ -883,7 +893,7 @@ int sofie_hip_quantize_linear(sofie_hip_ctx *ctx, int8_t *dst, const float *src,
    SOFIE_HIP_REQUIRE(dst && src, "sofie_hip_quantize_linear: NULL pointer");
    SOFIE_HIP_REQUIRE(scale > 0.0f, "sofie_hip_quantize_linear: scale must be positive");
    const int vec = (((uintptr_t)src & 15) == 0) && (((uintptr_t)dst & 3) == 0);
-   launch_kernel(quantize_linear_kernel, dim3(grid_for(vec ? (n + 15) / 16 : n)), dim3(256), 0, ctx->stream, dst, src, n, scale, vec);
+   launch_kernel(quantize_linear_kernel, dim3(grid_for(vec ? (n + 3) / 4 : n)), dim3(256), 0, ctx->stream, dst, src, n, scale, vec);
    return launch_status("quantize_linear_kernel");
 }
 
