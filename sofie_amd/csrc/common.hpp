@@ -40,7 +40,7 @@ struct LaunchCfg {
    hipStream_t stream;
    int tile;    // forced tile configuration, 0 = heuristic
    int variant; // alternative of the pipelined kernel
-   int swizzle; // tile order (tile_of_block)
+   int swizzle; // tile order (TileOrder)
 };
 inline LaunchCfg launch_cfg_i8(const sofie_hip_ctx *ctx) { return LaunchCfg{ctx->stream, ctx->opt.i8_tile, ctx->opt.gemm_variant, ctx->opt.swizzle}; }
 inline LaunchCfg launch_cfg_f8(const sofie_hip_ctx *ctx) { return LaunchCfg{ctx->stream, ctx->opt.f8_tile, ctx->opt.gemm_variant, ctx->opt.swizzle}; }

@@ -185,7 +185,7 @@ struct F32Conv3x3Shape {
 // that cover each other's trips to memory and barriers.  WAVES_K waves share a wave tile, each multiplying every WAVES_K-th step of
 // a slab: where there are few tiles, smaller ones keep as many matrix cores busy.
 template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int CS, int PLANE, int WVEC, bool PLAIN>
-__global__ __launch_bounds__(256, 2) void f32_conv3x3_kernel(F32Conv3x3 a, F32ConvStore out, int tiles_m, int tiles_n, int first_tile, int places_at)
+__global__ __launch_bounds__(256, 2) void f32_conv3x3_kernel(F32Conv3x3 a, F32ConvStore out, TileOrder order, int first_tile, int places_at)
 {
    typedef F32Conv3x3Shape<BM, BN, CS, PLANE, WVEC> S;
    constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N, MT = TM / 32, NT = TN / 32;
@@ -197,12 +197,12 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_kernel(F32Conv3x3 a, F32Co
    extern __shared__ __attribute__((aligned(16))) float f32_lds[];
    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
    const int wk = wave % WAVES_K, wm = wave / WAVES_K / WAVES_N, wn = wave / WAVES_K % WAVES_N, lk = lane >> 5, c = lane & 31;
-   const int wave_id = wave, z = blockIdx.z;
+   const int wave_id = wave;
+   int tm, tn, z;
+   order.place(first_tile + blockIdx.x, tm, tn, z);
    a.X += z * a.group;
    a.W += (long long)z * a.N * a.K;
    out.select_batch(z);
-   int tm, tn;
-   f32_tile_of_block(first_tile, tiles_m, tiles_n, tm, tn);
    const int m0 = tm * BM, n0 = tn * BN;
    const int VW = a.OW + 2, VH = a.OH + 2;
    auto quotient = [](int n, const Divisor31 &by) { return (int)by.over((unsigned)n); };
@@ -428,8 +428,9 @@ static int launch_f32_conv3x3_as(hipStream_t stream, const F32Conv3x3 &a, const 
       static bool configured[64] = {};
       if (int st = configure_lds_once(kern, std::max(stage * 2, parts) + PLANE * sizeof(int), configured))
          return st;
-      in_launches((long long)tiles_m * tiles_n, 256, [&](int first, unsigned count) {
-         launch_kernel(kern, dim3(count, 1, (unsigned)group), dim3(256), smem, stream, a, out, tiles_m, tiles_n, first, (int)(slabs / sizeof(int)));
+      const TileOrder order(tiles_m, tiles_n, 4, group);
+      in_launches(order.workgroups(group), 256, [&](int first, unsigned count) {
+         launch_kernel(kern, dim3(count, 1, order.depth(group)), dim3(256), smem, stream, a, out, order, first, (int)(slabs / sizeof(int)));
       });
       return launch_status("f32_conv3x3_kernel");
    };

@@ -70,19 +70,19 @@ struct F32Conv3x3SplitShape {
 // workgroups per CU, one of which splits while the other multiplies.  (One workgroup whose other four waves split for it, through two slabs of pieces, is no
 // faster: 36 us, bound by LDS.)  8 - 14 scalars are spilled, 48 - 70 in the kernels of activations with calls; 256 pixels with narrow weights fill the 256 vector registers.
 template <int BM, int PLANE, int WVEC, bool PLAIN>
-__global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a, F32ConvStore out, int tiles_m, int tiles_n, int first_tile)
+__global__ __launch_bounds__(256, 2) void f32_conv3x3_split_kernel(F32Conv3x3 a, F32ConvStore out, TileOrder order, int first_tile)
 {
    typedef F32Conv3x3SplitShape<PLANE, WVEC> S;
    constexpr int CS = S::CS, BN = S::BN, TM = BM / 4, MT = TM / 32;
    static_assert(TM % 32 == 0 && PLANE % 8 == 0, "wave tiles of 32 x 32 blocks");
    extern __shared__ __attribute__((aligned(16))) char split_lds[];
    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lk = lane >> 5, c = lane & 31;
-   const int wave_id = wave, z = blockIdx.z;
+   const int wave_id = wave;
+   int tm, tn, z;
+   order.place(first_tile + blockIdx.x, tm, tn, z);
    a.X += z * a.group;
    a.W += (long long)z * a.N * a.K;
    out.select_batch(z);
-   int tm, tn;
-   f32_tile_of_block(first_tile, tiles_m, tiles_n, tm, tn);
    const int m0 = tm * BM, n0 = tn * BN;
    const int VW = a.OW + 2, VH = a.OH + 2;
    auto quotient = [](int n, const Divisor31 &by) { return (int)by.over((unsigned)n); };
@@ -321,8 +321,9 @@ static int launch_f32_conv3x3_split_as(hipStream_t stream, const F32Conv3x3 &a, 
       static bool configured[64] = {};
       if (int st = configure_lds_once(kern, smem, configured))
          return st;
-      in_launches((long long)tiles_m * tiles_n, 256, [&](int first, unsigned count) {
-         launch_kernel(kern, dim3(count, 1, (unsigned)group), dim3(256), smem, stream, a, out, tiles_m, tiles_n, first);
+      const TileOrder order(tiles_m, tiles_n, 4, group);
+      in_launches(order.workgroups(group), 256, [&](int first, unsigned count) {
+         launch_kernel(kern, dim3(count, 1, order.depth(group)), dim3(256), smem, stream, a, out, order, first);
       });
       return launch_status("f32_conv3x3_split_kernel");
    };

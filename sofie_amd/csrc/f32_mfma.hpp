@@ -27,19 +27,6 @@ __device__ __forceinline__ v4f mfma_f32_step(const v4f &n_side, const v4f &m_sid
    return acc;
 }
 
-// tile_of_block for a launch of in_launches; a single column of tiles (the usual convolution) needs none of its divisions
-__device__ __forceinline__ void f32_tile_of_block(int first, int tiles_m, int tiles_n, int &tm, int &tn)
-{
-   const int bid = first + blockIdx.x;
-   if (tiles_n == 1) {
-      const int per = tiles_m / 8, rem = tiles_m % 8, xcd = bid % 8;
-      tm = xcd * per + (xcd < rem ? xcd : rem) + bid / 8;
-      tn = 0;
-   } else {
-      tile_of_block(bid, tiles_m * tiles_n, tiles_m, tiles_n, 4, tm, tn);
-   }
-}
-
 // a value that is the same in all lanes, in scalar registers
 __device__ __forceinline__ long long uniform(long long v)
 {
@@ -603,8 +590,7 @@ constexpr size_t f32_tile_lds_bytes(int stages)
 // filled round of tiles where there are not.  WAVES_K waves share a wave tile: each takes its part of the k of every slab,
 // which puts all four SIMDs of a CU to work on tiles smaller than four blocks of 32 x 32.
 template <class ASRC, class BSRC, class STORE, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int WAVES_K, int STAGES>
-__global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_kernel(ASRC A, BSRC B, STORE out, int M, int N, int K, int tiles_m,
-                                                                                   int tiles_n, int first_tile, long long strideA, long long strideB)
+__global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_kernel(ASRC A, BSRC B, STORE out, int M, int N, int K, TileOrder order, int first_tile, long long strideA, long long strideB)
 {
    constexpr int NW = WAVES_M * WAVES_N * WAVES_K;
    constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N, MT = TM / 32, NT = TN / 32;
@@ -617,13 +603,12 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_ke
    static_assert((STAGES - 1) * LPT < 64, "vmcnt counts fewer than 64 loads");
    extern __shared__ __attribute__((aligned(16))) float f32_lds[];
 
-   const int z = blockIdx.z;
+   int tm, tn, z;
+   order.place(first_tile + blockIdx.x, tm, tn, z);
    A.shift(z * strideA);
    B.shift(z * strideB);
    A.select_group(z);
    out.select_batch(z);
-   int tm, tn;
-   f32_tile_of_block(first_tile, tiles_m, tiles_n, tm, tn);
    const int m0 = tm * BM, n0 = tn * BN;
    const int lane = threadIdx.x & 63;
    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -851,18 +836,17 @@ __device__ __forceinline__ void f32_direct_store(const STORE &out, const v4f (&a
 // % 16) supplies k = 4 lk + j of row c to MFMA j); the partial tiles meet in LDS.  What such a product
 // costs is one trip to memory for its operands: every wave has UNROLL steps of loads in flight at once.
 template <class ASRC, class BSRC, class STORE, int MB, int NB, int W, int UNROLL>
-__global__ __launch_bounds__(W * 64) void f32_direct_kernel(ASRC A, BSRC B, STORE out, int M, int N, int K, int tiles_m, int tiles_n, int first_tile,
+__global__ __launch_bounds__(W * 64) void f32_direct_kernel(ASRC A, BSRC B, STORE out, int M, int N, int K, TileOrder order, int first_tile,
                                                             long long strideA, long long strideB)
 {
    constexpr int TM = MB * 16, TN = NB * 16, PITCH = TN + 4;
    __shared__ __attribute__((aligned(16))) float part[W][TM][PITCH];
-   const int z = blockIdx.z;
+   int tm, tn, z;
+   order.place(first_tile + blockIdx.x, tm, tn, z);
    A.shift(z * strideA);
    B.shift(z * strideB);
    A.select_group(z);
    out.select_batch(z);
-   int tm, tn;
-   f32_tile_of_block(first_tile, tiles_m, tiles_n, tm, tn);
    const int m0 = tm * TM, n0 = tn * TN;
    const int lane = threadIdx.x & 63;
    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -920,16 +904,15 @@ struct DirectF32 {
    }
 };
 template <class STORE, int MB, int NB, int W>
-__global__ __launch_bounds__(W * 64) void f32_direct_ring_kernel(RowMajorRows A, RowMajorRows B, STORE out, int M, int N, int K, int tiles_m, int tiles_n, int first_tile,
+__global__ __launch_bounds__(W * 64) void f32_direct_ring_kernel(RowMajorRows A, RowMajorRows B, STORE out, int M, int N, int K, TileOrder order, int first_tile,
                                                                  long long strideA, long long strideB, int depth)
 {
    extern __shared__ __attribute__((aligned(16))) int8_t smem[];
-   const int z = blockIdx.z;
+   int tm, tn, z;
+   order.place(first_tile + blockIdx.x, tm, tn, z);
    A.base += z * strideA;
    B.base += z * strideB;
    out.select_batch(z);
-   int tm, tn;
-   f32_tile_of_block(first_tile, tiles_m, tiles_n, tm, tn);
    const int m0 = tm * MB * 16, n0 = tn * NB * 16;
    const int lane = threadIdx.x & 63;
    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -964,8 +947,9 @@ static int launch_f32_tile(hipStream_t stream, const ASRC &A, const BSRC &B, con
    if (int st = configure_lds_once(kern, most, configured))
       return st;
    constexpr int NTHREADS = WAVES_M * WAVES_N * WAVES_K * 64;
-   in_launches(nwg, NTHREADS, [&](int first, unsigned count) {
-      launch_kernel(kern, dim3(count, 1, (unsigned)batch), dim3(NTHREADS), smem, stream, A, B, out, M, N, K, tiles_m, tiles_n, first, strideA, strideB);
+   const TileOrder order(tiles_m, tiles_n, 4, batch);
+   in_launches(order.workgroups(batch), NTHREADS, [&](int first, unsigned count) {
+      launch_kernel(kern, dim3(count, 1, order.depth(batch)), dim3(NTHREADS), smem, stream, A, B, out, M, N, K, order, first, strideA, strideB);
    });
    return launch_status("f32_tile_kernel");
 }
@@ -977,6 +961,7 @@ static int launch_f32_direct(hipStream_t stream, const ASRC &A, const BSRC &B, c
    const long long nwg = (long long)tiles_m * tiles_n;
    if (nwg > 0x7fffffffLL)
       return fail(SOFIE_HIP_ERR_INVALID, "fp32 product: too many tiles");
+   const TileOrder order(tiles_m, tiles_n, 4, batch);
    if constexpr (ASRC::KC && BSRC::KC && ASRC::VEC == 4 && BSRC::VEC == 4) {
       typedef DirectRing<MB, NB, W> Ring;
       // A single step has nothing to pipeline: 64 x 640 x 32 2.83 us, 2.89 through the ring, 130 x 1500 x 32 9 % longer.  Few rows that do not start on lines take two
@@ -989,16 +974,16 @@ static int launch_f32_direct(hipStream_t stream, const ASRC &A, const BSRC &B, c
          if (int st = configure_lds_once(kern, 128 * 1024, configured))
             return st;
          const RowMajorRows a{(const int8_t *)A.p, (int)(A.ld * 4)}, b{(const int8_t *)B.p, (int)(B.ld * 4)};
-         in_launches(nwg, W * 64, [&](int first, unsigned count) {
-            launch_kernel(kern, dim3(count, 1, (unsigned)batch), dim3(W * 64), ring.bytes, stream, a, b, out, M, N, K * 4, tiles_m, tiles_n, first, strideA * 4,
+         in_launches(order.workgroups(batch), W * 64, [&](int first, unsigned count) {
+            launch_kernel(kern, dim3(count, 1, order.depth(batch)), dim3(W * 64), ring.bytes, stream, a, b, out, M, N, K * 4, order, first, strideA * 4,
                           strideB * 4, ring.depth);
          });
          return launch_status("f32_direct_ring_kernel");
       }
    }
-   in_launches(nwg, W * 64, [&](int first, unsigned count) {
-      launch_kernel((f32_direct_kernel<ASRC, BSRC, STORE, MB, NB, W, UNROLL>), dim3(count, 1, (unsigned)batch), dim3(W * 64), 0, stream, A, B, out, M, N, K, tiles_m,
-                    tiles_n, first, strideA, strideB);
+   in_launches(order.workgroups(batch), W * 64, [&](int first, unsigned count) {
+      launch_kernel((f32_direct_kernel<ASRC, BSRC, STORE, MB, NB, W, UNROLL>), dim3(count, 1, order.depth(batch)), dim3(W * 64), 0, stream, A, B, out, M, N, K, order,
+                    first, strideA, strideB);
    });
    return launch_status("f32_direct_kernel");
 }

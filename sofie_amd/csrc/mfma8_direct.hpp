@@ -139,15 +139,14 @@ __device__ __forceinline__ void direct_store(const EPI &ep, const typename MMA::
 }
 
 template <class MMA, int MB, int NB, int W, int UNROLL, class EPI>
-__global__ __launch_bounds__(W * 64) void mfma8_direct_kernel(RowMajorRows A, RowMajorRows Bt, int M, int N, int K, EPI ep, int tiles_m, int tiles_n, int sw,
-                                                              int first_tile)
+__global__ __launch_bounds__(W * 64) void mfma8_direct_kernel(RowMajorRows A, RowMajorRows Bt, int M, int N, int K, EPI ep, TileOrder order, int first_tile)
 {
    constexpr int STEP = 128, TM = MB * 16, TN = NB * 16, PITCH = TN + 4;
    typedef typename MMA::acc_t acc_t;
    typedef typename MMA::elem_t elem_t;
    __shared__ __attribute__((aligned(16))) elem_t part[W][TM][PITCH];
    int tm, tn;
-   tile_of_block(first_tile + blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, sw, tm, tn);
+   order.place(first_tile + blockIdx.x, tm, tn);
    const int m0 = tm * TM, n0 = tn * TN;
    const int lane = threadIdx.x & 63;
    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -292,12 +291,11 @@ __device__ __forceinline__ void direct_ring_sums(typename MMA::acc_t (&acc)[MB][
 }
 
 template <class MMA, int MB, int NB, int W, class EPI>
-__global__ __launch_bounds__(W * 64) void mfma8_direct_ring_kernel(RowMajorRows A, RowMajorRows Bt, int M, int N, int K, EPI ep, int tiles_m, int tiles_n, int sw,
-                                                                   int first_tile, int depth)
+__global__ __launch_bounds__(W * 64) void mfma8_direct_ring_kernel(RowMajorRows A, RowMajorRows Bt, int M, int N, int K, EPI ep, TileOrder order, int first_tile, int depth)
 {
    extern __shared__ __attribute__((aligned(16))) int8_t smem[];
    int tm, tn;
-   tile_of_block(first_tile + blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, sw, tm, tn);
+   order.place(first_tile + blockIdx.x, tm, tn);
    const int m0 = tm * MB * 16, n0 = tn * NB * 16;
    const int lane = threadIdx.x & 63;
    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -349,6 +347,7 @@ static int launch_mfma8_direct(const LaunchCfg &lc, const int8_t *A, const int8_
    const long long nwg = (long long)tiles_m * tiles_n;
    if (nwg > 0x7fffffffLL)
       return fail(SOFIE_HIP_ERR_INVALID, "gemm: too many tiles");
+   const TileOrder order(tiles_m, tiles_n, lc.swizzle);
    typedef DirectRing<MB, NB, W> Ring;
    if (mfma8_direct_by_lines(MB * 16, M, N, K) && Ring::takes(A, Bt, lda, ldb, K)) {
       const Ring ring(nwg, K);
@@ -357,14 +356,14 @@ static int launch_mfma8_direct(const LaunchCfg &lc, const int8_t *A, const int8_
       if (int st = configure_lds_once(kern, 128 * 1024, configured))
          return st;
       in_launches(nwg, W * 64, [&](int first, unsigned count) {
-         launch_kernel(kern, dim3(count), dim3(W * 64), ring.bytes, lc.stream, RowMajorRows{A, lda}, RowMajorRows{Bt, ldb}, M, N, K, ep, tiles_m, tiles_n,
-                       lc.swizzle, first, ring.depth);
+         launch_kernel(kern, dim3(count), dim3(W * 64), ring.bytes, lc.stream, RowMajorRows{A, lda}, RowMajorRows{Bt, ldb}, M, N, K, ep, order, first,
+                       ring.depth);
       });
       return launch_status("mfma8_direct_ring_kernel");
    }
    in_launches(nwg, W * 64, [&](int first, unsigned count) {
       launch_kernel((mfma8_direct_kernel<MMA, MB, NB, W, UNROLL, EPI>), dim3(count), dim3(W * 64), 0, lc.stream, RowMajorRows{A, lda}, RowMajorRows{Bt, ldb}, M, N, K, ep,
-                    tiles_m, tiles_n, lc.swizzle, first);
+                    order, first);
    });
    return launch_status("mfma8_direct_kernel");
 }

@@ -9,8 +9,7 @@ namespace sofie_hip {
 
 // KP: the padded reduction length.  OCC: waves per SIMD the register allocation leaves room for.
 template <class MMA, int BM, int BN, int BK, int WAVES_M, int WAVES_N, class EPI, int KP, int OCC>
-__global__ __launch_bounds__(WAVES_M *WAVES_N * 64, OCC) void mfma8_gather_kernel(GatherConvRowsT<KP> A, RowMajorRows Bt, int M, int N, EPI ep, int tiles_m,
-                                                                                int tiles_n, int sw)
+__global__ __launch_bounds__(WAVES_M *WAVES_N * 64, OCC) void mfma8_gather_kernel(GatherConvRowsT<KP> A, RowMajorRows Bt, int M, int N, EPI ep, TileOrder order)
 {
    constexpr int NTHREADS = WAVES_M * WAVES_N * 64;
    constexpr int CPR = BK / 16;
@@ -28,7 +27,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, OCC) void mfma8_gather_kerne
    int8_t *sB = smem + BM * BK; // [BN*BK]
 
    int tm, tn;
-   tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, sw, tm, tn);
+   order.place(blockIdx.x, tm, tn);
    const int m0 = tm * BM, n0 = tn * BN;
    const int t = threadIdx.x;
    const int lane = t & 63, wave = t >> 6;
@@ -157,7 +156,7 @@ static int launch_mfma8_gather_kp(const LaunchCfg &lc, const GatherConvRows &a, 
       return st;
    GatherConvRowsT<KP> src;
    static_cast<GatherConvRows &>(src) = a;
-   launch_kernel(kern, dim3((unsigned)nwg), dim3(256), smem, lc.stream, src, RowMajorRows{Wp, KP}, M, N, ep, tiles_m, tiles_n, 0);
+   launch_kernel(kern, dim3((unsigned)nwg), dim3(256), smem, lc.stream, src, RowMajorRows{Wp, KP}, M, N, ep, TileOrder(tiles_m, tiles_n, 0));
    return launch_status("mfma8_gather_kernel");
 }
 

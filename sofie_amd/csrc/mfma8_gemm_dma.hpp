@@ -29,7 +29,7 @@ __device__ __forceinline__ void wait_vmcnt()
 // workgroup's tile store overlaps the other's K loop.
 template <class MMA, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int STAGES, class EPI, class ASRC = RowMajorRows, int OCC = 1>
 __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, OCC) void mfma8_gemm_dma_kernel(ASRC A, RowMajorRows Bt, int M, int N,
-                                                                                int K, EPI ep, int tiles_m, int tiles_n, int sw)
+                                                                                int K, EPI ep, TileOrder order)
 {
    constexpr int NW = WAVES_M * WAVES_N;
    constexpr int CPR = BK / 16;           // 16-byte chunks per LDS row
@@ -48,7 +48,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, OCC) void mfma8_gemm_dma_ker
    extern __shared__ __attribute__((aligned(16))) int8_t smem[];
 
    int tm, tn;
-   tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, sw, tm, tn);
+   order.place(blockIdx.x, tm, tn);
    const int m0 = tm * BM, n0 = tn * BN;
    const int t = threadIdx.x;
    const int lane = t & 63;
@@ -211,7 +211,7 @@ static int launch_mfma8_dma_src(const LaunchCfg &lc, const ASRC &a, const int8_t
    static bool configured[64] = {};
    if (int st = configure_lds_once(kern, smem, configured))
       return st;
-   launch_kernel(kern, dim3((unsigned)nwg), dim3(NTHREADS), smem, lc.stream, a, b, M, N, K, ep, tiles_m, tiles_n, lc.swizzle);
+   launch_kernel(kern, dim3((unsigned)nwg), dim3(NTHREADS), smem, lc.stream, a, b, M, N, K, ep, TileOrder(tiles_m, tiles_n, lc.swizzle));
    return launch_status("mfma8_gemm_dma_kernel");
 }
 

@@ -245,7 +245,7 @@ struct StagedSlab<StagedColumns, R, BK, NTHREADS> {
 };
 
 template <class MMA, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int DEPTH, class ASRC, class BSRC, class EPI>
-__global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void mfma8_staged_kernel(ASRC A, BSRC B, int M, int N, int K, EPI ep, int tiles_m, int tiles_n, int sw)
+__global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void mfma8_staged_kernel(ASRC A, BSRC B, int M, int N, int K, EPI ep, TileOrder order)
 {
    constexpr int NTHREADS = WAVES_M * WAVES_N * 64;
    constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N, MT = TM / 32, NT = TN / 32;
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void mfma8_staged_kernel(
    extern __shared__ __attribute__((aligned(16))) int8_t smem[];
 
    int tm, tn;
-   tile_of_block(blockIdx.x, gridDim.x, tiles_m, tiles_n, sw, tm, tn);
+   order.place(blockIdx.x, tm, tn);
    const int m0 = tm * BM, n0 = tn * BN;
    const int t = threadIdx.x, lane = t & 63;
    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -373,7 +373,7 @@ static int launch_mfma8_staged(const LaunchCfg &lc, const ASRC &A, const BSRC &B
    static bool configured[64] = {};
    if (int st = configure_lds_once(kern, smem, configured))
       return st;
-   launch_kernel(kern, dim3((unsigned)nwg), dim3(WAVES_M * WAVES_N * 64), smem, lc.stream, A, B, M, N, K, ep, tiles_m, tiles_n, lc.swizzle);
+   launch_kernel(kern, dim3((unsigned)nwg), dim3(WAVES_M * WAVES_N * 64), smem, lc.stream, A, B, M, N, K, ep, TileOrder(tiles_m, tiles_n, lc.swizzle));
    return launch_status("mfma8_staged_kernel");
 }
 
