@@ -57,9 +57,9 @@ int sofie_hip_ctx_destroy(sofie_hip_ctx *ctx);
  *   "swizzle"              tile order
  *   "conv_explicit"        1: int8 convolutions through a column matrix whenever the workspace holds one
  *   "f32_tile"             0 = heuristic; 16 the direct kernel; 32, 62, 64, 126, 128 the tile kernel with tiles of 32 x 32, 64 x 32,
- *                          64 x 64, 128 x 32 (convolutions), 128 x 128 (products); 3032, 3064, 3128 the kernel of 3 x 3 convolutions with
- *                          tiles of 32, 64, 128 pixels, 4128, 4256 the one that multiplies bf16 pieces, with 128, 256 (64 x 64 tiles for
- *                          what they do not take); a call refuses any other value
+ *                          64 x 64, 128 x 32 (convolutions), 128 x 128 (products); of 3 x 3 convolutions 3004 the kernel for up to
+ *                          four input channels, 3032, 3064, 3128 the one with tiles of 32, 64, 128 pixels, 4128, 4256 the one that
+ *                          multiplies bf16 pieces, with 128, 256 (64 x 64 tiles for what they do not take); a call refuses any other value
  *   "f32_skinny"           -1 = heuristic; 1 the direct kernel, 0 the 64 x 64 tiles where "f32_tile" is 0
  *   "f32_chain"            -1 = heuristic; 1 all layers of sofie_hip_gemm_chain_f32 in one launch if they allow it, 0 each by itself
  * Each is also read once, at sofie_hip_ctx_create, from the environment variable SOFIE_HIP_<NAME IN CAPITALS>; nothing reads the

@@ -1,5 +1,6 @@
 // fp32 Gemm / MatMul and fp32 convolution (implicit GEMM) with the bias + activation epilogue fused into the store: the entry
 // points and the choice among the kernels of f32_mfma.hpp, and the kernel that runs a chain of small products in one launch.
+#include "f32_conv3x3_few.hpp"
 #include "f32_conv3x3_split.hpp"
 #include <algorithm>
 #include <cmath>
@@ -192,7 +193,7 @@ namespace sofie_hip {
 // along k), 0.2 % and 0.2 % (16 bytes, along k) above the best kernel's time.  Costs without the rows were 2.1, 1.6, 0.7 and 0.7 % above, and a third on a few rows of long k
 // (4 x 3545 x 468, float by float: 6.6 us, now 4.9; 4 x 4096 x 192, 16 bytes: 4.2, now 3.7).  (Launches take 0.4 us more or less from one card to another; these are of
 // the shorter kind, as the chain's costs below are.)
-enum F32Tile { F32_CONV3X3_32 = 3032, F32_CONV3X3_64 = 3064, F32_CONV3X3_128 = 3128, F32_CONV3X3_SPLIT_128 = 4128, F32_CONV3X3_SPLIT_256 = 4256, F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
+enum F32Tile { F32_CONV3X3_FEW = 3004, F32_CONV3X3_32 = 3032, F32_CONV3X3_64 = 3064, F32_CONV3X3_128 = 3128, F32_CONV3X3_SPLIT_128 = 4128, F32_CONV3X3_SPLIT_256 = 4256, F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
 // Pixels of a tile of the 3 x 3 convolution kernels; 0 for any other kernel.
 static int conv3x3_pixels(int tile)
 {
@@ -277,7 +278,7 @@ static int launch_f32_product(sofie_hip_ctx *ctx, const ASRC &A, const BSRC &B, 
    constexpr bool CONV = ASRC::kLeastRows == 64;
    if (!tile)
       tile = CONV ? pick_f32_conv_tile(M, N, K, batch) : pick_f32_tile(M, N, K, batch, f32_loads(ASRC::VEC == 4 && BSRC::VEC == 4, ASRC::KC && BSRC::KC));
-   if (conv3x3_pixels(tile) || (CONV ? tile == F32_TILE_32 || tile == F32_TILE_128 : tile == F32_TILE_128x32))
+   if (conv3x3_pixels(tile) || tile == F32_CONV3X3_FEW || (CONV ? tile == F32_TILE_32 || tile == F32_TILE_128 : tile == F32_TILE_128x32))
       tile = F32_TILE_64; // a request for a tile that the other kind of product has
    if constexpr (CONV) {
       switch (tile) {
@@ -311,10 +312,14 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
    if ((most * s.C + s.Cg) * plane * 4 >= F32_BUFFER_BYTES || 128LL * K * 4 >= F32_BUFFER_BYTES)
       return SOFIE_HIP_OK;
    const bool vec = ((uintptr_t)W & 15) == 0 && K % 4 == 0;
+   F32Conv3x3 a{X, W, images, s.Cg, s.H, s.W, s.OH, s.OW, s.pad_h, s.pad_w, plane * s.C, plane * s.Cg, M, N, K, 0, 0, Divisor31(s.OW), Divisor31(s.OH),
+                Divisor31(s.OW + 2LL), Divisor31(s.OH + 2LL)};
    int tile = force;
-   if (!tile && s.Cg <= 4) {
-      tile = F32_CONV3X3_128; // slabs of four channels; half of any other kernel's slab would be zeros
-   } else if (!tile) {
+   if ((!tile || tile == F32_CONV3X3_FEW) && f32_conv3x3_few_takes(a, out)) {
+      *taken = true;
+      return launch_f32_conv3x3_few(ctx->stream, a, out, group);
+   }
+   if (!tile) {
       // us: a launch; a slab (8 channels, 16 of the split kernel) of a CU whose tiles wait for their loads, and of one with several tiles at work; a tile.  The
       // second set is for weights that come float by float.  Fitted to 156 layers (the split kernel's to 230 others) from 1 image of 6 x 6 to 64 of 64 x 64, 5 to 130
       // channels; holds to a sixth, and costs 0.4 % of the best of these kernels on average over the 260 layers, 14 % the most, 10 % but for that one.
@@ -347,8 +352,8 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
       return SOFIE_HIP_OK;
    // the images that 256 pixels touch, all their channels
    const int near = (255 / ((long long)s.OH * s.OW) + 2) * (long long)out.Cout * out.positions * 4 < F32_BUFFER_BYTES - (1 << 20);
-   const F32Conv3x3 a{X, W, images, s.Cg, s.H, s.W, s.OH, s.OW, s.pad_h, s.pad_w, plane * s.C, plane * s.Cg, M, N, K, (int)(patch + 63) / 64, near,
-                      Divisor31(s.OW), Divisor31(s.OH), Divisor31(s.OW + 2LL), Divisor31(s.OH + 2LL)};
+   a.chunks = (int)(patch + 63) / 64;
+   a.near = near;
    *taken = true;
    hipStream_t st = ctx->stream;
    if (split) {
@@ -363,12 +368,10 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
    }
    auto go = [&](auto room, auto wide) {
       constexpr int P = decltype(room)::value, V = decltype(wide)::value;
-      if (s.Cg <= 4 && tile == F32_CONV3X3_128)
-         return launch_f32_conv3x3_as<128, 32, 4, 1, 1, 4, P, 1>(st, a, out, group);
       switch (tile) {
-      case F32_CONV3X3_32: return launch_f32_conv3x3_as<32, 32, 1, 1, 4, 8, P, V>(st, a, out, group);
-      case F32_CONV3X3_64: return launch_f32_conv3x3_as<64, 32, 2, 1, 2, 8, P, V>(st, a, out, group);
-      default: return launch_f32_conv3x3_as<128, 32, 4, 1, 1, 8, P, V>(st, a, out, group);
+      case F32_CONV3X3_32: return launch_f32_conv3x3_as<32, 32, 1, 1, 4, P, V>(st, a, out, group);
+      case F32_CONV3X3_64: return launch_f32_conv3x3_as<64, 32, 2, 1, 2, P, V>(st, a, out, group);
+      default: return launch_f32_conv3x3_as<128, 32, 4, 1, 1, P, V>(st, a, out, group);
       }
    };
    auto with = [&](auto room) { return vec ? go(room, std::integral_constant<int, 4>{}) : go(room, std::integral_constant<int, 1>{}); };
