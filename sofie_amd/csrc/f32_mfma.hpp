@@ -115,20 +115,28 @@ struct F32Matrix {
       const int r = row < rows ? row : rows - 1;
       return row_state{KC ? p + (long long)r * ld : p + r};
    }
-   // `left`: how many k there are from k on, negative past K
+   // WHOLE: k..k+3 lie before K.  Otherwise `left` of them do, none if it is negative: what lies past K is read as the first k of the row, and dropped.  No branch
+   // stands between the loads.
+   template <bool WHOLE>
    __device__ __forceinline__ v4f fetch(const row_state &st, int k, int left) const
    {
-      v4f v = {0.f, 0.f, 0.f, 0.f};
-      if (KC && VEC == 4) {
-         if (left > 0)
-            v = *(const v4f *)(st.at + k);
+      typedef float v4f_by_floats __attribute__((ext_vector_type(4), aligned(4)));
+      if constexpr (KC && (VEC == 4 || WHOLE)) {
+         const v4f v = *(const v4f_by_floats *)(st.at + (WHOLE || left > 0 ? k : 0));
+         return WHOLE || left > 0 ? v : v4f{0.f, 0.f, 0.f, 0.f};
       } else {
+         v4f v;
+         const float *at = st.at + (KC ? (long long)k : (long long)k * ld);
+#pragma unroll
+         for (int j = 0; j < 4; ++j) {
+            const float *from = at + (KC ? (long long)j : j * ld);
+            v[j] = *(WHOLE || j < left ? from : st.at);
+         }
 #pragma unroll
          for (int j = 0; j < 4; ++j)
-            if (j < left)
-               v[j] = st.at[KC ? (long long)(k + j) : (long long)(k + j) * ld];
+            v[j] = WHOLE || j < left ? v[j] : 0.f;
+         return v;
       }
-      return v;
    }
 };
 
@@ -283,6 +291,7 @@ struct F32ConvRows {
          __builtin_amdgcn_global_load_lds((global_void_t *)at, to, 4, 0, 0);
       }
    }
+   template <bool>
    __device__ __forceinline__ v4f fetch(const row_state &st, int k, int) const
    {
       v4f v;
@@ -378,7 +387,36 @@ struct F32RowStore {
       if (ep.R)
          ep.R += b * strideY;
    }
-   __device__ __forceinline__ void put(float acc, int m, int n) const { Y[m * ldy + n] = f32_epilogue(ep, acc, m, n); }
+   // what is added to the element (m, n): asked for before the products it is there when they are done
+   struct added {
+      float bias, residual;
+   };
+   __device__ __forceinline__ added look_up(int m, int n) const
+   {
+      added a = {0.0f, 0.0f};
+      switch (ep.bias_mode) {
+      case SOFIE_BIAS_ROW: a.bias = ep.C[n]; break;
+      case SOFIE_BIAS_COL: a.bias = ep.C[m]; break;
+      case SOFIE_BIAS_SCALAR: a.bias = ep.C[0]; break;
+      case SOFIE_BIAS_FULL: a.bias = ep.C[m * ep.ldc + n]; break;
+      default: break;
+      }
+      if (ep.R)
+         a.residual = ep.R[m * ep.ldr + n];
+      return a;
+   }
+   // f32_epilogue
+   __device__ __forceinline__ void put(float acc, int m, int n, const added &a) const
+   {
+      float v = ep.alpha * acc;
+      if (ep.bias_mode == SOFIE_BIAS_FULL)
+         v += ep.beta * a.bias;
+      else if (ep.bias_mode >= SOFIE_BIAS_ROW && ep.bias_mode <= SOFIE_BIAS_SCALAR)
+         v += a.bias;
+      if (ep.R)
+         v += a.residual;
+      Y[m * ldy + n] = f32_activate(v, ep.chain);
+   }
    // the bias of columns n..n+3, where each has its own: asked for before the products it is there when they are done
    __device__ __forceinline__ v4f ahead(int n, int N) const
    {
@@ -479,7 +517,9 @@ struct F32ConvStore {
          if (n[i] < N)
             Y[at[i]] = v[i];
    }
-   __device__ __forceinline__ void put(float v, int m, int n) const
+   struct added {};
+   __device__ __forceinline__ added look_up(int, int) const { return added{}; }
+   __device__ __forceinline__ void put(float v, int m, int n, const added &) const
    {
       float one[1] = {v};
       const int col[1] = {n};
@@ -806,38 +846,53 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *WAVES_K * 64, 2) void f32_tile_ke
 }
 
 // ---- the direct kernel --------------------------------------------------------------------------------------------------------
-// The partial tiles of W waves meet in LDS and are stored.
+// The partial tiles of W waves meet in LDS and are stored, an element by a thread.
 template <int MB, int NB, int W, class STORE>
-__device__ __forceinline__ void f32_direct_store(const STORE &out, const v4f (&acc)[MB][NB], float (*part)[MB * 16][NB * 16 + 4], int m0, int n0, int M, int N, int wave, int lane)
-{
-   constexpr int TM = MB * 16, TN = NB * 16;
-   const int lk = lane >> 4, c = lane & 15;
-#pragma unroll
-   for (int i = 0; i < MB; ++i)
-#pragma unroll
-      for (int j = 0; j < NB; ++j)
-         *(v4f *)&part[wave][i * 16 + c][j * 16 + lk * 4] = acc[i][j];
-   __syncthreads();
-#pragma unroll 1
-   for (int e = threadIdx.x; e < TM * TN; e += W * 64) {
-      // neighbouring threads store neighbouring elements of the direction that is contiguous in the result
-      const int r = STORE::kAlongRows ? e % TM : e / TN, q = STORE::kAlongRows ? e / TM : e % TN;
-      float v = part[0][r][q];
-#pragma unroll
-      for (int w = 1; w < W; ++w)
-         v += part[w][r][q];
-      const int m = m0 + r, n = n0 + q;
-      if (m < M && n < N)
-         out.put(v, m, n);
+struct F32DirectStore {
+   static constexpr int TM = MB * 16, TN = NB * 16;
+   static_assert(TM * TN <= W * 64, "an element by a thread");
+   int r, q; // neighbouring threads store neighbouring elements of the direction that is contiguous in the result
+   bool live;
+   typename STORE::added added = {};
+   __device__ __forceinline__ F32DirectStore(int m0, int n0, int M, int N)
+   {
+      const int e = threadIdx.x;
+      r = STORE::kAlongRows ? e % TM : e / TN, q = STORE::kAlongRows ? e / TM : e % TN;
+      live = e < TM * TN && m0 + r < M && n0 + q < N;
    }
-}
+   // what is added to the element, behind the first loads of the operands
+   __device__ __forceinline__ void ask(const STORE &out, int m0, int n0)
+   {
+      if (live)
+         added = out.look_up(m0 + r, n0 + q);
+   }
+   __device__ __forceinline__ void store(const STORE &out, const v4f (&acc)[MB][NB], float (*part)[TM][TN + 4], int m0, int n0, int wave, int lane) const
+   {
+      const int lk = lane >> 4, c = lane & 15;
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+         for (int j = 0; j < NB; ++j)
+            *(v4f *)&part[wave][i * 16 + c][j * 16 + lk * 4] = acc[i][j];
+      __syncthreads();
+      if (live) {
+         float v = part[0][r][q];
+#pragma unroll
+         for (int w = 1; w < W; ++w)
+            v += part[w][r][q];
+         out.put(v, m0 + r, n0 + q, added);
+      }
+   }
+};
 
 // W waves split the reduction of one (16 MB) x (16 NB) tile in steps of 16 k (v_mfma_f32_16x16x4_f32: lane (lk = lane / 16, c = lane
 // % 16) supplies k = 4 lk + j of row c to MFMA j); the partial tiles meet in LDS.  What such a product
-// costs is one trip to memory for its operands: every wave has UNROLL steps of loads in flight at once.
+// costs is one trip to memory for its operands: every wave has UNROLL steps of loads in flight at once.  No step but the last looks at its k, and no branch stands
+// between loads: with one around each, a wave alone on its SIMD took as long for them as for the trip.  us, before -> after, with the bias asked for behind the first
+// loads: 64 x 10 x 64 3.09 -> 2.57, 256 x 10 x 256 4.2 -> 3.05, 16 x 10 x 333 4.4 -> 2.95, 100 x 33 x 77 3.7 -> 2.95, 200 x 17 x 50 3.5 -> 2.75, 1 x 1000 x 2048 5.9 -> 5.6.
 template <class ASRC, class BSRC, class STORE, int MB, int NB, int W, int UNROLL>
-__global__ __launch_bounds__(W * 64) void f32_direct_kernel(ASRC A, BSRC B, STORE out, int M, int N, int K, TileOrder order, int first_tile,
-                                                            long long strideA, long long strideB)
+__global__ __launch_bounds__(W * 64) void f32_direct_kernel(ASRC A, BSRC B, STORE out, int M, int N, int K, TileOrder order, int first_tile, long long strideA,
+                                                            long long strideB)
 {
    constexpr int TM = MB * 16, TN = NB * 16, PITCH = TN + 4;
    __shared__ __attribute__((aligned(16))) float part[W][TM][PITCH];
@@ -865,21 +920,38 @@ __global__ __launch_bounds__(W * 64) void f32_direct_kernel(ASRC A, BSRC B, STOR
 #pragma unroll
       for (int j = 0; j < NB; ++j)
          acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+   F32DirectStore<MB, NB, W, STORE> store(m0, n0, M, N);
    const int KS = (int)(((unsigned)K + 15) / 16);
    for (int s0 = wave; s0 < KS; s0 += W * UNROLL) {
       v4f fa[UNROLL][MB], fb[UNROLL][NB];
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
-         // steps past the end, whose k may leave 31 bits, fetch zeros
-         const unsigned first = (unsigned)(s0 + u * W) * 16;
-         const int k = (int)(first + lk * 4), left = (int)((unsigned)K - first) - lk * 4;
+         const unsigned first = (unsigned)(s0 + u * W) * 16; // of steps past the end it may leave 31 bits
+         auto load = [&](auto whole) {
+            constexpr bool WHOLE = decltype(whole)::value;
+            const int k = (int)(first + lk * 4), left = (int)((unsigned)K - first) - lk * 4;
 #pragma unroll
-         for (int i = 0; i < MB; ++i)
-            fa[u][i] = A.fetch(ra[i], k, left);
+            for (int i = 0; i < MB; ++i)
+               fa[u][i] = A.template fetch<WHOLE>(ra[i], k, left);
 #pragma unroll
-         for (int j = 0; j < NB; ++j)
-            fb[u][j] = B.fetch(rb[j], k, left);
+            for (int j = 0; j < NB; ++j)
+               fb[u][j] = B.template fetch<WHOLE>(rb[j], k, left);
+         };
+         if (first + 16 <= (unsigned)K) {
+            load(std::true_type{});
+         } else if (first < (unsigned)K) {
+            load(std::false_type{});
+         } else {
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+               fa[u][i] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+               fb[u][j] = v4f{0.f, 0.f, 0.f, 0.f};
+         }
       }
+      if (s0 == wave)
+         store.ask(out, m0, n0);
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
@@ -888,7 +960,9 @@ __global__ __launch_bounds__(W * 64) void f32_direct_kernel(ASRC A, BSRC B, STOR
             for (int j = 0; j < NB; ++j)
                acc[i][j] = mfma_f32_step(fb[u][j], fa[u][i], acc[i][j]);
    }
-   f32_direct_store<MB, NB, W>(out, acc, part, m0, n0, M, N, wave, lane);
+   if (wave >= KS)
+      store.ask(out, m0, n0);
+   store.store(out, acc, part, m0, n0, wave, lane);
 }
 
 // The same through LDS, where both operands are contiguous in k and their rows start on 16 bytes (see direct_ring_sums): 64 x 128 x 784 takes 4.1 us instead of
@@ -904,8 +978,8 @@ struct DirectF32 {
    }
 };
 template <class STORE, int MB, int NB, int W>
-__global__ __launch_bounds__(W * 64) void f32_direct_ring_kernel(RowMajorRows A, RowMajorRows B, STORE out, int M, int N, int K, TileOrder order, int first_tile,
-                                                                 long long strideA, long long strideB, int depth)
+__global__ __launch_bounds__(W * 64) void f32_direct_ring_kernel(RowMajorRows A, RowMajorRows B, STORE out, int M, int N, int K, TileOrder order, int first_tile, long long strideA,
+                                                                 long long strideB, int depth)
 {
    extern __shared__ __attribute__((aligned(16))) int8_t smem[];
    int tm, tn, z;
@@ -924,8 +998,10 @@ __global__ __launch_bounds__(W * 64) void f32_direct_ring_kernel(RowMajorRows A,
 #pragma unroll
       for (int j = 0; j < NB; ++j)
          acc[i][j] = __builtin_shufflevector(both[i][j], both[i][j], 0, 1, 2, 3) + __builtin_shufflevector(both[i][j], both[i][j], 4, 5, 6, 7);
+   F32DirectStore<MB, NB, W, STORE> store(m0, n0, M, N);
+   store.ask(out, m0, n0);
    __syncthreads();
-   f32_direct_store<MB, NB, W>(out, acc, (float(*)[MB * 16][NB * 16 + 4])smem, m0, n0, M, N, wave, lane);
+   store.store(out, acc, (float(*)[MB * 16][NB * 16 + 4])smem, m0, n0, wave, lane);
 }
 
 // ---- launches -----------------------------------------------------------------------------------------------------------------
