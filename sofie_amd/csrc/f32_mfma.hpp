@@ -370,6 +370,35 @@ __device__ __forceinline__ float f32_epilogue(const F32Epilogue &ep, float acc, 
 {
    return f32_activate(f32_linear(ep, acc, m, n), ep.chain);
 }
+// The same in two parts: what is added to the element (m, n), asked for before the products it is there when they are done, and the rest.
+struct F32Added {
+   float bias, residual;
+};
+__device__ __forceinline__ F32Added f32_look_up(const F32Epilogue &ep, int m, int n)
+{
+   F32Added a = {0.0f, 0.0f};
+   switch (ep.bias_mode) {
+   case SOFIE_BIAS_ROW: a.bias = ep.C[n]; break;
+   case SOFIE_BIAS_COL: a.bias = ep.C[m]; break;
+   case SOFIE_BIAS_SCALAR: a.bias = ep.C[0]; break;
+   case SOFIE_BIAS_FULL: a.bias = ep.C[m * ep.ldc + n]; break;
+   default: break;
+   }
+   if (ep.R)
+      a.residual = ep.R[m * ep.ldr + n];
+   return a;
+}
+__device__ __forceinline__ float f32_finish(const F32Epilogue &ep, float acc, const F32Added &a)
+{
+   float v = ep.alpha * acc;
+   if (ep.bias_mode == SOFIE_BIAS_FULL)
+      v += ep.beta * a.bias;
+   else if (ep.bias_mode >= SOFIE_BIAS_ROW && ep.bias_mode <= SOFIE_BIAS_SCALAR)
+      v += a.bias;
+   if (ep.R)
+      v += a.residual;
+   return f32_activate(v, ep.chain);
+}
 
 // Row-major results of a product.
 struct F32RowStore {
@@ -387,36 +416,9 @@ struct F32RowStore {
       if (ep.R)
          ep.R += b * strideY;
    }
-   // what is added to the element (m, n): asked for before the products it is there when they are done
-   struct added {
-      float bias, residual;
-   };
-   __device__ __forceinline__ added look_up(int m, int n) const
-   {
-      added a = {0.0f, 0.0f};
-      switch (ep.bias_mode) {
-      case SOFIE_BIAS_ROW: a.bias = ep.C[n]; break;
-      case SOFIE_BIAS_COL: a.bias = ep.C[m]; break;
-      case SOFIE_BIAS_SCALAR: a.bias = ep.C[0]; break;
-      case SOFIE_BIAS_FULL: a.bias = ep.C[m * ep.ldc + n]; break;
-      default: break;
-      }
-      if (ep.R)
-         a.residual = ep.R[m * ep.ldr + n];
-      return a;
-   }
-   // f32_epilogue
-   __device__ __forceinline__ void put(float acc, int m, int n, const added &a) const
-   {
-      float v = ep.alpha * acc;
-      if (ep.bias_mode == SOFIE_BIAS_FULL)
-         v += ep.beta * a.bias;
-      else if (ep.bias_mode >= SOFIE_BIAS_ROW && ep.bias_mode <= SOFIE_BIAS_SCALAR)
-         v += a.bias;
-      if (ep.R)
-         v += a.residual;
-      Y[m * ldy + n] = f32_activate(v, ep.chain);
-   }
+   typedef F32Added added;
+   __device__ __forceinline__ added look_up(int m, int n) const { return f32_look_up(ep, m, n); }
+   __device__ __forceinline__ void put(float acc, int m, int n, const added &a) const { Y[m * ldy + n] = f32_finish(ep, acc, a); }
    // the bias of columns n..n+3, where each has its own: asked for before the products it is there when they are done
    __device__ __forceinline__ v4f ahead(int n, int N) const
    {

@@ -11,8 +11,9 @@ namespace sofie_hip {
 // Layer l+1 reads what layer l wrote (an MLP at small batch): per layer launches cost more than the arithmetic, so one
 // workgroup takes RB rows through every layer, the rows of activations staying in LDS between layers (each layer's
 // output is also written to its Y, as separate launches would).  The weights stream from L2 once per workgroup:
-//   transB (W stored [N][K], the ONNX export of a Linear layer): a wave takes 4 outputs at a time, its lanes stride over k
-//     (coalesced 256-byte reads of each weight row), then the 64 partial sums are folded across the lanes;
+//   transB (W stored [N][K], the ONNX export of a Linear layer): groups of lanes take an output each, 16 bytes of its row a lane, then the partial sums are folded across the
+//     lanes (2 rows through 304-16-32-193 7.5 -> 6.1 us, 60 through 160-16-16-176 7.0 -> 5.9, 64 through 784-128-64-10, one launch, 9.7 -> 9.3; rows of W that do not start
+//     on 16 bytes: a wave takes 4 outputs at a time, 256 bytes of each);
 //   else (W stored [K][N]): a thread owns output n and walks k (lanes read consecutive n of one weight row); up to 512 outputs, whose threads alone
 //     would leave the others idle, k is dealt out over groups of threads, and their sums are added up through LDS (39 rows through
 //     256-137-1800-17: 28.6 -> 19.9 us, most of it by taking the first layer into the chain, whose waves were one in eight before; 4 rows through
@@ -64,6 +65,61 @@ __device__ __forceinline__ void chain_walk(float (&acc)[RB], const float *column
    some(std::integral_constant<int, 1>{});
 }
 
+// The sums of J * 64 / G outputs from n0 on, rows of W on 16 bytes: G lanes an output (as many as its row has 16-byte pieces, up to 64), so that a wave's load brings 64 / G rows, and
+// two pieces of J outputs are on their way in every lane.  Lane j of group s of G lanes ends up with output n0 + j 64 / G + s.
+// behind() is called once, with the first of them on their way.
+template <int RB, int G, int J, class F>
+__device__ __forceinline__ void chain_rows(float (&sums)[RB], const ChainLayerArgs &L, int n0, const float *in, int width, int lane, F &&behind)
+{
+   constexpr int P = 64 / G;
+   const int N = L.N, pieces = L.K / 4, sub = lane / G, l = lane % G;
+   const v4f *w[J]; // rows of W past N are read as row N - 1 and their sums dropped
+#pragma unroll
+   for (int j = 0; j < J; ++j)
+      w[j] = (const v4f *)(L.B + (long long)(n0 + j * P + sub < N ? n0 + j * P + sub : N - 1) * L.ldb);
+   float acc[J][RB];
+#pragma unroll
+   for (int j = 0; j < J; ++j)
+#pragma unroll
+      for (int r = 0; r < RB; ++r)
+         acc[j][r] = 0.0f;
+   constexpr int U = G < 64 ? 1 : 2; // rows of fewer than 64 pieces are read at once
+#pragma unroll 1
+   for (int k = l; k - l < pieces; k += U * G) {
+      v4f v[U][J];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+         if (k - l + u * G < pieces) // for some lane
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+               v[u][j] = w[j][k + u * G < pieces ? k + u * G : 0];
+      if (k == l)
+         behind();
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+         if (k + u * G < pieces) {
+#pragma unroll
+            for (int r = 0; r < RB; ++r) {
+               const v4f x = *(const v4f *)(in + r * width + 4 * (k + u * G));
+#pragma unroll
+               for (int j = 0; j < J; ++j)
+#pragma unroll
+                  for (int e = 0; e < 4; ++e)
+                     acc[j][r] = fmaf(v[u][j][e], x[e], acc[j][r]);
+            }
+         }
+   }
+#pragma unroll
+   for (int r = 0; r < RB; ++r) {
+      sums[r] = 0.0f;
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+         const float sum = sum_over_lanes(acc[j][r], G);
+         sums[r] = l == j ? sum : sums[r];
+      }
+   }
+}
+
 template <int RB>
 __global__ __launch_bounds__(CHAIN_THREADS) void gemm_chain_f32_kernel(ChainArgs a, int width)
 {
@@ -87,7 +143,38 @@ __global__ __launch_bounds__(CHAIN_THREADS) void gemm_chain_f32_kernel(ChainArgs
       const ChainLayerArgs &L = a.layer[l];
       const int N = L.N, K = L.K;
       const float *__restrict__ B = L.B;
-      if (L.transB) {
+      if (L.transB && K % 4 == 0 && L.ldb % 4 == 0 && ((uintptr_t)B & 15) == 0) {
+         // four outputs a wave, sixteen where one pass would not do and rows are short enough for as many loads
+         const int g_log2 = K <= 64 ? 4 : K <= 128 ? 5 : 6, j_log2 = N > 64 ? 2 : g_log2 - 4, per_wave = 64 >> g_log2 << j_log2;
+         for (int n0 = wave * per_wave; n0 < N; n0 += CHAIN_THREADS / 64 * per_wave) {
+            const int l = lane & ((1 << g_log2) - 1), n = n0 + (l << (6 - g_log2)) + (lane >> g_log2);
+            const bool mine = l >> j_log2 == 0 && n < N;
+            F32Added added[RB];
+            auto ask = [&]() {
+#pragma unroll
+               for (int r = 0; r < RB; ++r)
+                  added[r] = mine && r < rows ? f32_look_up(L.ep, m0 + r, n) : F32Added{0.0f, 0.0f};
+            };
+            float sums[RB];
+            if (g_log2 == 6)
+               chain_rows<RB, 64, 4>(sums, L, n0, in, width, lane, ask);
+            else if (g_log2 == 5 && j_log2 == 2)
+               chain_rows<RB, 32, 4>(sums, L, n0, in, width, lane, ask);
+            else if (g_log2 == 5)
+               chain_rows<RB, 32, 2>(sums, L, n0, in, width, lane, ask);
+            else if (j_log2 == 2)
+               chain_rows<RB, 16, 4>(sums, L, n0, in, width, lane, ask);
+            else
+               chain_rows<RB, 16, 1>(sums, L, n0, in, width, lane, ask);
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+               if (mine && r < rows) {
+                  const float v = f32_finish(L.ep, sums[r], added[r]);
+                  out[r * width + n] = v;
+                  L.Y[(long long)(m0 + r) * L.ldy + n] = v;
+               }
+         }
+      } else if (L.transB) {
          for (int n0 = wave * 4; n0 < N; n0 += CHAIN_THREADS / 16) {
             float acc[4][RB];
 #pragma unroll
@@ -189,10 +276,10 @@ namespace sofie_hip {
 // loads, and `slab` and `tile` in as many rounds as the tiles need over 256 CUs; operands that come float by float (ragged) take longer.  The direct
 // kernel takes a launch, `alone` per 128 k (16 of each wave) and `row` for every sixteenth of its 16 rows or, where there are many tiles, `slab` per 16 k and 256
 // tiles, and `tile` per 256 tiles; where both operands come line by line through its ring, 78 KB/us a CU and 0.48 us for the first 256 tiles, 73 and 0.49 a tile where
-// there are more.  Fitted to 1220 products of each kind of loads, 20 kFLOP to 30 GFLOP, 1 .. 4096 rows, K = 8 .. 2048: on average 0.5 % (float by float), 0.25 % (float by float
-// along k), 0.2 % and 0.2 % (16 bytes, along k) above the best kernel's time.  Costs without the rows were 2.1, 1.6, 0.7 and 0.7 % above, and a third on a few rows of long k
-// (4 x 3545 x 468, float by float: 6.6 us, now 4.9; 4 x 4096 x 192, 16 bytes: 4.2, now 3.7).  (Launches take 0.4 us more or less from one card to another; these are of
-// the shorter kind, as the chain's costs below are.)
+// there are more.  Fitted to 1220 products of each kind of 16-byte loads, and to 1384 that come float by float, 1 .. 4096 rows, K = 8 .. 2048; on 1500 other products on average 0.15 %
+// (float by float), 0.2 % (float by float along k), 0.13 % and 0.11 % (16 bytes, along k) above the best kernel's time, 18 % the most.  (With the costs of a direct kernel that branched
+// around its loads, those float by float were 7.8 and 9.5 % above, 90 % the most: 291 x 6 x 1532 11.2 us, now 5.9; 2 x 4 x 1991 11.6, now 6.3.  Launches take 0.4 us more or
+// less from one card to another; these are of the shorter kind, as the chain's costs below are.)
 enum F32Tile { F32_CONV3X3_FEW = 3004, F32_CONV3X3_32 = 3032, F32_CONV3X3_64 = 3064, F32_CONV3X3_128 = 3128, F32_CONV3X3_SPLIT_128 = 4128, F32_CONV3X3_SPLIT_256 = 4256, F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
 // Pixels of a tile of the 3 x 3 convolution kernels; 0 for any other kernel.
 static int conv3x3_pixels(int tile)
@@ -217,8 +304,8 @@ static int pick_f32_tile(int M, int N, int K, int batch, F32Loads loads, double 
       Cost direct, tile32, tile64x32, tile64, tile128;
    };
    static constexpr Costs COSTS[] = { // by F32Loads
-      {{2.77, 0.49, 0.096, 0.63, 0.336}, {3.80, 0.03, 0.136, 0.54}, {4.06, 0.26, 0.291, 0.86}, {4.17, 0.09, 0.526, 1.51}, {7.85, 0.37, 2.08, 3.06}},
-      {{2.11, 0.85, 0.284, 0.57, 0.210}, {3.62, 0.03, 0.140, 0.56}, {3.80, 0.39, 0.298, 0.92}, {3.73, 0.11, 0.545, 1.47}, {5.41, 0.39, 2.34, 4.67}},
+      {{2.75, 0.23, 0.063, 0.40, 0.092}, {3.12, 0.15, 0.152, 0.52}, {3.44, 0.32, 0.325, 0.94}, {2.66, 0.57, 0.548, 1.88}, {8.85, 1.77, 2.14, 1.88}},
+      {{2.75, 0.26, 0.066, 0.41, 0.080}, {3.11, 0.14, 0.144, 0.55}, {3.36, 0.25, 0.313, 0.99}, {2.55, 0.21, 0.547, 1.79}, {8.52, 1.81, 2.12, 1.10}},
       {{3.09, 0.31, 0.068, 0.38, 0.038}, {3.06, 0.09, 0.134, 0.53}, {3.64, 0.14, 0.262, 0.78}, {3.14, 0.34, 0.504, 1.53}, {5.94, 0.03, 2.01, 3.56}},
       {{}, {2.78, 0.10, 0.125, 0.49}, {3.45, 0.18, 0.251, 0.66}, {2.68, 0.48, 0.478, 1.47}, {5.36, 0.03, 1.80, 3.55}}};
    auto tiles = [&](int bm, int bn) { return std::ceil((double)M / bm) * std::ceil((double)N / bn) * batch; };
@@ -583,10 +670,10 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
    SOFIE_HIP_REQUIRE(count >= 1 && count <= SOFIE_MAX_GEMM_CHAIN, "sofie_hip_gemm_chain_f32: %d layers (1..%d allowed)", count, SOFIE_MAX_GEMM_CHAIN);
    for (int l = 1; l < count; ++l)
       SOFIE_HIP_REQUIRE(layers[l].A == layers[l - 1].Y && layers[l].A != nullptr, "sofie_hip_gemm_chain_f32: layer %d does not read the output of layer %d", l, l - 1);
-   // Which layers share a launch.  A launch of its own spreads a layer over the chip and costs about 3 us (what the host takes for
-   // it); in the chain kernel a workgroup does its rows' share alone: a pass over 64 outputs (W stored [N][K]) or a walk along k
-   // (W stored [K][N]) at a time.  So large layers run one by one, and small ones behind them share a launch.  (Fitted to 60 networks of two to four
-   // layers; of 40 others one is 1.5 us slower than the best split.)
+   // Which layers share a launch.  A launch of its own spreads a layer over the chip and costs 2.5 us or more; in the chain kernel a workgroup does its rows' share alone: a pass over
+   // the outputs that its waves take at once (W stored [N][K]) or a walk along k (W stored [K][N]) at a time.  So large layers run one by one, and small ones behind them share a
+   // launch.  (Fitted to 3100 networks of two to four layers, 1 .. 256 rows, all layers together or each by itself: 0.65 % above the better of the two on average, 39 % the most; with the costs
+   // of the kernel before 1.2 and 58 %.)
    const int M = layers[0].M;
    int first = count; // first layer of the shared launch
    if (ctx->opt.f32_chain == 1) {
@@ -596,24 +683,27 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
          const auto &d = layers[l];
          return f32_loads((d.transA ? d.M : d.K) % 4 == 0 && (d.transB ? d.K : d.N) % 4 == 0, d.transB && !d.transA);
       };
+      auto apart = [](double t) { return std::max(1.02 * t - 0.27, 2.5); }; // behind another layer
       double before = 0.0, least = 0.0;
       for (int l = 0; l < count; ++l) {
          double t = 0.0;
          pick_f32_tile(M, layers[l].N, layers[l].K, 1, loads(l), &t);
-         least += std::max(t, 3.0);
+         least += apart(t);
       }
       for (int s = 0; s + 2 <= count; ++s) {
          double together = 0.0, t = 0.0;
          for (int l = s; l < count; ++l) {
-            const double K = layers[l].K, N = layers[l].N, passes = std::ceil(N / (layers[l].transB ? 64.0 : 1024.0));
+            const double K = layers[l].K, N = layers[l].N;
+            const bool wide = layers[l].K % 4 == 0 && layers[l].ldb % 4 == 0; // chain_rows
+            const double outputs = !layers[l].transB ? 1024.0 : !wide || N <= 64 ? 64.0 : K <= 64 ? 256.0 : K <= 128 ? 128.0 : 64.0, passes = std::ceil(N / outputs);
             const double groups = N <= 64 ? 16.0 : N <= 128 ? 8.0 : N <= 256 ? 4.0 : N <= 512 ? 2.0 : 1.0; // that deal out k
-            together += 0.4 + passes * (layers[l].transB ? 0.7 + 0.002 * K : 1.3 + 0.023 * K / groups);
+            together += layers[l].transB ? wide ? 0.44 + passes * (0.81 + 0.0013 * K) : 0.43 + passes * (0.78 + 0.0023 * K) : passes * (1.55 + 0.025 * K / groups);
          }
-         together = before + 2.3 + together * (M <= 64 ? 1.0 : 1.8);
+         together = before + 1.76 + together * (M <= 64 ? 1.0 : M <= 128 ? 1.27 : 1.7);
          if (together < least)
             least = together, first = s;
          pick_f32_tile(M, layers[s].N, layers[s].K, 1, loads(s), &t);
-         before += std::max(t, 3.0);
+         before += apart(t);
       }
    }
    for (int l = 0; l < count; ++l) {
