@@ -11,7 +11,7 @@ namespace sofie_hip {
 
 // NT: blocks of 16 output channels.
 template <class EPI, int NT>
-__global__ __launch_bounds__(256) void conv_i8_windows_kernel(FewChannelConv g, int stride_w, const int8_t *__restrict__ Wp, int Kp, EPI ep, int M, int N, int ngroups)
+__global__ __launch_bounds__(256) void conv_i8_windows_kernel(FewChannelConv g, int stride_w, const int8_t *__restrict__ Wp, int Kp, EPI ep, int M, int N, int ngroups, int kh_mul, Divisor31 by_plane, Divisor31 by_ow)
 {
    typedef uint64_t u64_unaligned __attribute__((aligned(1)));
    __shared__ v4i wfrag[NT * 16 * 4]; // [column][quarter of the reduction]: 16 bytes each
@@ -20,27 +20,32 @@ __global__ __launch_bounds__(256) void conv_i8_windows_kernel(FewChannelConv g, 
    const int c = lane & 15, lk = lane >> 4;
    const int npairs = g.Cg * g.kh;
 
-   // ---- weights, re-ordered from k = (ky * kw + kx) * Cg + channel
+   auto channel_of = [&](int pair) { return pair * kh_mul >> 8; }; // pair / kh for the 16 pairs there may be
+   // ---- weights, re-ordered from k = (ky * kw + kx) * Cg + channel: sixteen bytes of a thread on their way at once, those that are none read as the first and dropped
    for (int e = t; e < NT * 16 * 4; e += 256) {
       const int col = e >> 2, q = e & 3;
-      uint32_t w[4] = {0, 0, 0, 0};
+      uint8_t v[4][4];
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
-         const int pair = q * 4 + p;
-         const int ch = g.pair_c[pair], ky = g.pair_ky[pair];
+         const int pair = q * 4 + p, ch = channel_of(pair), ky = pair - ch * g.kh;
 #pragma unroll
          for (int kx = 0; kx < 4; ++kx)
-            if (pair < npairs && kx < g.kw && col < N)
-               w[p] |= (uint32_t)(uint8_t)Wp[(size_t)col * Kp + (ky * g.kw + kx) * g.Cg + ch] << (8 * kx);
+            v[p][kx] = (uint8_t)Wp[pair < npairs && kx < g.kw && col < N ? (size_t)col * Kp + (ky * g.kw + kx) * g.Cg + ch : 0];
       }
+      __builtin_amdgcn_sched_barrier(0);
+      uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+#pragma unroll
+         for (int kx = 0; kx < 4; ++kx)
+            w[p] |= q * 4 + p < npairs && kx < g.kw && col < N ? (uint32_t)v[p][kx] << (8 * kx) : 0u;
       wfrag[e] = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
    }
    // ---- the lane's four pairs: plane and row offset, and the row distance (a pair past the end never lies inside the image)
    int pair_off[4], pair_dy[4];
 #pragma unroll
    for (int q = 0; q < 4; ++q) {
-      const int pair = lk * 4 + q;
-      const int ch = g.pair_c[pair], ky = g.pair_ky[pair];
+      const int pair = lk * 4 + q, ch = channel_of(pair), ky = pair - ch * g.kh;
       pair_off[q] = (ch * g.H + ky * g.dil_h) * g.W;
       pair_dy[q] = pair < npairs ? ky * g.dil_h : -(1 << 30); // above any image (rows of 8 bytes or more: at most 2^28 of them)
    }
@@ -55,13 +60,12 @@ __global__ __launch_bounds__(256) void conv_i8_windows_kernel(FewChannelConv g, 
       fb[j] = wfrag[(j * 16 + c) * 4 + lk];
 
    // the windows of a group are requested one group ahead
-   const int ohw = g.OH * g.OW;
    uint64_t chunk[4];
    bool ok[4];
    int shift;
    auto request = [&](int grp) {
       const int m = grp * 16 + c < M ? grp * 16 + c : M - 1;
-      const int img = m / ohw, r = m - img * ohw, oh = r / g.OW, ow = r - oh * g.OW;
+      const int img = (int)by_plane.over((unsigned)m), r = m - img * (int)by_plane.d, oh = (int)by_ow.over((unsigned)r), ow = r - oh * g.OW;
       const int ih0 = oh * g.stride_h - g.pad_h0, iw0 = ow * stride_w - g.pad_w0;
       // the 8 bytes lie inside the row; `shift` moves the window down (positive) or up
       const int cs = iw0 < 0 ? 0 : iw0 > g.W - 8 ? g.W - 8 : iw0;
@@ -108,20 +112,17 @@ inline bool conv_i8_windows_applies(const FewChannelConv &g, int N)
 }
 
 template <class EPI>
-static int launch_conv_i8_windows(const LaunchCfg &lc, FewChannelConv g, int stride_w, const int8_t *Wp, int M, int N, int Kp, const EPI &ep)
+static int launch_conv_i8_windows(const LaunchCfg &lc, const FewChannelConv &g, int stride_w, const int8_t *Wp, int M, int N, int Kp, const EPI &ep)
 {
    const int ngroups = (M + 15) / 16;
-   for (int pair = 0; pair < 16; ++pair) {
-      g.pair_c[pair] = (unsigned char)(pair / g.kh);
-      g.pair_ky[pair] = (unsigned char)(pair % g.kh);
-   }
    // up to 16 waves per CU, each with its next group of windows on the way
    int grid = (ngroups + 3) / 4;
    if (grid > 1024)
       grid = 1024;
    auto go = [&](auto nt) {
       constexpr int NT = decltype(nt)::value;
-      launch_kernel((conv_i8_windows_kernel<EPI, NT>), dim3((unsigned)grid), dim3(256), 0, lc.stream, g, stride_w, Wp, Kp, ep, M, N, ngroups);
+      launch_kernel((conv_i8_windows_kernel<EPI, NT>), dim3((unsigned)grid), dim3(256), 0, lc.stream, g, stride_w, Wp, Kp, ep, M, N, ngroups,
+                    (255 + g.kh) / g.kh, Divisor31((long long)g.OH * g.OW), Divisor31(g.OW));
       return launch_status("conv_i8_windows_kernel");
    };
    return N <= 16 ? go(std::integral_constant<int, 1>{}) : N <= 32 ? go(std::integral_constant<int, 2>{}) : go(std::integral_constant<int, 4>{});

@@ -71,9 +71,39 @@ int gemm_i8_nt(const LaunchCfg &lc, const int8_t *A, const int8_t *Bt, int M, in
    return launch_mfma8_best<MfmaI8, I8Epilogue>(lc, A, Bt, M, N, K, lda, ldb, ep);
 }
 
+// The direct kernel for a convolution over NHWC input, if it is estimated to be the fastest (*taken tells); `others` is what the caller's kernels take, in us.  A launch, a wait per
+// eight steps of 128 bytes of k, and for every 256 tiles their steps.  us, general and pipelined kernels -> direct: 5 images of 28 x 28, 16 -> 32 channels 4.5 -> 2.6, 32 -> 64 4.5 -> 2.8; 8 of 10 x
+// 10, 64 -> 256 4.8 -> 3.1; 1 of 15 x 15, 256 -> 256 8.9 -> 4.6; 10 of 45 x 45, 32 -> 64 5.2 -> 4.4; 185 of 41 x 41, 16 -> 32 24.4 -> 17.4 (where half of a tile of 64 columns is
+// empty); the line lies at 20 of 40 x 40, 24 -> 64, 5.75 and 5.79.  Fitted to 467 layers of 1 to 250 images: 0.4 % above the fastest on average, 13 % the most, and the layers 1.33 times as
+// fast as without it.
+static int conv_i8_direct(const LaunchCfg &lc, const ConvRows &g, int Cg, const int8_t *Wp, int M, int N, int K, int Kp, const I8Epilogue &ep, double others, bool *taken)
+{
+   auto time = [&](int b, double launch, double wait, double again, double step) {
+      const double tiles = (double)((M + b - 1) / b) * ((N + b - 1) / b) / 256.0, steps = std::ceil(K / 128.0), waits = std::ceil(steps / 8.0);
+      return launch + std::max(wait + again * (waits - 1.0), tiles * step * (1.3 + std::max(0.0, steps - 4.0)));
+   };
+   const double t16 = time(16, 2.35, 0.23, 1.0, 0.14), t32 = time(32, 2.41, 0.40, 1.9, 0.32);
+   *taken = ep.rows_per_plane == 0 && (lc.tile == 17 || lc.tile == 33 || (lc.tile == 0 && lc.variant == 0 && std::min(t16, t32) < others));
+   if (!*taken)
+      return SOFIE_HIP_OK;
+   auto go = [&](auto piece) {
+      constexpr int P = decltype(piece)::value;
+      const DirectConvRows<P> src{g.X, M, g.H, g.W, g.C, g.stride_h, g.stride_w, g.pad_h0, g.pad_w0, g.dil_h, g.dil_w, K,
+                                  Divisor31((long long)g.OH * g.OW), Divisor31(g.OW), Divisor31(Cg), Divisor31(g.kw)};
+      if (lc.tile ? lc.tile == 17 : t16 < t32)
+         return launch_conv_i8_direct<P, 1, 1, 4, I8Epilogue>(lc, src, Wp, M, N, Kp, ep);
+      return launch_conv_i8_direct<P, 2, 2, 4, I8Epilogue>(lc, src, Wp, M, N, Kp, ep);
+   };
+   return Cg % 16 == 0 ? go(std::integral_constant<int, 16>{}) : go(std::integral_constant<int, 8>{});
+}
+
 int conv_i8_implicit(const LaunchCfg &lc, const ConvRows &src, int Cg, const int8_t *Wp, int M, int N, int K, I8Epilogue ep)
 {
    derive_epilogue_fields(ep, N);
+   bool taken = false;
+   const double others = std::min(mfma8_time(M, N, K, 64, 64, 3.6, 0.0, 56e3), mfma8_time(M, N, K, 128, 128, 5.7, 0.0, 55e3)); // larger layers are the other kernels' in any case
+   if (int st = conv_i8_direct(lc, src, Cg, Wp, M, N, K, K, ep, others, &taken); st || taken)
+      return st;
    return launch_mfma8_conv<I8Epilogue>(lc, src, Cg, Wp, M, N, K, ep);
 }
 
@@ -86,6 +116,10 @@ int conv_i8_gather(const LaunchCfg &lc, const GatherConvRows &src, const int8_t 
 int conv_i8_staged(const LaunchCfg &lc, const ConvRows &g, int Cg, const int8_t *Wp, int M, int N, int K, int Kp, I8Epilogue ep)
 {
    derive_epilogue_fields(ep, N);
+   bool taken = false;
+   const double others = std::min(mfma8_time(M, N, K, 64, 64, 3.3, 0.95, 139e3), mfma8_time(M, N, K, 128, 128, 8.6, 3.6, 41e3));
+   if (int st = conv_i8_direct(lc, g, Cg, Wp, M, N, K, Kp, ep, others, &taken); st || taken)
+      return st;
    auto go = [&](auto src) {
       src.X = g.X;
       src.rows = M;

@@ -105,38 +105,44 @@ struct DirectF8 {
    }
 };
 
-// The partial tiles of W waves meet in LDS and are stored.
+// The partial tiles of W waves meet in LDS and are stored, four columns of a row by a thread.
 template <class MMA, int MB, int NB, int W, class EPI>
-__device__ __forceinline__ void direct_store(const EPI &ep, const typename MMA::acc_t (&acc)[MB][NB], typename MMA::elem_t (*part)[MB * 16][NB * 16 + 4], int m0, int n0,
-                                             int M, int N, int wave, int lane)
-{
-   constexpr int TM = MB * 16, TN = NB * 16;
-   typedef typename MMA::acc_t acc_t;
-   const int lk = lane >> 4, c = lane & 15;
+struct DirectStore {
+   static constexpr int TM = MB * 16, TN = NB * 16;
+   static_assert(TM * TN / 4 <= W * 64, "four elements by a thread");
+   int m0, n0, M, N, r, q;
+   bool live;
+   typename EPI::template col_params<4> prm;
+   __device__ __forceinline__ DirectStore(int m0, int n0, int M, int N) : m0(m0), n0(n0), M(M), N(N)
+   {
+      r = (int)threadIdx.x / (TN / 4), q = (int)threadIdx.x % (TN / 4) * 4;
+      live = r < TM && m0 + r < M && n0 + q < N;
+   }
+   // the columns' parameters
+   __device__ __forceinline__ void ask(const EPI &ep)
+   {
+      if (live)
+         ep.template load_params<4>(n0 + q, prm);
+   }
+   __device__ __forceinline__ void store(const EPI &ep, const typename MMA::acc_t (&acc)[MB][NB], typename MMA::elem_t (*part)[TM][TN + 4], int wave, int lane) const
+   {
+      typedef typename MMA::acc_t acc_t;
+      const int lk = lane >> 4, c = lane & 15;
 #pragma unroll
-   for (int i = 0; i < MB; ++i)
+      for (int i = 0; i < MB; ++i)
 #pragma unroll
-      for (int j = 0; j < NB; ++j)
-         *(acc_t *)&part[wave][i * 16 + c][j * 16 + lk * 4] = acc[i][j];
-   __syncthreads();
-   ep.dispatch([&](auto mode) {
-      constexpr int MODE = decltype(mode)::value;
-#pragma unroll 1
-      for (int e = threadIdx.x; e < TM * TN / 4; e += W * 64) {
-         const int r = e / (TN / 4), q = e % (TN / 4) * 4;
-         acc_t v = *(const acc_t *)&part[0][r][q];
+         for (int j = 0; j < NB; ++j)
+            *(acc_t *)&part[wave][i * 16 + c][j * 16 + lk * 4] = acc[i][j];
+      __syncthreads();
+      if (!live)
+         return;
+      acc_t v = *(const acc_t *)&part[0][r][q];
 #pragma unroll
-         for (int w = 1; w < W; ++w)
-            v += *(const acc_t *)&part[w][r][q];
-         const int m = m0 + r, n = n0 + q;
-         if (m >= M || n >= N)
-            continue;
-         typename EPI::template col_params<4> prm;
-         ep.template load_params<4>(n, prm);
-         store_four_columns<MODE>(ep, prm, v, m, n, N);
-      }
-   });
-}
+      for (int w = 1; w < W; ++w)
+         v += *(const acc_t *)&part[w][r][q];
+      ep.dispatch([&](auto mode) { store_four_columns<decltype(mode)::value>(ep, prm, v, m0 + r, n0 + q, N); });
+   }
+};
 
 template <class MMA, int MB, int NB, int W, int UNROLL, class EPI>
 __global__ __launch_bounds__(W * 64) void mfma8_direct_kernel(RowMajorRows A, RowMajorRows Bt, int M, int N, int K, EPI ep, TileOrder order, int first_tile)
@@ -214,7 +220,9 @@ __global__ __launch_bounds__(W * 64) void mfma8_direct_kernel(RowMajorRows A, Ro
             acc[i][j] = MMA::mma(fb[j], fa[i], acc[i][j]);
    }
 
-   direct_store<MMA, MB, NB, W>(ep, acc, part, m0, n0, M, N, wave, lane);
+   DirectStore<MMA, MB, NB, W, EPI> store(m0, n0, M, N);
+   store.ask(ep);
+   store.store(ep, acc, part, wave, lane);
 }
 
 // The same with the operands going through LDS, for rows that start on 16 bytes.  A vector L1 takes four cycles per line that a load instruction touches: fragments
@@ -301,8 +309,10 @@ __global__ __launch_bounds__(W * 64) void mfma8_direct_ring_kernel(RowMajorRows 
    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
    typename MMA::acc_t acc[MB][NB];
    direct_ring_sums<MMA, MB, NB, W>(acc, A, Bt, M, N, K, m0, n0, smem, depth, wave, lane);
+   DirectStore<MMA, MB, NB, W, EPI> store(m0, n0, M, N);
+   store.ask(ep);
    __syncthreads();
-   direct_store<MMA, MB, NB, W>(ep, acc, (typename MMA::elem_t(*)[MB * 16][NB * 16 + 4])smem, m0, n0, M, N, wave, lane);
+   store.store(ep, acc, (typename MMA::elem_t(*)[MB * 16][NB * 16 + 4])smem, wave, lane);
 }
 
 // The ring of a launch: places per wave (as many as fit and are used; half of them where a CU has several tiles), and bytes of LDS, in which the partial tiles

@@ -1,6 +1,7 @@
 // Kernel choice for the int8 / FP8 GEMM and the int8 convolution: which tile, which pipelined kernel, or the general one.
 #pragma once
 #include "conv_i8_resident.hpp"
+#include "conv_i8_direct.hpp"
 #include "mfma8_staged.hpp"
 #include <algorithm>
 #include <cmath>
