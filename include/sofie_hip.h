@@ -49,11 +49,12 @@ int sofie_hip_ctx_create(sofie_hip_ctx **out, int device, void *external_stream)
 int sofie_hip_ctx_destroy(sofie_hip_ctx *ctx);
 /* Kernel-choice overrides of one context, for tuning and for tests that must reach a particular kernel (no counterpart in the
  * reference, whose GPU path has no such choice).  A kernel that does not take a call's shape leaves it to the others.
- *   "i8_tile" / "f8_tile"  0 = heuristic; 64, 128, 256 the tile of the pipelined or general kernel; 258 and 512 the two-per-CU and the
- *                          persistent kernel; 16 and 32 the direct kernel with tiles of 16 x 16 and 32 x 32 (products only: an int8
- *                          convolution that reads its input directly refuses them); for int8 convolutions also 27 the window kernel of
- *                          few input channels, 257 the 256 x 128 tile with a ring of five, 576 the kernel with resident weights, 17 and 33
- *                          the direct kernel of small NHWC layers with tiles of 16 x 16 and 32 x 32
+ *   "i8_tile" / "f8_tile"  0 = heuristic; 64, 128, 256 the tile of the pipelined or general kernel; 164 the general kernel with tiles of
+ *                          128 x 64 (products only); 258 and 512 the two-per-CU and the persistent kernel; 16 and 32 the direct
+ *                          kernel with tiles of 16 x 16 and 32 x 32 (products only: an int8 convolution that reads its input directly
+ *                          refuses them); for int8 convolutions also 27 the window kernel of few input channels, 257 the 256 x 128
+ *                          tile with a ring of five, 576 the kernel with resident weights, 17 and 33 the direct kernel of small NHWC
+ *                          layers with tiles of 16 x 16 and 32 x 32
  *   "gemm_variant"         1: alternative pipelined kernel, -1: general kernel only
  *   "swizzle"              tile order
  *   "conv_explicit"        1: int8 convolutions through a column matrix whenever the workspace holds one

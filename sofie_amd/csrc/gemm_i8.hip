@@ -117,8 +117,7 @@ int conv_i8_staged(const LaunchCfg &lc, const ConvRows &g, int Cg, const int8_t 
 {
    derive_epilogue_fields(ep, N);
    bool taken = false;
-   const double others = std::min(mfma8_time(M, N, K, 64, 64, 3.3, 0.95, 139e3), mfma8_time(M, N, K, 128, 128, 8.6, 3.6, 41e3));
-   if (int st = conv_i8_direct(lc, g, Cg, Wp, M, N, K, Kp, ep, others, &taken); st || taken)
+   if (int st = conv_i8_direct(lc, g, Cg, Wp, M, N, K, Kp, ep, mfma8_general_time(M, N, K, MFMA8_PIXELS), &taken); st || taken)
       return st;
    auto go = [&](auto src) {
       src.X = g.X;
@@ -248,7 +247,7 @@ static int gemm_i8_with_workspace(sofie_hip_ctx *ctx, const sofie_gemm_i8_desc *
       SOFIE_HIP_REQUIRE(ws != nullptr && ws_left >= need,
                         "sofie_hip_gemm_i8: B is [K,N]; a workspace of %zu bytes is needed to re-lay it out", need);
       SOFIE_HIP_REQUIRE(((uintptr_t)ws & 255) == 0, "sofie_hip_gemm_i8: workspace must be 256-byte aligned");
-      if (!d->transA && mfma8_columns_preferred(launch_cfg_i8(ctx), M, N, K, K % 16 == 0 && lda % 16 == 0 && ((uintptr_t)A & 15) == 0)) {
+      if (!d->transA && mfma8_columns_preferred(launch_cfg_i8(ctx), M, N, K, ((K | lda) & 3) == 0 && ((uintptr_t)A & 3) == 0, K % 16 == 0 && lda % 16 == 0 && ((uintptr_t)A & 15) == 0)) {
          derive_epilogue_fields(ep, N);
          return launch_mfma8_general<MfmaI8, StagedRows, StagedColumns, I8Epilogue>(launch_cfg_i8(ctx), StagedRows{A, lda, M}, StagedColumns{d->B, ldb, N}, M, N, K, ep);
       }

@@ -9,12 +9,8 @@
 namespace sofie_hip {
 
 // ---- estimates ------------------------------------------------------------------------------------------------------------
-// Below the sizes that fill the matrix cores, all of these kernels are bound by the bytes a CU takes in (37 - 45 KB/us through
-// registers, 67 - 75 KB/us straight into LDS) and by what a tile costs besides (start, store).  Fitted to single launches from
-// 33 x 260 x 100 to 3001 x 3695 x 6991 and to the long, narrow products of small convolutions (200000 x 32 x 224), the estimates hold
-// to about a fifth where both operands are rows; they decide between kernels whose times differ by more than that almost everywhere.
-// The loader that transposes B (mfma8_columns_preferred) has no term of its own and takes up to half as long again: 1537 x 1000 x 777 7.6 us
-// estimated and 11.4 measured, 300 x 300 x 300 4.3 and 6.2.
+// Below the sizes that fill the matrix cores, all of these kernels are bound by the bytes a CU takes in (15 - 58 KB/us through
+// registers, by what the loads' alignment costs, 67 - 75 KB/us straight into LDS) and by what a tile costs besides (start, store).
 inline double mfma8_rounds(int M, int N, int bm, int bn)
 {
    const double rounds = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) / 256.0; // tiles per CU; a CU works on a few at a time
@@ -28,17 +24,42 @@ inline double mfma8_time(int M, int N, int K, int bm, int bn, double fixed_us, d
 // are asked for at once, and as much behind them while few CUs are at work, 20 TB/s from L2 over all of them (us, estimated / measured: 16 x 4096 x 4096
 // 4.4 / 4.2, 600 x 320 x 6144 6.7 / 6.4, 108 x 4096 x 8192 16.0 / 14.4); whole steps of a short K through registers at the rates below.  Fitted, int8 and FP8, to 1900
 // products of 1 .. 800 rows by 32 .. 4096 columns, K = 32 .. 8192, with what the 64 x 64 tiles took: the choice is 0.05 % above the fastest on average, 7 % the most.
-inline double mfma8_direct_time(int M, int N, int K, int b, bool lines)
+// `words`: rows start on four bytes; a load of 16 bytes at any other place takes a vector L1 three times as long (15 KB/us a CU).  Fitted to 482 and 500 products.
+inline double mfma8_direct_time(int M, int N, int K, int b, bool words, bool lines)
 {
    if (!lines)
-      return b == 16 ? mfma8_time(M, N, K, 16, 16, 2.5, 0.4, 41e3) : mfma8_time(M, N, K, 32, 32, 2.5, 0.8, 44e3);
+      return b == 16 ? mfma8_time(M, N, K, 16, 16, 2.75, 0.43, words ? 54e3 : 14.9e3) : mfma8_time(M, N, K, 32, 32, 2.85, words ? 1.0 : 1.1, words ? 51e3 : 16.2e3);
    if (!mfma8_direct_by_lines(b, M, N, K))
       return b == 16 ? mfma8_time(M, N, K, 16, 16, 2.5, 0.3, 41e3) : mfma8_time(M, N, K, 32, 32, 2.5, 0.45, 80e3);
    const double tiles = (double)((M + b - 1) / b) * ((N + b - 1) / b), ahead = std::min(K, 2048);
    return 2.5 + mfma8_rounds(M, N, b, b) * ((b == 16 ? 0.5 : 0.62) + 2.0 * b * (ahead / 120e3 + (K - ahead) / std::min(120e3, 20e6 / std::min(tiles, 256.0))));
 }
-inline double mfma8_staged64_time(int M, int N, int K) { return mfma8_time(M, N, K, 64, 64, 3.0, 0.4, 45e3); }
-inline double mfma8_staged128_time(int M, int N, int K) { return mfma8_time(M, N, K, 128, 128, 4.0, 2.5, 39e3); }
+// The general loop: tiles of 64 x 64, 128 x 64 and 128 x 128 (0, 1, 2).  By what it reads: rows that start on four bytes, rows that start anywhere, rows against a B that is
+// transposed on its way, a convolution's pixels.  Each fitted to 445 .. 1000 products of 1 .. 8192 rows and columns (int8 and FP8; 124 layers): the choice among the tiles is 0.4 - 1.3 % above the
+// fastest on average.  Between 64 x 64, of which a CU has one or two, and 128 x 128, of which the chip has too few, the tile in the middle: us, the better of those two -> 128 x 64,
+// 1537 x 1000 x 777 with B transposed 10.8 -> 9.7, 1000 x 2000 x 500 8.9 -> 7.7, 2048^3 22.6 -> 19.4, 384 x 2976 x 3500 23.8 -> 19.5; rows 1537 x 1000 x 777 9.6 -> 9.0.  (A convolution's
+// rows are worked out by each thread for its chunks: equal at best there.)
+enum Mfma8Source { MFMA8_WORD_ROWS, MFMA8_ROWS, MFMA8_COLUMNS, MFMA8_PIXELS };
+inline double mfma8_general_time(int M, int N, int K, Mfma8Source source, int *tile = nullptr)
+{
+   static constexpr struct {
+      double fixed, tile, rate;
+   } COSTS[4][3] = {{{3.0, 1.1, 58e3}, {1.6, 2.95, 58e3}, {1.5, 4.9, 52e3}},
+                    {{2.8, 1.55, 42.5e3}, {1.5, 3.5, 42.3e3}, {1.2, 6.0, 41e3}},
+                    {{3.5, 1.13, 34e3}, {1.5, 3.2, 40e3}, {0.0, 6.7, 34.5e3}},
+                    {{3.3, 0.95, 139e3}, {1e9, 0.0, 1.0}, {8.6, 3.6, 41e3}}};
+   double least = 1e30;
+   for (int t = 0; t < 3; ++t) {
+      const auto &c = COSTS[source][t];
+      const double time = mfma8_time(M, N, K, t ? 128 : 64, t == 2 ? 128 : 64, c.fixed, c.tile, c.rate);
+      if (time < least) {
+         least = time;
+         if (tile)
+            *tile = t;
+      }
+   }
+   return least;
+}
 inline double mfma8_ring_time(int M, int N, int K, int tile)
 {
    return tile >= 128 ? mfma8_time(M, N, K, 128, 128, 3.5, 3.4, 67e3) : mfma8_time(M, N, K, 64, 64, 2.9, 0.6, 75e3);
@@ -46,10 +67,18 @@ inline double mfma8_ring_time(int M, int N, int K, int tile)
 
 // The general loop (any alignment, a convolution's input or plain rows, B either way).
 template <class MMA, class ASRC, class BSRC, class EPI>
-static int launch_mfma8_general(const LaunchCfg &lc, const ASRC &A, const BSRC &B, int M, int N, int K, const EPI &ep)
+static int launch_mfma8_general(const LaunchCfg &lc, const ASRC &A, const BSRC &B, int M, int N, int K, const EPI &ep, bool words = false)
 {
-   const bool wide = lc.tile == 64 ? false : lc.tile >= 128 ? true : mfma8_staged128_time(M, N, K) < mfma8_staged64_time(M, N, K);
-   if (wide)
+   constexpr bool PIXELS = !std::is_same_v<ASRC, StagedRows>;
+   int tile = 0;
+   mfma8_general_time(M, N, K, PIXELS ? MFMA8_PIXELS : BSRC::kTransposed ? MFMA8_COLUMNS : words ? MFMA8_WORD_ROWS : MFMA8_ROWS, &tile);
+   if (lc.tile)
+      tile = lc.tile == 64 ? 0 : lc.tile >= 128 && (lc.tile != 164 || PIXELS) ? 2 : lc.tile == 164 ? 1 : tile;
+   if constexpr (!PIXELS) {
+      if (tile == 1)
+         return launch_mfma8_staged<MMA, 128, 64, 128, 4, 2, 2, ASRC, BSRC, EPI>(lc, A, B, M, N, K, ep);
+   }
+   if (tile == 2)
       return launch_mfma8_staged<MMA, 128, 128, 128, 4, 2, 2, ASRC, BSRC, EPI>(lc, A, B, M, N, K, ep);
    return launch_mfma8_staged<MMA, 64, 64, 128, 2, 2, 2, ASRC, BSRC, EPI>(lc, A, B, M, N, K, ep);
 }
@@ -64,17 +93,15 @@ static int launch_mfma8_best(const LaunchCfg &lc, const int8_t *A, const int8_t 
    typedef std::conditional_t<(MMA::KSTEP * 2 <= 64), DirectI8, DirectF8> Direct;
    const bool aligned = (lda % 16 == 0) && (ldb % 16 == 0) && (((uintptr_t)A & 15) == 0) && (((uintptr_t)Bt & 15) == 0);
    const bool ring = variant >= 0 && aligned && K >= 64 && K % 64 == 0 && (MMA::KSTEP * 2 <= 64 || K % 128 == 0);
-   const bool lines = aligned && K % 16 == 0;
-   const double t16 = mfma8_direct_time(M, N, K, 16, lines), t32 = mfma8_direct_time(M, N, K, 32, lines);
-   // (the general loop takes 0.4 - 0.7 us longer than estimated where few tiles of aligned rows are all there is: 300 x 1000 x 32 3.9 int8, 4.2 FP8, the direct kernel 3.8)
-   const double others = ring ? mfma8_ring_time(M, N, K, pick_tile(M, N, 0))
-                              : std::min(mfma8_staged64_time(M, N, K), mfma8_staged128_time(M, N, K)) + (lines ? 0.5 : 0.0);
+   const bool lines = aligned && K % 16 == 0, words = ((lda | ldb) & 3) == 0 && (((uintptr_t)A | (uintptr_t)Bt) & 3) == 0;
+   const double t16 = mfma8_direct_time(M, N, K, 16, words, lines), t32 = mfma8_direct_time(M, N, K, 32, words, lines);
+   const double others = ring ? mfma8_ring_time(M, N, K, pick_tile(M, N, 0)) : mfma8_general_time(M, N, K, words ? MFMA8_WORD_ROWS : MFMA8_ROWS);
    if (force_tile == 16 || K < 16 || (!force_tile && variant == 0 && t16 <= t32 && t16 < others))
       return launch_mfma8_direct<Direct, 1, 1, 8, 4, EPI>(lc, A, Bt, M, N, K, lda, ldb, ep);
    if (force_tile == 32 || (!force_tile && variant == 0 && t32 < others))
       return launch_mfma8_direct<Direct, 2, 2, 8, 2, EPI>(lc, A, Bt, M, N, K, lda, ldb, ep);
-   if (!ring)
-      return launch_mfma8_general<MMA, StagedRows, StagedRows, EPI>(lc, StagedRows{A, lda, M}, StagedRows{Bt, ldb, N}, M, N, K, ep);
+   if (!ring || force_tile == 164)
+      return launch_mfma8_general<MMA, StagedRows, StagedRows, EPI>(lc, StagedRows{A, lda, M}, StagedRows{Bt, ldb, N}, M, N, K, ep, words);
    const int tile = pick_tile(M, N, force_tile);
    const bool k128 = (K % 128 == 0);
    if constexpr (MMA::KSTEP * 2 <= 64) {
@@ -123,19 +150,20 @@ static int launch_mfma8_best(const LaunchCfg &lc, const int8_t *A, const int8_t 
 }
 
 // Whether a product whose B is stored [K,N] is better off with the general loop, which transposes B on its way into LDS, than
-// with a launch that re-lays B out and the kernels above: that launch takes about 2 us and 4.2 TB/s for the bytes it moves.  Both sides come out
-// low (above; two launches in a row take 4.0 us for B of 0.8 MB, 6.9 for 4.2 MB), so the line lies near the right place up to about
-// 2048^3: in the loop / re-laid out 1537 x 1000 x 777 11.4 / 14.1 us, 1000 x 2000 x 500 8.0 / 9.8, 100 x 4000 x 4000 17.5 / 21.8, 2048^3 19.3 / 19.3.
-// Past them the loop is taken although it is slower: 4096 x 4096 x 1000 42.8 / 37.4, 3001 x 3695 x 1999 68.8 / 60.5.
-static bool mfma8_columns_preferred(const LaunchCfg &lc, int M, int N, int K, bool aligned_behind)
+// with a launch that re-lays B out and the kernels above: that launch takes 2.7 us and 4.1 TB/s for the bytes it moves.  Fitted to 445 products; us, in the loop / re-laid out: 1537 x
+// 1000 x 777 9.7 / 13.2, 2048^3 19.4 / 22.6, 100 x 4000 x 4000 17.9 / 23.6, 5113 x 3917 x 1376 93.8 / 74.0, 2432 x 1125 x 3968 37.4 / 31.0.
+static bool mfma8_columns_preferred(const LaunchCfg &lc, int M, int N, int K, bool words_behind, bool aligned_behind)
 {
    if (K < 16 || N < 16 || lc.tile == 16 || lc.tile == 32)
       return false;
-   const double staged = std::min(mfma8_staged64_time(M, N, K), mfma8_staged128_time(M, N, K));
-   double behind = std::min(std::min(mfma8_direct_time(M, N, K, 16, aligned_behind), mfma8_direct_time(M, N, K, 32, aligned_behind)), staged);
+   if (lc.tile == 164)
+      return true;
+   const bool lines = aligned_behind && K % 16 == 0;
+   double behind = std::min(std::min(mfma8_direct_time(M, N, K, 16, words_behind, lines), mfma8_direct_time(M, N, K, 32, words_behind, lines)),
+                            mfma8_general_time(M, N, K, words_behind ? MFMA8_WORD_ROWS : MFMA8_ROWS));
    if (aligned_behind && K >= 64 && K % 64 == 0)
       behind = std::min(behind, mfma8_ring_time(M, N, K, pick_tile(M, N, 0)));
-   return lc.tile == 0 && lc.variant <= 0 && staged < 2.0 + 2.0 * K * N / 4.2e6 + behind;
+   return lc.tile == 0 && lc.variant <= 0 && mfma8_general_time(M, N, K, MFMA8_COLUMNS) < 2.66 + (double)K * N / 2.07e6 + behind;
 }
 
 } // namespace sofie_hip

@@ -175,18 +175,20 @@ __device__ __forceinline__ void transpose_4x4_bytes(unsigned r0, unsigned r1, un
 
 template <int R, int BK, int NTHREADS>
 struct StagedSlab<StagedColumns, R, BK, NTHREADS> {
-   // a thread carries blocks of 4 k of 8 rows: four 8-byte pieces, one per k
-   static constexpr int RB = R / 8; // blocks along the rows
+   // a thread carries blocks of 4 k of PR rows, eight or, where there are threads enough, four: four pieces of as many bytes, one per k
+   static constexpr int PR = R / 8 * (BK / 4) >= NTHREADS ? 8 : 4;
+   static constexpr int RB = R / PR; // blocks along the rows
    static constexpr int LD = RB * (BK / 4) / NTHREADS;
    static_assert(RB * (BK / 4) % NTHREADS == 0, "the slab divides over the threads");
-   typedef unsigned long long piece_t;
+   typedef std::conditional_t<PR == 8, unsigned long long, unsigned> piece_t;
    typedef piece_t piece_unaligned_t __attribute__((aligned(1)));
    piece_t v[LD][4];
    struct places {};
    static __device__ __forceinline__ void find(const StagedColumns &, int, int, places &) {}
-   static __device__ __forceinline__ int row_of(int i, int t) { return (t + i * NTHREADS) % RB * 8; }
+   static __device__ __forceinline__ unsigned word(piece_t v, int q) { return (unsigned)((unsigned long long)v >> (32 * q)); }
+   static __device__ __forceinline__ int row_of(int i, int t) { return (t + i * NTHREADS) % RB * PR; }
    static __device__ __forceinline__ int k_of(int i, int t) { return (t + i * NTHREADS) / RB * 4; }
-   // pieces past the last column are fetched from the last 8 columns (align_edge moves them), k past K from the last k (finish_last)
+   // pieces past the last column are fetched from the last columns (align_edge moves them), k past K from the last k (finish_last)
    __device__ __forceinline__ void load_last(const StagedColumns &s, const places &, int r0, int k0, int K, int t)
    {
 #pragma unroll
@@ -194,7 +196,7 @@ struct StagedSlab<StagedColumns, R, BK, NTHREADS> {
          const int r = r0 + row_of(i, t), k = k0 + k_of(i, t);
 #pragma unroll
          for (int j = 0; j < 4; ++j)
-            v[i][j] = *(const piece_unaligned_t *)(s.base + (size_t)(k + j < K ? k + j : K - 1) * (size_t)s.ld + (r + 8 <= s.rows ? r : s.rows - 8));
+            v[i][j] = *(const piece_unaligned_t *)(s.base + (size_t)(k + j < K ? k + j : K - 1) * (size_t)s.ld + (r + PR <= s.rows ? r : s.rows - PR));
       }
    }
    __device__ __forceinline__ void load(const StagedColumns &s, const places &, int r0, int k0, int K, int t)
@@ -202,7 +204,7 @@ struct StagedSlab<StagedColumns, R, BK, NTHREADS> {
 #pragma unroll
       for (int i = 0; i < LD; ++i) {
          const int r = r0 + row_of(i, t);
-         const int8_t *p = s.base + (size_t)(k0 + k_of(i, t)) * (size_t)s.ld + (r + 8 <= s.rows ? r : s.rows - 8);
+         const int8_t *p = s.base + (size_t)(k0 + k_of(i, t)) * (size_t)s.ld + (r + PR <= s.rows ? r : s.rows - PR);
 #pragma unroll
          for (int j = 0; j < 4; ++j)
             v[i][j] = *(const piece_unaligned_t *)(p + (size_t)j * (size_t)s.ld);
@@ -221,10 +223,10 @@ struct StagedSlab<StagedColumns, R, BK, NTHREADS> {
    {
 #pragma unroll
       for (int i = 0; i < LD; ++i) {
-         const int drop = (r0 + row_of(i, t) + 8 - s.rows) * 8; // bits that lie before the piece's first row
+         const int drop = (r0 + row_of(i, t) + PR - s.rows) * 8; // bits that lie before the piece's first row
 #pragma unroll
          for (int j = 0; j < 4; ++j)
-            v[i][j] = drop <= 0 ? v[i][j] : drop >= 64 ? 0 : v[i][j] >> drop;
+            v[i][j] = drop <= 0 ? v[i][j] : drop >= 8 * PR ? 0 : v[i][j] >> drop;
       }
    }
    __device__ __forceinline__ void store(int8_t *lds, int t) const
@@ -233,9 +235,9 @@ struct StagedSlab<StagedColumns, R, BK, NTHREADS> {
       for (int i = 0; i < LD; ++i) {
          const int r = row_of(i, t), k = k_of(i, t);
 #pragma unroll
-         for (int q = 0; q < 2; ++q) {
+         for (int q = 0; q < PR / 4; ++q) {
             unsigned w[4];
-            transpose_4x4_bytes((unsigned)(v[i][0] >> (32 * q)), (unsigned)(v[i][1] >> (32 * q)), (unsigned)(v[i][2] >> (32 * q)), (unsigned)(v[i][3] >> (32 * q)), w);
+            transpose_4x4_bytes(word(v[i][0], q), word(v[i][1], q), word(v[i][2], q), word(v[i][3], q), w);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                *(unsigned *)(lds + lds_chunk_offset<BK>(r + 4 * q + e, k / 16) + k % 16) = w[e];
