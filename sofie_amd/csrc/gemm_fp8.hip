@@ -248,7 +248,7 @@ int sofie_hip_gemm_fp8(sofie_hip_ctx *ctx, const sofie_gemm_fp8_desc *d)
       SOFIE_HIP_REQUIRE(d->workspace != nullptr && d->workspace_bytes >= need,
                         "sofie_hip_gemm_fp8: B is [K,N]; a workspace of %zu bytes is needed to re-lay it out", need);
       SOFIE_HIP_REQUIRE(((uintptr_t)d->workspace & 255) == 0, "sofie_hip_gemm_fp8: workspace must be 256-byte aligned");
-      if (mfma8_columns_preferred(launch_cfg_f8(ctx), M, N, K, ((K | lda) & 3) == 0 && ((uintptr_t)A & 3) == 0, K % 128 == 0 && lda % 16 == 0 && ((uintptr_t)A & 15) == 0))
+      if (mfma8_columns_preferred(launch_cfg_f8(ctx), A, lda, Bt, ldb, M, N, K, K % 128 == 0 && lda % 16 == 0 && ((uintptr_t)A & 15) == 0))
          return launch_mfma8_general<MfmaF8, StagedRows, StagedColumns, F8Epilogue>(launch_cfg_f8(ctx), StagedRows{A, lda, M}, StagedColumns{Bt, ldb, N}, M, N, K, ep);
       int st = transpose_i8(ctx->stream, (int8_t *)d->workspace, (const int8_t *)d->B, K, N, ldb, K);
       if (st)

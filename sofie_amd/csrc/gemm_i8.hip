@@ -247,7 +247,7 @@ static int gemm_i8_with_workspace(sofie_hip_ctx *ctx, const sofie_gemm_i8_desc *
       SOFIE_HIP_REQUIRE(ws != nullptr && ws_left >= need,
                         "sofie_hip_gemm_i8: B is [K,N]; a workspace of %zu bytes is needed to re-lay it out", need);
       SOFIE_HIP_REQUIRE(((uintptr_t)ws & 255) == 0, "sofie_hip_gemm_i8: workspace must be 256-byte aligned");
-      if (!d->transA && mfma8_columns_preferred(launch_cfg_i8(ctx), M, N, K, ((K | lda) & 3) == 0 && ((uintptr_t)A & 3) == 0, K % 16 == 0 && lda % 16 == 0 && ((uintptr_t)A & 15) == 0)) {
+      if (!d->transA && mfma8_columns_preferred(launch_cfg_i8(ctx), A, lda, d->B, ldb, M, N, K, K % 16 == 0 && lda % 16 == 0 && ((uintptr_t)A & 15) == 0)) {
          derive_epilogue_fields(ep, N);
          return launch_mfma8_general<MfmaI8, StagedRows, StagedColumns, I8Epilogue>(launch_cfg_i8(ctx), StagedRows{A, lda, M}, StagedColumns{d->B, ldb, N}, M, N, K, ep);
       }

@@ -2,7 +2,7 @@
 // split the reduction; every fragment is loaded from memory into the registers the MFMA reads, UNROLL steps of 128 bytes of k
 // ahead, and the partial tiles meet in LDS.  What such a product costs is the trip to memory for its operands, and one workgroup
 // has its whole share of them (tens of KB) on the way at once; the ring kernels wait for a few KB at a time.  A tile has as few
-// as 16 rows, where theirs have 64.  Rows may start at any byte: a chunk is one unaligned 16-byte load.
+// as 16 rows, where theirs have 64.  Rows may start at any byte: those that start on no word are read as the words they lie in.
 #pragma once
 #include "mfma8_gemm_dma.hpp"
 #include <algorithm>
@@ -11,36 +11,48 @@ namespace sofie_hip {
 
 typedef int v4i_unaligned __attribute__((ext_vector_type(4), aligned(1)));
 
-// The 16 bytes of a row from k on, zero from K on.  Never reads outside the row's K bytes.
-__device__ __forceinline__ v4i load_chunk_tail(const int8_t *row, int k, int K)
+// 16 bytes from any address as words: those they lie in, five of them (four where the address is a multiple of four, so that every word that is read has at least one of the
+// bytes).  One load of 16 bytes at an address that is no multiple of four takes the vector L1 three times as long as at one that is.
+struct AnyChunk {
+   typedef int words_t __attribute__((ext_vector_type(4), aligned(4)));
+   v4i v;
+   unsigned behind, shift;
+   __device__ __forceinline__ void load(const int8_t *p)
+   {
+      shift = (unsigned)(uintptr_t)p & 3u;
+      const int8_t *word = p - shift;
+      v = *(const words_t *)word;
+      behind = *(const unsigned *)(word + (shift ? 16 : 12));
+   }
+   static __device__ __forceinline__ v4i aligned(v4i v, unsigned behind, unsigned shift)
+   {
+      v4i out;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+         out[i] = (int)__builtin_amdgcn_alignbyte(i < 3 ? (unsigned)v[i + 1 < 4 ? i + 1 : 3] : behind, (unsigned)v[i], shift);
+      return out;
+   }
+   __device__ __forceinline__ v4i bytes() const { return aligned(v, behind, shift); }
+};
+
+inline bool rows_of_words(const int8_t *base, int ld) { return ((uintptr_t)base & 3) == 0 && (ld & 3) == 0; }
+
+// The chunk at k of a row of K >= 16 bytes as a load inside the row: where it crosses K, the last 16 bytes of the row instead,
+// which cut_chunk moves down to k, zeros behind them.
+__device__ __forceinline__ const int8_t *chunk_in_row(const int8_t *row, int k, int K) { return row + (k <= K - 16 ? k : K - 16); }
+__device__ __forceinline__ v4i cut_chunk(v4i v, int k, int K)
 {
-   if (k <= K - 16)
-      return *(const v4i_unaligned *)(row + k);
    union {
       v4i v;
       unsigned long long q[2];
-      int8_t b[16];
    } u;
-   u.v = v4i{0, 0, 0, 0};
-   if (k >= K)
-      return u.v;
-   if (K >= 16) {
-      // the last 16 bytes of the row, shifted down to where k lies
-      u.v = *(const v4i_unaligned *)(row + K - 16);
-      const int drop = (k - K + 16) * 8; // bits; 8 .. 120
-      if (drop >= 64) {
-         u.q[0] = u.q[1] >> (drop - 64);
-         u.q[1] = 0;
-      } else {
-         u.q[0] = (u.q[0] >> drop) | (u.q[1] << (64 - drop));
-         u.q[1] >>= drop;
-      }
-      return u.v;
+   u.v = v;
+   const int drop = (k - K + 16) * 8; // bits that lie before k
+   if (drop > 0) {
+      const unsigned long long hi = drop >= 128 ? 0 : u.q[1];
+      u.q[0] = drop >= 64 ? hi >> (drop & 63) : (u.q[0] >> drop) | (u.q[1] << (64 - drop));
+      u.q[1] = drop >= 64 ? 0 : u.q[1] >> drop;
    }
-#pragma unroll
-   for (int i = 0; i < 16; ++i)
-      if (k + i < K)
-         u.b[i] = row[k + i];
    return u.v;
 }
 
@@ -144,7 +156,79 @@ struct DirectStore {
    }
 };
 
-template <class MMA, int MB, int NB, int W, int UNROLL, class EPI>
+// What a lane reads of a row in a step: 32 bytes, as nine words of any row (BYTES) or two chunks of one that starts on four bytes.  The vector L1 bounds this kernel where rows start
+// at any byte: as two unaligned chunks 7 bytes a clock reached a CU, as words 15 - 26; 16 x 193 x 395 3.45 us before, 2.85 now, 2 x 900 x 4001 9.3 and 5.1, 16 x 4096 x 4093 12.9 and
+// 6.7, 50 x 1500 x 767 7.6 and 4.1.
+template <bool BYTES>
+struct DirectLane {
+   v4i v[2];
+   unsigned behind;
+   __device__ __forceinline__ void load(const int8_t *row, int k)
+   {
+      if constexpr (BYTES) {
+         const unsigned shift = (unsigned)(uintptr_t)row & 3u;
+         const int8_t *word = row - shift + k;
+         v[0] = *(const AnyChunk::words_t *)word;
+         v[1] = *(const AnyChunk::words_t *)(word + 16);
+         behind = *(const unsigned *)(word + (shift ? 32 : 28));
+      } else {
+         v[0] = *(const v4i_unaligned *)(row + k);
+         v[1] = *(const v4i_unaligned *)(row + k + 16);
+      }
+   }
+   __device__ __forceinline__ void finish(const int8_t *row)
+   {
+      if constexpr (BYTES) {
+         const unsigned shift = (unsigned)(uintptr_t)row & 3u;
+         v[0] = AnyChunk::aligned(v[0], (unsigned)v[1][0], shift);
+         v[1] = AnyChunk::aligned(v[1], behind, shift);
+      }
+   }
+};
+
+// The step that K cuts off.
+template <bool BYTES>
+struct DirectLast {
+   std::conditional_t<BYTES, AnyChunk, v4i> c[2];
+   v4i v[2];
+   __device__ __forceinline__ void load(const int8_t *row, int k, int K)
+   {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+         const int8_t *p = chunk_in_row(row, k + 16 * h, K);
+         if constexpr (BYTES)
+            c[h].load(p);
+         else
+            c[h] = *(const v4i_unaligned *)p;
+      }
+   }
+   __device__ __forceinline__ void finish(int k, int K)
+   {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+         if constexpr (BYTES)
+            v[h] = cut_chunk(c[h].bytes(), k + 16 * h, K);
+         else
+            v[h] = cut_chunk(c[h], k + 16 * h, K);
+      }
+   }
+   // rows of fewer than 16 bytes
+   __device__ __forceinline__ void load_short(const int8_t *row, int k, int K)
+   {
+      union {
+         v4i v[2];
+         int8_t b[32];
+      } u;
+      u.v[0] = u.v[1] = v4i{0, 0, 0, 0};
+#pragma unroll
+      for (int i = 0; i < 15; ++i)
+         if (k + i < K)
+            u.b[i] = row[k + i];
+      v[0] = u.v[0], v[1] = u.v[1];
+   }
+};
+
+template <class MMA, int MB, int NB, int W, int UNROLL, bool BYTES, class EPI>
 __global__ __launch_bounds__(W * 64) void mfma8_direct_kernel(RowMajorRows A, RowMajorRows Bt, int M, int N, int K, EPI ep, TileOrder order, int first_tile)
 {
    constexpr int STEP = 128, TM = MB * 16, TN = NB * 16, PITCH = TN + 4;
@@ -172,8 +256,29 @@ __global__ __launch_bounds__(W * 64) void mfma8_direct_kernel(RowMajorRows A, Ro
          acc[i][j] = acc_t{0, 0, 0, 0};
 
    const int whole = K / STEP; // steps without a chunk past K
+   // the step that K cuts off: asked for ahead of the others by the wave whose turn it is
+   const bool last = K % STEP != 0 && wave == whole % W;
+   const int last_k = whole * STEP + lk * 32;
+   DirectLast<BYTES> la[MB], lb[NB];
+   if (last) {
+      if (K >= 16) {
+#pragma unroll
+         for (int j = 0; j < NB; ++j)
+            lb[j].load(rb[j], last_k, K);
+#pragma unroll
+         for (int i = 0; i < MB; ++i)
+            la[i].load(ra[i], last_k, K);
+      } else {
+#pragma unroll
+         for (int j = 0; j < NB; ++j)
+            lb[j].load_short(rb[j], last_k, K);
+#pragma unroll
+         for (int i = 0; i < MB; ++i)
+            la[i].load_short(ra[i], last_k, K);
+      }
+   }
    for (int s0 = wave; s0 < whole; s0 += W * UNROLL) {
-      v4i fa[UNROLL][MB][2], fb[UNROLL][NB][2];
+      DirectLane<BYTES> fa[UNROLL][MB], fb[UNROLL][NB];
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
          const int s = s0 + u * W;
@@ -181,43 +286,42 @@ __global__ __launch_bounds__(W * 64) void mfma8_direct_kernel(RowMajorRows A, Ro
             const int k = s * STEP + lk * 32;
 #pragma unroll
             for (int j = 0; j < NB; ++j)
-#pragma unroll
-               for (int h = 0; h < 2; ++h)
-                  fb[u][j][h] = *(const v4i_unaligned *)(rb[j] + k + 16 * h);
+               fb[u][j].load(rb[j], k);
 #pragma unroll
             for (int i = 0; i < MB; ++i)
-#pragma unroll
-               for (int h = 0; h < 2; ++h)
-                  fa[u][i][h] = *(const v4i_unaligned *)(ra[i] + k + 16 * h);
+               fa[u][i].load(ra[i], k);
          }
       }
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u)
          if (s0 + u * W < whole) {
 #pragma unroll
+            for (int j = 0; j < NB; ++j)
+               fb[u][j].finish(rb[j]);
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+               fa[u][i].finish(ra[i]);
+#pragma unroll
             for (int i = 0; i < MB; ++i)
 #pragma unroll
                for (int j = 0; j < NB; ++j)
-                  acc[i][j] = MMA::mma(fb[u][j], fa[u][i], acc[i][j]);
+                  acc[i][j] = MMA::mma(fb[u][j].v, fa[u][i].v, acc[i][j]);
          }
    }
-   if (K % STEP != 0 && wave == whole % W) { // the wave whose turn it is
-      const int k = whole * STEP + lk * 32;
-      v4i fa[MB][2], fb[NB][2];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
+   if (last) {
+      if (K >= 16) {
 #pragma unroll
          for (int j = 0; j < NB; ++j)
-            fb[j][h] = load_chunk_tail(rb[j], k + 16 * h, K);
+            lb[j].finish(last_k, K);
 #pragma unroll
          for (int i = 0; i < MB; ++i)
-            fa[i][h] = load_chunk_tail(ra[i], k + 16 * h, K);
+            la[i].finish(last_k, K);
       }
 #pragma unroll
       for (int i = 0; i < MB; ++i)
 #pragma unroll
          for (int j = 0; j < NB; ++j)
-            acc[i][j] = MMA::mma(fb[j], fa[i], acc[i][j]);
+            acc[i][j] = MMA::mma(lb[j].v, la[i].v, acc[i][j]);
    }
 
    DirectStore<MMA, MB, NB, W, EPI> store(m0, n0, M, N);
@@ -371,8 +475,9 @@ static int launch_mfma8_direct(const LaunchCfg &lc, const int8_t *A, const int8_
       });
       return launch_status("mfma8_direct_ring_kernel");
    }
+   const bool bytes = !rows_of_words(A, lda) || !rows_of_words(Bt, ldb);
    in_launches(nwg, W * 64, [&](int first, unsigned count) {
-      launch_kernel((mfma8_direct_kernel<MMA, MB, NB, W, UNROLL, EPI>), dim3(count), dim3(W * 64), 0, lc.stream, RowMajorRows{A, lda}, RowMajorRows{Bt, ldb}, M, N, K, ep,
+      launch_kernel(bytes ? mfma8_direct_kernel<MMA, MB, NB, W, UNROLL, true, EPI> : mfma8_direct_kernel<MMA, MB, NB, W, UNROLL, false, EPI>, dim3(count), dim3(W * 64), 0, lc.stream, RowMajorRows{A, lda}, RowMajorRows{Bt, ldb}, M, N, K, ep,
                     order, first);
    });
    return launch_status("mfma8_direct_kernel");

@@ -9,7 +9,7 @@
 namespace sofie_hip {
 
 // ---- estimates ------------------------------------------------------------------------------------------------------------
-// Below the sizes that fill the matrix cores, all of these kernels are bound by the bytes a CU takes in (15 - 58 KB/us through
+// Below the sizes that fill the matrix cores, all of these kernels are bound by the bytes a CU takes in (33 - 58 KB/us through
 // registers, by what the loads' alignment costs, 67 - 75 KB/us straight into LDS) and by what a tile costs besides (start, store).
 inline double mfma8_rounds(int M, int N, int bm, int bn)
 {
@@ -24,29 +24,41 @@ inline double mfma8_time(int M, int N, int K, int bm, int bn, double fixed_us, d
 // are asked for at once, and as much behind them while few CUs are at work, 20 TB/s from L2 over all of them (us, estimated / measured: 16 x 4096 x 4096
 // 4.4 / 4.2, 600 x 320 x 6144 6.7 / 6.4, 108 x 4096 x 8192 16.0 / 14.4); whole steps of a short K through registers at the rates below.  Fitted, int8 and FP8, to 1900
 // products of 1 .. 800 rows by 32 .. 4096 columns, K = 32 .. 8192, with what the 64 x 64 tiles took: the choice is 0.05 % above the fastest on average, 7 % the most.
-// `words`: rows start on four bytes; a load of 16 bytes at any other place takes a vector L1 three times as long (15 KB/us a CU).  Fitted to 482 and 500 products.
+// `words`: rows start on four bytes; others are read as the words they lie in (33 KB/us a CU of the rows there are).  Fitted to 482 and 524 products.
 inline double mfma8_direct_time(int M, int N, int K, int b, bool words, bool lines)
 {
-   if (!lines)
-      return b == 16 ? mfma8_time(M, N, K, 16, 16, 2.75, 0.43, words ? 54e3 : 14.9e3) : mfma8_time(M, N, K, 32, 32, 2.85, words ? 1.0 : 1.1, words ? 51e3 : 16.2e3);
+   if (!lines) {
+      if (words)
+         return b == 16 ? mfma8_time(M, N, K, 16, 16, 2.75, 0.43, 54e3) : mfma8_time(M, N, K, 32, 32, 2.85, 1.0, 51e3);
+      const double bytes = (double)(std::min(M, b) + std::min(N, b)) * K;
+      return b == 16 ? 2.24 + mfma8_rounds(M, N, 16, 16) * (0.64 + bytes / 32.7e3) : 1.17 + mfma8_rounds(M, N, 32, 32) * (2.06 + bytes / 33.6e3);
+   }
    if (!mfma8_direct_by_lines(b, M, N, K))
       return b == 16 ? mfma8_time(M, N, K, 16, 16, 2.5, 0.3, 41e3) : mfma8_time(M, N, K, 32, 32, 2.5, 0.45, 80e3);
    const double tiles = (double)((M + b - 1) / b) * ((N + b - 1) / b), ahead = std::min(K, 2048);
    return 2.5 + mfma8_rounds(M, N, b, b) * ((b == 16 ? 0.5 : 0.62) + 2.0 * b * (ahead / 120e3 + (K - ahead) / std::min(120e3, 20e6 / std::min(tiles, 256.0))));
 }
 // The general loop: tiles of 64 x 64, 128 x 64 and 128 x 128 (0, 1, 2).  By what it reads: rows that start on four bytes, rows that start anywhere, rows against a B that is
-// transposed on its way, a convolution's pixels.  Each fitted to 445 .. 1000 products of 1 .. 8192 rows and columns (int8 and FP8; 124 layers): the choice among the tiles is 0.4 - 1.3 % above the
+// transposed on its way (its k start anywhere, only they start on four bytes, both do), a convolution's pixels.  Each fitted to 201 .. 1000 products of 1 .. 8192 rows and columns (int8 and FP8; 124 layers): the choice among the tiles is 0.4 - 1.3 % above the
 // fastest on average.  Between 64 x 64, of which a CU has one or two, and 128 x 128, of which the chip has too few, the tile in the middle: us, the better of those two -> 128 x 64,
-// 1537 x 1000 x 777 with B transposed 10.8 -> 9.7, 1000 x 2000 x 500 8.9 -> 7.7, 2048^3 22.6 -> 19.4, 384 x 2976 x 3500 23.8 -> 19.5; rows 1537 x 1000 x 777 9.6 -> 9.0.  (A convolution's
+// 1537 x 1000 x 777 with B transposed 10.8 -> 9.7, 1000 x 2000 x 500 8.9 -> 7.7, 2048^3 22.6 -> 19.4, 384 x 2976 x 3500 23.8 -> 19.5.  (A convolution's
 // rows are worked out by each thread for its chunks: equal at best there.)
-enum Mfma8Source { MFMA8_WORD_ROWS, MFMA8_ROWS, MFMA8_COLUMNS, MFMA8_PIXELS };
+enum Mfma8Source { MFMA8_WORD_ROWS, MFMA8_ROWS, MFMA8_COLUMNS, MFMA8_WORD_COLUMNS, MFMA8_WORD_ROWS_COLUMNS, MFMA8_PIXELS };
+inline Mfma8Source mfma8_source(bool a_words, bool b_words, bool columns)
+{
+   if (columns)
+      return !b_words ? MFMA8_COLUMNS : a_words ? MFMA8_WORD_ROWS_COLUMNS : MFMA8_WORD_COLUMNS;
+   return a_words && b_words ? MFMA8_WORD_ROWS : MFMA8_ROWS;
+}
 inline double mfma8_general_time(int M, int N, int K, Mfma8Source source, int *tile = nullptr)
 {
    static constexpr struct {
       double fixed, tile, rate;
-   } COSTS[4][3] = {{{3.0, 1.1, 58e3}, {1.6, 2.95, 58e3}, {1.5, 4.9, 52e3}},
-                    {{2.8, 1.55, 42.5e3}, {1.5, 3.5, 42.3e3}, {1.2, 6.0, 41e3}},
-                    {{3.5, 1.13, 34e3}, {1.5, 3.2, 40e3}, {0.0, 6.7, 34.5e3}},
+   } COSTS[6][3] = {{{3.0, 1.1, 58e3}, {1.6, 2.95, 58e3}, {1.5, 4.9, 52e3}},
+                    {{3.1, 1.25, 47.6e3}, {1.5, 3.1, 51e3}, {1.5, 5.6, 42e3}},
+                    {{3.5, 1.13, 32e3}, {1.9, 3.0, 37e3}, {0.0, 6.7, 33e3}},
+                    {{3.65, 1.03, 36e3}, {2.1, 2.68, 43.8e3}, {0.5, 6.4, 33e3}},
+                    {{3.36, 1.04, 37e3}, {1.9, 2.7, 49.8e3}, {0.3, 6.25, 38e3}},
                     {{3.3, 0.95, 139e3}, {1e9, 0.0, 1.0}, {8.6, 3.6, 41e3}}};
    double least = 1e30;
    for (int t = 0; t < 3; ++t) {
@@ -67,20 +79,40 @@ inline double mfma8_ring_time(int M, int N, int K, int tile)
 
 // The general loop (any alignment, a convolution's input or plain rows, B either way).
 template <class MMA, class ASRC, class BSRC, class EPI>
-static int launch_mfma8_general(const LaunchCfg &lc, const ASRC &A, const BSRC &B, int M, int N, int K, const EPI &ep, bool words = false)
+static int launch_mfma8_general(const LaunchCfg &lc, const ASRC &A, const BSRC &B, int M, int N, int K, const EPI &ep)
 {
    constexpr bool PIXELS = !std::is_same_v<ASRC, StagedRows>;
+   Mfma8Source source = MFMA8_PIXELS;
+   bool by_words = false; // whether rows that start on no word are read as words
+   if constexpr (!PIXELS) {
+      const bool a = rows_of_words(A.base, A.ld), b = rows_of_words(B.base, B.ld);
+      source = mfma8_source(a, b, BSRC::kTransposed);
+      by_words = BSRC::kTransposed ? !a && StagedAnyRows::takes(A.ld) : !(a && b) && StagedAnyRows::takes(A.ld) && StagedAnyRows::takes(B.ld);
+   }
    int tile = 0;
-   mfma8_general_time(M, N, K, PIXELS ? MFMA8_PIXELS : BSRC::kTransposed ? MFMA8_COLUMNS : words ? MFMA8_WORD_ROWS : MFMA8_ROWS, &tile);
+   mfma8_general_time(M, N, K, source, &tile);
    if (lc.tile)
       tile = lc.tile == 64 ? 0 : lc.tile >= 128 && (lc.tile != 164 || PIXELS) ? 2 : lc.tile == 164 ? 1 : tile;
-   if constexpr (!PIXELS) {
-      if (tile == 1)
-         return launch_mfma8_staged<MMA, 128, 64, 128, 4, 2, 2, ASRC, BSRC, EPI>(lc, A, B, M, N, K, ep);
-   }
    if (tile == 2)
       return launch_mfma8_staged<MMA, 128, 128, 128, 4, 2, 2, ASRC, BSRC, EPI>(lc, A, B, M, N, K, ep);
-   return launch_mfma8_staged<MMA, 64, 64, 128, 2, 2, 2, ASRC, BSRC, EPI>(lc, A, B, M, N, K, ep);
+   auto smaller = [&](const auto &a, const auto &b) {
+      typedef std::decay_t<decltype(a)> AT;
+      typedef std::decay_t<decltype(b)> BT;
+      if constexpr (!PIXELS) {
+         if (tile == 1)
+            return launch_mfma8_staged<MMA, 128, 64, 128, 4, 2, 2, AT, BT, EPI>(lc, a, b, M, N, K, ep);
+      }
+      return launch_mfma8_staged<MMA, 64, 64, 128, 2, 2, 2, AT, BT, EPI>(lc, a, b, M, N, K, ep);
+   };
+   if constexpr (!PIXELS) {
+      if (by_words) {
+         if constexpr (BSRC::kTransposed)
+            return smaller(StagedAnyRows{A}, B);
+         else
+            return smaller(StagedAnyRows{A}, StagedAnyRows{B});
+      }
+   }
+   return smaller(A, B);
 }
 
 // Chooses between the direct kernel (few rows or tiles, short rows), the pipelined kernels (aligned operands, K a multiple of 64) and the general one.
@@ -93,15 +125,15 @@ static int launch_mfma8_best(const LaunchCfg &lc, const int8_t *A, const int8_t 
    typedef std::conditional_t<(MMA::KSTEP * 2 <= 64), DirectI8, DirectF8> Direct;
    const bool aligned = (lda % 16 == 0) && (ldb % 16 == 0) && (((uintptr_t)A & 15) == 0) && (((uintptr_t)Bt & 15) == 0);
    const bool ring = variant >= 0 && aligned && K >= 64 && K % 64 == 0 && (MMA::KSTEP * 2 <= 64 || K % 128 == 0);
-   const bool lines = aligned && K % 16 == 0, words = ((lda | ldb) & 3) == 0 && (((uintptr_t)A | (uintptr_t)Bt) & 3) == 0;
+   const bool lines = aligned && K % 16 == 0, words = rows_of_words(A, lda) && rows_of_words(Bt, ldb);
    const double t16 = mfma8_direct_time(M, N, K, 16, words, lines), t32 = mfma8_direct_time(M, N, K, 32, words, lines);
-   const double others = ring ? mfma8_ring_time(M, N, K, pick_tile(M, N, 0)) : mfma8_general_time(M, N, K, words ? MFMA8_WORD_ROWS : MFMA8_ROWS);
+   const double others = ring ? mfma8_ring_time(M, N, K, pick_tile(M, N, 0)) : mfma8_general_time(M, N, K, mfma8_source(words, words, false));
    if (force_tile == 16 || K < 16 || (!force_tile && variant == 0 && t16 <= t32 && t16 < others))
       return launch_mfma8_direct<Direct, 1, 1, 8, 4, EPI>(lc, A, Bt, M, N, K, lda, ldb, ep);
    if (force_tile == 32 || (!force_tile && variant == 0 && t32 < others))
       return launch_mfma8_direct<Direct, 2, 2, 8, 2, EPI>(lc, A, Bt, M, N, K, lda, ldb, ep);
    if (!ring || force_tile == 164)
-      return launch_mfma8_general<MMA, StagedRows, StagedRows, EPI>(lc, StagedRows{A, lda, M}, StagedRows{Bt, ldb, N}, M, N, K, ep, words);
+      return launch_mfma8_general<MMA, StagedRows, StagedRows, EPI>(lc, StagedRows{A, lda, M}, StagedRows{Bt, ldb, N}, M, N, K, ep);
    const int tile = pick_tile(M, N, force_tile);
    const bool k128 = (K % 128 == 0);
    if constexpr (MMA::KSTEP * 2 <= 64) {
@@ -150,20 +182,20 @@ static int launch_mfma8_best(const LaunchCfg &lc, const int8_t *A, const int8_t 
 }
 
 // Whether a product whose B is stored [K,N] is better off with the general loop, which transposes B on its way into LDS, than
-// with a launch that re-lays B out and the kernels above: that launch takes 2.7 us and 4.1 TB/s for the bytes it moves.  Fitted to 445 products; us, in the loop / re-laid out: 1537 x
+// with a launch that re-lays B out and the kernels above: that launch takes 3.6 us and 3.6 TB/s for the bytes it moves.  Fitted to 445 products; us, in the loop / re-laid out: 1537 x
 // 1000 x 777 9.7 / 13.2, 2048^3 19.4 / 22.6, 100 x 4000 x 4000 17.9 / 23.6, 5113 x 3917 x 1376 93.8 / 74.0, 2432 x 1125 x 3968 37.4 / 31.0.
-static bool mfma8_columns_preferred(const LaunchCfg &lc, int M, int N, int K, bool words_behind, bool aligned_behind)
+static bool mfma8_columns_preferred(const LaunchCfg &lc, const int8_t *A, int lda, const int8_t *B, int ldb, int M, int N, int K, bool aligned_behind)
 {
    if (K < 16 || N < 16 || lc.tile == 16 || lc.tile == 32)
       return false;
    if (lc.tile == 164)
       return true;
-   const bool lines = aligned_behind && K % 16 == 0;
+   const bool lines = aligned_behind && K % 16 == 0, a_words = rows_of_words(A, lda), words_behind = a_words && K % 4 == 0;
    double behind = std::min(std::min(mfma8_direct_time(M, N, K, 16, words_behind, lines), mfma8_direct_time(M, N, K, 32, words_behind, lines)),
-                            mfma8_general_time(M, N, K, words_behind ? MFMA8_WORD_ROWS : MFMA8_ROWS));
+                            mfma8_general_time(M, N, K, mfma8_source(words_behind, words_behind, false)));
    if (aligned_behind && K >= 64 && K % 64 == 0)
       behind = std::min(behind, mfma8_ring_time(M, N, K, pick_tile(M, N, 0)));
-   return lc.tile == 0 && lc.variant <= 0 && mfma8_general_time(M, N, K, MFMA8_COLUMNS) < 2.66 + (double)K * N / 2.07e6 + behind;
+   return lc.tile == 0 && lc.variant <= 0 && mfma8_general_time(M, N, K, mfma8_source(a_words, rows_of_words(B, ldb), true)) < 3.6 + (double)K * N / 1.8e6 + behind;
 }
 
 } // namespace sofie_hip

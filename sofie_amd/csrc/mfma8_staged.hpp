@@ -1,6 +1,6 @@
 // General tile loop of the int8 and the FP8 GEMM: any K, any alignment, B stored either way.  The pipelined kernels load straight
 // into LDS, which takes rows that start on 16 bytes and a K of whole slabs; here the slabs go through registers, so that a chunk
-// may be an unaligned 16-byte load (the hardware takes any address), the last chunk of a row is cut off at K, and a B given as
+// may start at any byte, the last chunk of a row is cut off at K, and a B given as
 // [K,N] is transposed on its way into LDS, four bytes by four, instead of by a launch of its own.
 //
 // A workgroup owns a BM x BN tile of Y and walks K in slabs of BK bytes, DEPTH slabs of loads ahead in registers, two slabs of LDS in
@@ -11,33 +11,19 @@
 
 namespace sofie_hip {
 
-// The chunk at k of a row of K >= 16 bytes as a load inside the row: where it crosses K, the last 16 bytes of the row instead,
-// which cut_chunk moves down to k, zeros behind them.
-__device__ __forceinline__ v4i fetch_cut(const int8_t *row, int k, int K)
-{
-   return *(const v4i_unaligned *)(row + (k <= K - 16 ? k : K - 16));
-}
-__device__ __forceinline__ v4i cut_chunk(v4i v, int k, int K)
-{
-   union {
-      v4i v;
-      unsigned long long q[2];
-   } u;
-   u.v = v;
-   const int drop = (k - K + 16) * 8; // bits that lie before k
-   if (drop > 0) {
-      const unsigned long long hi = drop >= 128 ? 0 : u.q[1];
-      u.q[0] = drop >= 64 ? hi >> (drop & 63) : (u.q[0] >> drop) | (u.q[1] << (64 - drop));
-      u.q[1] = drop >= 64 ? 0 : u.q[1] >> drop;
-   }
-   return u.v;
-}
-
 // An operand of `rows` rows that are contiguous in k.
 struct StagedRows {
    static constexpr bool kTransposed = false;
+   static constexpr int kWaves = 2; // a SIMD at least
    const int8_t *base;
    int ld, rows;
+};
+// The same with rows that start at any byte, fewer than 2^24 bytes apart: read as words, which the vector L1 takes faster than chunks that start on none (us, chunks -> words: 1537 x
+// 1000 x 777 9.7 -> 8.7, 777 x 1555 x 1999 16.3 -> 14.6, 384 x 2976 x 3501 20.4 -> 17.3).  Not for tiles of 128 x 128, which have no registers left for it beside four waves a SIMD: 4001 x 4001
+// x 1001 57 as chunks, 61 as words by two waves; nor for columns, whose short pieces would be two loads each: 777 x 1555 x 1999 16.0 and 18.3.
+struct StagedAnyRows : StagedRows {
+   static constexpr int kWaves = 4;
+   static bool takes(int ld) { return ld < 1 << 24; } // offsets inside a slab in 32 bits
 };
 // An operand stored [K][rows]: contiguous along the rows.
 struct StagedColumns {
@@ -52,6 +38,7 @@ struct StagedColumns {
 template <int PIECE_>
 struct StagedConvRows {
    static constexpr bool kTransposed = false;
+   static constexpr int kWaves = 2;
    static constexpr int PIECE = PIECE_;
    const int8_t *X; // first channel of the group
    int rows, H, W, C, OH, OW, stride_h, stride_w, pad_h0, pad_w0, dil_h, dil_w, kw, Cg, K;
@@ -86,7 +73,7 @@ struct StagedSlab {
    {
 #pragma unroll
       for (int i = 0; i < LD; ++i)
-         v[i] = fetch_cut(row_of(s, r0, i, t), k_of(k0, i, t), K);
+         v[i] = *(const v4i_unaligned *)chunk_in_row(row_of(s, r0, i, t), k_of(k0, i, t), K);
    }
    __device__ __forceinline__ void finish_last(int k0, int K, int t)
    {
@@ -100,6 +87,65 @@ struct StagedSlab {
       for (int i = 0; i < LD; ++i) {
          const int id = t + i * NTHREADS;
          *(v4i *)(lds + lds_chunk_offset<BK>(id / CPR, id % CPR)) = v[i];
+      }
+   }
+};
+
+template <int R, int BK, int NTHREADS>
+struct StagedSlab<StagedAnyRows, R, BK, NTHREADS> {
+   typedef StagedAnyRows SRC;
+   typedef StagedSlab<StagedRows, R, BK, NTHREADS> Words;
+   static constexpr int CPR = Words::CPR, LD = Words::LD;
+   static_assert(CPR == 8, "half a row of lanes to a row of the slab");
+   // from the word that the tile starts in: a chunk's first word and the word behind the slab's row (the one its last byte lies in, where the row starts on a word)
+   struct places {
+      unsigned at[LD], behind[LD], shift[LD];
+   };
+   AnyChunk c[LD];
+   static __device__ __forceinline__ const int8_t *tile_of(const SRC &s, int r0) { return s.base + (size_t)r0 * (size_t)s.ld; }
+   static __device__ __forceinline__ void find(const SRC &s, int r0, int t, places &p)
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i) {
+         const int r = (t + i * NTHREADS) / CPR;
+         const unsigned from = ((unsigned)(uintptr_t)tile_of(s, r0) & 3u) + (unsigned)(r0 + r < s.rows ? r : s.rows - 1 - r0) * (unsigned)s.ld;
+         p.at[i] = (from & ~3u) + (unsigned)(t % CPR * 16);
+         p.behind[i] = (from + BK - 1) & ~3u;
+         p.shift[i] = from & 3u;
+      }
+   }
+   __device__ __forceinline__ void load(const SRC &s, const places &p, int r0, int k0, int, int)
+   {
+      const int8_t *tile = tile_of(s, r0);
+      tile += k0 - (int)((unsigned)(uintptr_t)tile & 3u);
+#pragma unroll
+      for (int i = 0; i < LD; ++i) {
+         c[i].v = *(const AnyChunk::words_t *)(tile + p.at[i]);
+         c[i].behind = *(const unsigned *)(tile + p.behind[i]);
+         c[i].shift = p.shift[i];
+      }
+   }
+   __device__ __forceinline__ void load_last(const SRC &s, const places &, int r0, int k0, int K, int t)
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i)
+         c[i].load(chunk_in_row(Words::row_of(s, r0, i, t), Words::k_of(k0, i, t), K));
+   }
+   __device__ __forceinline__ void finish_last(int k0, int K, int t)
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i) {
+         c[i].v = cut_chunk(c[i].bytes(), Words::k_of(k0, i, t), K);
+         c[i].shift = 0;
+      }
+   }
+   __device__ __forceinline__ void store(int8_t *lds, int t) const
+   {
+#pragma unroll
+      for (int i = 0; i < LD; ++i) {
+         const int id = t + i * NTHREADS;
+         const unsigned next = (unsigned)__builtin_amdgcn_mov_dpp(c[i].v[0], 0x101, 0xf, 0xf, true); // row_shl:1
+         *(v4i *)(lds + lds_chunk_offset<BK>(id / CPR, id % CPR)) = AnyChunk::aligned(c[i].v, id % CPR == CPR - 1 ? c[i].behind : next, c[i].shift);
       }
    }
 };
@@ -247,7 +293,7 @@ struct StagedSlab<StagedColumns, R, BK, NTHREADS> {
 };
 
 template <class MMA, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int DEPTH, class ASRC, class BSRC, class EPI>
-__global__ __launch_bounds__(WAVES_M *WAVES_N * 64, 2) void mfma8_staged_kernel(ASRC A, BSRC B, int M, int N, int K, EPI ep, TileOrder order)
+__global__ __launch_bounds__(WAVES_M *WAVES_N * 64, ASRC::kWaves) void mfma8_staged_kernel(ASRC A, BSRC B, int M, int N, int K, EPI ep, TileOrder order)
 {
    constexpr int NTHREADS = WAVES_M * WAVES_N * 64;
    constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N, MT = TM / 32, NT = TN / 32;
