@@ -4,8 +4,8 @@
 // floats touches three or four lines, and a slab of 32 k of a 64 x 64 tile took 0.60 us where its MFMAs take 0.43.  Here a tile is BM consecutive output pixels
 // (through rows and images) and BN output channels; what it reads of a channel is one run of rows, loaded once, and the nine kernel
 // positions read it from LDS at offsets that are known where the code is written.  64 images, us before -> after: 32 -> 64 channels at
-// 32 x 32 36.7 -> 26.8, 64 -> 64 57.2 -> 43.8 (110 TFLOP/s of the matrix cores' 157; on another card 44.7, with a residual 45.3);
-// one image, 48 -> 96 at 40 x 40 12.8 -> 8.4.  (Up to four channels are f32_conv3x3_few.hpp's.)  On 64 -> 64 the matrix cores work in 0.72 of the cycles and no bank conflicts are
+// 32 x 32 36.7 -> 26.8, 64 -> 64 57.2 -> 43.8 (110 TFLOP/s of the matrix cores' 157; on another card 44.7, with a residual 45.3), 3 -> 32 at
+// 64 x 64 24.2 -> 17.0 (14.9 with the stores below); one image, 48 -> 96 at 40 x 40 12.8 -> 8.4.  On 64 -> 64 the matrix cores work in 0.72 of the cycles and no bank conflicts are
 // counted; what is left is a patch that is loaded once per 32 output channels and one MFMA per value read from LDS.
 //
 // The images are taken as one column of OH + 2 rows each, padding included (row r of image i is row i (OH + 2) + r), and OW + 2 columns:
@@ -67,9 +67,11 @@ inline bool conv3x3_plain(const PostChain &chain) { return chain.count == 0 || (
 
 // The results that a lane holds of a block: E of the 16 channels first + 4 lk + e / 4 * 8 + e % 4, from element e0 (a multiple of 4) on, of one pixel.  32 neighbouring
 // lanes hold 32 neighbouring pixels of a channel: whole lines, loaded and stored straight from the registers.  Addresses are an offset per lane, one for all
-// channels, and a scalar per channel.  (With an address, a bound and a branch per channel, places of the patch worked out by every wave and more scalars spilled, a tile of
-// one slab had twice the vector instructions.)  Still spilled, in plain kernels: 20 - 32 scalars at 128 pixels, up to 66 where waves share a tile (none at 256 places
-// with wide weights).
+// channels, and a scalar per channel.  A tile of few input channels is bound by the instructions around its MFMAs: with an address, a bound and a branch per
+// channel, places of the patch worked out by every wave and more scalars spilled, 3 -> 32 channels had 18 MFMAs a wave among 573 vector and 357 scalar instructions, now
+// 303 and 298.  64 images of 64 x 64, us before -> after, for all of these together: 3 -> 32 channels 19.3 -> 14.9; 40 of 90 x 90, 3 -> 12 23.2 -> 16.7; 1 of 64 x 64
+// 5.5 -> 4.0.  Still spilled, in plain kernels: 6 scalars with few channels, 20 - 32 at 128 pixels, up to 66 where waves share a tile (none at 256 places with wide
+// weights).
 template <int E>
 struct Conv3x3Block {
    float *Y;         // result of channel `first`, pixel 0 of the tile's first image (scalar)
@@ -165,12 +167,12 @@ struct Conv3x3Block {
    }
 };
 
-// Eight channels per slab; lane half lk multiplies the four from 4 lk on, kernel position by kernel position.
-template <int BM, int BN, int PLANE, int WVEC>
+// CS channels per slab; lane half lk multiplies the channels from lk * CS / 2 on, kernel position by kernel position.
+template <int BM, int BN, int CS, int PLANE, int WVEC>
 struct F32Conv3x3Shape {
-   static constexpr int CS = 8, HALF = CS / 2 * 9;              // k per lane half and slab
-   static constexpr int PITCH = 76;                             // of a weight row in LDS: the rows of a fragment start in different banks
-   static constexpr int READ = 4;                               // floats of a weight row that a lane reads at once
+   static constexpr int HALF = CS / 2 * 9;                      // k per lane half and slab
+   static constexpr int PITCH = CS == 8 ? 76 : 38;              // of a weight row in LDS: the rows of a fragment start in different banks
+   static constexpr int READ = CS == 8 ? 4 : 2;                 // floats of a weight row that a lane reads at once
    static constexpr int PATCH = CS * PLANE + 32;                // the second half of the channels starts 32 banks on
    static constexpr int WEIGHTS = (BN * PITCH + 64 * WVEC - 1) / (64 * WVEC) * 64 * WVEC;
    static constexpr int STAGE = (PATCH + WEIGHTS + 3) / 4 * 4;
@@ -182,11 +184,10 @@ struct F32Conv3x3Shape {
 // Two slabs in LDS, the next on its way while one is multiplied (2304 cycles of MFMAs for 32 x 32 wave tiles), and several workgroups per CU
 // that cover each other's trips to memory and barriers.  WAVES_K waves share a wave tile, each multiplying every WAVES_K-th step of
 // a slab: where there are few tiles, smaller ones keep as many matrix cores busy.
-template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int PLANE, int WVEC, bool PLAIN>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int CS, int PLANE, int WVEC, bool PLAIN>
 __global__ __launch_bounds__(256, 2) void f32_conv3x3_kernel(F32Conv3x3 a, F32ConvStore out, TileOrder order, int first_tile, int places_at)
 {
-   typedef F32Conv3x3Shape<BM, BN, PLANE, WVEC> S;
-   constexpr int CS = S::CS;
+   typedef F32Conv3x3Shape<BM, BN, CS, PLANE, WVEC> S;
    constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N, MT = TM / 32, NT = TN / 32;
    // Waves that share a tile wait for their loads: bounds worked out again before each slab's cost more than their spills (2 images of 25 x 25, 128 -> 66 channels
    // 16.8 us against 15.9).  With a tile each they are what a slab's issue waits for.
@@ -239,7 +240,7 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_kernel(F32Conv3x3 a, F32Co
       weight_at[i] = n0 + row < a.N && k < 2 * S::HALF ? (row * a.K + k) * 4 : F32_OUTSIDE;
    }
 
-   const int slabs = (a.C + CS - 1) / CS;
+   const int slabs = CS == 4 ? 1 : (a.C + CS - 1) / CS; // slabs of 4 channels are for layers that have no more
    auto issue_weights = [&](int s, int stage) {
       float *lds = f32_lds + stage * S::STAGE;
       const bool whole = (s + 1) * CS <= a.C;
@@ -414,16 +415,16 @@ __global__ __launch_bounds__(256, 2) void f32_conv3x3_kernel(F32Conv3x3 a, F32Co
    });
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int PLANE, int WVEC>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int CS, int PLANE, int WVEC>
 static int launch_f32_conv3x3_as(hipStream_t stream, const F32Conv3x3 &a, const F32ConvStore &out, int group)
 {
    const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
    if ((long long)tiles_m * tiles_n > 0x7fffffffLL)
       return fail(SOFIE_HIP_ERR_INVALID, "fp32 convolution: too many tiles");
-   constexpr size_t stage = sizeof(float) * F32Conv3x3Shape<BM, BN, PLANE, WVEC>::STAGE, parts = WAVES_K > 1 ? 4 * 1024 * sizeof(float) : 0;
-   const size_t slabs = std::max(stage * (a.C > 8 ? 2 : 1), parts), smem = slabs + PLANE * sizeof(int);
+   constexpr size_t stage = sizeof(float) * F32Conv3x3Shape<BM, BN, CS, PLANE, WVEC>::STAGE, parts = WAVES_K > 1 ? 4 * 1024 * sizeof(float) : 0;
+   const size_t slabs = std::max(stage * (a.C > CS ? 2 : 1), parts), smem = slabs + PLANE * sizeof(int);
    auto go = [&](auto plain) {
-      auto kern = f32_conv3x3_kernel<BM, BN, WAVES_M, WAVES_N, WAVES_K, PLANE, WVEC, decltype(plain)::value>;
+      auto kern = f32_conv3x3_kernel<BM, BN, WAVES_M, WAVES_N, WAVES_K, CS, PLANE, WVEC, decltype(plain)::value>;
       static bool configured[64] = {};
       if (int st = configure_lds_once(kern, std::max(stage * 2, parts) + PLANE * sizeof(int), configured))
          return st;

@@ -5,10 +5,11 @@
 // channels wide.  Here the reduction is the layer's own 9 C, in the order the weights have in memory, padded to a multiple of four (v_mfma_f32_16x16x4_f32: seven MFMAs for
 // three channels, 32 cycles each), and a workgroup takes `span` consecutive pixels of an image: weights and the distances of a lane's products in the patch are worked out
 // once, and 32 pixels more cost two quotients, the reads of their fragments and the stores.  us, tiles of 128 pixels -> here: 64 images of 64 x 64, 3 -> 32 channels 14.6 ->
-// 12.1, 8 of 96 x 96, 3 -> 48 10.8 -> 10.0, 30 of 47 x 47, 3 -> 9 5.9 -> 4.6, 1 of 20 x 20, 3 -> 16 3.6 -> 2.9; 4096 of 6 x 6, 3 -> 16 14.3 -> 13.0 (eight channels wide there).  Of the
-// first, 7.1 are left without MFMAs and stores, 8.9 with the stores, 11.9 with the MFMAs: all its workgroups start together, and wait for the same things.
+// 12.1, 8 of 96 x 96, 3 -> 48 10.8 -> 10.0, 30 of 47 x 47, 3 -> 9 5.9 -> 4.6, 1 of 20 x 20, 3 -> 16 3.6 -> 2.9 (not for
+// many small images: f32_conv3x3_few_preferred).  Of the first, 7.1 are left without MFMAs and stores, 8.9 with the stores, 11.9 with the MFMAs: all its workgroups start together, and wait for the same things.
 #pragma once
 #include "f32_conv3x3.hpp"
+#include <cmath>
 
 namespace sofie_hip {
 
@@ -186,35 +187,59 @@ inline bool f32_conv3x3_few_takes(const F32Conv3x3 &a, const F32ConvStore &out)
    return a.C <= 4 && (long long)a.images * ((out.positions + 127) / 128) * ((a.N + 15) / 16) <= 0x7fffffffLL && 80LL * out.positions * 4 < bytes && 4LL * a.H * a.Wd * 4 < bytes && f32_conv3x3_few_patch(a.OH, a.OW, 128) * a.C <= F32_CONV3X3_FEW_PATCH;
 }
 
-static int launch_f32_conv3x3_few(hipStream_t stream, const F32Conv3x3 &a, const F32ConvStore &out, int group)
+// How a layer is split: pixels and blocks of channels of a workgroup, floats of a channel of its patch.
+struct F32Conv3x3FewSplit {
+   int span, chunks, nb, tiles_n, plane;
+   long long total; // workgroups of a group
+   F32Conv3x3FewSplit(const F32Conv3x3 &a, const F32ConvStore &out, int group)
+   {
+      // Channels of a tile: as many blocks of 16 as there are, or as few tiles as hold four each.  Pixels: as many as leave two workgroups for each CU, us with 128 / 256 / 512 / 1024:
+      // 64 images of 64 x 64, 3 -> 32 channels 16.2 / 13.5 / 12.6 / 13.8, 16 of 28 x 28, 1 -> 32 3.2 / 3.9 / 5.3 / 7.2, 64 of 96 x 96, 3 -> 16 18.9 / 15.0 / 14.5 / 15.6.
+      const int blocks = (a.N + 15) / 16;
+      tiles_n = (blocks + 3) / 4;
+      span = 512;
+      auto workgroups = [&] { return (long long)a.images * ((out.positions + span - 1) / span) * tiles_n; };
+      while (span > 128 && (workgroups() * group < 512 || f32_conv3x3_few_patch(a.OH, a.OW, span) * a.C > F32_CONV3X3_FEW_PATCH))
+         span /= 2;
+      while (tiles_n < blocks && workgroups() * group < 256)
+         ++tiles_n;
+      nb = (blocks + tiles_n - 1) / tiles_n;
+      tiles_n = (blocks + nb - 1) / nb;
+      chunks = (out.positions + span - 1) / span;
+      span = ((out.positions + chunks - 1) / chunks + 31) / 32 * 32; // as much for each
+      plane = (int)f32_conv3x3_few_patch(a.OH, a.OW, span);
+      total = workgroups();
+   }
+};
+
+// Whether the kernel is faster than tiles of 128 pixels, four channels wide, that run through images (f32_conv3x3.hpp; `patch`: their positions).  A workgroup here stays within an
+// image, so that one of 9 pixels is a workgroup of 128 places for each, and the four-channel kernel with four blocks spills: us, those tiles / here, 65536 images of 3 x 3, 4 -> 64 channels 60 / 614,
+// 16384 of 5 x 5, 3 -> 32 23 / 67, 124 of 14 x 14, 4 -> 48 6.0 / 7.5, 21 of 63 x 63, 4 -> 159 21.9 / 30.3, but 6311 of 8 x 8, 3 -> 2 17.2 / 13.2, and 64 of 64 x 64, 3 -> 32 14.6 /
+// 12.1.  Costs, us: a launch, the trip to memory, a CU's workgroups by their patches and MFMAs, the layer's bytes; a launch and a CU's tiles.  Fitted for the choice to 1161 layers
+// of 1 to 65536 images of 3 to 115 columns, up to 160 channels out, up to 256 groups: 0.2 % above the faster on average, 15 % the most (always here: 9.4 %, 5.7 times; always there: 50 %).
+inline bool f32_conv3x3_few_preferred(const F32Conv3x3 &a, const F32ConvStore &out, const F32Conv3x3FewSplit &split, int group, long long patch)
 {
-   // Channels of a tile: as many blocks of 16 as there are, or as few tiles as hold four each.  Pixels: as many as leave two workgroups for each CU, us with 128 / 256 / 512 / 1024:
-   // 64 images of 64 x 64, 3 -> 32 channels 16.2 / 13.5 / 12.6 / 13.8, 16 of 28 x 28, 1 -> 32 3.2 / 3.9 / 5.3 / 7.2, 64 of 96 x 96, 3 -> 16 18.9 / 15.0 / 14.5 / 15.6.
-   const int blocks = (a.N + 15) / 16;
-   int tiles_n = (blocks + 3) / 4;
-   int span = 512;
-   auto workgroups = [&] { return (long long)a.images * ((out.positions + span - 1) / span) * tiles_n; };
-   while (span > 128 && (workgroups() * group < 512 || f32_conv3x3_few_patch(a.OH, a.OW, span) * a.C > F32_CONV3X3_FEW_PATCH))
-      span /= 2;
-   while (tiles_n < blocks && workgroups() * group < 256)
-      ++tiles_n;
-   const int nb = (blocks + tiles_n - 1) / tiles_n;
-   tiles_n = (blocks + nb - 1) / nb;
-   const int chunks = (out.positions + span - 1) / span;
-   span = ((out.positions + chunks - 1) / chunks + 31) / 32 * 32; // as much for each
-   const int plane = (int)f32_conv3x3_few_patch(a.OH, a.OW, span);
-   const long long total = workgroups();
-   const size_t smem = (size_t)plane * a.C * 4;
+   const int steps = (9 * a.C + 3) / 4;
+   const double cus = 256.0, workgroups = std::ceil((double)split.total * group / cus), tiles = std::ceil((double)((a.M + 127LL) / 128) * ((a.N + 31LL) / 32) * group / cus);
+   const double trip = 0.106 * split.nb * steps, bytes = 4.0 * a.images * group * (a.C + a.N) * out.positions;
+   const double each = 0.036 + 0.000189 * split.plane * a.C + (split.span + 127) / 128 * split.nb * (0.0306 * steps + 0.126) * (a.C < 4 ? 1.0 : split.nb < 4 ? 1.13 : 1.82);
+   const double here = 2.89 + std::sqrt(trip * trip + workgroups * each * workgroups * each + bytes / 6.8e6 * (bytes / 6.8e6));
+   return here <= 3.47 + tiles * (1.07 + 0.000244 * patch);
+}
+
+static int launch_f32_conv3x3_few(hipStream_t stream, const F32Conv3x3 &a, const F32ConvStore &out, const F32Conv3x3FewSplit &split, int group)
+{
+   const size_t smem = (size_t)split.plane * a.C * 4;
    auto with = [&](auto steps, auto nbc, auto plain) {
       auto kern = f32_conv3x3_few_kernel<decltype(steps)::value, decltype(nbc)::value, decltype(plain)::value>;
-      const TileOrder order((int)(total / tiles_n), tiles_n, 0, group);
+      const TileOrder order((int)(split.total / split.tiles_n), split.tiles_n, 0, group);
       in_launches(order.workgroups(group), 256, [&](int first, unsigned count) {
-         launch_kernel(kern, dim3(count, 1, order.depth(group)), dim3(256), smem, stream, a, out, order, Divisor31(chunks), span, plane, first);
+         launch_kernel(kern, dim3(count, 1, order.depth(group)), dim3(256), smem, stream, a, out, order, Divisor31(split.chunks), split.span, split.plane, first);
       });
       return launch_status("f32_conv3x3_few_kernel");
    };
    auto blocks_of = [&](auto steps, auto plain) {
-      switch (nb) {
+      switch (split.nb) {
       case 1: return with(steps, std::integral_constant<int, 1>{}, plain);
       case 2: return with(steps, std::integral_constant<int, 2>{}, plain);
       case 3: return with(steps, std::integral_constant<int, 3>{}, plain);

@@ -403,10 +403,16 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
                 Divisor31(s.OW + 2LL), Divisor31(s.OH + 2LL)};
    int tile = force;
    if ((!tile || tile == F32_CONV3X3_FEW) && f32_conv3x3_few_takes(a, out)) {
-      *taken = true;
-      return launch_f32_conv3x3_few(ctx->stream, a, out, group);
+      const F32Conv3x3FewSplit split(a, out, group);
+      const long long patch = f32_conv3x3_patch(s.OH, s.OW, 128);
+      if (tile || patch > F32_CONV3X3_PATCH || f32_conv3x3_few_preferred(a, out, split, group, patch)) {
+         *taken = true;
+         return launch_f32_conv3x3_few(ctx->stream, a, out, split, group);
+      }
    }
-   if (!tile) {
+   if (!tile && s.Cg <= 4) {
+      tile = F32_CONV3X3_128; // slabs of four channels; half of any other kernel's slab would be zeros
+   } else if (!tile) {
       // us: a launch; a slab (8 channels, 16 of the split kernel) of a CU whose tiles wait for their loads, and of one with several tiles at work; a tile.  The
       // second set is for weights that come float by float.  Fitted to 156 layers (the split kernel's to 230 others) from 1 image of 6 x 6 to 64 of 64 x 64, 5 to 130
       // channels; holds to a sixth, and costs 0.4 % of the best of these kernels on average over the 260 layers, 14 % the most, 10 % but for that one.
@@ -455,10 +461,12 @@ static int launch_f32_conv3x3(sofie_hip_ctx *ctx, const float *X, const F32ConvS
    }
    auto go = [&](auto room, auto wide) {
       constexpr int P = decltype(room)::value, V = decltype(wide)::value;
+      if (s.Cg <= 4 && tile == F32_CONV3X3_128)
+         return launch_f32_conv3x3_as<128, 32, 4, 1, 1, 4, P, 1>(st, a, out, group);
       switch (tile) {
-      case F32_CONV3X3_32: return launch_f32_conv3x3_as<32, 32, 1, 1, 4, P, V>(st, a, out, group);
-      case F32_CONV3X3_64: return launch_f32_conv3x3_as<64, 32, 2, 1, 2, P, V>(st, a, out, group);
-      default: return launch_f32_conv3x3_as<128, 32, 4, 1, 1, P, V>(st, a, out, group);
+      case F32_CONV3X3_32: return launch_f32_conv3x3_as<32, 32, 1, 1, 4, 8, P, V>(st, a, out, group);
+      case F32_CONV3X3_64: return launch_f32_conv3x3_as<64, 32, 2, 1, 2, 8, P, V>(st, a, out, group);
+      default: return launch_f32_conv3x3_as<128, 32, 4, 1, 1, 8, P, V>(st, a, out, group);
       }
    };
    auto with = [&](auto room) { return vec ? go(room, std::integral_constant<int, 4>{}) : go(room, std::integral_constant<int, 1>{}); };
