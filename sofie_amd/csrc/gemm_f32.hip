@@ -120,7 +120,12 @@ __device__ __forceinline__ void chain_rows(float (&sums)[RB], const ChainLayerAr
    }
 }
 
-template <int RB>
+// Rows of W that chain_rows reads.
+__host__ __device__ __forceinline__ bool chain_layer_by_rows(const ChainLayerArgs &L) { return L.transB && L.K % 4 == 0 && L.ldb % 4 == 0 && ((uintptr_t)L.B & 15) == 0; }
+
+// ROWS: some layer goes through chain_rows.  Its code costs the others' registers (92 - 112 vector registers and up to 29 scalars spilled, 64 - 92 and up to two without): layers
+// with W stored [K][N] in the kernel with it / without, M x K-..-N, 40 x 256-128-128-1123-11 15.7 / 15.0 us, 3 x 4-128-5 5.10 / 4.98.
+template <int RB, bool ROWS>
 __global__ __launch_bounds__(CHAIN_THREADS) void gemm_chain_f32_kernel(ChainArgs a, int width)
 {
    extern __shared__ float chain_lds[]; // two buffers of RB rows x width, RB sums per thread
@@ -143,7 +148,7 @@ __global__ __launch_bounds__(CHAIN_THREADS) void gemm_chain_f32_kernel(ChainArgs
       const ChainLayerArgs &L = a.layer[l];
       const int N = L.N, K = L.K;
       const float *__restrict__ B = L.B;
-      if (L.transB && K % 4 == 0 && L.ldb % 4 == 0 && ((uintptr_t)B & 15) == 0) {
+      if (ROWS && chain_layer_by_rows(L)) {
          // four outputs a wave, sixteen where one pass would not do and rows are short enough for as many loads
          const int g_log2 = K <= 64 ? 4 : K <= 128 ? 5 : 6, j_log2 = N > 64 ? 2 : g_log2 - 4, per_wave = 64 >> g_log2 << j_log2;
          for (int n0 = wave * per_wave; n0 < N; n0 += CHAIN_THREADS / 64 * per_wave) {
@@ -598,15 +603,21 @@ static int launch_f32_chain(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *layer
    if (fused && (long long)RB * width <= 8192) {
       const size_t lds = ((size_t)2 * RB * width + RB * CHAIN_THREADS) * sizeof(float);
       const dim3 grid((unsigned)((M + RB - 1) / RB));
-      auto launch = [&](auto rows) -> int {
-         auto kern = gemm_chain_f32_kernel<decltype(rows)::value>;
+      bool any = false;
+      for (int l = 0; l < count; ++l)
+         any = any || chain_layer_by_rows(a.layer[l]);
+      auto launch = [&](auto rows, auto by_rows) -> int {
+         auto kern = gemm_chain_f32_kernel<decltype(rows)::value, decltype(by_rows)::value>;
          static bool configured[64] = {};
          if (int st = configure_lds_once(kern, (2 * 8192 + decltype(rows)::value * CHAIN_THREADS) * sizeof(float), configured))
             return st;
          launch_kernel(kern, grid, dim3(CHAIN_THREADS), lds, ctx->stream, a, width);
          return SOFIE_HIP_OK;
       };
-      if (int st = RB == 1 ? launch(std::integral_constant<int, 1>{}) : RB == 2 ? launch(std::integral_constant<int, 2>{}) : launch(std::integral_constant<int, 4>{}))
+      auto with = [&](auto by_rows) {
+         return RB == 1 ? launch(std::integral_constant<int, 1>{}, by_rows) : RB == 2 ? launch(std::integral_constant<int, 2>{}, by_rows) : launch(std::integral_constant<int, 4>{}, by_rows);
+      };
+      if (int st = any ? with(std::true_type{}) : with(std::false_type{}))
          return st;
       *launched = true;
       return launch_status("gemm_chain_f32_kernel");
