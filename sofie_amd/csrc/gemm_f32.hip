@@ -128,7 +128,8 @@ __host__ __device__ __forceinline__ bool chain_layer_by_rows(const ChainLayerArg
 template <int RB, bool ROWS>
 __global__ __launch_bounds__(CHAIN_THREADS) void gemm_chain_f32_kernel(ChainArgs a, int width)
 {
-   extern __shared__ float chain_lds[]; // two buffers of RB rows x width, RB sums per thread
+   // two buffers of RB rows x width, RB sums per thread; chain_rows reads 16 bytes at a time: width is a multiple of four
+   extern __shared__ __attribute__((aligned(16))) float chain_lds[];
    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
    const int m0 = blockIdx.x * RB;
    const int rows = (a.M - m0) < RB ? (a.M - m0) : RB;
