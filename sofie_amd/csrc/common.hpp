@@ -7,6 +7,7 @@
 #include <cstring>
 #include <type_traits>
 #include "sofie_hip.h"
+#include "tile_order.hpp"
 
 // Kernel-choice overrides of a context (tuning and tests).  Read from the environment ONCE, when the context is created
 // (SOFIE_HIP_SWIZZLE, SOFIE_HIP_I8_TILE, SOFIE_HIP_F8_TILE, SOFIE_HIP_GEMM_VARIANT, SOFIE_HIP_CONV_EXPLICIT,
@@ -96,22 +97,6 @@ inline int launch_status(const char *what)
 
 // The longest M or N of a product: rows are counted in 32 bits up to the end of the last tile, of at most 256.
 constexpr long long MOST_ROWS = 0x7fffffffLL - 255;
-
-// Index arithmetic by an extent that the launch knows: a multiplication while every index fits 31 bits (a 64-bit division by a
-// run-time value is some hundred instructions per element, several times what the memory traffic of most kernels leaves room for).
-struct Divisor31 {
-   // with s = ceil(log2 d) and mul = ceil(2^(31 + s) / d), mul d - 2^(31 + s) < 2^s: below 2^31 the error of n mul / 2^(31 + s) is
-   // smaller than 1 / d, and mul < 2^32
-   unsigned d, mul, shift;
-   explicit Divisor31(long long extent) : d((unsigned)extent), shift(0)
-   {
-      while ((1ull << shift) < d)
-         ++shift;
-      mul = (unsigned)(((1ull << (31 + shift)) + d - 1) / d);
-   }
-   typedef unsigned index;
-   __device__ __forceinline__ index over(index n) const { return __umulhi(2 * n, mul) >> shift; }
-};
 
 // ---- scalar formulas shared by every epilogue --------------------------------------------------
 

@@ -120,51 +120,6 @@ __device__ __forceinline__ void tile_of_block(int bid, int nwg, int tiles_m, int
    tn = (id % width) / gsz;
 }
 
-// The same for a launch whose tiles are known to the host, which works out the divisors: four divisions by run-time values are 400 cycles that a small product waits for before its
-// first load.  The products of a batch are laid side by side in the same list, so that those of one product meet in one XCD's L2: 96 products of 128 x 128 x 64
-// read 18 MB through eight L2s, whose operands are 6.
-struct TileOrder {
-   int tiles_m, tiles_n, band, last; // last: rows of the last band
-   int per, rem;                     // workgroups of an XCD, XCDs with one more; per < 0: no regrouping
-   int tiles;                        // of a product of a batch; 0: the products are the grid's z
-   Divisor31 by_width, by_band, by_last, by_tiles;
-   TileOrder(int tiles_m, int tiles_n, int mode, int batch = 1)
-      : tiles_m(tiles_m), tiles_n(tiles_n), band(std::max(1, std::min(mode & 0xff, tiles_m))), last(tiles_m % band ? tiles_m % band : band), by_width((long long)band * tiles_n),
-        by_band(band), by_last(last), by_tiles(1)
-   {
-      const long long one = (long long)tiles_m * tiles_n, all = one * batch;
-      tiles = batch > 1 && all <= 0x7fffffffLL ? (int)one : 0;
-      if (tiles)
-         by_tiles = Divisor31(tiles);
-      per = mode & 0x100 ? -1 : (int)((tiles ? all : one) / 8);
-      rem = (int)((tiles ? all : one) % 8);
-   }
-   long long workgroups(int batch) const { return (long long)tiles_m * tiles_n * (tiles ? batch : 1); } // of the grid's x
-   unsigned depth(int batch) const { return tiles ? 1u : (unsigned)batch; }                            // its z
-   __device__ __forceinline__ void place(int bid, int &tm, int &tn, int &product) const
-   {
-      int id = bid;
-      if (per >= 0) {
-         const int xcd = bid & 7;
-         id = xcd * per + (xcd < rem ? xcd : rem) + (bid >> 3);
-      }
-      product = blockIdx.z;
-      if (tiles) {
-         product = (int)by_tiles.over((unsigned)id);
-         id -= product * tiles;
-      }
-      const int group = (int)by_width.over((unsigned)id), first = group * band, in = id - group * band * tiles_n;
-      const bool whole = first + band <= tiles_m;
-      tn = whole ? (int)by_band.over((unsigned)in) : (int)by_last.over((unsigned)in);
-      tm = first + in - tn * (whole ? band : last);
-   }
-   __device__ __forceinline__ void place(int bid, int &tm, int &tn) const
-   {
-      int product;
-      place(bid, tm, tn, product);
-   }
-};
-
 // Byte offset of 16-byte chunk c of row r in an LDS slab of BK-byte rows.  Chunk c is stored at chunk
 // position c ^ ((r / rows_per_256B) % chunks_per_row): the 16 lanes served together by one ds_read_b128
 // (16 consecutive rows, same logical chunk) then fall into 16 different 16-byte bank groups.
