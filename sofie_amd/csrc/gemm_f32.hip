@@ -284,8 +284,10 @@ namespace sofie_hip {
 // tiles, and `tile` per 256 tiles; where both operands come line by line through its ring, 78 KB/us a CU and 0.48 us for the first 256 tiles, 73 and 0.49 a tile where
 // there are more.  Fitted to 1220 products of each kind of 16-byte loads, and to 1384 that come float by float, 1 .. 4096 rows, K = 8 .. 2048; on 1500 other products on average 0.15 %
 // (float by float), 0.2 % (float by float along k), 0.13 % and 0.11 % (16 bytes, along k) above the best kernel's time, 18 % the most.  (With the costs of a direct kernel that branched
-// around its loads, those float by float were 7.8 and 9.5 % above, 90 % the most: 291 x 6 x 1532 11.2 us, now 5.9; 2 x 4 x 1991 11.6, now 6.3.  Launches take 0.4 us more or
-// less from one card to another; these are of the shorter kind, as the chain's costs below are.)
+// around its loads, those float by float were 7.8 and 9.5 % above, 90 % the most: 291 x 6 x 1532 11.2 us, now 5.9; 2 x 4 x 1991 11.6, now 6.3.  The two larger tiles' costs are fitted to
+// 2700 products of either float by float kind, half of them batches of up to 128: on 1000 others each 0.12 and 0.19 % above the best, batches 0.54 and 0.41 %, 31 % the most; fitted to
+// single products alone they had batches 1.3 % above, 2.1 times the most: 63 products of 693 x 163 x 19 47 us on tiles of 128, now 24 on 64.  Launches take 0.4 us more or less from one
+// card to another; these are of the shorter kind, as the chain's costs below are.)
 enum F32Tile { F32_CONV3X3_FEW = 3004, F32_CONV3X3_32 = 3032, F32_CONV3X3_64 = 3064, F32_CONV3X3_128 = 3128, F32_CONV3X3_SPLIT_128 = 4128, F32_CONV3X3_SPLIT_256 = 4256, F32_DIRECT = 16, F32_TILE_32 = 32, F32_TILE_64x32 = 62, F32_TILE_64 = 64, F32_TILE_128x32 = 126, F32_TILE_128 = 128 };
 // Pixels of a tile of the 3 x 3 convolution kernels; 0 for any other kernel.
 static int conv3x3_pixels(int tile)
@@ -310,8 +312,8 @@ static int pick_f32_tile(int M, int N, int K, int batch, F32Loads loads, double 
       Cost direct, tile32, tile64x32, tile64, tile128;
    };
    static constexpr Costs COSTS[] = { // by F32Loads
-      {{2.75, 0.23, 0.063, 0.40, 0.092}, {3.12, 0.15, 0.152, 0.52}, {3.44, 0.32, 0.325, 0.94}, {2.66, 0.57, 0.548, 1.88}, {8.85, 1.77, 2.14, 1.88}},
-      {{2.75, 0.26, 0.066, 0.41, 0.080}, {3.11, 0.14, 0.144, 0.55}, {3.36, 0.25, 0.313, 0.99}, {2.55, 0.21, 0.547, 1.79}, {8.52, 1.81, 2.12, 1.10}},
+      {{2.75, 0.23, 0.063, 0.40, 0.092}, {3.12, 0.15, 0.152, 0.52}, {3.44, 0.32, 0.325, 0.94}, {3.54, 0.59, 0.566, 1.44}, {5.13, 0.05, 2.48, 4.64}},
+      {{2.75, 0.26, 0.066, 0.41, 0.080}, {3.11, 0.14, 0.144, 0.55}, {3.36, 0.25, 0.313, 0.99}, {3.62, 0.195, 0.504, 1.37}, {5.88, 2.25, 2.12, 3.49}},
       {{3.09, 0.31, 0.068, 0.38, 0.038}, {3.06, 0.09, 0.134, 0.53}, {3.64, 0.14, 0.262, 0.78}, {3.14, 0.34, 0.504, 1.53}, {5.94, 0.03, 2.01, 3.56}},
       {{}, {2.78, 0.10, 0.125, 0.49}, {3.45, 0.18, 0.251, 0.66}, {2.68, 0.48, 0.478, 1.47}, {5.36, 0.03, 1.80, 3.55}}};
    auto tiles = [&](int bm, int bn) { return std::ceil((double)M / bm) * std::ceil((double)N / bn) * batch; };

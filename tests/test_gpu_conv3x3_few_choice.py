@@ -49,6 +49,7 @@ def test_the_faster_kernel_is_chosen(rt, opt, images, channels, H, W, out):
                 rt.call("sofie_hip_conv_f32", C.byref(d), util.ptr(dX), util.ptr(dW), None, R.ACT_NONE, C.c_float(0.0), util.ptr(dY), None, None)
             best = min(best, rt.timer_stop() * 1e3 / 20)
         return best
+    us(0)   # the card awake
     chosen, within, through = us(0), us(3004), us(3128)
     print(chosen, within, through, flush=True)
     assert chosen <= 1.2 * min(within, through)
