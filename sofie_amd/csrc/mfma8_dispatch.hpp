@@ -92,7 +92,7 @@ static int launch_mfma8_general(const LaunchCfg &lc, const ASRC &A, const BSRC &
    int tile = 0;
    mfma8_general_time(M, N, K, source, &tile);
    if (lc.tile)
-      tile = lc.tile == 64 ? 0 : lc.tile >= 128 && (lc.tile != 164 || PIXELS) ? 2 : lc.tile == 164 ? 1 : tile;
+      tile = lc.tile == 64 ? 0 : lc.tile == 164 ? PIXELS ? tile : 1 : lc.tile >= 128 ? 2 : tile;
    if (tile == 2)
       return launch_mfma8_staged<MMA, 128, 128, 128, 4, 2, 2, ASRC, BSRC, EPI>(lc, A, B, M, N, K, ep);
    auto smaller = [&](const auto &a, const auto &b) {
@@ -207,7 +207,8 @@ namespace sofie_hip {
 template <class EPI>
 static int launch_mfma8_conv(const LaunchCfg &lc, const ConvRows &a, int Cg, const int8_t *Wp, int M, int N, int K, const EPI &ep)
 {
-   const int force_tile = lc.tile;
+   // requests for kernels of other layers, or that have turned this one down: no request here
+   const int force_tile = lc.tile == 17 || lc.tile == 33 || lc.tile == 27 || lc.tile == 164 ? 0 : lc.tile;
    auto tiles = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
    const bool pairs = (Cg % 128 == 0);
    int tile = force_tile;
