@@ -61,3 +61,21 @@ def test_fp8(rt, opt, M, N, K, ba, bb, pa, pb, tile):
     rt.call("sofie_hip_gemm_fp8", C.byref(g))
     rt.sync()
     assert np.array_equal(util.to_host(dY), (a @ b.T + bias).astype(np.float32))
+
+
+@pytest.mark.parametrize("tile", [0, 16, 32, 64, 164])
+@pytest.mark.parametrize("M,N,K,ba,bb,pa,pb", CASES)
+def test_fp8_columns(rt, opt, M, N, K, ba, bb, pa, pb, tile):
+    """A B stored [K,N]: transposed on its way against rows read as words (as chosen, and by force in tiles of 128 x 64), or by a launch of its own (the other requests)."""
+    a, b, bias = whole(30 + tile, (M, K + pa), 8), whole(31 + tile, (K, N + pb), 8), whole(32 + tile, (N,), 100)
+    code = lambda v: torch.from_numpy(v.astype(np.float32)).to(torch.float8_e4m3fn).view(torch.uint8).numpy()
+    (dA, pA), (dB, pB) = placed(a, ba, code), placed(b, bb, code)
+    dC, dY, ws = util.to_dev(bias.astype(np.float32)), util.dev_empty((M, N), np.float32), util.dev_empty(((N * K + 255) // 256 * 256,), np.int8)
+    g = R.GemmFp8Desc()
+    g.M, g.N, g.K, g.transB, g.lda, g.ldb, g.scale, g.act, g.out = M, N, K, 0, K + pa, N + pb, 1.0, R.ACT_NONE, R.F8OUT_F32
+    g.A, g.B, g.bias, g.Y, g.workspace, g.workspace_bytes = pA, pB, util.ptr(dC), util.ptr(dY), util.ptr(ws), ws.numel()
+    torch.cuda.synchronize()
+    opt("f8_tile", tile)
+    rt.call("sofie_hip_gemm_fp8", C.byref(g))
+    rt.sync()
+    assert np.array_equal(util.to_host(dY), (a[:, :K] @ b[:, :N] + bias).astype(np.float32))

@@ -46,3 +46,23 @@ def test_fp8(rt, opt, M, N, K):
     rt.call("sofie_hip_gemm_fp8", C.byref(g))
     rt.sync()
     assert np.array_equal(util.to_host(dY), (a @ b.T + bias).astype(np.float32))
+
+
+@pytest.mark.parametrize("tile", [0, 164])
+@pytest.mark.parametrize("pad_a, pad_b", [(0, 0), (3, 0), (4, 5)])
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_fp8_columns(rt, opt, M, N, K, pad_a, pad_b, tile):
+    """A B stored [K,N], by force in tiles of 128 x 64 and as chosen."""
+    seed = 40 + tile + pad_a
+    a, b, bias = whole(seed, (M, K + pad_a), 8), whole(seed + 1, (K, N + pad_b), 8), whole(seed + 2, (N,), 100)
+    e4m3 = lambda v: util.to_dev(torch.from_numpy(v.astype(np.float32)).to(torch.float8_e4m3fn).view(torch.uint8).numpy())
+    dA, dB, dC, dY = e4m3(a), e4m3(b), util.to_dev(bias.astype(np.float32)), util.dev_empty((M, N), np.float32)
+    ws = util.dev_empty(((N * K + 255) // 256 * 256,), np.int8)
+    g = R.GemmFp8Desc()
+    g.M, g.N, g.K, g.transB, g.lda, g.ldb, g.scale, g.act, g.out = M, N, K, 0, K + pad_a, N + pad_b, 1.0, R.ACT_NONE, R.F8OUT_F32
+    g.A, g.B, g.bias, g.Y, g.workspace, g.workspace_bytes = util.ptr(dA), util.ptr(dB), util.ptr(dC), util.ptr(dY), util.ptr(ws), ws.numel()
+    torch.cuda.synchronize()
+    opt("f8_tile", tile)
+    rt.call("sofie_hip_gemm_fp8", C.byref(g))
+    rt.sync()
+    assert np.array_equal(util.to_host(dY), (a[:, :K] @ b[:, :N] + bias).astype(np.float32))
