@@ -29,7 +29,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // q = sat8(rne(x / scale)), fp32 division (ONNX QuantizeLinear, zero point 0)
 // A load per thread: the divisions of four values take a wave that is alone on its SIMD as long as the trip to memory, and sixteen of them, with four loads in flight,
-// three times as long.  us with sixteen -> four: 16 K values 2.35 -> 1.83, 1 M 2.65 -> 2.13, 3 M 3.76 -> 3.41.
+// three times as long.  us with sixteen -> four, launches of a captured loop: over data in the caches 16 K values 2.74 -> 2.27, 1 M 2.97 -> 2.58, 3 M 4.08 -> 3.77, 50 M 38.4 -> 35.9; over
+// data that is not (600 MB in turn) 2.37 -> 1.85, 3.66 -> 3.19, 5.56 -> 5.36, 47.3 -> 46.1 (past 8 M values a thread takes several, one after the other).  Behind the other kernels of a
+// network, traced: 16 K 2.7 -> 2.2, 1 M 4.1 .. 4.8 and 4.5 .. 4.8, 3 M 5.2 -> 5.1: what bounds the larger ones there is the trip.
 __global__ __launch_bounds__(256) void quantize_linear_kernel(int8_t *__restrict__ dst, const float *__restrict__ src,
                                                                size_t n, float scale, int vec)
 {

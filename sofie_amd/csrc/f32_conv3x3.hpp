@@ -5,7 +5,7 @@
 // (through rows and images) and BN output channels; what it reads of a channel is one run of rows, loaded once, and the nine kernel
 // positions read it from LDS at offsets that are known where the code is written.  64 images, us before -> after: 32 -> 64 channels at
 // 32 x 32 36.7 -> 26.8, 64 -> 64 57.2 -> 43.8 (110 TFLOP/s of the matrix cores' 157; on another card 44.7, with a residual 45.3), 3 -> 32 at
-// 64 x 64 24.2 -> 17.0 (14.9 with the stores below); one image, 48 -> 96 at 40 x 40 12.8 -> 8.4.  On 64 -> 64 the matrix cores work in 0.72 of the cycles and no bank conflicts are
+// 64 x 64 24.2 -> 17.0 (14.9 with the stores below); one image, 48 -> 96 at 40 x 40 12.8 -> 8.4.  (Up to four channels: a slab of four, or f32_conv3x3_few.hpp.)  On 64 -> 64 the matrix cores work in 0.72 of the cycles and no bank conflicts are
 // counted; what is left is a patch that is loaded once per 32 output channels and one MFMA per value read from LDS.
 //
 // The images are taken as one column of OH + 2 rows each, padding included (row r of image i is row i (OH + 2) + r), and OW + 2 columns:

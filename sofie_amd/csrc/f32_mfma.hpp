@@ -892,7 +892,7 @@ struct F32DirectStore {
 // W waves split the reduction of one (16 MB) x (16 NB) tile in steps of 16 k (v_mfma_f32_16x16x4_f32: lane (lk = lane / 16, c = lane
 // % 16) supplies k = 4 lk + j of row c to MFMA j); the partial tiles meet in LDS.  What such a product
 // costs is one trip to memory for its operands: every wave has UNROLL steps of loads in flight at once.  No step but the last looks at its k, and no branch stands
-// between loads: with one around each, a wave alone on its SIMD took as long for them as for the trip.  us, before -> after, with the bias asked for behind the first
+// between loads of single floats: with one around each, a wave alone on its SIMD took as long for them as for the trip.  us, before -> after, with the bias asked for behind the first
 // loads: 64 x 10 x 64 3.09 -> 2.57, 256 x 10 x 256 4.2 -> 3.05, 16 x 10 x 333 4.4 -> 2.95, 100 x 33 x 77 3.7 -> 2.95, 200 x 17 x 50 3.5 -> 2.75, 1 x 1000 x 2048 5.9 -> 5.6.
 template <class ASRC, class BSRC, class STORE, int MB, int NB, int W, int UNROLL>
 __global__ __launch_bounds__(W * 64) void f32_direct_kernel(ASRC A, BSRC B, STORE out, int M, int N, int K, TileOrder order, int first_tile, long long strideA,
