@@ -694,8 +694,9 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
       SOFIE_HIP_REQUIRE(layers[l].A == layers[l - 1].Y && layers[l].A != nullptr, "sofie_hip_gemm_chain_f32: layer %d does not read the output of layer %d", l, l - 1);
    // Which layers share a launch.  A launch of its own spreads a layer over the chip and costs 2.5 us or more; in the chain kernel a workgroup does its rows' share alone: a pass over
    // the outputs that its waves take at once (W stored [N][K]) or a walk along k (W stored [K][N]) at a time.  So large layers run one by one, and small ones behind them share a
-   // launch.  (Fitted to 3100 networks of two to four layers, 1 .. 256 rows, all layers together or each by itself: 0.65 % above the better of the two on average, 39 % the most; with the costs
-   // of the kernel before 1.2 and 58 %.)
+   // launch.  Costs by the rows of a workgroup, one, two or four (M <= 64, <= 128, <= 256).  Fitted to 4000 networks of two to four layers, all layers together or each by itself: 0.2 %
+   // above the better of the two on average where W is stored [N][K], 0.3 % where it is [K][N].  (With one factor of 1.27 and 1.7 for both, from 65 and 129 rows on, 0.7 - 1.8 % there, 36 % the
+   // most: 183 x 128-112-94-48-3, [N][K], 16.7 us together, 12.3 apart; 232 x 16-36-9-128-37, [K][N], 12.1 apart, 9.7 together.)
    const int M = layers[0].M;
    int first = count; // first layer of the shared launch
    if (ctx->opt.f32_chain == 1) {
@@ -706,6 +707,12 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
          return f32_loads((d.transA ? d.M : d.K) % 4 == 0 && (d.transB ? d.K : d.N) % 4 == 0, d.transB && !d.transA);
       };
       auto apart = [](double t) { return std::max(1.02 * t - 0.27, 2.5); }; // behind another layer
+      struct Costs {
+         double launch, layer, pass, k;                  // W stored [N][K]
+         double columns_launch, columns_pass, columns_k; // W stored [K][N]
+      };
+      static constexpr Costs COSTS[] = {{1.76, 0.44, 0.81, 0.0013, 2.13, 1.21, 0.030}, {1.56, 0.15, 1.76, 0.0014, 1.88, 1.57, 0.0393}, {2.30, 0.23, 2.80, 0.0020, 3.55, 1.28, 0.0664}};
+      const Costs &cost = COSTS[M <= 64 ? 0 : M <= 128 ? 1 : 2];
       double before = 0.0, least = 0.0;
       for (int l = 0; l < count; ++l) {
          double t = 0.0;
@@ -719,9 +726,10 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
             const bool wide = layers[l].K % 4 == 0 && layers[l].ldb % 4 == 0; // chain_rows
             const double outputs = !layers[l].transB ? 1024.0 : !wide || N <= 64 ? 64.0 : K <= 64 ? 256.0 : K <= 128 ? 128.0 : 64.0, passes = std::ceil(N / outputs);
             const double groups = N <= 64 ? 16.0 : N <= 128 ? 8.0 : N <= 256 ? 4.0 : N <= 512 ? 2.0 : 1.0; // that deal out k
-            together += layers[l].transB ? wide ? 0.44 + passes * (0.81 + 0.0013 * K) : 0.43 + passes * (0.78 + 0.0023 * K) : passes * (1.55 + 0.025 * K / groups);
+            // (rows of W that are no whole 16-byte pieces: a little less a pass, more for its k)
+            together += layers[l].transB ? cost.layer + passes * (wide ? cost.pass + cost.k * K : 0.96 * cost.pass + 1.8 * cost.k * K) : passes * (cost.columns_pass + cost.columns_k * K / groups);
          }
-         together = before + 1.76 + together * (M <= 64 ? 1.0 : M <= 128 ? 1.27 : 1.7);
+         together += before + (layers[count - 1].transB ? cost.launch : cost.columns_launch);
          if (together < least)
             least = together, first = s;
          pick_f32_tile(M, layers[s].N, layers[s].K, 1, loads(s), &t);
