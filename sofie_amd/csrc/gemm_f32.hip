@@ -694,9 +694,9 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
       SOFIE_HIP_REQUIRE(layers[l].A == layers[l - 1].Y && layers[l].A != nullptr, "sofie_hip_gemm_chain_f32: layer %d does not read the output of layer %d", l, l - 1);
    // Which layers share a launch.  A launch of its own spreads a layer over the chip and costs 2.5 us or more; in the chain kernel a workgroup does its rows' share alone: a pass over
    // the outputs that its waves take at once (W stored [N][K]) or a walk along k (W stored [K][N]) at a time.  So large layers run one by one, and small ones behind them share a
-   // launch.  Costs by the rows of a workgroup, one, two or four (M <= 64, <= 128, <= 256).  Fitted to 4000 networks of two to four layers, all layers together or each by itself: 0.2 %
-   // above the better of the two on average where W is stored [N][K], 0.3 % where it is [K][N].  (With one factor of 1.27 and 1.7 for both, from 65 and 129 rows on, 0.7 - 1.8 % there, 36 % the
-   // most: 183 x 128-112-94-48-3, [N][K], 16.7 us together, 12.3 apart; 232 x 16-36-9-128-37, [K][N], 12.1 apart, 9.7 together.)
+   // launch.  Costs by the rows of a workgroup, one, two or four (M <= 64, <= 128, <= 256).  Of 4000 networks of two to four layers, all layers together or each by itself, the choice is 0.1 %
+   // above the better of the two on average where W is stored [N][K] (0.2, 0.7 and 1.0 % with factors of 1, 1.27 and 1.7 for the rows, 36 % the most: 183 x 128-112-94-48-3 16.7 us together,
+   // 12.3 apart) and 0.5, 0.7 and 1.8 % where it is [K][N] (25 % the most: more than 128 rows are taken together too seldom).
    const int M = layers[0].M;
    int first = count; // first layer of the shared launch
    if (ctx->opt.f32_chain == 1) {
@@ -711,7 +711,7 @@ int sofie_hip_gemm_chain_f32(sofie_hip_ctx *ctx, const sofie_gemm_f32_desc *laye
          double launch, layer, pass, k;                  // W stored [N][K]
          double columns_launch, columns_pass, columns_k; // W stored [K][N]
       };
-      static constexpr Costs COSTS[] = {{1.76, 0.44, 0.81, 0.0013, 2.13, 1.21, 0.030}, {1.56, 0.15, 1.76, 0.0014, 1.88, 1.57, 0.0393}, {2.30, 0.23, 2.80, 0.0020, 3.55, 1.28, 0.0664}};
+      static constexpr Costs COSTS[] = {{1.76, 0.44, 0.81, 0.0013, 1.76, 1.55, 0.025}, {1.56, 0.15, 1.76, 0.0014, 1.76, 1.97, 0.0318}, {2.30, 0.23, 2.80, 0.0020, 1.76, 2.64, 0.0425}};
       const Costs &cost = COSTS[M <= 64 ? 0 : M <= 128 ? 1 : 2];
       double before = 0.0, least = 0.0;
       for (int l = 0; l < count; ++l) {

@@ -8,8 +8,8 @@ from tests import util
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M, transB, dims", [(183, 1, (128, 112, 94, 48, 3)), (202, 1, (160, 32, 104, 112, 1)), (130, 1, (128, 16, 21, 48, 107)), (232, 0, (16, 36, 9, 128, 37)),
-                                             (207, 0, (128, 16, 144, 17, 31)), (181, 0, (128, 33, 32, 128, 4)), (33, 0, (16, 24, 16, 5, 5)), (20, 1, (304, 16, 32, 193))])
+@pytest.mark.parametrize("M, transB, dims", [(183, 1, (128, 112, 94, 48, 3)), (202, 1, (160, 32, 104, 112, 1)), (175, 1, (6, 16, 80, 7)), (130, 1, (128, 16, 21, 48, 107)),
+                                             (146, 1, (64, 48, 40, 10)), (33, 0, (16, 24, 16, 5, 5)), (20, 1, (304, 16, 32, 193))])
 def test_a_fast_split_is_chosen(rt, opt, M, transB, dims):
     layers, keep, src = (R.GemmF32Desc * (len(dims) - 1))(), [], torch.randn(M * dims[0], device="cuda")
     for l, (k, n) in enumerate(zip(dims, dims[1:])):
