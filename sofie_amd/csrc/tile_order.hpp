@@ -35,9 +35,9 @@ struct Divisor31 {
 
 // Tiles in bands of `mode & 0xff` rows, column by column inside a band, and workgroups regrouped so that the eight XCDs, which take them in turn, each have a run of them (not
 // with `mode & 0x100`).  The tiles are known to the host, which works out the divisors: four divisions by run-time values are 400 cycles that a small product waits for before its
-// first load, and a single column of tiles (small fp32 products, most fp32 convolutions) needs none of them: 0.07 us of 2.5 where a few tiles are all there is.  The products
-// of a batch are laid side by side in the same list, so that those of one product meet in one XCD's L2: 96 products of 128 x 128 x 64 read 18 MB through eight L2s, whose
-// operands are 6.
+// first load.  What is left is the trip to the scalar cache for the fields, and a branch around some of them makes it two: 0.05 us of a small product's 2.5.  So no case has a way of its
+// own (one without divisions for a single column of tiles made products of several columns 1.2 % slower, and int8 and FP8 0.5 %).  The products of a batch are laid side by side in the same
+// list, so that those of one product meet in one XCD's L2: 96 products of 128 x 128 x 64 read 18 MB through eight L2s, whose operands are 6.
 struct TileOrder {
    int tiles_m, tiles_n, band, last; // last: rows of the last band
    int per, rem;                     // workgroups of an XCD, XCDs with one more; per < 0: no regrouping
@@ -56,8 +56,6 @@ struct TileOrder {
    }
    long long workgroups(int batch) const { return (long long)tiles_m * tiles_n * (tiles ? batch : 1); } // of the grid's x
    unsigned depth(int batch) const { return tiles ? 1u : (unsigned)batch; }                            // its z
-   // F32: with a branch around the divisions of a single column.  The int8 and FP8 kernels, whose columns are more, take 0.5 % longer with it.
-   template <bool F32>
    SOFIE_ORDER_FN void place_of(int bid, int z, int &tm, int &tn, int &product) const
    {
       int id = bid;
@@ -70,22 +68,17 @@ struct TileOrder {
          product = (int)by_tiles.over((unsigned)id);
          id -= product * tiles;
       }
-      if (F32 && tiles_n == 1) {
-         tm = id;
-         tn = 0;
-         return;
-      }
       const int group = (int)by_width.over((unsigned)id), first = group * band, in = id - group * band * tiles_n;
       const bool whole = first + band <= tiles_m;
       tn = whole ? (int)by_band.over((unsigned)in) : (int)by_last.over((unsigned)in);
       tm = first + in - tn * (whole ? band : last);
    }
 #if defined(__HIPCC__)
-   __device__ __forceinline__ void place(int bid, int &tm, int &tn, int &product) const { place_of<true>(bid, blockIdx.z, tm, tn, product); }
+   __device__ __forceinline__ void place(int bid, int &tm, int &tn, int &product) const { place_of(bid, blockIdx.z, tm, tn, product); }
    __device__ __forceinline__ void place(int bid, int &tm, int &tn) const
    {
       int product;
-      place_of<false>(bid, 0, tm, tn, product);
+      place_of(bid, 0, tm, tn, product);
    }
 #endif
 };

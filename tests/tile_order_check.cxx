@@ -26,15 +26,9 @@ int main()
    long long compared = 0, bad = 0;
    auto check = [&](const TileOrder &o, long long bid, int z, long long tiles_m, long long tiles_n, int mode, long long batch) {
       int tm = -1, tn = -1, product = -1;
-      o.place_of<true>((int)bid, z, tm, tn, product);
+      o.place_of((int)bid, z, tm, tn, product);
       const Place p = plain(bid, z, tiles_m, tiles_n, mode, o.tiles != 0, batch);
       ++compared;
-      if (batch == 1) { // the kernels without batches
-         int tm1 = -1, tn1 = -1, none = -1;
-         o.place_of<false>((int)bid, z, tm1, tn1, none);
-         if (tm1 != p.tm || tn1 != p.tn)
-            ++bad;
-      }
       if (tm != p.tm || tn != p.tn || product != p.product)
          ++bad;
       return Place{tm, tn, product};
