@@ -35,8 +35,8 @@ struct Divisor31 {
 
 // Tiles in bands of `mode & 0xff` rows, column by column inside a band, and workgroups regrouped so that the eight XCDs, which take them in turn, each have a run of them (not
 // with `mode & 0x100`).  The tiles are known to the host, which works out the divisors: four divisions by run-time values are 400 cycles that a small product waits for before its
-// first load.  What is left is the trip to the scalar cache for the fields, and a branch around some of them makes it two: 0.05 us of a small product's 2.5.  So no case has a way of its
-// own (one without divisions for a single column of tiles made products of several columns 1.2 % slower, and int8 and FP8 0.5 %).  The products of a batch are laid side by side in the same
+// first load.  What is left is the trip to the scalar cache for the fields, and a branch around some of them makes it two: 0.05 us of a small product's 2.5.  So a single column of tiles has no way of
+// its own (one without the divisions made products of several columns 1.2 % slower, int8 and FP8 0.5 %).  The products of a batch are laid side by side in the same
 // list, so that those of one product meet in one XCD's L2: 96 products of 128 x 128 x 64 read 18 MB through eight L2s, whose operands are 6.
 struct TileOrder {
    int tiles_m, tiles_n, band, last; // last: rows of the last band
@@ -56,6 +56,8 @@ struct TileOrder {
    }
    long long workgroups(int batch) const { return (long long)tiles_m * tiles_n * (tiles ? batch : 1); } // of the grid's x
    unsigned depth(int batch) const { return tiles ? 1u : (unsigned)batch; }                            // its z
+   // BATCHES: for the fp32 kernels, without a branch (above): 3 % of a small product of a batch.  The int8 and FP8 kernels, which have no batches, take 1 % longer without it.
+   template <bool BATCHES>
    SOFIE_ORDER_FN void place_of(int bid, int z, int &tm, int &tn, int &product) const
    {
       int id = bid;
@@ -64,7 +66,11 @@ struct TileOrder {
          id = xcd * per + (xcd < rem ? xcd : rem) + (bid >> 3);
       }
       product = z;
-      if (tiles) {
+      if (BATCHES) {
+         const int listed = (int)by_tiles.over((unsigned)id);
+         product = tiles ? listed : z;
+         id -= listed * tiles;
+      } else if (tiles) {
          product = (int)by_tiles.over((unsigned)id);
          id -= product * tiles;
       }
@@ -74,11 +80,11 @@ struct TileOrder {
       tm = first + in - tn * (whole ? band : last);
    }
 #if defined(__HIPCC__)
-   __device__ __forceinline__ void place(int bid, int &tm, int &tn, int &product) const { place_of(bid, blockIdx.z, tm, tn, product); }
+   __device__ __forceinline__ void place(int bid, int &tm, int &tn, int &product) const { place_of<true>(bid, blockIdx.z, tm, tn, product); }
    __device__ __forceinline__ void place(int bid, int &tm, int &tn) const
    {
       int product;
-      place_of(bid, 0, tm, tn, product);
+      place_of<false>(bid, 0, tm, tn, product);
    }
 #endif
 };

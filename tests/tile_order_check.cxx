@@ -26,9 +26,13 @@ int main()
    long long compared = 0, bad = 0;
    auto check = [&](const TileOrder &o, long long bid, int z, long long tiles_m, long long tiles_n, int mode, long long batch) {
       int tm = -1, tn = -1, product = -1;
-      o.place_of((int)bid, z, tm, tn, product);
+      o.place_of<true>((int)bid, z, tm, tn, product);
       const Place p = plain(bid, z, tiles_m, tiles_n, mode, o.tiles != 0, batch);
       ++compared;
+      int tm2 = -1, tn2 = -1, product2 = -1;
+      o.place_of<false>((int)bid, z, tm2, tn2, product2);
+      if (tm2 != tm || tn2 != tn || product2 != product)
+         ++bad;
       if (tm != p.tm || tn != p.tn || product != p.product)
          ++bad;
       return Place{tm, tn, product};
